@@ -142,8 +142,8 @@ __device__ __forceinline__ double shap_from_fixed(unsigned long long v, double s
     return static_cast<double>(static_cast<long long>(v)) / scale * static_cast<double>(lr);
 }
 
-// KM: compile-time bound on the path length (8 covers depth-8 trees), so every per-path
-// array lives in registers.
+// Serves the ensembles the tree form (below) does not take.  KM: compile-time bound on the
+// path length, so every per-path array lives in registers.
 template <int KM>
 __global__ __launch_bounds__(256) void k_shap(u8 const *__restrict__ bins, u64 n, u64 stride, u32 F,
                                               SElem const *__restrict__ elems, SHead const *__restrict__ heads,
@@ -169,8 +169,7 @@ __global__ __launch_bounds__(256) void k_shap(u8 const *__restrict__ bins, u64 n
     for (u32 g = blockIdx.y * NW + wave; g < n_groups; g += NW * gridDim.y) {
         SHead const hd = heads[static_cast<size_t>(g) * 64u + lane];
         u32 const nel = hd.n;
-        // The group's longest path (wave-uniform): the KM = 16 body skips element slots
-        // past it; the KM = 8 body runs all eight.
+        // The group's longest path (wave-uniform): element slots past it are skipped.
         u32 nmax = nel;
         for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, static_cast<u32>(__shfl_xor(static_cast<int>(nmax), o)));
         nmax = __builtin_amdgcn_readfirstlane(nmax);
@@ -222,7 +221,7 @@ __global__ __launch_bounds__(256) void k_shap(u8 const *__restrict__ bins, u64 n
 #pragma unroll
             for (int j = 0; j < KM; ++j) {
                 sat[j] = false;
-                if (KM <= 8 || static_cast<u32>(j) < nmax) {
+                if (static_cast<u32>(j) < nmax) {
                     u32 const b = row[feat[j]];
                     bool const one = b == lst[j] ? miss[j] : (b >= lo[j] && b <= hi[j]);
                     sat[j] = one;
@@ -240,7 +239,7 @@ __global__ __launch_bounds__(256) void k_shap(u8 const *__restrict__ bins, u64 n
             float const nu = -vs * unsat;
 #pragma unroll
             for (int k = 0; k < KM; ++k) {
-                if (KM <= 8 || static_cast<u32>(k) < nmax) {
+                if (static_cast<u32>(k) < nmax) {
                     // synthetic division by (t + z_k), from the top: deflated[i] =
                     // P[i+1] - z_k deflated[i+1], zero above the path's degree; used only
                     // where element k is satisfied (P then holds the factor t + z_k)
@@ -248,7 +247,7 @@ __global__ __launch_bounds__(256) void k_shap(u8 const *__restrict__ bins, u64 n
                     float sdef = 0.0F, prev = 0.0F;
 #pragma unroll
                     for (int i = KM - 1; i >= 0; --i) {
-                        if (KM <= 8 || static_cast<u32>(i) < nmax) {
+                        if (static_cast<u32>(i) < nmax) {
                             prev = __builtin_fmaf(nzk, prev, poly[i + 1]);
                             sdef = __builtin_fmaf(wl[i], prev, sdef);
                         }
@@ -277,6 +276,417 @@ __global__ __launch_bounds__(256) void k_shap(u8 const *__restrict__ bins, u64 n
         out[(r0 + rr) * (F + 1) + f] = shap_from_fixed(s_phi[k], scale, lr);
     }
     for (u32 rr = threadIdx.x; rr < nr; rr += blockDim.x) out[(r0 + rr) * (F + 1) + F] = bias;
+}
+
+// ---------------------------------------------------------------------------------
+// TreeSHAP, tree form: one row per lane, a wave walks whole trees.
+//
+// The closed form's sum over coefficients is an integral: w_i = 1 / (n C(n-1, i)) is
+// the Beta integral of x^i (1-x)^(n-1-i) over [0, 1], so element k's term is
+//   value (o_k - z_k) * integral of prod_{j != k} (z_j (1-x) + o_j x) dx,
+// a polynomial of degree n - 1 that M >= n/2 Gauss-Legendre nodes x_q integrate exactly.
+// At a fixed x_q the paths' products factor over the tree's edges, so they are formed
+// once per edge and shared by every path through it (the edge-sharing of Linear
+// TreeSHAP, Yu et al. 2022, at quadrature points instead of in coefficient form).  For
+// an internal node whose child c holds the cover fraction z_c and s_c = 1 on the row's
+// side, with T_q the product above the node and H_q(c) the values below c:
+//   M = sum_c z_c H(c), S = sum_c s_c H(c), d = S - M,
+//   H(node) = M + k_q d,  T(c) = T(node) (z_c + k_q (s_c - z_c)),
+//   phi[feature] += sum_q T_q(node) l_q d_q,
+// k_q = x_q and l_q = 1 when no edge above splits on the node's feature.  When one does,
+// its edge carries the merged fraction z' and satisfaction o' of that feature: o' = 0
+// turns k and l into 0, o' = 1 gives k_q = x_q / a, l_q = z' / a^2, a = z' + x_q (1 - z').
+// Nodes past 1/2 use 1 - k_q, which floats hold more exactly: H = S - (1 - k) d,
+// T(c) = T(node) (s_c - (1 - k) (s_c - z_c)); the weights carry a common factor that
+// makes them nearly exact in float (tree_quad), so neither adds a systematic error.
+//
+// Lanes are rows and a wave's control flow and node records are uniform.  Bound by vector
+// issue: 14,900 wave instructions per 255-node tree and 64 rows (about 58 a node, against
+// some 265 a path of the packed form) at 4 clocks each are 6.2 of the 7.6 ms that 16,384
+// rows of 1,000 such trees take (packed form 28.4 ms).  Contributions go through float to
+// 64-bit fixed point (one FP64 add against 1.5 * 2^52)
+// and into LDS with conflict-free integer atomics: exact in any order, so a row's result
+// depends neither on the batch nor on how trees are dealt to waves and workgroups.
+// ---------------------------------------------------------------------------------
+// A tree is stored as the steps of its depth-first walk, read as one sequential stream:
+//   block    a subtree of at most three levels, as seven nodes in one straight run of
+//            instructions (a shallower leaf becomes nodes that split it into itself)
+//   enter    a node above the blocks: its decision, T of the child walked first
+//   turn     its left child is done: keep its value, T of the right child
+//   combine  its right child is done (or is a leaf): the node's value and contribution
+// so one product T and one left value per level above the blocks stay in registers.  A wave holds 64 consecutive
+// 32-byte slots of the stream in registers, one per lane (the next 64 in flight), and
+// broadcasts the words a step needs with v_readlane.  A node with a same-feature edge
+// above has its k and l in slots after the step's own; a step never crosses a group of
+// 64 slots (kTSkip pads).
+// ---------------------------------------------------------------------------------
+struct TSlot {
+    u32 w[8];
+};
+// Words of a step.  op: kind | level << 2 | dup bit of node i << (8 + i).
+// lv: level of the same-feature edge above node i << 4 i.  Splits: byte offset of the
+// bin column (shifted plane where the missing bin goes left) | first bin going right << 16.
+enum : u32 {
+    kTEnter = 0, kTTurn = 1, kTCombine = 2, kTBlock = 3, kTSkip = 15,
+    kTLeafL = 0x10000u, kTLeafR = 0x20000u, // enter / combine: that child is a leaf
+    kTwOp = 0, kTwLv = 1, kTwSplit = 2,
+    kTwZl = 3, kTwZr = 4, kTwVl = 5, kTwVr = 6,          // enter, turn, combine
+    kTwZ = 9, kTwMean = 15, kTwLeaf = 19, kTwBlock = 27, // block: z of 3 nodes, means of 4, 8 leaves
+};
+constexpr u32 kTBlockLevels = 3;
+constexpr u32 tree_dup_slots(u32 m) { return (2u * m + 7u) / 8u; }
+constexpr u32 tree_step_slots(u32 kind) { return kind == kTBlock ? (kTwBlock + 7u) / 8u : 1u; }
+constexpr u32 kTreeShapRows = 64; // rows of a workgroup, one per lane
+// Four waves a workgroup, three workgroups a CU (168 registers a lane; with 512-thread
+// workgroups and two waves per SIMD the batch above takes 9.0 ms); deep trees keep more
+// levels in registers and run one.
+constexpr u32 kTreeShapThreads = 256;
+constexpr u32 tree_shap_waves(u32 upper) { return upper <= 5u ? 3u : 1u; }
+constexpr u32 kTreeShapMaxM = 6;      // quadrature nodes: paths of up to 12 features
+constexpr u32 kTreeShapMaxDepth = 12;
+// LDS of a workgroup: 64-bit sums, bins, and bins with the missing bin moved to 0.
+constexpr size_t tree_shap_lds(u32 F) { return static_cast<size_t>(kTreeShapRows) * F * 10u; }
+
+// Quadrature of M nodes, ascending: y = x for the first half, 1 - x past 1/2; weights
+// times a common factor.
+struct TQuad {
+    float y[kTreeShapMaxM], w[kTreeShapMaxM];
+};
+
+// U: levels above the blocks.
+template <int M, int U> struct TreeShap {
+    typedef float V[M];
+    u8 const *bins;      // LDS: this lane's column of the bins
+    unsigned char *phi;  // LDS: this lane's column of the sums
+    u32 plane;           // bytes of one plane of bins
+    TSlot const *ahead;  // this lane's slot of the group after the next
+    uint4 nx0, nx1;      // its slot of the next group, in flight
+    u32 cur[8];          // its slot of the current group
+    u32 at, op;          // the running step's slot in it and its first word (uniform)
+    V y;                 // quadrature nodes (TQuad)
+    u32 sat;             // bit l: the row satisfies the merged feature of the edge below level l
+
+    __device__ __forceinline__ void load()
+    {
+        uint4 const *p = reinterpret_cast<uint4 const *>(ahead);
+        nx0 = p[0];
+        nx1 = p[1];
+        ahead += 64;
+    }
+    __device__ __forceinline__ void shift()
+    {
+        cur[0] = nx0.x;
+        cur[1] = nx0.y;
+        cur[2] = nx0.z;
+        cur[3] = nx0.w;
+        cur[4] = nx1.x;
+        cur[5] = nx1.y;
+        cur[6] = nx1.z;
+        cur[7] = nx1.w;
+        load(); // whole groups of 64 slots are allocated, and two past the last
+    }
+    // The step at `at`: a skip or the group's end moves on to the next group.
+    __device__ __forceinline__ void fetch()
+    {
+        op = at < 64u ? __builtin_amdgcn_readlane(cur[kTwOp], at & 63u) : kTSkip << 2;
+        if ((op >> 2 & 15u) == kTSkip) {
+            shift();
+            at = 0;
+            op = __builtin_amdgcn_readlane(cur[kTwOp], 0);
+        }
+    }
+    __device__ __forceinline__ void advance(u32 slots)
+    {
+        at += slots + __popc(op >> 8 & 0x7Fu) * tree_dup_slots(M);
+    }
+
+    // word j (a constant) of the slots from `slot` after the step's first
+    __device__ __forceinline__ u32 word(u32 j, u32 slot = 0) const
+    {
+        return __builtin_amdgcn_readlane(cur[j & 7u], at + slot + (j >> 3));
+    }
+    __device__ __forceinline__ float fword(u32 j, u32 slot = 0) const { return __uint_as_float(word(j, slot)); }
+    static __device__ __forceinline__ float keep(float v, u32 m) { return __uint_as_float(__float_as_uint(v) & m); }
+    static __device__ __forceinline__ float pick(u32 m, float a, float b)
+    {
+        return __uint_as_float((__float_as_uint(a) & m) | (__float_as_uint(b) & ~m));
+    }
+
+    __device__ __forceinline__ u32 goes_left(u32 split) const { return bins[split & 0xFFFFu] < split >> 16 ? ~0u : 0u; }
+
+    __device__ __forceinline__ void add(u32 split, float c)
+    {
+        u32 const col = split & 0xFFFFu;
+        // |c| < 2^51: the sum's low 52 bits hold round(c) beside 1.5 * 2^52's own
+        double const v = static_cast<double>(c) + 6755399441055744.0;
+        atomicAdd(reinterpret_cast<unsigned long long *>(phi + min(col, col - plane) * 8u),
+                  static_cast<unsigned long long>(__double_as_longlong(v)) - 0x4338000000000000ull);
+    }
+
+    static constexpr bool past_half(int q) { return 2 * q >= M + (M & 1); }
+    // value at k_q between a (k = 0) and b (k = 1), slope = b - a
+    static __device__ __forceinline__ float mix(int q, float k, float slope, float a, float b)
+    {
+        return past_half(q) ? __builtin_fmaf(-k, slope, b) : __builtin_fmaf(k, slope, a);
+    }
+
+    // A node's same-feature edge above: none, or where its constants are.  Lane masks are
+    // words and constants are read before use: selects of bools would become branches.
+    struct Dup {
+        bool is;
+        u32 slot, level;
+    };
+    // all ones where the row satisfies the merged feature of that edge
+    __device__ __forceinline__ u32 dup_sat(Dup const &u) const
+    {
+        return static_cast<u32>(__builtin_amdgcn_sbfe(static_cast<int>(sat), u.level, 1u));
+    }
+    // its k_q (or 1 - k_q) there, else k_q = 0
+    __device__ __forceinline__ float dup_k(Dup const &u, int q, u32 o) const
+    {
+        u32 const k = word(q, u.slot);
+        return __uint_as_float(past_half(q) ? (k & o) | (0x3F800000u & ~o) : k & o);
+    }
+    __device__ __forceinline__ float dup_l(Dup const &u, int q) const { return fword(M + q, u.slot); }
+
+    // A node's k_q (1 - k_q past the half) for every row.
+    __device__ __forceinline__ void consts(V &k, Dup const &u) const
+    {
+        if (u.is) {
+            u32 const o = dup_sat(u);
+#pragma unroll
+            for (int q = 0; q < M; ++q) k[q] = dup_k(u, q, o);
+        } else {
+#pragma unroll
+            for (int q = 0; q < M; ++q) k[q] = y[q];
+        }
+    }
+
+    // T of the child taken by the rows of m, with cover fraction zc
+    static __device__ __forceinline__ void descend(V const &Tn, V &Tc, V const &k, u32 m, float zc)
+    {
+        float const sc = keep(1.0F, m);
+        float const e = sc - zc;
+#pragma unroll
+        for (int q = 0; q < M; ++q) Tc[q] = Tn[q] * mix(q, k[q], e, zc, sc);
+    }
+    // the edge to that child at `level`: what same-feature nodes below it test
+    __device__ __forceinline__ void mark(u32 m, u32 level, Dup const &u)
+    {
+        if (u.is) m &= dup_sat(u);
+        u32 const bit = 1u << level;
+        sat = (m & bit) | (sat & ~bit);
+    }
+
+    // Value and contribution of a node from its children's values.
+    __device__ __forceinline__ void join(V const &Tn, V const &k, V const &L, V const &R, V &out, u32 m, float zl,
+                                         float zr, u32 split, Dup const &u)
+    {
+        V d;
+#pragma unroll
+        for (int q = 0; q < M; ++q) {
+            float const mean = __builtin_fmaf(zr, R[q], zl * L[q]);
+            float const S = pick(m, L[q], R[q]);
+            d[q] = S - mean;
+            out[q] = mix(q, k[q], d[q], mean, S);
+        }
+        float c = 0.0F;
+        if (u.is) {
+#pragma unroll
+            for (int q = 0; q < M; ++q) c = __builtin_fmaf(Tn[q] * dup_l(u, q), d[q], c);
+            c = keep(c, dup_sat(u));
+        } else {
+#pragma unroll
+            for (int q = 0; q < M; ++q) c = __builtin_fmaf(Tn[q], d[q], c);
+        }
+        add(split, c);
+    }
+
+    // Value and contribution of a node whose children are leaves, below the edge of the
+    // rows of em (fraction ze) of a node with product Tn and constants k: without a
+    // same-feature edge above, its product is only needed summed over q, which is
+    // ze a0 + e a1 with a0 = sum Tn_q, a1 = sum Tn_q k_q.
+    __device__ __forceinline__ void leaves(V const &Tn, V const &k, float a0, float a1, u32 em, float ze, V &out,
+                                           u32 m, float vl, float vr, float mean, u32 split, Dup const &u)
+    {
+        float const S = pick(m, vl, vr);
+        float const d = S - mean;
+        float t;
+        if (u.is) {
+            V Tc;
+            descend(Tn, Tc, k, em, ze);
+            u32 const o = dup_sat(u);
+            t = 0.0F;
+#pragma unroll
+            for (int q = 0; q < M; ++q) {
+                t = __builtin_fmaf(Tc[q], dup_l(u, q), t);
+                out[q] = mix(q, dup_k(u, q, o), d, mean, S);
+            }
+            t = keep(t, o);
+        } else {
+            t = __builtin_fmaf(ze, a0 - a1, keep(a1, em));
+#pragma unroll
+            for (int q = 0; q < M; ++q) out[q] = mix(q, y[q], d, mean, S);
+        }
+        add(split, t * d);
+    }
+
+    // Seven nodes in preorder (r; a, a0, a1; b, b0, b1) below the product Tr.
+    __device__ __forceinline__ void block(V const &Tr, V &H, u32 level)
+    {
+        u32 const lv = word(kTwLv);
+        u32 split[7], m[7];
+        Dup u[7];
+        u32 slot = tree_step_slots(kTBlock);
+#pragma unroll
+        for (int i = 0; i < 7; ++i) {
+            split[i] = word(kTwSplit + i);
+            m[i] = goes_left(split[i]);
+            u[i] = Dup{(op >> (8 + i) & 1u) != 0, slot, lv >> (4 * i) & 15u};
+            slot += u[i].is ? tree_dup_slots(M) : 0u;
+        }
+        float z[6];
+#pragma unroll
+        for (int i = 0; i < 6; ++i) z[i] = fword(kTwZ + i);
+        V kr, ka, Ta, H0, H1, Ha;
+        consts(kr, u[0]);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            int const n = 1 + 3 * s; // a, then b
+            u32 const me = s ? ~m[0] : m[0];
+            descend(Tr, Ta, kr, me, z[s]);
+            mark(me, level, u[0]);
+            consts(ka, u[n]);
+            float a0 = 0.0F, a1 = 0.0F;
+#pragma unroll
+            for (int q = 0; q < M; ++q) {
+                a0 += Ta[q];
+                a1 = past_half(q) ? a1 + __builtin_fmaf(-ka[q], Ta[q], Ta[q]) : __builtin_fmaf(ka[q], Ta[q], a1);
+            }
+            mark(m[n], level + 1u, u[n]);
+            leaves(Ta, ka, a0, a1, m[n], z[2 + 2 * s], H0, m[n + 1], fword(kTwLeaf + 4 * s), fword(kTwLeaf + 4 * s + 1),
+                   fword(kTwMean + 2 * s), split[n + 1], u[n + 1]);
+            mark(~m[n], level + 1u, u[n]);
+            leaves(Ta, ka, a0, a1, ~m[n], z[3 + 2 * s], H1, m[n + 2], fword(kTwLeaf + 4 * s + 2),
+                   fword(kTwLeaf + 4 * s + 3), fword(kTwMean + 2 * s + 1), split[n + 2], u[n + 2]);
+            join(Ta, ka, H0, H1, s ? H : Ha, m[n], z[2 + 2 * s], z[3 + 2 * s], split[n], u[n]);
+        }
+        join(Tr, kr, Ha, H, H, m[0], z[0], z[1], split[0], u[0]);
+    }
+
+    // The subtree whose first step is fetched, at level L below the product Tn.  Each
+    // level is one copy of this code: its two children are two trips of a loop.
+    template <int L> __device__ __forceinline__ void walk(V const &Tn, V &H)
+    {
+        if (L == U || (op & 3u) == kTBlock) {
+            block(Tn, H, L);
+            advance(tree_step_slots(kTBlock));
+            return;
+        }
+        if constexpr (L < U) {
+            u32 const m = goes_left(word(kTwSplit));
+            V HL;
+#pragma clang loop unroll(disable)
+            for (u32 side = 0; side < 2u; ++side) {
+                if (op & (kTLeafL << side)) {
+                    float const v = side ? fword(kTwVr) : fword(kTwVl);
+#pragma unroll
+                    for (int q = 0; q < M; ++q) H[q] = v;
+                } else {
+                    V Tc;
+                    V k;
+                    u32 const me = side ? ~m : m;
+                    consts(k, dup_of<L>());
+                    descend(Tn, Tc, k, me, side ? fword(kTwZr) : fword(kTwZl));
+                    mark(me, L, dup_of<L>());
+                    advance(1);
+                    fetch();
+                    walk<L + 1>(Tc, H);
+                    fetch();
+                }
+                if (side == 0) {
+#pragma unroll
+                    for (int q = 0; q < M; ++q) HL[q] = H[q];
+                }
+            }
+            V k;
+            consts(k, dup_of<L>());
+            join(Tn, k, HL, H, H, m, fword(kTwZl), fword(kTwZr), word(kTwSplit), dup_of<L>());
+            advance(1);
+        }
+    }
+    template <int L> __device__ __forceinline__ Dup dup_of() const
+    {
+        return Dup{L > 0 && (op & 0x100u) != 0, 1u, word(kTwLv)};
+    }
+};
+
+// gridDim.y workgroups share a row block; each of their waves walks a run of trees.
+template <int M, int U>
+__global__ __launch_bounds__(kTreeShapThreads, tree_shap_waves(U)) void k_shap_tree(
+    u8 const *__restrict__ bins, u64 n, u64 stride, u32 F, u16 const *__restrict__ last,
+    TSlot const *__restrict__ slots, u32 const *__restrict__ first, u32 n_trees, TQuad quad, float lr, double bias,
+    double scale, double *__restrict__ out)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned long long *s_phi = reinterpret_cast<unsigned long long *>(smem); // [F][64] fixed point
+    u8 *s_bins = reinterpret_cast<u8 *>(s_phi + kTreeShapRows * F);            // [2][F][64]
+    constexpr u32 threads = kTreeShapThreads, nw = threads / 64u;
+    u64 const r0 = static_cast<u64>(blockIdx.x) * kTreeShapRows;
+    u32 const nr = static_cast<u32>(min<u64>(kTreeShapRows, n - r0));
+    u32 const plane = kTreeShapRows * F;
+    for (u32 k = threadIdx.x; k < plane; k += threads) {
+        u32 const rr = k / F, f = k - rr * F;
+        u32 const b = rr < nr ? bins[(r0 + rr) * stride + f] : 0u;
+        s_phi[k] = 0ull;
+        s_bins[f * kTreeShapRows + rr] = static_cast<u8>(b);
+        s_bins[plane + f * kTreeShapRows + rr] = static_cast<u8>(b == last[f] ? 0u : min(b + 1u, 255u));
+    }
+    __syncthreads();
+    u32 const lane = threadIdx.x & 63u;
+    u32 const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    TreeShap<M, U> w;
+    w.bins = s_bins + lane;
+    w.phi = reinterpret_cast<unsigned char *>(s_phi + lane);
+    w.plane = plane;
+    w.sat = 0;
+    float T[M];
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        w.y[q] = quad.y[q];
+        T[q] = quad.w[q];
+    }
+    u32 const wi = blockIdx.y * nw + wave, waves = gridDim.y * nw;
+    u32 const per = n_trees / waves, more = n_trees - per * waves;
+    u32 const t0 = wi * per + min(wi, more), t1 = t0 + per + (wi < more ? 1u : 0u);
+    if (t0 < t1) {
+        u32 const pc = __builtin_amdgcn_readfirstlane(first[t0]);
+        w.ahead = slots + (pc & ~63u) + lane;
+        w.load();
+        w.shift();
+        w.at = pc & 63u;
+        for (u32 t = t0; t < t1; ++t) {
+            float H[M];
+            w.fetch();
+            w.template walk<0>(T, H);
+        }
+    }
+    __syncthreads();
+    if (gridDim.y > 1) {
+        // Shares of one row block meet in the zeroed output cells (exact in any order);
+        // k_shap_to_double converts them once every workgroup has added its own.
+        unsigned long long *acc = reinterpret_cast<unsigned long long *>(out);
+        for (u32 k = threadIdx.x; k < nr * F; k += threads) {
+            u32 const rr = k / F, f = k - rr * F;
+            unsigned long long const v = s_phi[f * kTreeShapRows + rr];
+            if (v != 0ull) atomicAdd(acc + (r0 + rr) * (F + 1) + f, v);
+        }
+        return;
+    }
+    for (u32 k = threadIdx.x; k < nr * (F + 1); k += threads) {
+        u32 const rr = k / (F + 1), f = k - rr * (F + 1);
+        out[(r0 + rr) * (F + 1) + f] = f == F ? bias : shap_from_fixed(s_phi[f * kTreeShapRows + rr], scale, lr);
+    }
 }
 
 // Split launches: the output cells start at zero (a fill kernel, so the sequence stays
@@ -363,6 +773,238 @@ void pack_paths(bh_node const *t, u16 const *last, u32 id, std::vector<ActiveEle
     else act[idx] = saved;
 }
 
+// Levels of splits below every node of a tree, and the most distinct features on a path.
+u32 tree_levels(bh_node const *t, u32 id, std::vector<u32> &levels, std::vector<u32> &feats, size_t &max_len)
+{
+    if (levels.size() <= id) levels.resize(id + 1, 0u);
+    bh_node const &nd = t[id];
+    if (nd.feature < 0) {
+        max_len = std::max(max_len, feats.size());
+        return 0;
+    }
+    u32 const f = static_cast<u32>(nd.feature);
+    bool const fresh = std::find(feats.begin(), feats.end(), f) == feats.end();
+    if (fresh) feats.push_back(f);
+    u32 const l = tree_levels(t, nd.left, levels, feats, max_len);
+    u32 const r = tree_levels(t, nd.right, levels, feats, max_len);
+    if (fresh) feats.pop_back();
+    return levels[id] = 1u + std::max(l, r);
+}
+
+struct GaussRule { // m nodes on [0, 1], ascending
+    u32 m;
+    double x[kTreeShapMaxM], w[kTreeShapMaxM];
+};
+bool past_half(u32 i, u32 m) { return 2u * i >= m + (m & 1u); }
+
+// Tree-form steps of an ensemble (TSlot stream).
+struct TreePacker {
+    bh_node const *t = nullptr;   // current tree
+    u32 const *levels = nullptr;  // and its nodes' levels of splits below
+    u16 const *last;
+    u32 F;
+    double scale;
+    GaussRule rule;
+    std::vector<TSlot> out;
+    struct Edge { // on the way down: feature, level and merged cover fraction of its latest edge
+        u32 feature, level;
+        double z;
+    };
+    std::vector<Edge> above;
+
+    // What the kernel reads of one node; a leaf taken as a node splits into itself.
+    struct Node {
+        u32 split = 0, level = 0; // level: of the same-feature edge above
+        bool dup = false, leaf = false;
+        double z = 1.0;           // and its merged fraction
+        double zl = 0.5, zr = 0.5, value = 0.0;
+    };
+    Node node(u32 id) const
+    {
+        bh_node const &nd = t[id];
+        Node r;
+        if (nd.feature < 0) {
+            r.leaf = true;
+            r.value = static_cast<double>(nd.value) * scale;
+            return r;
+        }
+        u32 const f = static_cast<u32>(nd.feature), lb = last[f];
+        // rows go left below the bound on the plane where the missing bin sorts last
+        // (bound bin + 1) or first (bin + 2); a split past the missing bin takes every
+        // other row left
+        u32 const bin = std::min<u32>(nd.bin + 1u, lb);
+        r.split = nd.default_left ? (F + f) * kTreeShapRows | (bin + 1u) << 16 : f * kTreeShapRows | bin << 16;
+        double const cover = nd.cover;
+        r.zl = cover > 0.0 ? static_cast<double>(t[nd.left].cover) / cover : 0.0;
+        r.zr = cover > 0.0 ? static_cast<double>(t[nd.right].cover) / cover : 0.0;
+        for (size_t k = above.size(); k-- > 0;)
+            if (above[k].feature == f) {
+                r.dup = true;
+                r.level = above[k].level;
+                r.z = above[k].z;
+                break;
+            }
+        return r;
+    }
+    static void put(TSlot *s, u32 word, float v) { std::memcpy(&s[word / 8u].w[word % 8u], &v, sizeof(v)); }
+    static void put(TSlot *s, u32 word, double v) { put(s, word, static_cast<float>(v)); }
+
+    // Room for a step and the constants of its n nodes; returns its first slot.
+    size_t open(u32 kind, Node const *nodes, u32 n)
+    {
+        u32 const ds = tree_dup_slots(rule.m);
+        u32 need = tree_step_slots(kind);
+        for (u32 i = 0; i < n; ++i) need += nodes[i].dup ? ds : 0u;
+        while ((out.size() & 63u) + need > 64u) {
+            TSlot skip{};
+            skip.w[kTwOp] = kTSkip << 2;
+            out.push_back(skip);
+        }
+        size_t const at = out.size();
+        out.resize(at + need);
+        size_t o = at + tree_step_slots(kind);
+        for (u32 i = 0; i < n; ++i) {
+            if (!nodes[i].dup) continue;
+            double const z = nodes[i].z;
+            for (u32 q = 0; q < rule.m; ++q) {
+                double const x = rule.x[q], a = z + x * (1.0 - z);
+                put(&out[o], q, past_half(q, rule.m) ? z * (1.0 - x) / a : x / a);
+                put(&out[o], rule.m + q, z / (a * a));
+            }
+            o += ds;
+        }
+        return at;
+    }
+
+    void step(u32 kind, u32 level, Node const &nd, u32 flags, double vl, double vr)
+    {
+        size_t const at = open(kind, &nd, 1);
+        TSlot *s = &out[at];
+        s->w[kTwOp] = kind | level << 2 | (nd.dup ? 0x100u : 0u) | flags;
+        s->w[kTwLv] = nd.level;
+        s->w[kTwSplit] = nd.split;
+        put(s, kTwZl, nd.zl);
+        put(s, kTwZr, nd.zr);
+        put(s, kTwVl, vl);
+        put(s, kTwVr, vr);
+    }
+
+    // Nodes of a block in preorder: `depth` more levels below id.
+    void collect(u32 id, u32 level, u32 depth, Node *&nodes, double *&leaf)
+    {
+        Node const nd = node(id);
+        if (depth == 0) {
+            *leaf++ = nd.value;
+            return;
+        }
+        *nodes++ = nd;
+        bool const self = nd.leaf; // its two children are itself
+        for (u32 side = 0; side < 2; ++side) {
+            if (!self) above.push_back({static_cast<u32>(t[id].feature), level, nd.z * (side ? nd.zr : nd.zl)});
+            collect(self ? id : (side ? t[id].right : t[id].left), level + 1, depth - 1, nodes, leaf);
+            if (!self) above.pop_back();
+        }
+    }
+
+    void block(u32 id, u32 level)
+    {
+        Node nd[7], *np = nd;
+        double leaf[8], *lp = leaf;
+        collect(id, level, kTBlockLevels, np, lp);
+        size_t const at = open(kTBlock, nd, 7);
+        TSlot *s = &out[at];
+        u32 op = kTBlock | level << 2, lv = 0;
+        for (u32 i = 0; i < 7; ++i) {
+            op |= nd[i].dup ? 0x100u << i : 0u;
+            lv |= nd[i].level << (4 * i);
+            s[(kTwSplit + i) / 8].w[(kTwSplit + i) % 8] = nd[i].split;
+        }
+        s->w[kTwOp] = op;
+        s->w[kTwLv] = lv;
+        static const u32 inner[3] = {0, 1, 4}, low[4] = {2, 3, 5, 6};
+        for (u32 i = 0; i < 3; ++i) {
+            put(s, kTwZ + 2 * i, nd[inner[i]].zl);
+            put(s, kTwZ + 2 * i + 1, nd[inner[i]].zr);
+        }
+        for (u32 i = 0; i < 4; ++i) {
+            put(s, kTwMean + i, nd[low[i]].zl * leaf[2 * i] + nd[low[i]].zr * leaf[2 * i + 1]);
+            put(s, kTwLeaf + 2 * i, leaf[2 * i]);
+            put(s, kTwLeaf + 2 * i + 1, leaf[2 * i + 1]);
+        }
+    }
+
+    void walk(u32 id, u32 level)
+    {
+        if (levels[id] <= kTBlockLevels) {
+            block(id, level);
+            return;
+        }
+        bh_node const &n = t[id];
+        Node const nd = node(id);
+        bool const ll = t[n.left].feature < 0, rl = t[n.right].feature < 0;
+        double const vl = ll ? static_cast<double>(t[n.left].value) * scale : 0.0;
+        double const vr = rl ? static_cast<double>(t[n.right].value) * scale : 0.0;
+        u32 const flags = (ll ? kTLeafL : 0u) | (rl ? kTLeafR : 0u);
+        step(kTEnter, level, nd, flags, vl, vr);
+        for (u32 side = 0; side < 2; ++side) {
+            if (side ? rl : ll) continue;
+            if (side && !ll) step(kTTurn, level, nd, flags, vl, vr);
+            above.push_back({static_cast<u32>(n.feature), level, nd.z * (side ? nd.zr : nd.zl)});
+            walk(side ? n.right : n.left, level + 1);
+            above.pop_back();
+        }
+        step(kTCombine, level, nd, flags, vl, vr);
+    }
+};
+
+// Gauss-Legendre nodes on [0, 1], ascending (Newton's method on the Legendre polynomial),
+// and their weights times a common factor `g` searched so that every weight lands
+// within 2^-29 of a float (or the nearest found): a weight's rounding would be the same
+// relative error in every contribution.
+GaussRule gauss_legendre(u32 m)
+{
+    GaussRule r{};
+    r.m = m;
+    for (u32 i = 0; i < m; ++i) {
+        double x = std::cos(3.14159265358979323846 * (m - 1 - i + 0.75) / (m + 0.5)), d = 1.0;
+        for (int it = 0; it < 60; ++it) {
+            double p0 = 1.0, p1 = x;
+            for (u32 k = 2; k <= m; ++k) {
+                double const p2 = ((2.0 * k - 1.0) * x * p1 - (k - 1.0) * p0) / k;
+                p0 = p1;
+                p1 = p2;
+            }
+            d = m * (x * p1 - p0) / (x * x - 1.0);
+            x -= p1 / d;
+        }
+        r.x[i] = 0.5 * (1.0 + x);
+        r.w[i] = 1.0 / ((1.0 - x * x) * d * d);
+    }
+    return r;
+}
+TQuad tree_quad(GaussRule const &r, double &g)
+{
+    u32 const m = r.m;
+    TQuad q{};
+    for (u32 i = 0; i < m; ++i) q.y[i] = static_cast<float>(past_half(i, m) ? 1.0 - r.x[i] : r.x[i]);
+    double best = 1.0;
+    g = 1.0;
+    for (u32 k = 0; k < 200000 && best > 0x1p-29; ++k) {
+        double const c = 1.0 + k * 0x1p-18;
+        double worst = 0.0;
+        for (u32 i = 0; i < (m + 1) / 2; ++i) { // the rule is symmetric
+            double const v = r.w[i] * c;
+            worst = std::max(worst, std::fabs(static_cast<double>(static_cast<float>(v)) - v) / v);
+        }
+        if (worst < best) {
+            best = worst;
+            g = c;
+        }
+    }
+    for (u32 i = 0; i < m; ++i) q.w[i] = static_cast<float>(r.w[std::min(i, m - 1 - i)] * g);
+    return q;
+}
+
 // tree_expected_value (src/shap.cpp:246-292): cover-weighted mean of the leaves.
 double expected_value(bh_node const *t, u32 id)
 {
@@ -385,6 +1027,12 @@ struct bh_predictor {
     u32 n_heads = 0, max_len = 0;
     u32 n_groups = 0;          // TreeSHAP path groups of 64
     double shap_scale = 1.0;   // fixed-point scale of the TreeSHAP accumulators
+    // tree-form TreeSHAP (tree_m quadrature nodes; 0: the packed form serves the ensemble)
+    u32 tree_m = 0, tree_depth = 0, n_ttrees = 0;
+    double tree_scale = 1.0;   // its fixed-point scale, times the weights' common factor
+    TQuad quad{};
+    TSlot *d_tslots = nullptr;
+    u32 *d_tfirst = nullptr;
     PNode *d_nodes = nullptr;
     u32 *d_roots = nullptr;
     u16 *d_last = nullptr;
@@ -407,9 +1055,54 @@ int launch_predict(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, float *
     return 0;
 }
 
+// Workgroups that fill the chip with tree-form waves: smaller batches split their trees.
+constexpr u32 kTreeShapFill = 768;
+
+int launch_shap_tree(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, double *d_out, hipStream_t s)
+{
+    u32 const blocks = static_cast<u32>((n + kTreeShapRows - 1) / kTreeShapRows);
+    u32 const upper = p->tree_depth > kTBlockLevels ? p->tree_depth - kTBlockLevels : 0u;
+    u32 const threads = kTreeShapThreads, waves = threads / 64u;
+    u32 split = 1;
+    if (blocks < kTreeShapFill)
+        split = std::min((kTreeShapFill + blocks - 1) / blocks, std::max(1u, (p->n_ttrees + waves - 1) / waves));
+    u64 const cells = n * (p->F + 1);
+    u32 const cgrid = static_cast<u32>(std::min<u64>((cells + 255) / 256, 4096));
+    if (split > 1) {
+        hipLaunchKernelGGL(k_shap_zero, dim3(cgrid), dim3(256), 0, s, reinterpret_cast<unsigned long long *>(d_out),
+                           cells);
+        SHIP(hipGetLastError());
+    }
+    size_t const lds = tree_shap_lds(p->F);
+    dim3 const grid(blocks, split);
+#define BH_TS(MV, UV)                                                                                              \
+    hipLaunchKernelGGL((k_shap_tree<MV, UV>), grid, dim3(threads), lds, s, d_bins, n, stride, p->F, p->d_last,     \
+                       p->d_tslots, p->d_tfirst, p->n_ttrees, p->quad, p->lr, p->shap_bias, p->tree_scale, d_out)
+    if (upper <= 5) {
+        if (p->tree_m <= 2) BH_TS(2, 5);
+        else if (p->tree_m == 3) BH_TS(3, 5);
+        else BH_TS(4, 5);
+    } else if (p->tree_m <= 4) {
+        BH_TS(4, 9);
+    } else if (p->tree_m == 5) {
+        BH_TS(5, 9);
+    } else {
+        BH_TS(6, 9);
+    }
+#undef BH_TS
+    SHIP(hipGetLastError());
+    if (split > 1) {
+        hipLaunchKernelGGL(k_shap_to_double, dim3(cgrid), dim3(256), 0, s, d_out, n, p->F, p->lr, p->shap_bias,
+                           p->tree_scale);
+        SHIP(hipGetLastError());
+    }
+    return 0;
+}
+
 int launch_shap(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, double *d_out, hipStream_t s)
 {
     if (n == 0) return 0;
+    if (p->tree_m) return launch_shap_tree(p, d_bins, n, stride, d_out, s);
     size_t const lds = static_cast<size_t>(kShapRows) * p->F * (sizeof(unsigned long long) + 1u);
     if (lds > 160u * 1024u) return sfail(1, "TreeSHAP: too many features for the LDS accumulators");
     u32 const blocks = static_cast<u32>((n + kShapRows - 1) / kShapRows);
@@ -426,13 +1119,8 @@ int launch_shap(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, double *d_
         SHIP(hipGetLastError());
     }
     dim3 const grid(blocks, split);
-    if (p->max_len <= 8)
-        hipLaunchKernelGGL(k_shap<8>, grid, dim3(256), lds, s, d_bins, n, stride, p->F, p->d_elems, p->d_heads,
-                           p->n_groups, p->max_len, p->d_w, p->d_last, p->lr, p->shap_bias, p->shap_scale, d_out);
-    else
-        hipLaunchKernelGGL(k_shap<kMaxPath>, grid, dim3(256), lds, s, d_bins, n, stride, p->F, p->d_elems,
-                           p->d_heads, p->n_groups, p->max_len, p->d_w, p->d_last, p->lr, p->shap_bias,
-                           p->shap_scale, d_out);
+    hipLaunchKernelGGL(k_shap<kMaxPath>, grid, dim3(256), lds, s, d_bins, n, stride, p->F, p->d_elems, p->d_heads,
+                       p->n_groups, p->max_len, p->d_w, p->d_last, p->lr, p->shap_bias, p->shap_scale, d_out);
     SHIP(hipGetLastError());
     if (split > 1) {
         hipLaunchKernelGGL(k_shap_to_double, dim3(cgrid), dim3(256), 0, s, d_out, n, p->F, p->lr, p->shap_bias,
@@ -465,7 +1153,9 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     std::vector<SHead> hd;
     size_t max_len = 0;
     double ev_sum = 0.0;
-    std::vector<ActiveElem> act;
+    std::vector<std::vector<u32>> levels(n_trees);
+    std::vector<u32> feats;
+    u32 deepest = 0;
     for (u32 t = 0; t < n_trees; ++t) {
         bh_node const *tn = nodes + tree_offsets[t];
         u32 const end = t + 1 < n_trees ? tree_offsets[t + 1] : 0;
@@ -505,8 +1195,8 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
             }
             pn.push_back(q);
         }
-        act.clear();
-        pack_paths(tn, last_bin, 0, act, el, hd, max_len);
+        levels[t].assign(count, 0u);
+        deepest = std::max(deepest, tree_levels(tn, 0, levels[t], feats, max_len));
         ev_sum += expected_value(tn, 0);
     }
     if (max_len > static_cast<size_t>(kMaxPath)) {
@@ -516,8 +1206,17 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     // bias column: sum of per-tree expected values, times lr, plus init
     // (include/bonsai/booster.hpp:902-925).
     p->shap_bias = ev_sum * static_cast<double>(learning_rate) + static_cast<double>(init_score);
-    p->n_heads = static_cast<u32>(hd.size());
     p->max_len = static_cast<u32>(std::max<size_t>(max_len, 1));
+    // The tree form serves every ensemble whose trees, paths and feature count fit its
+    // kernels; the packed form the rest.
+    bool const tree_form = deepest <= kTreeShapMaxDepth && max_len <= 2 * kTreeShapMaxM &&
+                           tree_shap_lds(n_features) <= 160u * 1024u;
+    if (!tree_form) {
+        std::vector<ActiveElem> act;
+        size_t longest = 0;
+        for (u32 t = 0; t < n_trees; ++t) pack_paths(nodes + tree_offsets[t], last_bin, 0, act, el, hd, longest);
+    }
+    p->n_heads = static_cast<u32>(hd.size());
     // Interleave the paths in groups of 64: element j of the group's paths contiguous.
     u32 const K = p->max_len;
     p->n_groups = (p->n_heads + 63u) / 64u;
@@ -551,6 +1250,51 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
                 w[rr * nn / 2 + i] = static_cast<float>(1.0 / (static_cast<double>(nn) * binom[i]));
         }
     }
+    TreePacker pack{};
+    std::vector<u32> tfirst;
+    if (tree_form) {
+        // kernels' node counts: 2, 3, 4 (up to 8 levels), 4, 5, 6 (more)
+        u32 const m = std::max<u32>(deepest <= 8 ? 2u : 4u, (p->max_len + 1u) / 2u);
+        // A contribution is at most 4 max|leaf| of its tree, and one level's together too.
+        double top = 0.0, sum = 0.0;
+        for (u32 t = 0; t < n_trees; ++t) {
+            u32 const count = (t + 1 < n_trees ? roots[t + 1] : static_cast<u32>(pn.size())) - roots[t];
+            double v = 0.0;
+            for (u32 i = 0; i < count; ++i)
+                if (nodes[tree_offsets[t] + i].feature < 0) {
+                    double const a = std::fabs(static_cast<double>(nodes[tree_offsets[t] + i].value));
+                    v = a <= v ? v : a; // keeps a NaN
+                }
+            top = v <= top ? top : v;
+            sum += v;
+        }
+        double scale = 1.0;
+        if (std::isfinite(sum) && sum > 0.0) {
+            int e1 = 0, e2 = 0;
+            (void)std::frexp(top, &e1);
+            (void)std::frexp(sum * std::max(1u, deepest), &e2);
+            scale = std::ldexp(1.0, std::min(48 - e1, 60 - e2));
+        }
+        pack.last = last_bin;
+        pack.F = n_features;
+        pack.scale = scale;
+        pack.rule = gauss_legendre(m);
+        for (u32 t = 0; t < n_trees; ++t) {
+            pack.t = nodes + tree_offsets[t];
+            pack.levels = levels[t].data();
+            if (pack.t[0].feature < 0) continue; // a single leaf has no contributions
+            tfirst.push_back(static_cast<u32>(pack.out.size()));
+            pack.walk(0, 0);
+        }
+        tfirst.push_back(static_cast<u32>(pack.out.size()));
+        pack.out.resize((pack.out.size() / 64u + 3u) * 64u); // the kernel reads whole groups, two ahead
+        double g = 1.0;
+        p->quad = tree_quad(pack.rule, g);
+        p->tree_m = m;
+        p->tree_depth = deepest;
+        p->n_ttrees = static_cast<u32>(tfirst.size() - 1);
+        p->tree_scale = std::isfinite(sum) ? scale * g : std::nan("");
+    }
     hipError_t e = hipSuccess;
     auto al = [&](void **ptr, size_t bytes) {
         if (e == hipSuccess) e = hipMalloc(ptr, std::max<size_t>(bytes, 16));
@@ -567,6 +1311,12 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     if (e == hipSuccess && !el.empty()) e = hipMemcpy(p->d_elems, el.data(), el.size() * sizeof(SElem), hipMemcpyHostToDevice);
     if (e == hipSuccess && !hd.empty()) e = hipMemcpy(p->d_heads, hd.data(), hd.size() * sizeof(SHead), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->d_w, w.data(), w.size() * sizeof(float), hipMemcpyHostToDevice);
+    if (p->tree_m) {
+        al(reinterpret_cast<void **>(&p->d_tslots), pack.out.size() * sizeof(TSlot));
+        al(reinterpret_cast<void **>(&p->d_tfirst), tfirst.size() * sizeof(u32));
+        if (e == hipSuccess) e = hipMemcpy(p->d_tslots, pack.out.data(), pack.out.size() * sizeof(TSlot), hipMemcpyHostToDevice);
+        if (e == hipSuccess && !tfirst.empty()) e = hipMemcpy(p->d_tfirst, tfirst.data(), tfirst.size() * sizeof(u32), hipMemcpyHostToDevice);
+    }
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
         bh_predictor_destroy(p);
@@ -580,7 +1330,7 @@ int bh_predictor_destroy(bh_predictor *p)
 {
     if (!p) return 0;
     (void)hipSetDevice(p->device);
-    void *ptrs[] = {p->d_nodes, p->d_roots, p->d_last, p->d_elems, p->d_heads, p->d_w};
+    void *ptrs[] = {p->d_nodes, p->d_roots, p->d_last, p->d_elems, p->d_heads, p->d_w, p->d_tslots, p->d_tfirst};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     if (p->stream) (void)hipStreamDestroy(p->stream);

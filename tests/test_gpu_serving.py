@@ -161,3 +161,64 @@ def test_shap_split_launch_equals_single_pass(hip, orc, model):
     scale = np.abs(ref).sum(axis=1, keepdims=True)
     assert np.max(np.abs(whole[:64] - ref) / scale) <= 1e-5
     p.close()
+
+
+def random_trees(rng, n_trees, depth, n_features, nb, p_leaf, zero_cover=False):
+    """Trees of exactly `depth` levels on one path, other nodes leaves with p_leaf."""
+    trees = []
+    for _ in range(n_trees):
+        nodes = []
+
+        def grow(level, cover, spine):
+            i = len(nodes)
+            nodes.append(None)
+            if level == depth or (not spine and rng.random() < p_leaf):
+                nodes[i] = (-1, 0, 0, 0, 0, rng.normal(0, 0.1), cover, 0.0)
+                return i
+            f = int(rng.integers(0, n_features))
+            b = int(rng.integers(0, max(1, nb[f] - 1)))
+            cl = float(np.round(cover * rng.uniform(0.05, 0.95)))
+            if zero_cover and rng.random() < 0.2:
+                cl = 0.0
+            side = rng.random() < 0.5
+            left = grow(level + 1, cl, spine and side)
+            right = grow(level + 1, cover - cl, spine and not side)
+            nodes[i] = (f, b, int(rng.integers(0, 2)), left, right, 0.0, cover, 1.0)
+            return i
+
+        grow(0, 1e6, True)
+        trees.append(np.array(nodes, NODE_DTYPE))
+    return trees
+
+
+@pytest.mark.parametrize("depth,n_features,used,n_rows,p_leaf", [
+    (1, 1, 1, 1, 0.0), (2, 3, 3, 64, 0.0), (3, 5, 5, 65, 0.3), (4, 28, 28, 63, 0.0), (5, 28, 4, 130, 0.2),
+    (8, 28, 28, 257, 0.0), (8, 28, 6, 100, 0.1), (8, 256, 256, 31, 0.0), (9, 28, 28, 70, 0.3), (10, 10, 10, 33, 0.2),
+    (12, 40, 40, 65, 0.35), (12, 28, 3, 20, 0.3), (13, 28, 12, 20, 0.4)])
+def test_shap_tree_form_matches_packed_form(hip, orc, depth, n_features, used, n_rows, p_leaf):
+    """Ensembles of up to 12 levels, 12 features per path and 256 features are served by
+    the tree form, others by the packed form: a plane with unused features up to 257 takes
+    the same trees through the packed form.  Both sum float path terms exactly, so they
+    agree with the double oracle to a few float roundings per path element (1e-5 of the
+    row's mass, the bound of the other TreeSHAP tests)."""
+    rng = np.random.default_rng([depth, n_features, used])
+    nb = rng.integers(2, 257, n_features).astype(np.uint16)
+    nb[0] = 2
+    for zero_cover in (False, True):
+        trees = random_trees(rng, 5, depth, used, nb, p_leaf, zero_cover)
+        trees.append(np.array([(-1, 0, 0, 0, 0, 0.5, 10.0, 0.0)], NODE_DTYPE))   # a single leaf
+        rows = (rng.random((n_rows, n_features)) * nb).astype(np.uint8)
+        p = hip.Predictor(trees, nb, 0.3, 0.25)
+        got = p.shap(rows)
+        wide = np.zeros((n_rows, 257), np.uint8)
+        wide[:, :n_features] = rows
+        wnb = np.full(257, 2, np.uint16)
+        wnb[:n_features] = nb
+        packed = hip.Predictor(trees, wnb, 0.3, 0.25).shap(wide)
+        mass = np.abs(packed).sum(axis=1, keepdims=True)
+        assert np.max(np.abs(got[:, :n_features] - packed[:, :n_features]) / mass) <= 1e-5
+        assert np.array_equal(got[:, -1], packed[:, -1])
+        assert np.array_equal(p.shap(rows[-1:])[0], got[-1])
+        if not zero_cover:
+            ref = orc.pred_contribs(trees, rows, nb, 0.3, 0.25, depth)
+            assert np.max(np.abs(got - ref) / mass) <= 1e-5
