@@ -72,31 +72,38 @@ constexpr int kMaxPath = 16;
 // ---------------------------------------------------------------------------------
 // Predict: init + lr * sum_t leaf_t(row), the tree sum in tree order, multiply then
 // add each rounded (predict_walk_kernel, src/cuda/predict.cu:50-85; host
-// predict_at_binned, include/bonsai/booster.hpp:831-846).  A workgroup takes kPR rows;
-// its threads walk (row, tree) pairs of one tree tile into LDS, then one thread per row
-// adds the tile in tree order.
+// predict_at_binned, include/bonsai/booster.hpp:831-846).
+//
+// Small batches (and any ensemble): a workgroup takes a few rows, its threads walk (row,
+// tree) pairs of one tree tile from global memory into LDS, then one thread per row adds
+// the tile in tree order.  Latency bound: the walk's dependent node loads and the ordered
+// float sum (about 3 us per 1,000 trees); one row per workgroup while the rows alone do
+// not fill the chip.
 // ---------------------------------------------------------------------------------
-constexpr u32 kPR = 16, kPT = 256;
+constexpr u32 kPredTile = 1024;    // trees whose values wait in LDS
+constexpr u32 kPredMaxRows = 8;    // rows of a workgroup
 
-__global__ __launch_bounds__(256) void k_predict(u8 const *__restrict__ bins, u64 n, u64 stride, u32 F,
-                                                 PNode const *__restrict__ nodes, u32 const *__restrict__ roots,
-                                                 u32 n_trees, u16 const *__restrict__ last, float lr, float init,
-                                                 float *__restrict__ out)
+__global__ __launch_bounds__(1024) void k_predict_direct(u8 const *__restrict__ bins, u64 n, u64 stride, u32 F,
+                                                         u32 rows, PNode const *__restrict__ nodes,
+                                                         u32 const *__restrict__ roots, u32 n_trees,
+                                                         u16 const *__restrict__ last, float lr, float init,
+                                                         float *__restrict__ out)
 {
-    __shared__ float s_val[kPR][kPT];
-    __shared__ float s_acc[kPR];
-    extern __shared__ __align__(16) unsigned char s_rows[]; // kPR * F bytes
-    u64 const r0 = static_cast<u64>(blockIdx.x) * kPR;
-    if (r0 >= n) return;
-    u32 const nr = static_cast<u32>(min<u64>(kPR, n - r0));
+    extern __shared__ __align__(16) unsigned char smem[];
+    float *s_val = reinterpret_cast<float *>(smem);                          // [rows][kPredTile]
+    u16 *s_last = reinterpret_cast<u16 *>(s_val + rows * kPredTile);         // [F]
+    u8 *s_rows = reinterpret_cast<u8 *>(s_last + F);                         // [rows][F]
+    u64 const r0 = static_cast<u64>(blockIdx.x) * rows;
+    u32 const nr = static_cast<u32>(min<u64>(rows, n - r0));
     for (u32 k = threadIdx.x; k < nr * F; k += blockDim.x) {
         u32 const rr = k / F, f = k - rr * F;
         s_rows[k] = bins[(r0 + rr) * stride + f];
     }
-    if (threadIdx.x < kPR) s_acc[threadIdx.x] = 0.0F;
+    for (u32 f = threadIdx.x; f < F; f += blockDim.x) s_last[f] = last[f];
     __syncthreads();
-    for (u32 t0 = 0; t0 < n_trees; t0 += kPT) {
-        u32 const tt = min(kPT, n_trees - t0);
+    float acc = 0.0F;
+    for (u32 t0 = 0; t0 < n_trees; t0 += kPredTile) {
+        u32 const tt = min(kPredTile, n_trees - t0);
         for (u32 k = threadIdx.x; k < nr * tt; k += blockDim.x) {
             u32 const rr = k / tt, t = k - rr * tt;
             PNode const *tn = nodes + roots[t0 + t];
@@ -104,20 +111,182 @@ __global__ __launch_bounds__(256) void k_predict(u8 const *__restrict__ bins, u6
             PNode nd = tn[0];
             while (nd.feature != 0xFFFFu) {
                 u32 const b = row[nd.feature];
-                bool const left = b == last[nd.feature] ? (nd.dl != 0) : (b <= nd.bin);
+                bool const left = b == s_last[nd.feature] ? (nd.dl != 0) : (b <= nd.bin);
                 nd = tn[left ? nd.u.c.left : nd.u.c.right];
             }
-            s_val[rr][t] = nd.u.value;
+            s_val[rr * kPredTile + t] = nd.u.value;
         }
         __syncthreads();
         if (threadIdx.x < nr) {
-            float acc = s_acc[threadIdx.x];
-            for (u32 t = 0; t < tt; ++t) acc += s_val[threadIdx.x][t];
-            s_acc[threadIdx.x] = acc;
+            float const *v = s_val + threadIdx.x * kPredTile;
+            u32 t = 0;
+            for (; t + 16 <= tt; t += 16) {
+                float4 q[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) q[k] = reinterpret_cast<float4 const *>(v + t)[k];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    acc += q[k].x;
+                    acc += q[k].y;
+                    acc += q[k].z;
+                    acc += q[k].w;
+                }
+            }
+            for (; t < tt; ++t) acc += v[t];
         }
         __syncthreads();
     }
-    if (threadIdx.x < nr) out[r0 + threadIdx.x] = __fadd_rn(init, __fmul_rn(lr, s_acc[threadIdx.x]));
+    if (threadIdx.x < nr) out[r0 + threadIdx.x] = __fadd_rn(init, __fmul_rn(lr, acc));
+}
+
+// Larger batches: one row per lane, trees walked from LDS.  The ensemble is laid out in
+// tiles of at most kTileNodes 4-byte nodes (and their values); a workgroup keeps ROWS rows
+// in LDS and streams the tiles through it, the next tile's loads in flight in registers.
+// A leaf is a node whose comparison always holds and whose left child is itself, so a
+// walk is a fixed number of steps (the deepest of its trees): one random 4-byte read of
+// a node, one random byte of the row and seven vector instructions.  LDS bound: about 11
+// clocks per wave step.  With fewer than 1,024 rows the workgroup's 16 waves split each
+// tile's trees, leave the values in LDS and the first waves add them in tree order.
+// A row's bins are stored shifted, the missing bin as 0, others as bin + 1: with d = 1
+// where the missing bin goes right, the row goes left when (shifted - d) as unsigned is
+// at most bin + 1 - d.
+constexpr u32 kTileNodes = 8192;
+constexpr u32 kTileThreads = 1024;
+// node: feature | bin + 1 - d (at most 255) << 8 | left child's index in the tile << 16 | d << 31
+constexpr u32 tile_row_stride(u32 F) { return ((F + 3u) / 4u | 1u) * 4u; } // odd dwords: lanes' rows spread over banks
+
+struct TileTree {
+    u32 root; // index in the tile | levels << 16
+};
+struct Tile {
+    u32 off, count; // first word of its nodes (count of them, then count values), count a multiple of 4
+    u32 tree0, n_trees;
+};
+
+template <int G> __device__ __forceinline__ void tile_walk(u32 const *s_nodes, u32 count, u8 const *row,
+                                                           TileTree const *__restrict__ tt, float (&v)[G])
+{
+    u32 at[G], steps = 0;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        u32 const r = __builtin_amdgcn_readfirstlane(tt[g].root);
+        at[g] = r & 0xFFFFu;
+        steps = max(steps, r >> 16);
+    }
+    for (u32 k = 0; k < steps; ++k) {
+        u32 nd[G], b[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) nd[g] = s_nodes[at[g]];
+#pragma unroll
+        for (int g = 0; g < G; ++g) b[g] = row[nd[g] & 0xFFu];
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            at[g] = (nd[g] >> 16 & 0x7FFFu) + (b[g] - (nd[g] >> 31) <= (nd[g] >> 8 & 0xFFu) ? 0u : 1u);
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) v[g] = reinterpret_cast<float const *>(s_nodes + count)[at[g]];
+}
+
+template <u32 ROWS>
+__global__ __launch_bounds__(kTileThreads) void k_predict_tile(u8 const *__restrict__ bins, u64 n, u64 stride, u32 F,
+                                                               u32 const *__restrict__ words,
+                                                               Tile const *__restrict__ tiles, u32 n_tiles,
+                                                               TileTree const *__restrict__ trees,
+                                                               u16 const *__restrict__ last, float lr, float init,
+                                                               float *__restrict__ out)
+{
+    constexpr u32 S = kTileThreads / ROWS; // waves of one row group that split a tile's trees
+    constexpr u32 NW = 2 * kTileNodes / 4 / kTileThreads; // 16-byte words of a tile per thread
+    extern __shared__ __align__(16) unsigned char smem[];
+    u32 *s_nodes = reinterpret_cast<u32 *>(smem);                       // 2 * kTileNodes: nodes, then values
+    float *s_out = reinterpret_cast<float *>(s_nodes + 2 * kTileNodes); // S > 1: [2][S * 4][ROWS]
+    u8 *s_rows = reinterpret_cast<u8 *>(s_out + (S > 1 ? 2 * S * 4 * ROWS : 0)); // [ROWS][RS]
+    u32 const RS = tile_row_stride(F);
+    u64 const r0 = static_cast<u64>(blockIdx.x) * ROWS;
+    u32 const nr = static_cast<u32>(min<u64>(ROWS, n - r0));
+    uint4 pf[NW];
+    auto fetch = [&](Tile const &t) {
+        uint4 const *src = reinterpret_cast<uint4 const *>(words + t.off);
+#pragma unroll
+        for (u32 k = 0; k < NW; ++k) {
+            u32 const i = threadIdx.x + k * kTileThreads;
+            pf[k] = i < t.count / 2u ? src[i] : make_uint4(0, 0, 0, 0);
+        }
+    };
+    Tile tile = tiles[0];
+    fetch(tile);
+    for (u32 k = threadIdx.x; k < ROWS * F; k += kTileThreads) {
+        u32 const rr = k / F, f = k - rr * F;
+        u32 const b = rr < nr ? bins[(r0 + rr) * stride + f] : 0u;
+        s_rows[rr * RS + f] = static_cast<u8>(b == last[f] ? 0u : min(b + 1u, 255u));
+    }
+    u32 const rr = threadIdx.x % ROWS;
+    u32 const s = __builtin_amdgcn_readfirstlane(threadIdx.x / ROWS);
+    u8 const *row = s_rows + rr * RS;
+    float acc = 0.0F;
+    u32 buf = 0;
+    for (u32 i = 0; i < n_tiles; ++i) {
+        __syncthreads(); // the previous tile is walked
+#pragma unroll
+        for (u32 k = 0; k < NW; ++k) {
+            u32 const w = threadIdx.x + k * kTileThreads;
+            if (w < tile.count / 2u) reinterpret_cast<uint4 *>(s_nodes)[w] = pf[k];
+        }
+        u32 const count = tile.count, t0 = tile.tree0, t1 = tile.tree0 + tile.n_trees;
+        if (i + 1 < n_tiles) {
+            tile = tiles[i + 1];
+            fetch(tile);
+        }
+        __syncthreads();
+        if constexpr (S == 1) {
+            u32 t = t0;
+            for (; t + 4 <= t1; t += 4) {
+                float v[4];
+                tile_walk<4>(s_nodes, count, row, trees + t, v);
+                acc += v[0];
+                acc += v[1];
+                acc += v[2];
+                acc += v[3];
+            }
+            for (; t < t1; ++t) {
+                float v[1];
+                tile_walk<1>(s_nodes, count, row, trees + t, v);
+                acc += v[0];
+            }
+        } else {
+            // g trees per wave and round; a round's values are added while the next is
+            // walked into the other buffer
+            u32 const g = t1 - t0 >= 4u * S ? 4u : (t1 - t0 >= 2u * S ? 2u : 1u);
+            for (u32 t = t0; t < t1; t += g * S) {
+                float *o = s_out + buf * (S * 4 * ROWS);
+                u32 const mine = t + s * g, end = min(t1, mine + g);
+                if (mine + 4 <= end) {
+                    float v[4];
+                    tile_walk<4>(s_nodes, count, row, trees + mine, v);
+#pragma unroll
+                    for (u32 k = 0; k < 4; ++k) o[(s * g + k) * ROWS + rr] = v[k];
+                } else if (mine + 2 == end) {
+                    float v[2];
+                    tile_walk<2>(s_nodes, count, row, trees + mine, v);
+                    o[s * g * ROWS + rr] = v[0];
+                    o[(s * g + 1) * ROWS + rr] = v[1];
+                } else {
+                    for (u32 k = mine; k < end; ++k) {
+                        float v[1];
+                        tile_walk<1>(s_nodes, count, row, trees + k, v);
+                        o[(k - t) * ROWS + rr] = v[0];
+                    }
+                }
+                __syncthreads();
+                if (s == 0) {
+                    u32 const m = min(g * S, t1 - t);
+                    for (u32 k = 0; k < m; ++k) acc += o[k * ROWS + rr];
+                }
+                buf ^= 1u;
+            }
+        }
+    }
+    if (s == 0 && rr < nr) out[r0 + rr] = __fadd_rn(init, __fmul_rn(lr, acc));
 }
 
 // ---------------------------------------------------------------------------------
@@ -712,6 +881,67 @@ __global__ __launch_bounds__(256) void k_shap_to_double(double *__restrict__ out
     }
 }
 
+// Tiles of an ensemble (k_predict_tile); false when a tree or the features do not fit.
+bool pack_tiles(bh_node const *nodes, uint32_t const *offsets, u32 n_trees, u32 F,
+                std::vector<u32> &words, std::vector<Tile> &tiles, std::vector<TileTree> &trees)
+{
+    if (F > 256u || n_trees == 0) return false;
+    std::vector<u32> nd, order; // the open tile's nodes; a tree's node ids, siblings adjacent
+    std::vector<float> val;
+    auto close = [&] {
+        if (tiles.empty() || tiles.back().count != 0) return;
+        while (nd.size() & 3u) {
+            nd.push_back(0u);
+            val.push_back(0.0F);
+        }
+        Tile &t = tiles.back();
+        t.off = static_cast<u32>(words.size());
+        t.count = static_cast<u32>(nd.size());
+        t.n_trees = static_cast<u32>(trees.size()) - t.tree0;
+        words.insert(words.end(), nd.begin(), nd.end());
+        words.resize(words.size() + val.size());
+        std::memcpy(words.data() + t.off + t.count, val.data(), val.size() * sizeof(float));
+        nd.clear();
+        val.clear();
+    };
+    for (u32 k = 0; k < n_trees; ++k) {
+        bh_node const *t = nodes + offsets[k];
+        order.assign(1, 0u);
+        u32 levels = 0;
+        for (size_t i = 0, end = 1; i < order.size();) { // breadth first, level by level
+            for (; i < end; ++i)
+                if (t[order[i]].feature >= 0) {
+                    order.push_back(t[order[i]].left);
+                    order.push_back(t[order[i]].right);
+                    if (order.size() > kTileNodes) return false;
+                }
+            if (order.size() > end) ++levels;
+            end = order.size();
+        }
+        if (tiles.empty() || nd.size() + order.size() > kTileNodes) {
+            close();
+            tiles.push_back(Tile{0u, 0u, static_cast<u32>(trees.size()), 0u});
+        }
+        u32 const base = static_cast<u32>(nd.size());
+        trees.push_back(TileTree{base | levels << 16});
+        u32 child = base + 1u;
+        for (size_t i = 0; i < order.size(); ++i) {
+            bh_node const &n = t[order[i]];
+            if (n.feature < 0) {
+                nd.push_back(255u << 8 | (base + static_cast<u32>(i)) << 16);
+                val.push_back(n.value);
+                continue;
+            }
+            u32 const d = n.default_left ? 0u : 1u;
+            nd.push_back(static_cast<u32>(n.feature) | std::min(255u, n.bin + 1u - d) << 8 | child << 16 | d << 31);
+            val.push_back(0.0F);
+            child += 2u;
+        }
+    }
+    close();
+    return true;
+}
+
 struct ActiveElem {
     u32 feature;
     int lo, hi;
@@ -1035,6 +1265,11 @@ struct bh_predictor {
     u32 *d_tfirst = nullptr;
     PNode *d_nodes = nullptr;
     u32 *d_roots = nullptr;
+    // tile form (n_tiles 0: the ensemble does not fit it)
+    u32 n_tiles = 0;
+    u32 *d_words = nullptr;
+    Tile *d_tiles = nullptr;
+    TileTree *d_ttrees = nullptr;
     u16 *d_last = nullptr;
     SElem *d_elems = nullptr;
     SHead *d_heads = nullptr;
@@ -1044,13 +1279,44 @@ struct bh_predictor {
 
 namespace {
 
+// Rows from which a batch is served from tiles: below, walking from global memory with a
+// few rows per workgroup answers sooner.
+constexpr u64 kPredTileRows = 4096;
+
 int launch_predict(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, float *d_out, hipStream_t s)
 {
     if (n == 0) return 0;
-    u32 const blocks = static_cast<u32>((n + kPR - 1) / kPR);
-    size_t const lds = static_cast<size_t>(kPR) * p->F;
-    hipLaunchKernelGGL(k_predict, dim3(blocks), dim3(256), lds, s, d_bins, n, stride, p->F, p->d_nodes, p->d_roots,
-                       p->n_trees, p->d_last, p->lr, p->init, d_out);
+    constexpr size_t kLdsMax = 160u * 1024u;
+    if (p->n_tiles && n >= kPredTileRows) {
+        auto const lds = [&](u32 rows) {
+            u32 const split = kTileThreads / rows;
+            return static_cast<size_t>(2u * kTileNodes * 4u) + (split > 1 ? 2u * split * 4u * rows * 4u : 0u) +
+                   rows * tile_row_stride(p->F);
+        };
+#define BH_PT(R)                                                                                                    \
+    hipLaunchKernelGGL(k_predict_tile<R>, dim3(static_cast<u32>((n + R - 1) / R)), dim3(kTileThreads), lds(R), s,   \
+                       d_bins, n, stride, p->F, p->d_words, p->d_tiles, p->n_tiles, p->d_ttrees, p->d_last, p->lr,  \
+                       p->init, d_out)
+        // the most rows per workgroup whose workgroups still give every CU two
+        if (n > 1024u * 512u && lds(1024) <= kLdsMax) BH_PT(1024);
+        else if (n > 256u * 512u && lds(256) <= kLdsMax) BH_PT(256);
+        else BH_PT(64);
+#undef BH_PT
+        SHIP(hipGetLastError());
+        return 0;
+    }
+    u32 rows = static_cast<u32>(std::min<u64>(kPredMaxRows, std::max<u64>(1, n / 1024)));
+    auto const lds_of = [&](u32 r) {
+        return static_cast<size_t>(r) * (kPredTile * sizeof(float) + p->F) + p->F * sizeof(u16);
+    };
+    while (rows > 1 && lds_of(rows) > kLdsMax / 4) rows /= 2;
+    size_t const lds = lds_of(rows);
+    if (lds > kLdsMax) return sfail(1, "predict: too many features for one row in LDS");
+    u32 const blocks = static_cast<u32>((n + rows - 1) / rows);
+    u32 const walks = rows * std::min(kPredTile, std::max(1u, p->n_trees));
+    u32 const threads = std::min(1024u, (walks + 63u) / 64u * 64u);
+    hipLaunchKernelGGL(k_predict_direct, dim3(blocks), dim3(threads), lds, s, d_bins, n, stride, p->F, rows, p->d_nodes,
+                       p->d_roots, p->n_trees, p->d_last, p->lr, p->init, d_out);
     SHIP(hipGetLastError());
     return 0;
 }
@@ -1295,6 +1561,11 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
         p->n_ttrees = static_cast<u32>(tfirst.size() - 1);
         p->tree_scale = std::isfinite(sum) ? scale * g : std::nan("");
     }
+    std::vector<u32> words;
+    std::vector<Tile> tiles;
+    std::vector<TileTree> ttrees;
+    if (pack_tiles(nodes, tree_offsets, n_trees, n_features, words, tiles, ttrees))
+        p->n_tiles = static_cast<u32>(tiles.size());
     hipError_t e = hipSuccess;
     auto al = [&](void **ptr, size_t bytes) {
         if (e == hipSuccess) e = hipMalloc(ptr, std::max<size_t>(bytes, 16));
@@ -1311,6 +1582,14 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     if (e == hipSuccess && !el.empty()) e = hipMemcpy(p->d_elems, el.data(), el.size() * sizeof(SElem), hipMemcpyHostToDevice);
     if (e == hipSuccess && !hd.empty()) e = hipMemcpy(p->d_heads, hd.data(), hd.size() * sizeof(SHead), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->d_w, w.data(), w.size() * sizeof(float), hipMemcpyHostToDevice);
+    if (p->n_tiles) {
+        al(reinterpret_cast<void **>(&p->d_words), words.size() * sizeof(u32));
+        al(reinterpret_cast<void **>(&p->d_tiles), tiles.size() * sizeof(Tile));
+        al(reinterpret_cast<void **>(&p->d_ttrees), ttrees.size() * sizeof(TileTree));
+        if (e == hipSuccess) e = hipMemcpy(p->d_words, words.data(), words.size() * sizeof(u32), hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(p->d_tiles, tiles.data(), tiles.size() * sizeof(Tile), hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(p->d_ttrees, ttrees.data(), ttrees.size() * sizeof(TileTree), hipMemcpyHostToDevice);
+    }
     if (p->tree_m) {
         al(reinterpret_cast<void **>(&p->d_tslots), pack.out.size() * sizeof(TSlot));
         al(reinterpret_cast<void **>(&p->d_tfirst), tfirst.size() * sizeof(u32));
@@ -1330,7 +1609,8 @@ int bh_predictor_destroy(bh_predictor *p)
 {
     if (!p) return 0;
     (void)hipSetDevice(p->device);
-    void *ptrs[] = {p->d_nodes, p->d_roots, p->d_last, p->d_elems, p->d_heads, p->d_w, p->d_tslots, p->d_tfirst};
+    void *ptrs[] = {p->d_nodes, p->d_roots, p->d_last,   p->d_elems, p->d_heads, p->d_w,
+                    p->d_words, p->d_tiles, p->d_ttrees, p->d_tslots, p->d_tfirst};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     if (p->stream) (void)hipStreamDestroy(p->stream);
