@@ -1280,8 +1280,9 @@ struct bh_predictor {
 namespace {
 
 // Rows from which a batch is served from tiles: below, walking from global memory with a
-// few rows per workgroup answers sooner.
-constexpr u64 kPredTileRows = 4096;
+// few rows per workgroup answers sooner (2,000 rows x 1,000 depth-8 trees: 153 us against
+// 145 from tiles, whose time is flat up to 16,384 rows; 1,000 rows: 82 us).
+constexpr u64 kPredTileRows = 2048;
 
 int launch_predict(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, float *d_out, hipStream_t s)
 {
@@ -1297,10 +1298,15 @@ int launch_predict(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, float *
     hipLaunchKernelGGL(k_predict_tile<R>, dim3(static_cast<u32>((n + R - 1) / R)), dim3(kTileThreads), lds(R), s,   \
                        d_bins, n, stride, p->F, p->d_words, p->d_tiles, p->n_tiles, p->d_ttrees, p->d_last, p->lr,  \
                        p->init, d_out)
-        // the most rows per workgroup whose workgroups still give every CU two
-        if (n > 1024u * 512u && lds(1024) <= kLdsMax) BH_PT(1024);
-        else if (n > 256u * 512u && lds(256) <= kLdsMax) BH_PT(256);
-        else BH_PT(64);
+        // One workgroup per CU (LDS): a round of 256 workgroups over 1,000 depth-8 trees
+        // takes 145 us with 64 rows each, 235 with 256 and 595 with 1,024.  The cheapest
+        // rounds win.
+        auto const cost = [&](u32 rows, u64 round) { return ((n + rows - 1) / rows + 255) / 256 * round; };
+        u64 const c64 = cost(64, 145), c256 = lds(256) <= kLdsMax ? cost(256, 235) : ~0ull,
+                  c1024 = lds(1024) <= kLdsMax ? cost(1024, 595) : ~0ull;
+        if (c64 <= c256 && c64 <= c1024) BH_PT(64);
+        else if (c256 <= c1024) BH_PT(256);
+        else BH_PT(1024);
 #undef BH_PT
         SHIP(hipGetLastError());
         return 0;
@@ -1329,9 +1335,19 @@ int launch_shap_tree(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, doubl
     u32 const blocks = static_cast<u32>((n + kTreeShapRows - 1) / kTreeShapRows);
     u32 const upper = p->tree_depth > kTBlockLevels ? p->tree_depth - kTBlockLevels : 0u;
     u32 const threads = kTreeShapThreads, waves = threads / 64u;
+    // Trees of a row block over `split` workgroups: the fewest rounds of kTreeShapFill
+    // workgroups per share of the trees, then the fewest shares.
+    u32 const most = std::min(std::max(1u, kTreeShapFill / std::min(blocks, kTreeShapFill)) + 7u,
+                              std::max(1u, (p->n_ttrees + waves - 1) / waves));
     u32 split = 1;
-    if (blocks < kTreeShapFill)
-        split = std::min((kTreeShapFill + blocks - 1) / blocks, std::max(1u, (p->n_ttrees + waves - 1) / waves));
+    u64 rounds = (static_cast<u64>(blocks) + kTreeShapFill - 1) / kTreeShapFill;
+    for (u32 k = 2; k <= most && blocks < 16u * kTreeShapFill; ++k) {
+        u64 const r = (static_cast<u64>(blocks) * k + kTreeShapFill - 1) / kTreeShapFill;
+        if (r * split < rounds * k) {
+            rounds = r;
+            split = k;
+        }
+    }
     u64 const cells = n * (p->F + 1);
     u32 const cgrid = static_cast<u32>(std::min<u64>((cells + 255) / 256, 4096));
     if (split > 1) {

@@ -228,7 +228,7 @@ def test_shap_tree_form_matches_packed_form(hip, orc, depth, n_features, used, n
     (1, 1, 3, 0.0), (4, 28, 1, 0.0), (8, 28, 37, 0.0), (9, 28, 130, 0.3), (6, 256, 70, 0.1), (12, 60, 9, 0.2),
     (3, 257, 5, 0.0), (13, 5, 2, 0.0)])
 def test_predict_tiles_match_the_walk(hip, orc, depth, n_features, n_trees, p_leaf):
-    """Batches from 4,096 rows walk trees from LDS tiles (64, 256 or 1,024 rows per
+    """Batches from 2,048 rows walk trees from LDS tiles (64, 256 or 1,024 rows per
     workgroup); smaller ones, more than 256 features and trees past a tile walk from
     memory.  Every row is bit-equal to the oracle's walk in each."""
     rng = np.random.default_rng([depth, n_features, n_trees])
@@ -239,8 +239,8 @@ def test_predict_tiles_match_the_walk(hip, orc, depth, n_features, n_trees, p_le
         inner = t["feature"] >= 0
         t["bin"][inner] = np.maximum(t["bin"][inner], nb[t["feature"][inner]].astype(np.uint32) - 1)  # past every cut
     p = hip.Predictor(trees, nb, 0.1, -0.5)
-    for n in (1, 33, 1_025, 4_095, 4_097, 131_073, 524_289):
-        if n > 5_000 and (n_trees > 40 or n_features > 30):
+    for n in (1, 33, 1_025, 2_047, 2_049, 20_001, 131_073, 262_145):
+        if n > 3_000 and (n_trees > 40 or n_features > 30):
             continue
         rows = (rng.random((n, n_features)) * nb).astype(np.uint8)
         dev = p.predict(rows)
