@@ -3,7 +3,8 @@
 // Data layout in HBM (one context = one resident training set):
 //   plane0   u8 [N][Fs]   pristine bin plane, original row order (Fs = F rounded up to 4)
 //   work0/1  u8 [N][Fs]   ping-pong planes: rows physically partitioned per node, each
-//                         node's rows one contiguous segment, ascending original order
+//                         node's rows one contiguous segment, ascending original order;
+//                         u32 [N] row ids of plane0 in that order for rows wider than 64 B
 //   gh0      gradient pairs in original order (f32x2, or one packed u32 when quantized:
 //                         high 16 bits int16 g in [-127,127], low 16 bits uint16 h)
 //   ghw0/1   gradient pairs travelling with the partitioned rows
@@ -40,9 +41,8 @@ constexpr u32 kHistGroupMax = 4;
 constexpr u32 kPartChunk  = 4096;  // rows per partition work unit
 constexpr u32 kCursorStride = 16;  // u32 between the class cursors of four-way partitions (64 B)
 constexpr u32 kCursorMinOps = 8;   // four-way ops of a level from which tiles reserve their runs
-// Rows wider than 64 bytes: partition chunks shrink (powers of two, at least 64 rows) to
-// about this many bytes, so a level of wide rows still has many chunks.
-constexpr u64 kPartChunkBytes = 256u * 1024u;
+// Rows wider than 64 bytes (only ids and gradient words move): rows per partition chunk.
+constexpr u32 kWideChunk = 1024;
 // Leafwise rounds partition one leaf and build one child's histogram; the work units are
 // sized to the leaf so that a small leaf is still spread over many workgroups: partition
 // chunks of kLwMinChunk..kPartChunk rows, about kLwChunkTarget of them, and histogram
@@ -99,6 +99,8 @@ struct SplitRec {
 };
 static_assert(sizeof(SplitRec) == 96, "SplitRec");
 
+constexpr u32 kFusedUnit = 0xFFFFFFFEu; // HistChunk::route
+
 // A histogram work unit: rows [begin, end) of one node's segment, or of its parent's
 // segment when the node's rows have not been moved yet (route != kNone): then only the
 // rows that the parent's split (ops[route]) sends to `side` (0 left, 1 right) count.
@@ -107,8 +109,9 @@ struct HistChunk {
     u32 src;   // which plane/gh buffer holds the rows
     u32 begin, end;
     u32 part;  // partial index, or kNone when the chunk is the node's only one
-    u32 route = kNone; // PartOp index of the parent's split, kNone: every row counts
-    u32 side = 0;
+    u32 route = kNone; // PartOp index of the parent's split, kNone: every row counts; kFusedUnit (wide
+                       // rows): the node's only unit, its sibling (slot `wide`) is completed with it
+    u32 side = 0;      // kFusedUnit: the parent's slot
     u32 wide = 0;      // quantized partial format: 1 wide (g, h, count planes), 0 packed 64-bit cells
 };
 
@@ -122,7 +125,8 @@ struct FinishOp {
     u32 small_off, small_cnt, src; // rows the units scan (the parent's segment when routed)
     u32 route = kNone, side = 0; // HistChunk::route / side of the units
     u32 wide = 0;                // HistChunk::wide of the units
-    u32 pad[2];
+    u32 fused = 0;               // the histogram kernel completes both children (kFusedUnit)
+    u32 pad;
 };
 static_assert(sizeof(FinishOp) == 64, "FinishOp");
 

@@ -243,12 +243,22 @@ struct bh_context {
     std::vector<float> iter_ms;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 
-    // Features per histogram slice: all of them up to 64, else up to 128, as long as the
-    // slice's LDS cells fit 128 KiB (8 B per quantized cell, 16 B per FP32 g / h pair).
+    // Features per histogram slice: all of them up to 64, as long as the slice's LDS cells
+    // fit 128 KiB (8 B per quantized cell, 16 B per FP32 g / h pair).  Wide rows: 128 or 64
+    // features (a line of the row or half of one) while two workgroups share a CU's LDS,
+    // else the most (a power of two) that one can hold.
     u32 hist_fsl() const
     {
         u32 const cell = quant ? 8u : 16u;
-        u32 f = F <= 64 ? round_up4(F) : 128u;
+        if (Fs > 64) {
+            size_t const per = static_cast<size_t>(SB | 1u) * cell;
+            for (u32 f : {128u, 64u})
+                if (f * per <= (80u << 10)) return f;
+            u32 f = 64;
+            while (f > 4 && f * per > (136u << 10)) f /= 2;
+            return f;
+        }
+        u32 f = round_up4(F);
         while (f > 4 && static_cast<size_t>(f) * SB * cell > (128u << 10)) f -= 4;
         return f;
     }
@@ -1001,8 +1011,9 @@ static int alloc_plane(bh_context *c, uint64_t n_rows, uint32_t n_features, cons
     c->n_bins.assign(n_bins, n_bins + n_features);
     size_t const bytes = static_cast<size_t>(n_rows) * c->Fs;
     HIP_TRY(hipMalloc(&c->plane0, bytes + kTailPadBytes));
-    HIP_TRY(hipMalloc(&c->work[0], bytes + kTailPadBytes));
-    HIP_TRY(hipMalloc(&c->work[1], bytes + kTailPadBytes));
+    size_t const work_bytes = c->Fs > 64 ? n_rows * sizeof(u32) : bytes; // wide rows: ids
+    HIP_TRY(hipMalloc(&c->work[0], work_bytes + kTailPadBytes));
+    HIP_TRY(hipMalloc(&c->work[1], work_bytes + kTailPadBytes));
     HIP_TRY(hipMemset(c->plane0, 0, bytes + kTailPadBytes));
     HIP_TRY(dalloc(&c->d_nbins, n_features));
     HIP_TRY(hipMemcpy(c->d_nbins, n_bins, n_features * sizeof(u16), hipMemcpyHostToDevice));

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <algorithm>
+#include <type_traits>
 #include "bh_common.hpp"
 #include "bh_device.hpp"
 #include "bh_find.hpp"
@@ -613,6 +614,139 @@ __global__ __launch_bounds__(kHqThreads) void k_hist_q(
     }
 }
 
+// Rows wider than 64 bytes never move: a partition orders 4-byte row ids (the work planes
+// hold them, wide_row_id) and their gradient words, and the histogram reads each row's
+// slice of the pristine plane through the id.  Moving 2,000-byte rows took 0.95 ms of a
+// 1M-row level; ordering the ids takes about 0.03.
+__device__ __forceinline__ u32 const *wide_ids(u32 src, u8 const *pl0, u8 const *pl1)
+{
+    return src == kSrcPlane0 ? nullptr : reinterpret_cast<u32 const *>(src == 0 ? pl0 : pl1);
+}
+__device__ __forceinline__ u32 wide_row_id(u32 const *ids, u32 r) { return ids ? ids[r] : r; }
+
+// Histogram build over wide rows (H6, unit contract of k_hist_q / k_hist_fx; FP32 cells are
+// k_hist_fx's fixed-point sums rounded once per unit).  One workgroup per feature slice
+// and unit, slices fastest so a row's lines are read together.  Lane l takes dword
+// d = l mod Dw of row l / Dw.  Feature 4 d + k of the slice has its cells at slot
+// k Dw + d with an odd stride, so the lanes of one atomic instruction start on distinct
+// banks: mostly-zero columns put most lanes on the same bin, which with the plain
+// [feature][bin] order is four bank pairs for 32 dwords (1M x 2,000 root: 1,666 us).
+// A single-unit node's larger sibling (kFusedUnit) is completed here, parent - small, while
+// the cells are in LDS.
+constexpr int kHwUnroll = 8;
+constexpr u32 hist_wide_stride(u32 SB) { return SB | 1u; }
+
+template <bool Q>
+__global__ __launch_bounds__(1024) void k_hist_wide(
+    HistChunk const *__restrict__ chunks, TreeCtl const *__restrict__ ctl,
+    u8 const *__restrict__ pl0, u8 const *__restrict__ pl1, u8 const *__restrict__ plp,
+    void const *__restrict__ gw0, void const *__restrict__ gw1, void const *__restrict__ gwp,
+    u32 Fs, u32 F, u32 SB, u32 sb_magic, u32 fsl, void *__restrict__ partials, void const *__restrict__ hist_cur,
+    void *__restrict__ hist_next, u32 *__restrict__ cnt_next, u32 const *__restrict__ fx)
+{
+    typedef typename std::conditional<Q, u32, float2>::type G;
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned long long *lh = reinterpret_cast<unsigned long long *>(smem);
+    u32 const f_begin = blockIdx.x * fsl;
+    u32 const nf = min(F - f_begin, fsl);
+    u32 const SL = hist_wide_stride(SB);
+    u32 const Dw = (nf + 3u) / 4u; // dwords of the slice per row (<= 32)
+    u32 const R = 64u / Dw;        // rows per wave instruction
+    u32 const lcells = 4u * Dw * SL, cells = nf * SB;
+    u32 const lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, NW = blockDim.x >> 6;
+    u32 const lr = lane / Dw, d = lane - lr * Dw;
+    bool const lane_ok = lr < R;
+    u32 const n_units = ctl->n_hist_chunks;
+    size_t const node_cells = static_cast<size_t>(F) * SB, cell0 = static_cast<size_t>(f_begin) * SB;
+    int const sg = Q ? 0 : static_cast<int>(fx[2]), sh = Q ? 0 : static_cast<int>(fx[3]);
+    unsigned long long *lc[4]; // the lane's four features
+#pragma unroll
+    for (u32 k = 0; k < 4; ++k) lc[k] = lh + (k * Dw + d) * SL;
+    u32 const live = min(4u, nf - min(nf, 4u * d)); // features of the lane's dword inside the slice
+    for (u32 c = blockIdx.y; c < n_units; c += gridDim.y) {
+        HistChunk const ch = chunks[c];
+        for (u32 i = threadIdx.x; i < (Q ? 1u : 2u) * lcells; i += blockDim.x) lh[i] = 0ull;
+        __syncthreads();
+        u32 const *ids = wide_ids(ch.src, pl0, pl1);
+        G const *gh = static_cast<G const *>(ch.src == 0 ? gw0 : (ch.src == 1 ? gw1 : gwp));
+        u8 const *cb = plp + f_begin + 4u * d;
+        u32 const stride = NW * R;
+        auto add = [&](u32 dw, G v) {
+            unsigned long long q0, q1 = 0;
+            if constexpr (Q) {
+                q0 = pack_q(v);
+            } else {
+                q0 = static_cast<unsigned long long>(fx_quant(v.x, sg));
+                q1 = static_cast<unsigned long long>(fx_quant(v.y, sh));
+            }
+#pragma unroll
+            for (u32 k = 0; k < 4; ++k)
+                if (k < live) {
+                    unsigned long long *p = lc[k] + ((dw >> (8u * k)) & 0xFFu);
+                    atomicAdd(p, q0);
+                    if (!Q) atomicAdd(p + lcells, q1);
+                }
+        };
+        if (lane_ok) {
+            u32 r = ch.begin + wave * R + lr;
+            for (; r + (kHwUnroll - 1) * stride < ch.end; r += kHwUnroll * stride) {
+                u32 dw[kHwUnroll], id[kHwUnroll];
+                G v[kHwUnroll];
+#pragma unroll
+                for (int u = 0; u < kHwUnroll; ++u) {
+                    id[u] = wide_row_id(ids, r + u * stride);
+                    v[u] = gh[r + u * stride];
+                }
+#pragma unroll
+                for (int u = 0; u < kHwUnroll; ++u)
+                    dw[u] = *reinterpret_cast<u32 const *>(cb + static_cast<size_t>(id[u]) * Fs);
+#pragma unroll
+                for (int u = 0; u < kHwUnroll; ++u) add(dw[u], v[u]);
+            }
+            for (; r < ch.end; r += stride)
+                add(*reinterpret_cast<u32 const *>(cb + static_cast<size_t>(wide_row_id(ids, r)) * Fs), gh[r]);
+        }
+        __syncthreads();
+        for (u32 i = threadIdx.x; i < cells; i += blockDim.x) {
+            u32 const fl = __umulhi(i, sb_magic), b = i - fl * SB; // i / SB
+            unsigned long long const *p = lh + ((fl & 3u) * Dw + (fl >> 2)) * SL + b;
+            if (ch.part != kNone) {
+                size_t const o = static_cast<size_t>(ch.part) * node_cells + cell0 + i;
+                if constexpr (Q)
+                    static_cast<u64 *>(partials)[o] = p[0];
+                else
+                    static_cast<float2 *>(partials)[o] = make_float2(fx_dequant(static_cast<long long>(p[0]), sg),
+                                                                     fx_dequant(static_cast<long long>(p[lcells]), sh));
+                continue;
+            }
+            size_t const o = static_cast<size_t>(ch.slot) * node_cells + cell0 + i;
+            bool const fused = ch.route == kFusedUnit;
+            size_t const lo = static_cast<size_t>(ch.wide) * node_cells + cell0 + i;
+            size_t const po = static_cast<size_t>(ch.side) * node_cells + cell0 + i;
+            if constexpr (Q) {
+                longlong2 *dst = static_cast<longlong2 *>(hist_next);
+                longlong2 const s = make_longlong2(unpack_g(p[0]), unpack_h(p[0]));
+                dst[o] = s;
+                if (cnt_next) cnt_next[o] = unpack_cnt(p[0]);
+                if (fused) {
+                    longlong2 const q = static_cast<longlong2 const *>(hist_cur)[po];
+                    dst[lo] = make_longlong2(q.x - s.x, q.y - s.y);
+                }
+            } else {
+                float2 *dst = static_cast<float2 *>(hist_next);
+                float2 const s = make_float2(fx_dequant(static_cast<long long>(p[0]), sg),
+                                             fx_dequant(static_cast<long long>(p[lcells]), sh));
+                dst[o] = s;
+                if (fused) {
+                    float2 const q = static_cast<float2 const *>(hist_cur)[po];
+                    dst[lo] = make_float2(q.x - s.x, q.y - s.y);
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
 // Quantized histogram, rotated row-dword lanes (rows of at most 64 bytes, all features in
 // one slice, single 8192-row sub-units; same contract as k_hist_q otherwise).  Loads are
 // k_hist_q's: lane (r, d) reads dword d of row r, so one wave load is 64 / Dw whole rows
@@ -1035,6 +1169,7 @@ __global__ void k_finish(FinishOp const *__restrict__ ops, TreeCtl const *__rest
     u32 const n_ops = ctl->n_finish;
     for (u32 o = blockIdx.y; o < n_ops; o += gridDim.y) {
         FinishOp const op = ops[o];
+        if (op.fused) continue; // the histogram kernel completed both children
         for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < node_cells; i += gridDim.x * blockDim.x) {
             if (Q) {
                 i64 *nx = reinterpret_cast<i64 *>(hist_next);
@@ -1150,6 +1285,7 @@ __global__ __launch_bounds__(256) void k_finish_q(FinishOp const *__restrict__ o
     u32 const n_tiles = (node_cells + kFqCells - 1) / kFqCells;
     for (u32 o = blockIdx.y; o < n_ops; o += gridDim.y) {
         FinishOp const op = ops[o];
+        if (op.fused) continue; // the histogram kernel completed both children
         i64 *nx = reinterpret_cast<i64 *>(hist_next);
         for (u32 tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
             u32 const pi_ = tile * kFqCells + j;          // cell index in the partials' order
@@ -1441,7 +1577,7 @@ __global__ __launch_bounds__(1024) void k_part_scan(
     TreeCtl *__restrict__ ctl, NodeInfo const *__restrict__ front, NodeInfo *__restrict__ next,
     SplitRec const *__restrict__ splits, DevNode *__restrict__ tree, HistChunk *__restrict__ hch,
     FinishOp *__restrict__ fops, GrowCfg cfg, double const *__restrict__ scales, u32 is_last,
-    u32 oblivious)
+    u32 oblivious, u32 fuse)
 {
     __shared__ u32 scratch[1024];
     __shared__ u32 s_run, s_alive, s_hch, s_parts;
@@ -1555,6 +1691,7 @@ __global__ __launch_bounds__(1024) void k_part_scan(
                 fo.small_off = left_small ? L.off : R.off;
                 fo.small_cnt = small_cnt;
                 fo.src = op.dst;
+                fo.fused = fuse && n_units == 1u ? 1u : 0u;
                 fops[rank] = fo;
             }
         }
@@ -1578,6 +1715,11 @@ __global__ __launch_bounds__(1024) void k_part_scan(
             hc.begin = fo.small_off + k * kHistChunk;
             hc.end = fo.small_off + min(fo.small_cnt, (k + 1) * kHistChunk);
             hc.part = fo.part_count ? fo.part_first + k : kNone;
+            if (fo.fused) {
+                hc.route = kFusedUnit;
+                hc.wide = fo.large_slot;
+                hc.side = fo.parent_slot;
+            }
             hch[c] = hc;
         }
     }
@@ -1617,85 +1759,106 @@ __device__ __forceinline__ bool chunk_fits(PartOp const &op, PartChunk const &ch
            (ch.begin - left_before) + (rows - n_left_chunk) <= op.cnt - op.n_left;
 }
 
-constexpr u32 kCopyRows = 8;
+// Partition of wide rows: their ids and gradient words (see wide_row_id).  A chunk is at
+// most kWideChunk rows, every thread's rows in flight at once: the routing bytes are one
+// random line each.
+constexpr u32 kWideRows = kWideChunk / 256;
 
-__global__ __launch_bounds__(256) void k_part_scatter(
+__device__ __forceinline__ u32 wide_route(PartOp const &op, PartChunk const &ch, u32 const *ids,
+                                          u8 const *__restrict__ plane, u32 Fs, u32 (&id)[kWideRows])
+{
+    u32 const rows = ch.end - ch.begin;
+    u32 b[kWideRows], bits = 0;
+#pragma unroll
+    for (u32 u = 0; u < kWideRows; ++u) {
+        u32 const k = threadIdx.x + u * 256u;
+        id[u] = k < rows ? wide_row_id(ids, op.off + ch.begin + k) : 0u;
+    }
+#pragma unroll
+    for (u32 u = 0; u < kWideRows; ++u) b[u] = plane[static_cast<size_t>(id[u]) * Fs + op.feature];
+#pragma unroll
+    for (u32 u = 0; u < kWideRows; ++u)
+        if (threadIdx.x + u * 256u < rows && routes_left(b[u], op.last_bin, op.bin, op.default_left)) bits |= 1u << u;
+    return bits; // bit u: row threadIdx.x + 256 u goes left
+}
+
+__global__ __launch_bounds__(256) void k_part_count_wide(PartChunk const *__restrict__ pch,
+                                                         PartOp const *__restrict__ ops,
+                                                         TreeCtl const *__restrict__ ctl, u8 const *__restrict__ pl0,
+                                                         u8 const *__restrict__ pl1, u8 const *__restrict__ plp, u32 Fs,
+                                                         u32 *__restrict__ chunk_left)
+{
+    __shared__ u32 red[4];
+    u32 const n = ctl->n_part_chunks;
+    for (u32 c = blockIdx.x; c < n; c += gridDim.x) {
+        PartChunk const ch = pch[c];
+        PartOp const op = ops[ch.op];
+        u32 id[kWideRows];
+        u32 cnt = __popc(wide_route(op, ch, wide_ids(op.src, pl0, pl1), plp, Fs, id));
+        for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = cnt;
+        __syncthreads();
+        if (threadIdx.x == 0) chunk_left[c] = red[0] + red[1] + red[2] + red[3];
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(256) void k_part_scatter_wide(
     PartChunk const *__restrict__ pch, PartOp const *__restrict__ ops, TreeCtl const *__restrict__ ctl,
     u8 const *__restrict__ pl0, u8 const *__restrict__ pl1, u8 const *__restrict__ plp,
     void const *__restrict__ gw0, void const *__restrict__ gw1, void const *__restrict__ gwp,
     u8 *__restrict__ out0, u8 *__restrict__ out1, void *__restrict__ go0, void *__restrict__ go1, u32 Fs,
-    u32 gh_bytes, u32 tpr_log2, u32 const *__restrict__ chunk_left, TreeCtl *ctl_err)
+    u32 gh_bytes, u32 const *__restrict__ chunk_left, TreeCtl *ctl_err)
 {
-    __shared__ u32 dest[kPartChunk];
-    __shared__ u32 scratch[256];
-    constexpr u32 RPT = kPartChunk / 256; // rows per thread
+    __shared__ u32 s_w[kWideRows][4], s_sum[4];
     u32 const n = ctl->n_part_chunks;
-    u32 const D = Fs / 4u;
-    u32 const tpr = 1u << tpr_log2;
+    u32 const lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     for (u32 c = blockIdx.x; c < n; c += gridDim.x) {
         PartChunk const ch = pch[c];
         PartOp const op = ops[ch.op];
         if (!op.alive) continue; // uniform across the block
-        u8 const *plane = op.src == 0 ? pl0 : (op.src == 1 ? pl1 : plp);
-        u8 const *gin = reinterpret_cast<u8 const *>(op.src == 0 ? gw0 : (op.src == 1 ? gw1 : gwp));
-        u8 *oplane = op.dst == 0 ? out0 : out1;
-        u8 *gout = reinterpret_cast<u8 *>(op.dst == 0 ? go0 : go1);
+        void const *gin = op.src == 0 ? gw0 : (op.src == 1 ? gw1 : gwp);
+        u32 *oid = reinterpret_cast<u32 *>(op.dst == 0 ? out0 : out1);
+        void *gout = op.dst == 0 ? go0 : go1;
         u32 const rows = ch.end - ch.begin;
-        u32 const r0 = threadIdx.x * RPT;
-        u32 bits = 0;
-        for (u32 k = 0; k < RPT; ++k) {
-            u32 const r = r0 + k;
-            if (r < rows) {
-                u32 const b = plane[static_cast<size_t>(op.off + ch.begin + r) * Fs + op.feature];
-                if (routes_left(b, op.last_bin, op.bin, op.default_left)) bits |= 1u << k;
-            }
+        u32 id[kWideRows], rank[kWideRows];
+        u32 const bits = wide_route(op, ch, wide_ids(op.src, pl0, pl1), plp, Fs, id);
+        __syncthreads(); // the previous chunk is done with s_w
+#pragma unroll
+        for (u32 u = 0; u < kWideRows; ++u) {
+            u64 const bal = __ballot((bits >> u) & 1u);
+            rank[u] = static_cast<u32>(__popcll(bal & ((1ull << lane) - 1ull)));
+            if (lane == 0) s_w[u][wave] = static_cast<u32>(__popcll(bal));
         }
-        u32 tot;
-        u32 const pre = block_exscan(__popc(bits), scratch, &tot);
+        __syncthreads();
+        u32 tot = 0;
+#pragma unroll
+        for (u32 u = 0; u < kWideRows; ++u)
+#pragma unroll
+            for (u32 k = 0; k < 4; ++k) {
+                if (k == wave) rank[u] += tot;
+                tot += s_w[u][k];
+            }
         u32 left_before = ch.left_before;
         if (chunk_left) {
-            left_before = chunk_prefix(chunk_left, op.chunk_first, c, scratch + 64);
+            left_before = chunk_prefix(chunk_left, op.chunk_first, c, s_sum);
             if (!chunk_fits(op, ch, left_before, tot)) {
                 if (threadIdx.x == 0) atomicExch(&ctl_err->part_error, 1u);
                 continue; // uniform across the block
             }
         }
-        u32 lpos = op.off + left_before + pre;
-        u32 rpos = op.off + op.n_left + (ch.begin + r0 - left_before - pre);
-        for (u32 k = 0; k < RPT; ++k) {
-            u32 const r = r0 + k;
-            if (r < rows) dest[r] = ((bits >> k) & 1u) ? lpos++ : rpos++;
-        }
-        __syncthreads();
-        // Row bytes: tpr threads per row, dword granularity, kCopyRows rows' loads in
-        // flight per thread (a wide row is a long latency chain otherwise).
-        u32 const rows_per_pass = 256u >> tpr_log2;
-        u32 const sub = threadIdx.x & (tpr - 1u), rsub = threadIdx.x >> tpr_log2;
-        size_t const sbase = static_cast<size_t>(op.off) + ch.begin;
-        for (u32 r0 = 0; r0 < rows; r0 += rows_per_pass * kCopyRows) {
-            for (u32 dw = sub; dw < D; dw += tpr) {
-                u32 v[kCopyRows];
 #pragma unroll
-                for (u32 u = 0; u < kCopyRows; ++u) {
-                    u32 const r = r0 + rsub + u * rows_per_pass;
-                    v[u] = r < rows ? reinterpret_cast<u32 const *>(plane + (sbase + r) * Fs)[dw] : 0u;
-                }
-#pragma unroll
-                for (u32 u = 0; u < kCopyRows; ++u) {
-                    u32 const r = r0 + rsub + u * rows_per_pass;
-                    if (r < rows) reinterpret_cast<u32 *>(oplane + static_cast<size_t>(dest[r]) * Fs)[dw] = v[u];
-                }
-            }
+        for (u32 u = 0; u < kWideRows; ++u) {
+            u32 const k = threadIdx.x + u * 256u;
+            if (k >= rows) continue;
+            size_t const src = static_cast<size_t>(op.off) + ch.begin + k;
+            // left rows keep their order from off + left_before, right rows from off + n_left
+            u32 const dst = op.off + ((bits >> u) & 1u ? left_before + rank[u]
+                                                       : op.n_left + (ch.begin - left_before) + (k - rank[u]));
+            oid[dst] = id[u];
+            if (gh_bytes == 8) static_cast<uint2 *>(gout)[dst] = static_cast<uint2 const *>(gin)[src];
+            else static_cast<u32 *>(gout)[dst] = static_cast<u32 const *>(gin)[src];
         }
-        // Gradient pairs.
-        for (u32 r = threadIdx.x; r < rows; r += 256u) {
-            size_t const s = static_cast<size_t>(op.off + ch.begin + r);
-            if (gh_bytes == 8)
-                reinterpret_cast<uint2 *>(gout)[dest[r]] = reinterpret_cast<uint2 const *>(gin)[s];
-            else
-                reinterpret_cast<u32 *>(gout)[dest[r]] = reinterpret_cast<u32 const *>(gin)[s];
-        }
-        __syncthreads();
     }
 }
 
@@ -2756,9 +2919,13 @@ __global__ __launch_bounds__(256) void k_bern_gather(TreeCtl const *__restrict__
             __syncthreads();
             if (keep) {
                 size_t const dst = pre + static_cast<u32>(__popcll(bal & ((1ull << lane) - 1ull)));
-                u32 const *src = reinterpret_cast<u32 const *>(plane + static_cast<size_t>(r) * Fs);
-                u32 *o = reinterpret_cast<u32 *>(out_plane + dst * Fs);
-                for (u32 d = 0; d < D; ++d) o[d] = src[d];
+                if (D > 16u) { // wide rows: the id
+                    reinterpret_cast<u32 *>(out_plane)[dst] = r;
+                } else {
+                    u32 const *src = reinterpret_cast<u32 const *>(plane + static_cast<size_t>(r) * Fs);
+                    u32 *o = reinterpret_cast<u32 *>(out_plane + dst * Fs);
+                    for (u32 d = 0; d < D; ++d) o[d] = src[d];
+                }
                 if (gh_bytes == 8) reinterpret_cast<uint2 *>(out_gh)[dst] = reinterpret_cast<uint2 const *>(gh)[r];
                 else reinterpret_cast<u32 *>(out_gh)[dst] = reinterpret_cast<u32 const *>(gh)[r];
             }
@@ -2844,9 +3011,13 @@ __global__ void k_gather_rows(u8 const *__restrict__ plane, u32 Fs, void const *
     for (u64 i = blockIdx.x * static_cast<u64>(blockDim.x) + threadIdx.x; i < n;
          i += static_cast<u64>(gridDim.x) * blockDim.x) {
         u32 const r = rows[i];
-        u32 const *src = reinterpret_cast<u32 const *>(plane + static_cast<size_t>(r) * Fs);
-        u32 *dst = reinterpret_cast<u32 *>(out_plane + i * Fs);
-        for (u32 d = 0; d < D; ++d) dst[d] = src[d];
+        if (D > 16u) { // wide rows: the id
+            reinterpret_cast<u32 *>(out_plane)[i] = r;
+        } else {
+            u32 const *src = reinterpret_cast<u32 const *>(plane + static_cast<size_t>(r) * Fs);
+            u32 *dst = reinterpret_cast<u32 *>(out_plane + i * Fs);
+            for (u32 d = 0; d < D; ++d) dst[d] = src[d];
+        }
         if (gh_is_row_id) {
             if (gh_bytes == 8) reinterpret_cast<uint2 *>(out_gh)[i] = make_uint2(r, 0u);
             else reinterpret_cast<u32 *>(out_gh)[i] = r;
@@ -3103,8 +3274,18 @@ u32 hist_transpose_F(bool q, u32 Fs, u32 F, bool group)
 hipError_t launch_hist(hipStream_t s, bool q, HistChunk const *chunks, TreeCtl const *ctl, u8 const *pl0,
                        u8 const *pl1, u8 const *plp, void const *g0, void const *g1, void const *gp, u32 Fs, u32 F,
                        u32 SB, u32 fsl, u32 n_waves, u32 grid_x, void *partials, void *hist_next, u32 const *fx,
-                       u32 *cnt_next, PartOp const *routes, bool group)
+                       u32 *cnt_next, PartOp const *routes, bool group, void const *hist_cur)
 {
+    if (Fs > 64u) {
+        if (!q && !fx) return hipErrorInvalidValue;
+        size_t const wlds = static_cast<size_t>((fsl + 3u) / 4u * 4u) * hist_wide_stride(SB) * (q ? 8u : 16u);
+        dim3 const wgrid((F + fsl - 1) / fsl, grid_x);
+        u32 const magic = static_cast<u32>(((1ull << 32) + SB - 1u) / SB); // exact quotients below 2^16 cells
+        hipLaunchKernelGGL(q ? k_hist_wide<true> : k_hist_wide<false>, wgrid, dim3(t_tune.hist_threads), wlds, s, chunks,
+                           ctl, pl0, pl1, plp, g0, g1, gp, Fs, F, SB, magic, fsl, partials, hist_cur, hist_next,
+                           cnt_next, fx);
+        return hipGetLastError();
+    }
     // group: units may span several 8192-row sub-units (the row-dword and row-in-lane
     // quantized kernels add each sub-unit into the unit's cells; the feature-in-lane one
     // takes single sub-units only).
@@ -3205,6 +3386,8 @@ hipError_t set_hist_lds_limits()
     raise_lds(reinterpret_cast<void const *>(&k_hist_q2), max_shared);
     raise_lds(reinterpret_cast<void const *>(&k_hist_q5), max_shared);
     raise_lds(reinterpret_cast<void const *>(&k_hist_fx), max_shared);
+    raise_lds(reinterpret_cast<void const *>(&k_hist_wide<true>), max_shared);
+    raise_lds(reinterpret_cast<void const *>(&k_hist_wide<false>), max_shared);
     raise_lds(reinterpret_cast<void const *>(&k_find<true, false>), max_shared);
     raise_lds(reinterpret_cast<void const *>(&k_find<false, false>), max_shared);
     raise_lds(reinterpret_cast<void const *>(&k_find<true, true>), max_shared);
@@ -3267,30 +3450,28 @@ void launch_plan_level(hipStream_t s, NodeInfo const *front, SplitRec const *spl
                        scales, dst, chunk_rows);
 }
 
-u32 part_chunk_rows(u32 Fs)
-{
-    if (Fs <= 64) return kPartChunk;
-    u32 r = kPartChunk;
-    while (r > 64u && static_cast<u64>(r) * Fs > kPartChunkBytes) r >>= 1;
-    return r;
-}
+u32 part_chunk_rows(u32 Fs) { return Fs <= 64 ? kPartChunk : kWideChunk; }
 
 void launch_part_count(hipStream_t s, PartChunk const *pch, PartOp const *ops, TreeCtl const *ctl, u8 const *pl0,
                        u8 const *pl1, u8 const *plp, u32 Fs, u32 *chunk_left, u32 grid)
 {
-    hipLaunchKernelGGL(k_part_count, dim3(grid), dim3(256), 0, s, pch, ops, ctl, pl0, pl1, plp, Fs, chunk_left);
+    if (Fs > 64)
+        hipLaunchKernelGGL(k_part_count_wide, dim3(grid), dim3(256), 0, s, pch, ops, ctl, pl0, pl1, plp, Fs,
+                           chunk_left);
+    else
+        hipLaunchKernelGGL(k_part_count, dim3(grid), dim3(256), 0, s, pch, ops, ctl, pl0, pl1, plp, Fs, chunk_left);
 }
 
 void launch_part_scan(hipStream_t s, bool q, PartOp *ops, PartChunk *pch, u32 const *chunk_left, TreeCtl *ctl,
                       NodeInfo const *front, NodeInfo *next, SplitRec const *splits, DevNode *tree, HistChunk *hch,
-                      FinishOp *fops, GrowCfg const &cfg, double const *scales, u32 is_last, u32 oblivious)
+                      FinishOp *fops, GrowCfg const &cfg, double const *scales, u32 is_last, u32 oblivious, u32 fuse)
 {
     if (q)
         hipLaunchKernelGGL(k_part_scan<true>, dim3(1), dim3(1024), 0, s, ops, pch, chunk_left, ctl, front, next,
-                           splits, tree, hch, fops, cfg, scales, is_last, oblivious);
+                           splits, tree, hch, fops, cfg, scales, is_last, oblivious, fuse);
     else
         hipLaunchKernelGGL(k_part_scan<false>, dim3(1), dim3(1024), 0, s, ops, pch, chunk_left, ctl, front, next,
-                           splits, tree, hch, fops, cfg, scales, is_last, oblivious);
+                           splits, tree, hch, fops, cfg, scales, is_last, oblivious, fuse);
 }
 
 void launch_part_scatter(hipStream_t s, PartChunk const *pch, PartOp const *ops, TreeCtl const *ctl,
@@ -3310,10 +3491,8 @@ void launch_part_scatter(hipStream_t s, PartChunk const *pch, PartOp const *ops,
                            const_cast<TreeCtl *>(ctl));
         return;
     }
-    u32 tl = 0;
-    while ((1u << tl) < D && tl < 8) ++tl;
-    hipLaunchKernelGGL(k_part_scatter, dim3(grid), dim3(256), 0, s, pch, ops, ctl, pl0, pl1, plp, g0, g1, gp, o0,
-                       o1, go0, go1, Fs, gh_bytes, tl, chunk_left, const_cast<TreeCtl *>(ctl));
+    hipLaunchKernelGGL(k_part_scatter_wide, dim3(grid), dim3(256), 0, s, pch, ops, ctl, pl0, pl1, plp, g0, g1, gp, o0,
+                       o1, go0, go1, Fs, gh_bytes, chunk_left, const_cast<TreeCtl *>(ctl));
 }
 
 u32 scatter_tile_rows(u32 Fs, u32 gh_bytes)

@@ -26,7 +26,8 @@ void launch_quant_from(hipStream_t s, float2 const *gh, u64 n, u32 *maxbits, u64
 hipError_t launch_hist(hipStream_t s, bool q, HistChunk const *chunks, TreeCtl const *ctl, u8 const *pl0,
                        u8 const *pl1, u8 const *plp, void const *g0, void const *g1, void const *gp, u32 Fs, u32 F,
                        u32 SB, u32 fsl, u32 n_waves, u32 grid_x, void *partials, void *hist_next, u32 const *fx,
-                       u32 *cnt_next = nullptr, PartOp const *routes = nullptr, bool group = false);
+                       u32 *cnt_next = nullptr, PartOp const *routes = nullptr, bool group = false,
+                       void const *hist_cur = nullptr);
 hipError_t set_hist_lds_limits();
 // F when launch_hist with these arguments runs the rotated row-in-lane kernel, whose unit
 // partials are in (bin, feature) order (launch_finish's tF), else 0.
@@ -42,13 +43,16 @@ u32 find_blocks_per_node(u32 F, u32 tile); // workgroups per node for tile-featu
 void launch_plan_level(hipStream_t s, NodeInfo const *front, SplitRec const *splits, TreeCtl *ctl, DevNode *tree,
                        PartOp *ops, PartChunk *pch, u16 const *n_bins, GrowCfg const &cfg, double const *scales,
                        u32 dst, u32 chunk_rows);
+// fuse (wide rows): single-unit nodes name their sibling and parent for the histogram
+// kernel, which then completes both children (launch_hist's hist_cur).
 // Rows per partition chunk for rows of Fs bytes (kPartChunk, smaller for wide rows).
 u32 part_chunk_rows(u32 Fs);
 void launch_part_count(hipStream_t s, PartChunk const *pch, PartOp const *ops, TreeCtl const *ctl, u8 const *pl0,
                        u8 const *pl1, u8 const *plp, u32 Fs, u32 *chunk_left, u32 grid);
 void launch_part_scan(hipStream_t s, bool q, PartOp *ops, PartChunk *pch, u32 const *chunk_left, TreeCtl *ctl,
                       NodeInfo const *front, NodeInfo *next, SplitRec const *splits, DevNode *tree, HistChunk *hch,
-                      FinishOp *fops, GrowCfg const &cfg, double const *scales, u32 is_last, u32 oblivious);
+                      FinishOp *fops, GrowCfg const &cfg, double const *scales, u32 is_last, u32 oblivious,
+                      u32 fuse = 0);
 void launch_part_scatter(hipStream_t s, PartChunk const *pch, PartOp const *ops, TreeCtl const *ctl,
                          u8 const *pl0, u8 const *pl1, u8 const *plp, void const *g0, void const *g1,
                          void const *gp, u8 *o0, u8 *o1, void *go0, void *go1, u32 Fs, u32 gh_bytes, u32 grid,

@@ -531,8 +531,8 @@ struct LwCtl {
 };
 
 // Rows per partition chunk of a leaf of `rows` rows: about kLwChunkTarget chunks,
-// multiples of 256 rows, kLwMinChunk..kPartChunk, and at most cap (the byte-sized chunk
-// of wide rows).
+// multiples of 256 rows, kLwMinChunk..kPartChunk, and at most cap (the chunk of wide
+// rows).
 __device__ __forceinline__ u32 lw_chunk_rows(u32 rows, u32 cap)
 {
     u32 const per = ((rows + kLwChunkTarget - 1u) / kLwChunkTarget + 255u) & ~255u;
@@ -1148,13 +1148,14 @@ void enqueue_levelwise(ExtState &s, hipStream_t st, bool q, GrowView const &v)
         launch_part_count(st, v.pch, v.ops, v.ctl, v.work[0], v.work[1], v.plane0, v.Fs, v.chunk_left,
                           std::max(1u, std::min(v.max_pch, tuning().part_grid)));
         launch_part_scan(st, q, v.ops, v.pch, v.chunk_left, v.ctl, cur, nxt, v.splits, v.tree, v.hch, v.fops, v.gc,
-                         v.scales, last ? 1u : 0u, 1u);
+                         v.scales, last ? 1u : 0u, 1u, v.Fs > 64 ? 1u : 0u);
         if (!last) {
             launch_part_scatter(st, v.pch, v.ops, v.ctl, v.work[0], v.work[1], v.plane0, v.gh[0], v.gh[1], v.gh[2],
                                 v.work[0], v.work[1], const_cast<void *>(v.gh[0]), const_cast<void *>(v.gh[1]), v.Fs,
                                 gh_bytes, std::max(1u, std::min(v.max_pch, tuning().part_grid)));
             launch_hist(st, q, v.hch, v.ctl, v.work[0], v.work[1], v.plane0, v.gh[0], v.gh[1], v.gh[2], v.Fs, v.F,
-                        v.SB, v.fsl, v.waves, std::max(1u, std::min(v.max_hch, 4096u)), v.partials, hnext, v.fx);
+                        v.SB, v.fsl, v.waves, std::max(1u, std::min(v.max_hch, 4096u)), v.partials, hnext, v.fx,
+                        nullptr, nullptr, false, hcur);
             launch_finish(st, q, v.fops, v.ctl, v.partials, hcur, hnext, v.F * v.SB, std::min(width, v.max_ops),
                           nullptr, nullptr, false, hist_transpose_F(q, v.Fs, v.F));
         }
