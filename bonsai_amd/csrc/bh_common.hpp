@@ -120,12 +120,13 @@ struct HistChunk {
 struct FinishOp {
     u32 small_slot, large_slot, parent_slot;
     u32 part_first, part_count; // part_count == 0: written directly (or empty)
-    u32 empty;                  // small child has no rows: zero its histogram
+    u32 empty;                  // small child has no rows: zero its histogram (2: leave it)
     u32 unit_first, unit_count; // histogram units of the small child
     u32 small_off, small_cnt, src; // rows the units scan (the parent's segment when routed)
     u32 route = kNone, side = 0; // HistChunk::route / side of the units
     u32 wide = 0;                // HistChunk::wide of the units
-    u32 fused = 0;               // the histogram kernel completes both children (kFusedUnit)
+    u32 fused = 0;               // nothing to do: the histogram kernel completes both children
+                                 // (kFusedUnit), or neither has rows
     u32 pad;
 };
 static_assert(sizeof(FinishOp) == 64, "FinishOp");

@@ -663,6 +663,7 @@ __global__ __launch_bounds__(1024) void k_hist_wide(
 #pragma unroll
     for (u32 k = 0; k < 4; ++k) lc[k] = lh + (k * Dw + d) * SL;
     u32 const live = min(4u, nf - min(nf, 4u * d)); // features of the lane's dword inside the slice
+    bool const whole = (nf & 3u) == 0u;
     for (u32 c = blockIdx.y; c < n_units; c += gridDim.y) {
         HistChunk const ch = chunks[c];
         for (u32 i = threadIdx.x; i < (Q ? 1u : 2u) * lcells; i += blockDim.x) lh[i] = 0ull;
@@ -681,30 +682,52 @@ __global__ __launch_bounds__(1024) void k_hist_wide(
             }
 #pragma unroll
             for (u32 k = 0; k < 4; ++k)
-                if (k < live) {
+                if (whole || k < live) {
                     unsigned long long *p = lc[k] + ((dw >> (8u * k)) & 0xFFu);
                     atomicAdd(p, q0);
                     if (!Q) atomicAdd(p + lcells, q1);
                 }
         };
         if (lane_ok) {
+            // The next step's row dwords and the ids of the one after are in flight while
+            // a step's rows are added (rows past the end read the last row, unused).
             u32 r = ch.begin + wave * R + lr;
-            for (; r + (kHwUnroll - 1) * stride < ch.end; r += kHwUnroll * stride) {
-                u32 dw[kHwUnroll], id[kHwUnroll];
-                G v[kHwUnroll];
+            u32 const last = ch.end - 1u, span = kHwUnroll * stride;
+            u32 id[kHwUnroll], dw[kHwUnroll];
+            G v[kHwUnroll];
+            auto get_ids = [&](u32 r0) {
+#pragma unroll
+                for (int u = 0; u < kHwUnroll; ++u) id[u] = wide_row_id(ids, min(r0 + u * stride, last));
+            };
+            auto get_rows = [&](u32 r0) {
 #pragma unroll
                 for (int u = 0; u < kHwUnroll; ++u) {
-                    id[u] = wide_row_id(ids, r + u * stride);
-                    v[u] = gh[r + u * stride];
-                }
-#pragma unroll
-                for (int u = 0; u < kHwUnroll; ++u)
                     dw[u] = *reinterpret_cast<u32 const *>(cb + static_cast<size_t>(id[u]) * Fs);
+                    v[u] = gh[min(r0 + u * stride, last)];
+                }
+            };
+            get_ids(r);
+            get_rows(r);
+            get_ids(r + span);
+            for (; r < ch.end; r += span) {
+                u32 cdw[kHwUnroll];
+                G cv[kHwUnroll];
 #pragma unroll
-                for (int u = 0; u < kHwUnroll; ++u) add(dw[u], v[u]);
+                for (int u = 0; u < kHwUnroll; ++u) {
+                    cdw[u] = dw[u];
+                    cv[u] = v[u];
+                }
+                get_rows(r + span);
+                get_ids(r + 2 * span);
+                if (r + (kHwUnroll - 1) * stride < ch.end) {
+#pragma unroll
+                    for (int u = 0; u < kHwUnroll; ++u) add(cdw[u], cv[u]);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < kHwUnroll; ++u)
+                        if (r + u * stride < ch.end) add(cdw[u], cv[u]);
+                }
             }
-            for (; r < ch.end; r += stride)
-                add(*reinterpret_cast<u32 const *>(cb + static_cast<size_t>(wide_row_id(ids, r)) * Fs), gh[r]);
         }
         __syncthreads();
         for (u32 i = threadIdx.x; i < cells; i += blockDim.x) {
@@ -1221,7 +1244,7 @@ __global__ void k_finish(FinishOp const *__restrict__ ops, TreeCtl const *__rest
                 float2 *nx = reinterpret_cast<float2 *>(hist_next);
                 float2 s = make_float2(0.0F, 0.0F);
                 if (op.empty) {
-                    nx[static_cast<size_t>(op.small_slot) * node_cells + i] = s;
+                    if (op.empty == 1u) nx[static_cast<size_t>(op.small_slot) * node_cells + i] = s;
                 } else if (op.part_count == 0) {
                     s = nx[static_cast<size_t>(op.small_slot) * node_cells + i];
                 } else {
@@ -1355,9 +1378,11 @@ __global__ __launch_bounds__(256) void k_finish_q(FinishOp const *__restrict__ o
                 if (op.empty) {
                     g = h = 0;
                     n = 0;
-                    nx[si * 2] = 0;
-                    nx[si * 2 + 1] = 0;
-                    if (cnt_next) cnt_next[si] = 0;
+                    if (op.empty == 1u) {
+                        nx[si * 2] = 0;
+                        nx[si * 2 + 1] = 0;
+                        if (cnt_next) cnt_next[si] = 0;
+                    }
                 } else if (op.part_count == 0) {
                     g = nx[si * 2];
                     h = nx[si * 2 + 1];
@@ -1691,7 +1716,9 @@ __global__ __launch_bounds__(1024) void k_part_scan(
                 fo.small_off = left_small ? L.off : R.off;
                 fo.small_cnt = small_cnt;
                 fo.src = op.dst;
-                fo.fused = fuse && n_units == 1u ? 1u : 0u;
+                // levelwise: nobody reads an empty node's cells (NodeInfo::cnt 0)
+                if (oblivious && small_cnt == 0) fo.empty = 2u;
+                fo.fused = (fuse && n_units == 1u) || (oblivious && op.cnt == 0) ? 1u : 0u;
                 fops[rank] = fo;
             }
         }

@@ -65,12 +65,21 @@ __device__ __forceinline__ void put_leaf(DevNode *tree, u32 id, float v)
 template <bool Q>
 __global__ __launch_bounds__(64) void k_totals(NodeInfo *__restrict__ front, TreeCtl const *__restrict__ ctl,
                                                void const *__restrict__ hist, u16 const *__restrict__ n_bins, u32 F,
-                                               u32 SB, u8 const *__restrict__ fmask)
+                                               u32 SB, u8 const *__restrict__ fmask, u32 local)
 {
     u32 const i = blockIdx.x;
     if (i >= ctl->n_front || ctl->done) return;
     NodeInfo nd = front[i];
     if (nd.totals_ready) return;
+    if (local && nd.cnt == 0) { // no cells
+        if (threadIdx.x == 0) {
+            nd.itg = nd.ith = 0;
+            nd.tg = nd.th = 0.0F;
+            nd.totals_ready = 1;
+            front[i] = nd;
+        }
+        return;
+    }
     size_t const nc = static_cast<size_t>(F) * SB;
     u32 f0 = 0;
     if (fmask)
@@ -123,22 +132,34 @@ __global__ __launch_bounds__(64) void k_totals(NodeInfo *__restrict__ front, Tre
 // Level (oblivious) finder: HistogramLevelSplitFinder::find (src/split.cpp:164-235,
 // :350-372).  One workgroup per feature.  Frontier nodes are taken in tiles: the tile's
 // prefix sums (fill_prefix: double running sums stored as float, or exact integers) go
-// to LDS, then each (bin, direction) candidate adds the tile's child scores to its
-// running sum in node order; an infeasible node contributes its parent score.
+// to LDS, every (node, bin, direction) child score is computed in parallel, and each
+// (bin, direction) candidate adds the tile's scores to its running sum in node order; an
+// infeasible node contributes its parent score.
+//
+// FP64 bound at deep levels (two divisions per candidate and node; 512 nodes of 2,000
+// features x 64 bins: 720 us when every candidate's thread also ran its divisions in node
+// order, 550 so).  Where every cell comes from the nodes' own rows (local: a grower's level, not a
+// caller's step over histograms it may have summed elsewhere), a node without rows adds
+// exactly 0 to every sum and is left out.  A feature whose missing cells are all empty
+// scans one direction (the other's sums are the same).
 // ---------------------------------------------------------------------------------
-constexpr u32 kLevelTileF32 = 16, kLevelTileQ = 8;
+constexpr u32 kLevelTile = 8;
+constexpr u32 kLevelMaxNodes = 1024; // split levels of a levelwise tree (max_depth <= 11)
+// LDS bytes per bin: the tile's prefix cells and both directions' scores.
+constexpr u32 level_lds_per_bin(bool q) { return kLevelTile * ((q ? 16u : 8u) + 16u); }
 
 template <bool Q>
 __global__ __launch_bounds__(256) void k_find_level(NodeInfo const *__restrict__ front,
                                                     TreeCtl const *__restrict__ ctl, void const *__restrict__ hist,
                                                     u16 const *__restrict__ n_bins, u32 F, u32 SB, GrowCfg cfg,
-                                                    double const *__restrict__ scales, SplitRec *__restrict__ fbest)
+                                                    double const *__restrict__ scales, SplitRec *__restrict__ fbest,
+                                                    u32 local)
 {
+    typedef typename CellT<Q>::T Cell;
     extern __shared__ __align__(16) unsigned char smem[];
     u32 const f = blockIdx.x;
     if (f >= F) return;
     if (ctl->done) return;
-    u32 const TN = Q ? kLevelTileQ : kLevelTileF32;
     u32 const P = ctl->n_front;
     u32 const nb = (cfg.fmask && !cfg.fmask[f]) ? 0u : n_bins[f]; // unselected: no cut
     u32 const ncut = nb >= 2 ? nb - 2 : 0;
@@ -148,116 +169,164 @@ __global__ __launch_bounds__(256) void k_find_level(NodeInfo const *__restrict__
         if (threadIdx.x == 0) fbest[f] = best;
         return;
     }
-    // LDS: per tile node prefix (g, h) over the cut bins + node scalars.
-    float2 *pf = reinterpret_cast<float2 *>(smem);  // F32: [TN][ncut]
-    i64 *pq = reinterpret_cast<i64 *>(smem);        // Q:   [TN][ncut][2]
-    __shared__ double s_ps[kLevelTileF32], s_rg[kLevelTileF32], s_rh[kLevelTileF32], s_mg[kLevelTileF32],
-        s_mh[kLevelTileF32];
-    __shared__ i64 s_itg[kLevelTileF32], s_ith[kLevelTileF32], s_img[kLevelTileF32], s_imh[kLevelTileF32];
+    Cell *s_pre = reinterpret_cast<Cell *>(smem);                       // [kLevelTile][SB] prefix over the cut bins
+    double *s_cs = reinterpret_cast<double *>(s_pre + kLevelTile * SB); // [kLevelTile][candidates]
+    __shared__ double s_ps[kLevelTile], s_rg[kLevelTile], s_rh[kLevelTile], s_mg[kLevelTile], s_mh[kLevelTile];
+    __shared__ i64 s_itg[kLevelTile], s_ith[kLevelTile], s_img[kLevelTile], s_imh[kLevelTile];
     __shared__ double s_sum_parent;
-    __shared__ u32 s_nonempty;
+    __shared__ u32 s_nonempty, s_live, s_wave[4];
+    __shared__ u16 s_list[kLevelMaxNodes];
     size_t const nc = static_cast<size_t>(F) * SB;
+    Cell const *cells = reinterpret_cast<Cell const *>(hist) + static_cast<size_t>(f) * SB;
     double const sg = Q ? scales[0] : 0.0, sh = Q ? scales[1] : 0.0;
-    // Two candidates per thread at most (ncut <= 254): k = threadIdx.x and + 256.
-    double acc[2] = {0.0, 0.0};
+    u32 const lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     if (threadIdx.x == 0) {
         s_sum_parent = 0.0;
         s_nonempty = 0;
+        s_live = 0;
     }
     __syncthreads();
-    for (u32 p0 = 0; p0 < P; p0 += TN) {
-        u32 const tn = min(TN, P - p0);
-        u32 const t = threadIdx.x;
-        if (t < tn) {
-            NodeInfo const nd = front[p0 + t];
-            if (Q) {
-                i64 const *c = reinterpret_cast<i64 const *>(hist) +
-                               (static_cast<size_t>(nd.slot) * nc + static_cast<size_t>(f) * SB) * 2;
-                i64 g = 0, h = 0;
-                for (u32 b = 0; b < ncut; ++b) {
-                    g += c[2 * b];
-                    h += c[2 * b + 1];
-                    pq[(t * ncut + b) * 2] = g;
-                    pq[(t * ncut + b) * 2 + 1] = h;
+    // The nodes with rows, in order, and whether any has a missing cell.
+    for (u32 p0 = 0; p0 < P; p0 += blockDim.x) {
+        u32 const p = p0 + threadIdx.x;
+        NodeInfo nd{};
+        if (p < P) nd = front[p];
+        bool const live = p < P && (!local || nd.cnt != 0);
+        u64 const bal = __ballot(live);
+        if (lane == 0) s_wave[wave] = static_cast<u32>(__popcll(bal));
+        __syncthreads();
+        u32 at = s_live + static_cast<u32>(__popcll(bal & ((1ull << lane) - 1ull)));
+        for (u32 w = 0; w < wave; ++w) at += s_wave[w];
+        if (live) {
+            if (local) s_list[at] = static_cast<u16>(p);
+            Cell const m = cells[static_cast<size_t>(nd.slot) * nc + nb - 1u];
+            if (m.x != 0 || m.y != 0) atomicOr(&s_nonempty, 1u);
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) s_live += s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+        __syncthreads();
+    }
+    u32 const n_live = s_live;
+    auto node_at = [&](u32 i) { return local ? static_cast<u32>(s_list[i]) : i; };
+    // candidate c: bin c, missing left (one direction) or bin c / 2, missing left first
+    bool const one_dir = s_nonempty == 0;
+    u32 const ncand = one_dir ? ncut : 2u * ncut;
+    double acc[2] = {0.0, 0.0}; // candidates threadIdx.x and + 256 (ncut <= 254)
+    for (u32 p0 = 0; p0 < n_live; p0 += kLevelTile) {
+        u32 const tn = min(kLevelTile, n_live - p0);
+        if (Q) {
+            // exact integers: a wave scans a node's cells in parallel
+            for (u32 t = wave; t < tn; t += 4u) {
+                i64 const *c = reinterpret_cast<i64 const *>(cells + static_cast<size_t>(front[node_at(p0 + t)].slot) * nc);
+                i64 *out = reinterpret_cast<i64 *>(s_pre + t * SB);
+                i64 g0 = 0, h0 = 0;
+                for (u32 b0 = 0; b0 < ncut; b0 += 64u) {
+                    u32 const b = b0 + lane;
+                    i64 g = b < ncut ? c[2 * b] : 0, h = b < ncut ? c[2 * b + 1] : 0;
+                    for (int o = 1; o < 64; o <<= 1) {
+                        i64 const ug = __shfl_up(g, o), uh = __shfl_up(h, o);
+                        if (static_cast<int>(lane) >= o) {
+                            g += ug;
+                            h += uh;
+                        }
+                    }
+                    if (b < ncut) {
+                        out[2 * b] = g0 + g;
+                        out[2 * b + 1] = h0 + h;
+                    }
+                    g0 += __shfl(g, 63);
+                    h0 += __shfl(h, 63);
                 }
-                i64 const mg = c[2 * (nb - 1)], mh = c[2 * (nb - 1) + 1];
-                s_img[t] = mg;
-                s_imh[t] = mh;
-                s_itg[t] = nd.itg;
-                s_ith[t] = nd.ith;
-                s_ps[t] = score_of(static_cast<double>(nd.itg) * sg, static_cast<double>(nd.ith) * sh, cfg.l1,
-                                   cfg.l2);
-                if (mg != 0 || mh != 0) atomicOr(&s_nonempty, 1u);
-            } else {
-                float2 const *c = reinterpret_cast<float2 const *>(hist) + static_cast<size_t>(nd.slot) * nc +
-                                  static_cast<size_t>(f) * SB;
+            }
+        } else {
+            // coalesced into LDS, then a thread per node sums in bin order
+            for (u32 k = threadIdx.x; k < tn * ncut; k += blockDim.x) {
+                u32 const t = k / ncut, b = k - t * ncut;
+                s_pre[t * SB + b] = cells[static_cast<size_t>(front[node_at(p0 + t)].slot) * nc + b];
+            }
+            __syncthreads();
+            if (threadIdx.x < tn) {
+                float2 *c = reinterpret_cast<float2 *>(s_pre + threadIdx.x * SB);
                 double g = 0.0, h = 0.0;
                 for (u32 b = 0; b < ncut; ++b) {
                     g = g + c[b].x;
                     h = h + c[b].y;
-                    pf[t * ncut + b] = make_float2(static_cast<float>(g), static_cast<float>(h));
+                    c[b] = make_float2(static_cast<float>(g), static_cast<float>(h));
                 }
-                float2 const m = c[nb - 1];
+            }
+        }
+        if (threadIdx.x < tn) {
+            u32 const t = threadIdx.x;
+            NodeInfo const nd = front[node_at(p0 + t)];
+            Cell const m = cells[static_cast<size_t>(nd.slot) * nc + nb - 1u];
+            if (Q) {
+                s_img[t] = static_cast<i64>(m.x);
+                s_imh[t] = static_cast<i64>(m.y);
+                s_itg[t] = nd.itg;
+                s_ith[t] = nd.ith;
+                s_ps[t] = score_of(static_cast<double>(nd.itg) * sg, static_cast<double>(nd.ith) * sh, cfg.l1, cfg.l2);
+            } else {
                 s_mg[t] = m.x;
                 s_mh[t] = m.y;
                 s_ps[t] = score_of(nd.tg, nd.th, cfg.l1, cfg.l2);
                 s_rg[t] = static_cast<double>(nd.tg) - m.x;
                 s_rh[t] = static_cast<double>(nd.th) - m.y;
-                if (m.x != 0.0F || m.y != 0.0F) atomicOr(&s_nonempty, 1u);
             }
         }
         __syncthreads();
         if (threadIdx.x == 0)
             for (u32 k = 0; k < tn; ++k) s_sum_parent += s_ps[k];
+        for (u32 i = threadIdx.x; i < tn * ncand; i += blockDim.x) {
+            u32 const p = i / ncand, k = i - p * ncand;
+            u32 const b = one_dir ? k : k >> 1;
+            bool const dl = one_dir || (k & 1u) == 0;
+            double cs;
+            bool ok;
+            if (Q) {
+                i64 const *pq = reinterpret_cast<i64 const *>(s_pre + p * SB + b);
+                i64 const lg = pq[0], lh = pq[1];
+                i64 const mg = s_img[p], mh = s_imh[p];
+                i64 const hL = lh + (dl ? mh : 0);
+                i64 const hR = ((s_ith[p] - mh) - lh) + (!dl ? mh : 0);
+                i64 const gL = lg + (dl ? mg : 0);
+                i64 const gR = ((s_itg[p] - mg) - lg) + (!dl ? mg : 0);
+                double const dhL = static_cast<double>(hL) * sh, dhR = static_cast<double>(hR) * sh;
+                ok = !(dhL < cfg.min_child_hess || dhR < cfg.min_child_hess);
+                cs = ok ? score_of(static_cast<double>(gL) * sg, dhL, cfg.l1, cfg.l2) +
+                              score_of(static_cast<double>(gR) * sg, dhR, cfg.l1, cfg.l2)
+                        : 0.0;
+            } else {
+                float2 const lp = reinterpret_cast<float2 const *>(s_pre)[p * SB + b];
+                double const lg = lp.x, lh = lp.y;
+                double const mg = s_mg[p], mh = s_mh[p];
+                double const right_g = s_rg[p] - lg, right_h = s_rh[p] - lh;
+                double const gL = lg + (dl ? mg : 0.0), hL = lh + (dl ? mh : 0.0);
+                double const gR = right_g + (!dl ? mg : 0.0), hR = right_h + (!dl ? mh : 0.0);
+                ok = !(hL < cfg.min_child_hess || hR < cfg.min_child_hess);
+                cs = ok ? score_of(gL, hL, cfg.l1, cfg.l2) + score_of(gR, hR, cfg.l1, cfg.l2) : 0.0;
+            }
+            s_cs[i] = ok ? cs : s_ps[p];
+        }
+        __syncthreads();
         for (u32 s = 0; s < 2; ++s) {
             u32 const k = threadIdx.x + s * blockDim.x;
-            if (k >= 2 * ncut) continue;
-            u32 const b = k >> 1;
-            bool const dl = (k & 1u) == 0;
+            if (k >= ncand) continue;
             double sum = acc[s];
-            for (u32 p = 0; p < tn; ++p) {
-                double cs;
-                bool ok;
-                if (Q) {
-                    i64 const lg = pq[(p * ncut + b) * 2], lh = pq[(p * ncut + b) * 2 + 1];
-                    i64 const mg = s_img[p], mh = s_imh[p];
-                    i64 const hL = lh + (dl ? mh : 0);
-                    i64 const hR = ((s_ith[p] - mh) - lh) + (!dl ? mh : 0);
-                    i64 const gL = lg + (dl ? mg : 0);
-                    i64 const gR = ((s_itg[p] - mg) - lg) + (!dl ? mg : 0);
-                    double const dhL = static_cast<double>(hL) * sh, dhR = static_cast<double>(hR) * sh;
-                    ok = !(dhL < cfg.min_child_hess || dhR < cfg.min_child_hess);
-                    cs = ok ? score_of(static_cast<double>(gL) * sg, dhL, cfg.l1, cfg.l2) +
-                                  score_of(static_cast<double>(gR) * sg, dhR, cfg.l1, cfg.l2)
-                            : 0.0;
-                } else {
-                    float2 const lp = pf[p * ncut + b];
-                    double const lg = lp.x, lh = lp.y;
-                    double const mg = s_mg[p], mh = s_mh[p];
-                    double const right_g = s_rg[p] - lg, right_h = s_rh[p] - lh;
-                    double const gL = lg + (dl ? mg : 0.0), hL = lh + (dl ? mh : 0.0);
-                    double const gR = right_g + (!dl ? mg : 0.0), hR = right_h + (!dl ? mh : 0.0);
-                    ok = !(hL < cfg.min_child_hess || hR < cfg.min_child_hess);
-                    cs = ok ? score_of(gL, hL, cfg.l1, cfg.l2) + score_of(gR, hR, cfg.l1, cfg.l2) : 0.0;
-                }
-                sum += ok ? cs : s_ps[p];
-            }
+            for (u32 p = 0; p < tn; ++p) sum += s_cs[p * ncand + k];
             acc[s] = sum;
         }
         __syncthreads();
     }
-    // Per-feature winner: max gain, earliest (bin, dl=true first); an all-empty missing
-    // cell set scans one direction (identical sums, so the first direction wins anyway).
+    // Per-feature winner: max gain, earliest (bin, dl=true first).
     __shared__ double s_g[256];
     __shared__ u32 s_k[256];
     double bg = 0.0;
     u32 bk = kNone;
     double const sp = s_sum_parent;
-    bool const one_dir = s_nonempty == 0;
     for (u32 s = 0; s < 2; ++s) {
-        u32 const k = threadIdx.x + s * blockDim.x;
-        if (k >= 2 * ncut) continue;
-        if (one_dir && (k & 1u)) continue;
+        u32 const c = threadIdx.x + s * blockDim.x;
+        if (c >= ncand) continue;
+        u32 const k = one_dir ? 2u * c : c; // bin << 1 | missing right
         double const gain = acc[s] - sp;
         if (!(gain > 0.0 && gain >= cfg.min_gain)) continue;
         if (gain > bg || (gain == bg && k < bk)) {
@@ -354,7 +423,7 @@ __global__ __launch_bounds__(1024) void k_plan_oblivious(NodeInfo const *__restr
                                                          void const *__restrict__ hist, u16 const *__restrict__ n_bins,
                                                          u32 F, u32 SB, SplitRec *__restrict__ splits,
                                                          PartOp *__restrict__ ops, PartChunk *__restrict__ pch, u32 dst,
-                                                         u32 is_last, u32 chunk_rows)
+                                                         u32 is_last, u32 chunk_rows, u32 local)
 {
     __shared__ u32 scratch[1024];
     __shared__ u32 s_chunks;
@@ -387,6 +456,9 @@ __global__ __launch_bounds__(1024) void k_plan_oblivious(NodeInfo const *__restr
             SplitRec r = s;
             if (!is_last) {
                 // child sums are only read for leaves made at the last level
+            } else if (local && nd.cnt == 0) { // no cells: every sum is zero
+                r.gL = r.hL = r.gR = r.hR = 0.0;
+                r.igL = r.ihL = r.igR = r.ihR = 0;
             } else if (Q) {
                 i64 const *c = reinterpret_cast<i64 const *>(hist) +
                                (static_cast<size_t>(nd.slot) * nc + static_cast<size_t>(s.feature) * SB) * 2;
@@ -1117,8 +1189,7 @@ void enqueue_levelwise(ExtState &s, hipStream_t st, bool q, GrowView const &v)
                 v.fsl, v.waves, std::max(1u, std::min(v.max_hch, 4096u)), v.partials, v.hist[0], v.fx);
     launch_finish(st, q, v.fops, v.ctl, v.partials, v.hist[1], v.hist[0], v.F * v.SB, 1, nullptr, nullptr, false,
                   hist_transpose_F(q, v.Fs, v.F));
-    u32 const TN = q ? kLevelTileQ : kLevelTileF32;
-    size_t const lds_level = static_cast<size_t>(TN) * v.SB * (q ? 16 : 8);
+    size_t const lds_level = static_cast<size_t>(v.SB) * level_lds_per_bin(q);
     for (u32 d = 0; d < D; ++d) {
         NodeInfo *cur = v.front[d & 1u], *nxt = v.front[(d + 1) & 1u];
         void *hcur = v.hist[d & 1u], *hnext = v.hist[(d + 1) & 1u];
@@ -1126,25 +1197,25 @@ void enqueue_levelwise(ExtState &s, hipStream_t st, bool q, GrowView const &v)
         bool const last = d + 1 == D;
         if (q)
             hipLaunchKernelGGL(k_totals<true>, dim3(width), dim3(64), 0, st, cur, v.ctl, hcur, v.d_nbins, v.F, v.SB,
-                               v.gc.fmask);
+                               v.gc.fmask, 1u);
         else
             hipLaunchKernelGGL(k_totals<false>, dim3(width), dim3(64), 0, st, cur, v.ctl, hcur, v.d_nbins, v.F, v.SB,
-                               v.gc.fmask);
+                               v.gc.fmask, 1u);
         if (q)
             hipLaunchKernelGGL(k_find_level<true>, dim3(v.F), dim3(256), lds_level, st, cur, v.ctl, hcur, v.d_nbins, v.F,
-                               v.SB, v.gc, v.scales, s.feat_best);
+                               v.SB, v.gc, v.scales, s.feat_best, 1u);
         else
             hipLaunchKernelGGL(k_find_level<false>, dim3(v.F), dim3(256), lds_level, st, cur, v.ctl, hcur, v.d_nbins,
-                               v.F, v.SB, v.gc, v.scales, s.feat_best);
+                               v.F, v.SB, v.gc, v.scales, s.feat_best, 1u);
         hipLaunchKernelGGL(k_level_pick, dim3(1), dim3(256), 0, st, s.feat_best, v.F, v.ctl, s.level_splits,
                            s.level_gains, pick);
         if (q)
             hipLaunchKernelGGL(k_plan_oblivious<true>, dim3(1), dim3(1024), 0, st, cur, v.ctl, pick, hcur, v.d_nbins,
-                               v.F, v.SB, v.splits, v.ops, v.pch, d & 1u, last ? 1u : 0u, part_chunk_rows(v.Fs));
+                               v.F, v.SB, v.splits, v.ops, v.pch, d & 1u, last ? 1u : 0u, part_chunk_rows(v.Fs), 1u);
         else
             hipLaunchKernelGGL(k_plan_oblivious<false>, dim3(1), dim3(1024), 0, st, cur, v.ctl, pick, hcur,
                                v.d_nbins, v.F, v.SB, v.splits, v.ops, v.pch, d & 1u, last ? 1u : 0u,
-                               part_chunk_rows(v.Fs));
+                               part_chunk_rows(v.Fs), 1u);
         launch_part_count(st, v.pch, v.ops, v.ctl, v.work[0], v.work[1], v.plane0, v.Fs, v.chunk_left,
                           std::max(1u, std::min(v.max_pch, tuning().part_grid)));
         launch_part_scan(st, q, v.ops, v.pch, v.chunk_left, v.ctl, cur, nxt, v.splits, v.tree, v.hch, v.fops, v.gc,
@@ -1177,28 +1248,27 @@ void enqueue_levelwise(ExtState &s, hipStream_t st, bool q, GrowView const &v)
 void launch_level_find_step(ExtState &s, hipStream_t st, bool q, GrowView const &v, NodeInfo *front, u32 n,
                             void const *hist, SplitRec *pick)
 {
-    u32 const TN = q ? kLevelTileQ : kLevelTileF32;
-    size_t const lds_level = static_cast<size_t>(TN) * v.SB * (q ? 16 : 8);
+    size_t const lds_level = static_cast<size_t>(v.SB) * level_lds_per_bin(q);
     hipLaunchKernelGGL(k_obl_begin, dim3(1), dim3(64), 0, st, v.ctl);
     if (q) {
         hipLaunchKernelGGL(k_totals<true>, dim3(n), dim3(64), 0, st, front, v.ctl, hist, v.d_nbins, v.F, v.SB,
-                           v.gc.fmask);
+                           v.gc.fmask, 0u);
         hipLaunchKernelGGL(k_find_level<true>, dim3(v.F), dim3(256), lds_level, st, front, v.ctl, hist, v.d_nbins,
-                           v.F, v.SB, v.gc, v.scales, s.feat_best);
+                           v.F, v.SB, v.gc, v.scales, s.feat_best, 0u);
     } else {
         hipLaunchKernelGGL(k_totals<false>, dim3(n), dim3(64), 0, st, front, v.ctl, hist, v.d_nbins, v.F, v.SB,
-                           v.gc.fmask);
+                           v.gc.fmask, 0u);
         hipLaunchKernelGGL(k_find_level<false>, dim3(v.F), dim3(256), lds_level, st, front, v.ctl, hist, v.d_nbins,
-                           v.F, v.SB, v.gc, v.scales, s.feat_best);
+                           v.F, v.SB, v.gc, v.scales, s.feat_best, 0u);
     }
     hipLaunchKernelGGL(k_level_pick, dim3(1), dim3(256), 0, st, s.feat_best, v.F, v.ctl, s.level_splits, s.level_gains,
                        pick);
     if (q)
         hipLaunchKernelGGL(k_plan_oblivious<true>, dim3(1), dim3(1024), 0, st, front, v.ctl, pick, hist, v.d_nbins, v.F,
-                           v.SB, v.splits, v.ops, v.pch, 0u, 1u, part_chunk_rows(v.Fs));
+                           v.SB, v.splits, v.ops, v.pch, 0u, 1u, part_chunk_rows(v.Fs), 0u);
     else
         hipLaunchKernelGGL(k_plan_oblivious<false>, dim3(1), dim3(1024), 0, st, front, v.ctl, pick, hist, v.d_nbins,
-                           v.F, v.SB, v.splits, v.ops, v.pch, 0u, 1u, part_chunk_rows(v.Fs));
+                           v.F, v.SB, v.splits, v.ops, v.pch, 0u, 1u, part_chunk_rows(v.Fs), 0u);
 }
 
 // LeafwiseGrower::grow as a launch sequence: the root, then max_leaves - 1 rounds

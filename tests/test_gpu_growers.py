@@ -176,6 +176,38 @@ def test_grow_depthwise_int_50_features(hip, orc, pair):
     assert np.array_equal(lor, rlor)
 
 
+@pytest.mark.parametrize("quantized", [True, False])
+@pytest.mark.parametrize("f,n,depth", [(65, 1025, 3), (127, 3001, 7), (128, 9000, 6), (129, 2047, 9), (257, 900, 8)])
+def test_wide_row_edges(hip, orc, f, n, depth, quantized):
+    """Rows of row ids (over 64 bytes) at slice and chunk edges: feature counts around the
+    histogram's slices, bin counts 2 .. 256 with and without missing cells, levels deep
+    enough for nodes without rows; a levelwise tree, a depthwise tree and one on a row
+    subset, all bit-exact."""
+    rng = np.random.default_rng(f)
+    nb = rng.choice([2, 3, 17, 64, 255, 256], f).astype(np.uint16)
+    bins = np.stack([rng.integers(0, int(b) - (j & 1), n) if b > 2 else np.full(n, j & 1)
+                     for j, b in enumerate(nb)], axis=1).astype(np.uint8)
+    y = (bins[:, 3] > nb[3] // 3).astype(np.float32) + rng.normal(0, 0.3, n).astype(np.float32)
+    g, h = orc.mse_grad(np.zeros(n, np.float32), y)
+    check_levelwise(hip, orc, bins, nb, g, h, depth, quantized)
+    c = orc_cfg(max_depth=depth, min_data=3)
+    for rows in (np.arange(n), np.sort(rng.permutation(n)[:n // 2 + 1])):
+        ctx = ctx_for(hip, bins, nb, quantized=quantized, max_depth=depth, min_data_in_leaf=3)
+        if quantized:
+            gq, hq, sc = ctx.set_gradients(g, h)
+            ref, rlor = orc.grow_depthwise(bins[rows], nb, gq=gq[rows], hq=hq[rows], scales=sc, c=c, mode=HIST_INT)
+        else:
+            ctx.set_gradients(g, h)
+            ref, rlor = orc.grow_depthwise(bins[rows], nb, g=g[rows], h=h[rows], c=c, mode=HIST_F32_FIXED,
+                                           scales=(orc.fx_shift(g), orc.fx_shift(h)))
+        if rows.size < n:
+            ctx.set_row_subset(rows.astype(np.uint32))
+        nodes, lor = ctx.grow_tree()
+        ctx.close()
+        assert_same_tree(nodes, ref)
+        assert np.array_equal(lor[rows], rlor)
+
+
 @pytest.mark.parametrize("grower", ["hip_leafwise", "hip_levelwise"])
 def test_train_graph_equals_eager(hip, orc, tall, grower):
     bins, nb, X, y = tall
