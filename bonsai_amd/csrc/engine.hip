@@ -277,7 +277,21 @@ struct bh_context {
     // sub-units, unless the feature-in-lane layout (single sub-units) is set.  Levels that
     // build the small children only keep single sub-units: their fewer units would leave
     // workgroup slots idle.
-    u32 unit_rows() const { return quant && tune.hist_layout != 1u ? kHistChunk * tune.hist_group : kHistChunk; }
+    u32 unit_rows() const
+    {
+        return quant && tune.hist_layout != 1u && tune.hist_group > 1u ? kHistChunk * tune.hist_group : small_unit();
+    }
+    // Rows per unit of its other levels: kHistChunk, halved down to kHistUnitMin until
+    // the rows make kHistUnitFill units (exact integer sums: the unit size does not show;
+    // FP32 units are part of the summation order and stay).  Wide rows have their feature
+    // slices to fill the chip with.
+    u32 small_unit() const
+    {
+        u32 rows = kHistChunk;
+        if (quant && Fs <= 64u)
+            while (rows > kHistUnitMin && N / rows < kHistUnitFill) rows /= 2u;
+        return rows;
+    }
     u32 node_cells() const { return F * SB; }
 };
 
@@ -405,9 +419,10 @@ int alloc_fit(bh_context *c)
     u32 const depth = static_cast<u32>(f.max_depth);
     c->max_front = f.grower == BH_LEAFWISE ? 2u : (1u << std::min(depth, 14u));
     c->max_ops = std::max(1u, c->max_front);
-    c->max_pch = N / part_chunk_rows(c->Fs) + c->max_ops + 2;
-    c->max_hch = N / kHistChunk + c->max_ops + 2;
-    c->max_parts = N / kHistChunk + c->max_ops + 2;
+    c->max_pch = N / part_chunk_rows(c->Fs, c->N) + c->max_ops + 2;
+    u32 const unit = f.grower == BH_DEPTHWISE ? c->small_unit() : kHistChunk;
+    c->max_hch = N / unit + c->max_ops + 2;
+    c->max_parts = N / unit + c->max_ops + 2;
     c->hist_slots = f.grower == BH_LEAFWISE ? static_cast<u32>(f.max_leaves) + 4u : std::max(1u, c->max_front / 2u);
     c->max_nodes = tree_capacity(f);
     size_t const nc = c->node_cells();
@@ -662,8 +677,8 @@ void enqueue_depthwise_counted(bh_context *c)
         launch_find(s, true, cur, c->ctl, hcur, c->d_nbins, c->F, c->SB, c->gc, c->scales, c->splits, width, 0, 0,
                     c->fscr, ccur);
         launch_plan_counted(s, cur, c->splits, c->ctl, c->tree, c->ops, c->pch, nxt, c->hch, c->fops, c->d_nbins,
-                            c->gc, c->scales, dst, last ? 1u : 0u, part_chunk_rows(c->Fs), mode, c->ops4,
-                            mode == 1 ? unit_rows : kHistChunk, c->cursors4);
+                            c->gc, c->scales, dst, last ? 1u : 0u, part_chunk_rows(c->Fs, c->N), mode, c->ops4,
+                            mode == 1 ? unit_rows : c->small_unit(), c->cursors4);
         if (c->fc.host_sync) host_sync_point(c);
         if (!last) {
             if (mode == 0) {
@@ -720,7 +735,7 @@ void enqueue_depthwise(bh_context *c)
         launch_find(s, c->quant, cur, c->ctl, hcur, c->d_nbins, c->F, c->SB, c->gc, c->scales, c->splits, width, 0, 0,
                     c->fscr);
         launch_plan_level(s, cur, c->splits, c->ctl, c->tree, c->ops, c->pch, c->d_nbins, c->gc, c->scales, d & 1u,
-                          part_chunk_rows(c->Fs));
+                          part_chunk_rows(c->Fs, c->N));
         if (c->fc.host_sync) host_sync_point(c);
         launch_part_count(s, c->pch, c->ops, c->ctl, c->work[0], c->work[1], c->plane0, c->Fs, c->chunk_left,
                           part_grid(c));
@@ -1961,7 +1976,7 @@ int bh_partition(bh_context *c, const uint32_t *rows, uint64_t n, uint32_t featu
     HIP_TRY(hipMemcpy(c->tree, &root, sizeof(root), hipMemcpyHostToDevice));
     GrowCfg gc = c->gc;
     launch_plan_level(c->stream, c->front[0], c->splits, c->ctl, c->tree, c->ops, c->pch, c->d_nbins, gc, c->scales,
-                      1, part_chunk_rows(c->Fs));
+                      1, part_chunk_rows(c->Fs, c->N));
     launch_part_count(c->stream, c->pch, c->ops, c->ctl, c->work[0], c->work[1], c->plane0, c->Fs, c->chunk_left,
                       part_grid(c));
     // oblivious = 1: no demotion, so an all-one-side split still scatters.
@@ -2150,7 +2165,7 @@ struct StepPart {
 };
 int step_partition(bh_context *c, std::vector<StepPart> const &parts, std::vector<u32> &n_left)
 {
-    u32 const chunk_rows = part_chunk_rows(c->Fs);
+    u32 const chunk_rows = part_chunk_rows(c->Fs, c->N);
     std::vector<PartOp> ops(parts.size());
     std::vector<PartChunk> pch;
     for (size_t i = 0; i < parts.size(); ++i) {

@@ -3491,7 +3491,13 @@ void launch_plan_level(hipStream_t s, NodeInfo const *front, SplitRec const *spl
                        scales, dst, chunk_rows);
 }
 
-u32 part_chunk_rows(u32 Fs) { return Fs <= 64 ? kPartChunk : kWideChunk; }
+u32 part_chunk_rows(u32 Fs, u64 n)
+{
+    if (Fs > 64) return kWideChunk;
+    u32 rows = kPartChunk;
+    while (rows > kPartChunkMin && n / rows < kPartChunkFill) rows /= 2u;
+    return rows;
+}
 
 void launch_part_count(hipStream_t s, PartChunk const *pch, PartOp const *ops, TreeCtl const *ctl, u8 const *pl0,
                        u8 const *pl1, u8 const *plp, u32 Fs, u32 *chunk_left, u32 grid)

@@ -1211,11 +1211,11 @@ void enqueue_levelwise(ExtState &s, hipStream_t st, bool q, GrowView const &v)
                            s.level_gains, pick);
         if (q)
             hipLaunchKernelGGL(k_plan_oblivious<true>, dim3(1), dim3(1024), 0, st, cur, v.ctl, pick, hcur, v.d_nbins,
-                               v.F, v.SB, v.splits, v.ops, v.pch, d & 1u, last ? 1u : 0u, part_chunk_rows(v.Fs), 1u);
+                               v.F, v.SB, v.splits, v.ops, v.pch, d & 1u, last ? 1u : 0u, part_chunk_rows(v.Fs, v.N), 1u);
         else
             hipLaunchKernelGGL(k_plan_oblivious<false>, dim3(1), dim3(1024), 0, st, cur, v.ctl, pick, hcur,
                                v.d_nbins, v.F, v.SB, v.splits, v.ops, v.pch, d & 1u, last ? 1u : 0u,
-                               part_chunk_rows(v.Fs), 1u);
+                               part_chunk_rows(v.Fs, v.N), 1u);
         launch_part_count(st, v.pch, v.ops, v.ctl, v.work[0], v.work[1], v.plane0, v.Fs, v.chunk_left,
                           std::max(1u, std::min(v.max_pch, tuning().part_grid)));
         launch_part_scan(st, q, v.ops, v.pch, v.chunk_left, v.ctl, cur, nxt, v.splits, v.tree, v.hch, v.fops, v.gc,
@@ -1265,10 +1265,10 @@ void launch_level_find_step(ExtState &s, hipStream_t st, bool q, GrowView const 
                        pick);
     if (q)
         hipLaunchKernelGGL(k_plan_oblivious<true>, dim3(1), dim3(1024), 0, st, front, v.ctl, pick, hist, v.d_nbins, v.F,
-                           v.SB, v.splits, v.ops, v.pch, 0u, 1u, part_chunk_rows(v.Fs), 0u);
+                           v.SB, v.splits, v.ops, v.pch, 0u, 1u, part_chunk_rows(v.Fs, v.N), 0u);
     else
         hipLaunchKernelGGL(k_plan_oblivious<false>, dim3(1), dim3(1024), 0, st, front, v.ctl, pick, hist, v.d_nbins,
-                           v.F, v.SB, v.splits, v.ops, v.pch, 0u, 1u, part_chunk_rows(v.Fs), 0u);
+                           v.F, v.SB, v.splits, v.ops, v.pch, 0u, 1u, part_chunk_rows(v.Fs, v.N), 0u);
 }
 
 // LeafwiseGrower::grow as a launch sequence: the root, then max_leaves - 1 rounds
@@ -1312,11 +1312,11 @@ void enqueue_leafwise(ExtState &s, hipStream_t st, bool q, GrowView const &v)
     if (q)
         hipLaunchKernelGGL(k_lw_select<true>, dim3(1), dim3(256), 0, st, v.ctl, lw, s.cands, kids, v.splits,
                            s.free_slots, parent, psplit, v.tree, v.ops, v.pch, v.hch, v.d_nbins, v.fops, v.gc, v.scales,
-                           v.lw_units, part_chunk_rows(v.Fs));
+                           v.lw_units, part_chunk_rows(v.Fs, v.N));
     else
         hipLaunchKernelGGL(k_lw_select<false>, dim3(1), dim3(256), 0, st, v.ctl, lw, s.cands, kids, v.splits,
                            s.free_slots, parent, psplit, v.tree, v.ops, v.pch, v.hch, v.d_nbins, v.fops, v.gc, v.scales,
-                           0u, part_chunk_rows(v.Fs));
+                           0u, part_chunk_rows(v.Fs, v.N));
     u32 const rounds = static_cast<u32>(v.fc.max_leaves) - 1u + 8u;
     for (u32 r = 0; r < rounds; ++r) {
         launch_part_count(st, v.pch, v.ops, v.ctl, v.work[0], v.work[1], v.plane0, v.Fs, v.chunk_left, pgrid);
@@ -1336,7 +1336,7 @@ void enqueue_leafwise(ExtState &s, hipStream_t st, bool q, GrowView const &v)
         launch_finish(st, q, v.fops, v.ctl, v.partials, pool, pool, v.F * v.SB, 1, cnt, cnt, false,
                       hist_transpose_F(q, v.Fs, v.F));
         LwNext const nx{s.cands, s.free_slots, parent, psplit, v.tree, v.ops, v.pch, v.hch, v.fops, v.lw_units,
-                        part_chunk_rows(v.Fs), r + 1 < rounds ? 1u : 0u};
+                        part_chunk_rows(v.Fs, v.N), r + 1 < rounds ? 1u : 0u};
         if (q) launch_lw_find<true, true>(st, v, lw, cnt, nx);
         else launch_lw_find<false, false>(st, v, lw, cnt, nx);
         if (v.host_sync) (void)hipStreamSynchronize(st);

@@ -175,6 +175,30 @@ def test_grow_depthwise_int_bit_exact(hip, orc, tall, depth, pair):
     assert np.array_equal(lor, rlor)
 
 
+@pytest.mark.parametrize("pair", [1, 0])
+@pytest.mark.parametrize("n", [255, 1025, 16385, 140001, 524289])
+def test_grow_depthwise_int_unit_sizes(hip, orc, n, pair):
+    """Row counts on both sides of the steps of the unit and partition chunk sizes
+    (1,024 .. 8,192 rows and 256 .. 4,096): the gradient maxima of every row count, then
+    the tree, bit-exact."""
+    rng = np.random.default_rng(n)
+    bins = rng.integers(0, 64, (n, 7)).astype(np.uint8)
+    nb = np.full(7, 64, np.uint16)
+    y = (bins[:, 2] > 30).astype(np.float32)
+    g, h = grad_of(orc, y, seed=n)
+    ctx = ctx_for(hip, bins, nb, quantized=True, max_depth=5, min_data_in_leaf=2, seed=9)
+    ctx.set_tuning(pair_levels=pair)
+    gq, hq, sc = ctx.set_gradients(g, h, it=1)
+    ogq, ohq, osc = orc.quantize(g, h, 9, 1)
+    assert np.array_equal(sc, osc) and np.array_equal(gq, ogq) and np.array_equal(hq, ohq)
+    ref, rlor = orc.grow_depthwise(bins, nb, gq=gq, hq=hq, scales=sc, c=orc_cfg(max_depth=5, min_data=2),
+                                   mode=HIST_INT)
+    nodes, lor = ctx.grow_tree()
+    ctx.close()
+    assert_same_tree(nodes, ref)
+    assert np.array_equal(lor, rlor)
+
+
 @pytest.mark.parametrize("width", [10, 60])
 def test_grow_depthwise_int_paired_row_widths(hip, orc, tall, width):
     """Rows of 12 and 60 bytes through the four-way partitions, whose tiles reserve
