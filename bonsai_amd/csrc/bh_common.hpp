@@ -214,12 +214,16 @@ struct RootSel {
     u32 n_from_ctl; // 1: the count is TreeCtl::root_n
 };
 
-// Launch-shape knobs of one context, picked by the autotuner (bh_autotune).
+// Launch-shape knobs of one context, picked by the autotuner (bh_autotune).  The
+// partition defaults hold 1,024 rows of 28 bytes and their gradients in one tile (a tile
+// costs its barriers and partly filled runs whatever it holds) and four chunks a CU over
+// 4 rounds: 16M x 28, depth 8, 20 rounds 56.7 -> 52.3 ms against 20 KiB and 2,048
+// (four-way scatters 381 -> 248 and 267 -> 220 us); 48 KiB loses a workgroup a CU.
 struct Tuning {
-    u32 scatter_lds = 20u * 1024u; // LDS bytes per partition-scatter workgroup (sets its tile rows)
+    u32 scatter_lds = 40992u;      // LDS bytes per partition-scatter workgroup (sets its tile rows)
     u32 find_blocks = kFindMaxBlocks; // workgroups sharing one node's split find (1..kFindMaxBlocks)
     u32 hist_threads = 512;      // quantized histogram workgroup size (256, 512 or 1024)
-    u32 part_grid = 2048;        // partition count / scatter workgroups
+    u32 part_grid = 4096;        // partition count / scatter workgroups
     u32 hist_layout = 0;         // quantized histogram: 0 row-dword lanes, 1 feature-in-lane (rows <= 32 B),
                                  // 2 row-in-lane (rows <= 64 B; routed levels always use it)
     u32 pair_levels = 1;         // quantized depthwise, rows <= 64 bytes: move rows every second level
