@@ -62,6 +62,12 @@ constexpr u32 kLwMinChunk = 256;
 constexpr u32 kLwUnitTarget = 256;
 constexpr u32 kLwMinUnit = 1024;
 constexpr u32 kMaxTreeNodes = 8192;
+constexpr u32 kLwBatch = 8;       // leaves a leafwise round expands at most
+constexpr u32 kLwAhead = 32;      // leaves expanded before their pop at most (each holds one more slot)
+constexpr u32 kLwMoreRounds = 4;  // rounds added at a time to a tree the first ones left unfinished
+constexpr u32 kLwPoolCap = 1024 + 8;                       // max_leaves and its last round's children
+constexpr u32 kLwListCap = kLwPoolCap + kLwAhead + 2 * kLwBatch;
+constexpr u32 kLwRecCap = 1 + 2 * (kLwPoolCap + kLwAhead + kLwBatch); // two a leaf expanded
 // Tail padding of planes (bytes) and gradient buffers (elements): kernels that read
 // aligned 16-byte words around a row range may touch up to 15 bytes past its end.
 constexpr size_t kTailPadBytes = 64;

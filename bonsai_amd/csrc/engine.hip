@@ -197,6 +197,7 @@ struct bh_context {
     u32 trees_cap = 0, trees_done = 0, max_nodes = 0;
     // capacities
     u32 max_front = 0, max_ops = 0, max_pch = 0, max_hch = 0, max_parts = 0, hist_slots = 0;
+    u32 lw_parts = 0, lw_pch = 0; // leafwise rounds
     u32 lw_units = 0; // quantized leafwise: histogram units per child at most
     // row sampling of the tree's root (bh_set_row_subset / bh_set_bernoulli)
     u32 samp_kind = 0;           // 0 every row, 1 a fixed subset, 2 a Bernoulli draw per iteration
@@ -226,6 +227,9 @@ struct bh_context {
     // graph
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
+    // leafwise: the iteration past its growth, and the extra rounds of an unfinished tree
+    hipGraph_t graph_tail = nullptr, graph_more = nullptr;
+    hipGraphExec_t tail_exec = nullptr, more_exec = nullptr;
     // histogram profiling (per-launch hipEvents, non-graph iterations only)
     bool prof = false;
     double prof_ms = 0.0, prof_bytes = 0.0, prof_scanned_bytes = 0.0;
@@ -297,12 +301,23 @@ struct bh_context {
 
 namespace {
 
+void drop_graphs(bh_context *c)
+{
+    hipGraphExec_t *const execs[] = {&c->graph_exec, &c->tail_exec, &c->more_exec};
+    hipGraph_t *const graphs[] = {&c->graph, &c->graph_tail, &c->graph_more};
+    for (hipGraphExec_t *e : execs) {
+        if (*e) (void)hipGraphExecDestroy(*e);
+        *e = nullptr;
+    }
+    for (hipGraph_t *g : graphs) {
+        if (*g) (void)hipGraphDestroy(*g);
+        *g = nullptr;
+    }
+}
+
 void free_fit(bh_context *c)
 {
-    if (c->graph_exec) hipGraphExecDestroy(c->graph_exec);
-    if (c->graph) hipGraphDestroy(c->graph);
-    c->graph_exec = nullptr;
-    c->graph = nullptr;
+    drop_graphs(c);
     void *ptrs[] = {c->gh0f, c->ghwf[0], c->ghwf[1], c->gh0q, c->ghwq[0], c->ghwq[1], c->maxbits, c->scales, c->fx,
                     c->hist[0], c->hist[1], c->partials, c->ctl, c->front[0], c->front[1], c->splits, c->tree,
                     c->ops, c->pch, c->chunk_left, c->hch, c->fops, c->trees_out, c->tree_sizes, c->leaf_rows,
@@ -437,7 +452,13 @@ int alloc_fit(bh_context *c)
         c->max_hch = std::max(c->max_hch, c->lw_units + 2u);
         c->max_parts = std::max(c->max_parts, c->lw_units + 2u);
     }
-    size_t const hist_bytes = static_cast<size_t>(c->hist_slots) * nc * c->cell_bytes();
+    // A leafwise round's leaves hold more slots, units and chunks than the engine steps'
+    // limits (hist_slots, max_parts, max_pch) name.
+    bool const leafwise = f.grower == BH_LEAFWISE;
+    u32 const slots = c->hist_slots + (leafwise ? kLwAhead + kLwBatch : 0u);
+    c->lw_parts = leafwise ? std::max(c->max_parts, 2u * c->lw_units + 2u) : 0u;
+    c->lw_pch = leafwise ? c->max_pch + kLwBatch * (kLwChunkTarget + 1u) : 0u;
+    size_t const hist_bytes = static_cast<size_t>(slots) * nc * c->cell_bytes();
     if (c->quant) {
         HIP_TRY(dalloc(&c->gh0q, N + kTailPad));
         HIP_TRY(dalloc(&c->ghwq[0], N + kTailPad));
@@ -454,7 +475,7 @@ int alloc_fit(bh_context *c)
     HIP_TRY(hipMemset(c->fx, 0, 4 * sizeof(u32)));
     HIP_TRY(hipMalloc(&c->hist[0], hist_bytes));
     if (f.grower != BH_LEAFWISE) HIP_TRY(hipMalloc(&c->hist[1], hist_bytes));
-    HIP_TRY(hipMalloc(&c->partials, static_cast<size_t>(c->max_parts) * nc * c->part_bytes()));
+    HIP_TRY(hipMalloc(&c->partials, static_cast<size_t>(std::max(c->max_parts, c->lw_parts)) * nc * c->part_bytes()));
     if (c->quant && f.grower == BH_DEPTHWISE) {
         size_t const cells = static_cast<size_t>(c->hist_slots) * nc;
         HIP_TRY(dalloc(&c->cnt[0], cells));
@@ -463,10 +484,10 @@ int alloc_fit(bh_context *c)
         HIP_TRY(dalloc(&c->chunk_cls, c->max_pch));
         HIP_TRY(dalloc(&c->cursors4, (static_cast<size_t>(c->max_ops) / 2 + 2) * 4u * kCursorStride));
     }
-    if (c->quant && f.grower == BH_LEAFWISE) HIP_TRY(dalloc(&c->cnt[0], static_cast<size_t>(c->hist_slots) * nc));
+    if (c->quant && f.grower == BH_LEAFWISE) HIP_TRY(dalloc(&c->cnt[0], static_cast<size_t>(slots) * nc));
     HIP_TRY(dalloc(&c->ctl, 1));
     HIP_TRY(hipMemset(c->ctl, 0, sizeof(TreeCtl)));
-    u32 const fcap = std::max(c->max_front * 2u, 4u);
+    u32 const fcap = std::max(std::max(c->max_front * 2u, 4u), leafwise ? 2u * kLwBatch : 0u);
     HIP_TRY(dalloc(&c->front[0], fcap));
     HIP_TRY(dalloc(&c->front[1], fcap));
     HIP_TRY(dalloc(&c->splits, fcap));
@@ -474,13 +495,13 @@ int alloc_fit(bh_context *c)
     HIP_TRY(dalloc(&c->fscr.done, fcap));
     HIP_TRY(hipMemset(c->fscr.done, 0, fcap * sizeof(u32)));
     HIP_TRY(dalloc(&c->tree, c->max_nodes));
-    HIP_TRY(dalloc(&c->ops, c->max_ops + 2));
-    HIP_TRY(dalloc(&c->pch, c->max_pch));
-    HIP_TRY(dalloc(&c->chunk_left, c->max_pch));
-    HIP_TRY(dalloc(&c->hch, c->max_hch));
-    HIP_TRY(dalloc(&c->fops, c->max_ops + 2));
+    HIP_TRY(dalloc(&c->ops, std::max(c->max_ops + 2, kLwBatch)));
+    HIP_TRY(dalloc(&c->pch, std::max(c->max_pch, c->lw_pch)));
+    HIP_TRY(dalloc(&c->chunk_left, std::max(c->max_pch, c->lw_pch)));
+    HIP_TRY(dalloc(&c->hch, std::max(c->max_hch, c->lw_parts)));
+    HIP_TRY(dalloc(&c->fops, std::max(c->max_ops + 2, kLwBatch)));
     HIP_TRY(dalloc(&c->leaf_rows, N));
-    if (ext_alloc(c->ext, f, c->F, c->SB, c->max_front, c->hist_slots) != hipSuccess)
+    if (ext_alloc(c->ext, f, c->F, slots) != hipSuccess)
         return fail(-1, "hip: extension buffers");
     c->gc.min_child_hess = f.min_child_hess;
     c->gc.min_gain = f.min_gain_to_split;
@@ -517,10 +538,7 @@ int ensure_tree_out(bh_context *c, u32 n_more)
     c->tree_sizes = ns;
     c->trees_cap = cap;
     // the captured graph holds the old pointers
-    if (c->graph_exec) hipGraphExecDestroy(c->graph_exec);
-    if (c->graph) hipGraphDestroy(c->graph);
-    c->graph_exec = nullptr;
-    c->graph = nullptr;
+    drop_graphs(c);
     return 0;
 }
 
@@ -764,6 +782,28 @@ void enqueue_grow(bh_context *c)
     else enqueue_leafwise(c->ext, c->stream, c->quant, grow_view(c));
 }
 
+void enqueue_more_rounds(bh_context *c)
+{
+    enqueue_leafwise_rounds(c->ext, c->stream, c->quant, grow_view(c), kLwMoreRounds);
+}
+
+// Leafwise: waits for the rounds enqueued so far and adds more until the tree is complete
+// (every round pops a leaf at least, so max_leaves + 7 are enough).
+int finish_growth(bh_context *c)
+{
+    if (c->fc.grower != BH_LEAFWISE) return 0;
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    u32 const most = static_cast<u32>(c->fc.max_leaves) / kLwMoreRounds + 2u;
+    for (u32 k = 0; *c->ext.report == 0u; ++k) {
+        if (k == most) return fail(-2, "leafwise growth did not complete");
+        if (c->more_exec) HIP_TRY(hipGraphLaunch(c->more_exec, c->stream));
+        else enqueue_more_rounds(c);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(c->stream));
+    }
+    return 0;
+}
+
 // Quantized fits: the first iteration after scores, labels or the fit were set takes
 // its gradient maxima from a pass of its own (later ones from the score update).
 void prime_gradients(bh_context *c)
@@ -783,10 +823,13 @@ void enqueue_gradients(bh_context *c)
 }
 
 // One boosting iteration: gradients, tree, score epilogue, tree copy-out.
-void enqueue_iteration(bh_context *c)
+void enqueue_iteration_head(bh_context *c)
 {
     enqueue_gradients(c);
     enqueue_grow(c);
+}
+void enqueue_iteration_tail(bh_context *c)
+{
     launch_score_update(c->stream, c->plane0, c->Fs, c->N, c->tree, c->ctl, c->d_nbins, c->F, c->fc.learning_rate,
                         c->score, nullptr, c->max_nodes, c->label, c->fc.objective, c->quant ? c->maxbits : nullptr,
                         c->weight);
@@ -800,6 +843,45 @@ void enqueue_iteration(bh_context *c)
     }
     launch_copy_tree(c->stream, c->tree, c->ctl, c->trees_out, c->tree_sizes, c->max_nodes);
     launch_iter_advance(c->stream, c->ctl);
+}
+int enqueue_iteration(bh_context *c)
+{
+    enqueue_iteration_head(c);
+    if (int r = finish_growth(c)) return r;
+    enqueue_iteration_tail(c);
+    return 0;
+}
+
+int capture(bh_context *c, hipGraph_t &g, hipGraphExec_t &ge, void (*enqueue)(bh_context *))
+{
+    HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+    enqueue(c);
+    hipError_t const e = hipStreamEndCapture(c->stream, &g);
+    if (e != hipSuccess) return fail(-1, std::string("hip: capture: ") + hipGetErrorString(e));
+    HIP_TRY(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
+    return 0;
+}
+
+// The iteration's graph: whole, or (leafwise) cut where the host looks at the growth.
+int capture_iteration(bh_context *c)
+{
+    if (c->graph_exec && (c->fc.grower != BH_LEAFWISE || c->tail_exec)) return 0;
+    drop_graphs(c);
+    if (c->fc.grower != BH_LEAFWISE)
+        return capture(c, c->graph, c->graph_exec, [](bh_context *x) {
+            enqueue_iteration_head(x);
+            enqueue_iteration_tail(x);
+        });
+    if (int r = capture(c, c->graph, c->graph_exec, enqueue_iteration_head)) return r;
+    if (int r = capture(c, c->graph_more, c->more_exec, enqueue_more_rounds)) return r;
+    return capture(c, c->graph_tail, c->tail_exec, enqueue_iteration_tail);
+}
+int launch_iteration(bh_context *c)
+{
+    HIP_TRY(hipGraphLaunch(c->graph_exec, c->stream));
+    if (int r = finish_growth(c)) return r;
+    if (c->tail_exec) HIP_TRY(hipGraphLaunch(c->tail_exec, c->stream));
+    return 0;
 }
 
 // The counted scatter reports a chunk whose prefix disagrees with its op's row counts
@@ -865,6 +947,8 @@ GrowView grow_view(bh_context *c)
     v.max_ops = c->max_ops;
     v.cnt = c->cnt[0];
     v.lw_units = c->lw_units;
+    v.lw_parts = c->lw_parts;
+    v.lw_pch = c->lw_pch;
     v.root = root_sel(c);
     v.fsl = c->hist_fsl();
     v.fx = c->fx;
@@ -1218,7 +1302,6 @@ int bh_upload_labels(bh_context *c, const float *labels)
     return 0;
 }
 
-static void drop_graph(bh_context *c);
 
 int bh_upload_weights(bh_context *c, const float *weights)
 {
@@ -1235,7 +1318,7 @@ int bh_upload_weights(bh_context *c, const float *weights)
         HIP_TRY(hipFree(c->weight));
         c->weight = nullptr;
     }
-    drop_graph(c); // the gradient kernels' arguments change
+    drop_graphs(c); // the gradient kernels' arguments change
     c->max_stale = true;
     return 0;
 }
@@ -1282,7 +1365,7 @@ int bh_set_scores(bh_context *c, const float *scores)
     if (c->have_valid) {
         c->have_valid = false;
         c->es_done = false;
-        drop_graph(c);
+        drop_graphs(c);
     }
     return 0;
 }
@@ -1326,7 +1409,7 @@ int bh_set_validation(bh_context *c, const uint8_t *bins, uint64_t n_rows, uint6
     c->es_base = c->trees_done;
     c->es_done = false;
     c->have_valid = true;
-    drop_graph(c); // the iteration graph gains the validation launches
+    drop_graphs(c); // the iteration graph gains the validation launches
     return 0;
 }
 
@@ -1355,7 +1438,7 @@ int bh_set_row_subset(bh_context *c, const uint32_t *rows, uint64_t n)
     if (c->samp_rows) (void)hipFree(c->samp_rows);
     c->samp_rows = nullptr;
     c->samp_kind = c->samp_n = 0;
-    drop_graph(c); // the iteration graph gains or loses the gather
+    drop_graphs(c); // the iteration graph gains or loses the gather
     if (!rows || n == 0 || n == c->N) {
         if (rows && n == c->N)
             for (u64 i = 0; i < n; ++i)
@@ -1383,7 +1466,7 @@ int bh_set_bernoulli(bh_context *c, float subsample, uint64_t seed)
     if (c->samp_rows) (void)hipFree(c->samp_rows);
     c->samp_rows = nullptr;
     c->samp_kind = c->samp_n = 0;
-    drop_graph(c);
+    drop_graphs(c);
     if (subsample >= 1.0F) return 0; // the reference keeps every row for p >= 1
     if (!c->samp_cnt) HIP_TRY(dalloc(&c->samp_cnt, c->N / kPartChunk + 2));
     double const t = std::floor(static_cast<double>(subsample) * 4294967296.0);
@@ -1402,7 +1485,7 @@ int bh_set_monotone(bh_context *c, const int8_t *dirs, uint32_t n)
     std::vector<int8_t> prev = std::move(c->mono_host);
     c->mono_host.clear();
     for (u32 f = 0; f < n; ++f) c->mono_host.push_back(dirs[f] > 0 ? 1 : (dirs[f] < 0 ? -1 : 0));
-    drop_graph(c); // the finders' configuration changes
+    drop_graphs(c); // the finders' configuration changes
     if (int r = arm_monotone(c)) {
         c->mono_host = std::move(prev);
         (void)arm_monotone(c);
@@ -1426,7 +1509,7 @@ int bh_set_interaction(bh_context *c, const uint32_t *members, const uint32_t *g
         k += group_sizes[g];
         if (!grp.empty()) c->groups_host.push_back(std::move(grp)); // empty entries are dropped
     }
-    drop_graph(c);
+    drop_graphs(c);
     if (int r = arm_interaction(c)) {
         c->groups_host = std::move(prev);
         (void)arm_interaction(c);
@@ -1443,7 +1526,7 @@ int reset_feature_sampling(bh_context *c)
     HIP_TRY(hipStreamSynchronize(c->stream));
     c->fsamp_kind = 0;
     c->gc.fmask = nullptr;
-    drop_graph(c);
+    drop_graphs(c);
     if (!c->fmask) HIP_TRY(dalloc(&c->fmask, c->F));
     return 0;
 }
@@ -1515,13 +1598,8 @@ int bh_train(bh_context *c, uint32_t n_iters)
     c->iter_ms.clear();
     bool const graph = c->fc.use_graph && !c->fc.host_sync;
     prime_gradients(c);
-    if (graph && !c->graph_exec) {
-        HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        enqueue_iteration(c);
-        hipError_t const e = hipStreamEndCapture(c->stream, &c->graph);
-        if (e != hipSuccess) return fail(-1, std::string("hip: capture: ") + hipGetErrorString(e));
-        HIP_TRY(hipGraphInstantiate(&c->graph_exec, c->graph, nullptr, nullptr, 0));
-    }
+    if (graph)
+        if (int r = capture_iteration(c)) return r;
     // With early stopping the device records the rule's verdict every round; the host
     // looks at it every kEsCheck rounds, so at most kEsCheck - 1 rounds past the stop
     // are grown and dropped.
@@ -1532,8 +1610,7 @@ int bh_train(bh_context *c, uint32_t n_iters)
         u32 const k = std::min(step, n_iters - done);
         for (u32 it = 0; it < k; ++it) {
             if (c->timing) HIP_TRY(hipEventRecord(c->ev0, c->stream));
-            if (graph) HIP_TRY(hipGraphLaunch(c->graph_exec, c->stream));
-            else enqueue_iteration(c);
+            if (int r = graph ? launch_iteration(c) : enqueue_iteration(c)) return r;
             if (c->timing) {
                 HIP_TRY(hipEventRecord(c->ev1, c->stream));
                 HIP_TRY(hipEventSynchronize(c->ev1));
@@ -1561,14 +1638,6 @@ int bh_train(bh_context *c, uint32_t n_iters)
     return 0;
 }
 
-static void drop_graph(bh_context *c)
-{
-    if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
-    if (c->graph) (void)hipGraphDestroy(c->graph);
-    c->graph_exec = nullptr;
-    c->graph = nullptr;
-}
-
 static int validate_tuning(bh_tuning const *t)
 {
     if (t->scatter_lds_bytes < 4096u || t->scatter_lds_bytes > 162816u)
@@ -1591,7 +1660,7 @@ int bh_set_tuning(bh_context *c, const bh_tuning *t)
     HIP_TRY(hipStreamSynchronize(c->stream));
     c->tune = Tuning{t->scatter_lds_bytes, t->find_blocks, t->hist_threads, t->part_grid, t->hist_layout,
                      t->pair_levels, t->hist_group};
-    drop_graph(c); // the iteration graph is re-captured with the new shapes
+    drop_graphs(c); // the iteration graph is re-captured with the new shapes
     return 0;
 }
 
@@ -1636,7 +1705,7 @@ int bh_autotune(bh_context *c, uint32_t iters, bh_tuning *chosen, float *ms_per_
     };
     auto trial = [&](Tuning const &t, float *ms) -> int {
         c->tune = t;
-        drop_graph(c);
+        drop_graphs(c);
         if (int r = restore()) return r;
         if (int r = bh_train(c, 1)) return r;
         if (int r = restore()) return r;
@@ -1683,7 +1752,7 @@ int bh_autotune(bh_context *c, uint32_t iters, bh_tuning *chosen, float *ms_per_
         }
     }
     c->tune = best;
-    drop_graph(c);
+    drop_graphs(c);
     int const rr = restore();
     (void)hipFree(saved);
     c->timing = saved_timing;
@@ -1803,6 +1872,7 @@ int bh_grow_tree(bh_context *c, bh_node *nodes, uint32_t cap, uint32_t *n_nodes,
     if (int r = check_ready(c)) return r;
     HIP_TRY(hipSetDevice(c->device));
     enqueue_grow(c);
+    if (int r = finish_growth(c)) return r;
     launch_score_update(c->stream, c->plane0, c->Fs, c->N, c->tree, c->ctl, c->d_nbins, c->F, 0.0F, nullptr,
                         c->leaf_rows, c->max_nodes);
     HIP_TRY(hipGetLastError());
@@ -2012,7 +2082,8 @@ int bh_profile_hist(bh_context *c, uint32_t n_iters, double *ms_total, double *b
     c->prof_ms = c->prof_bytes = c->prof_scanned_bytes = 0.0;
     c->prof_launches = c->prof_rows = c->prof_scanned = 0;
     prime_gradients(c);
-    for (u32 it = 0; it < n_iters; ++it) enqueue_iteration(c);
+    for (u32 it = 0; it < n_iters; ++it)
+        if (int r = enqueue_iteration(c)) return r;
     c->prof = false;
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(c->stream));

@@ -590,18 +590,20 @@ __global__ __launch_bounds__(1024) void k_oblivious_tree(NodeInfo const *__restr
 
 // ---------------------------------------------------------------------------------
 // Leafwise rounds.
+//
+// Growth pops the pool's best leaf (gain, ties to the lower node id), and each pop needs
+// its children's splits before the next one is known: as one leaf a round that is five
+// launches of mostly idle chip, 254 times for 255 leaves (57 us a round, nearly all
+// launch and latency).  A round here expands up to kLwBatch leaves: the one the pops wait
+// for and the best of the others, children of expanded but not yet popped leaves
+// included; what is expanded early is popped later without a round of its own.  Pops and
+// node ids follow the one-leaf order exactly, and a leaf expanded but never popped stays
+// the leaf it is (its rows only moved inside their segment).  255 leaves take 33 rounds on
+// the logistic table (of 32 possible), 31 take 7; 16M x 28: LWFIG.
+//
+// Constrained fits (monotone or interaction) keep one leaf a round: their split finder
+// reads per-node bounds and paths, which exist under the final node ids only.
 // ---------------------------------------------------------------------------------
-struct LwCtl {
-    u32 n_cand;
-    u32 n_free;
-    u32 parent_slot;
-    u32 demoted;
-    u32 small_left;
-    u32 n_push;      // children of the last round that still have to join the pool
-    u32 grid_done;   // workgroups of the running split find that have finished
-    u32 pad[9];
-};
-
 // Rows per partition chunk of a leaf of `rows` rows: about kLwChunkTarget chunks,
 // multiples of 256 rows, kLwMinChunk..kPartChunk, and at most cap (the chunk of wide
 // rows).
@@ -622,198 +624,27 @@ __device__ __forceinline__ u32 lw_unit_rows(u32 rows, u32 target)
     return min(kHistChunk, max(kLwMinUnit, per));
 }
 
-// queue_children (src/grower_impl.hpp:404-428): a child with a valid split joins the
-// pool; one without becomes a leaf now and frees its slot.  One thread.
-__device__ __forceinline__ void lw_push(LwCtl *lw, NodeInfo const *kids, SplitRec const *splits, u32 n, bool is_root, Cand *cands,
-                        u32 *free_slots, DevNode *tree, GrowCfg const &cfg, double const *scales)
+// Upper bound of a built node's unit count over all its row counts up to `rows`.
+__device__ __forceinline__ u32 lw_unit_bound(u32 rows, u32 target)
 {
-    for (u32 k = 0; k < n; ++k) {
-        NodeInfo const nd = kids[k];
-        SplitRec const s = splits[k];
-        bool const ok = s.valid && (!is_root || cfg.max_depth > 0);
-        if (ok) {
-            Cand c;
-            c.node = nd;
-            c.split = s;
-            cands[lw->n_cand++] = c;
-        } else {
-            put_leaf(tree, nd.id, node_value(nd, cfg, scales));
-            if (nd.slot != kNone) free_slots[lw->n_free++] = nd.slot;
-        }
-    }
+    u32 const whole = (rows + kHistChunk - 1u) / kHistChunk;
+    return max(whole, min(target, (rows + kLwMinUnit - 1u) / kLwMinUnit));
 }
 
-// The partitioned leaf's children (commit_pop, src/grower_impl.hpp:370-400), one
-// thread: demotion when every row went one way; else two children, the larger keeping
-// the parent's histogram slot (completed in place) and the smaller getting a fresh slot
-// and the histogram units in *fo, unless the children sit at max_depth (then they only
-// need totals, from the parent split's sums).  split_totals: the children's totals are
-// the split's exact integer sums (quantized), so the finder need not derive them.
-// Returns the smaller child's unit count (0: no histogram this round).
-template <bool Q>
-__device__ __forceinline__ u32 lw_children(PartOp &op, u32 nL, TreeCtl *ctl, LwCtl *lw, NodeInfo const &par, SplitRec const &s,
-                           u32 *free_slots, NodeInfo *kids, DevNode *tree, GrowCfg const &cfg,
-                           double const *scales, bool split_totals, u32 unit_target, FinishOp &fo,
-                           u32 &unit_rows)
-{
-    u32 const nR = op.cnt - nL;
-    op.n_left = nL;
-    bool const demote = (nL == 0) != (nR == 0);
-    op.alive = demote ? 0u : 1u;
-    lw->n_push = 0;
-    if (demote) {
-        put_leaf(tree, par.id, node_value(par, cfg, scales));
-        tree[par.id].gain = 0.0F;
-        free_slots[lw->n_free++] = par.slot;
-        ctl->n_front = 0;
-        ctl->n_finish = 0;
-        ctl->n_hist_chunks = 0;
-        lw->demoted = 1;
-        return 0;
-    }
-    lw->demoted = 0;
-    tree[op.left_id].cover = static_cast<float>(nL);
-    tree[op.right_id].cover = static_cast<float>(nR);
-    NodeInfo L{}, R{};
-    L.id = op.left_id;
-    R.id = op.right_id;
-    L.off = op.off;
-    L.cnt = nL;
-    R.off = op.off + nL;
-    R.cnt = nR;
-    L.src = R.src = op.dst;
-    L.depth = R.depth = par.depth + 1;
-    bool const left_small = nL <= nR;
-    bool const leaves = static_cast<int>(L.depth) >= cfg.max_depth;
-    ctl->live += 1;
-    ctl->max_depth_seen = max(ctl->max_depth_seen, L.depth);
-    if (leaves || split_totals) {
-        L.totals_ready = R.totals_ready = 1;
-        if (Q) {
-            L.itg = s.igL;
-            L.ith = s.ihL;
-            R.itg = s.igR;
-            R.ith = s.ihR;
-        } else {
-            L.tg = static_cast<float>(s.gL);
-            L.th = static_cast<float>(s.hL);
-            R.tg = static_cast<float>(s.gR);
-            R.th = static_cast<float>(s.hR);
-        }
-    }
-    u32 units = 0;
-    if (leaves) {
-        L.slot = R.slot = kNone;
-        free_slots[lw->n_free++] = par.slot;
-        ctl->n_finish = 0;
-        ctl->n_hist_chunks = 0;
-    } else {
-        u32 const fresh = free_slots[--lw->n_free];
-        L.slot = left_small ? fresh : par.slot;
-        R.slot = left_small ? par.slot : fresh;
-        u32 const small_cnt = left_small ? nL : nR;
-        unit_rows = lw_unit_rows(small_cnt, unit_target);
-        units = (small_cnt + unit_rows - 1) / unit_rows;
-        fo = FinishOp{};
-        fo.small_slot = fresh;
-        fo.large_slot = par.slot;
-        fo.parent_slot = par.slot;
-        fo.part_first = 0;
-        fo.part_count = units > 1 ? units : 0;
-        fo.empty = small_cnt == 0;
-        fo.unit_first = 0;
-        fo.unit_count = units;
-        fo.small_off = left_small ? L.off : R.off;
-        fo.small_cnt = small_cnt;
-        fo.src = op.dst;
-        ctl->n_finish = 1;
-        ctl->n_hist_chunks = units;
-    }
-    lw->small_left = left_small ? 1u : 0u;
-    lw->n_push = 2;
-    kids[0] = L;
-    kids[1] = R;
-    ctl->n_front = 2;
-    return units;
-}
+enum : u32 { kLwPlain = 0, kLwExpanded = 1, kLwDemoted = 2 };
 
-// Histogram units of the smaller child: rows [off, off + cnt) of plane `src` in
-// unit_rows pieces, each with its own partial when there is more than one.  u[] holds
-// (slot, src, off, cnt) in LDS.
-__device__ __forceinline__ void lw_expand_units(u32 const *u, u32 units, u32 unit_rows, HistChunk *hch)
+// Argmax over an LDS list (value, then lower key: a total order, so the butterfly is
+// exact) by one wave; every lane receives the index.
+__device__ __forceinline__ u32 lw_argmax(double const *val, u32 const *key, u32 n)
 {
-    for (u32 k = threadIdx.x; k < units; k += blockDim.x) {
-        HistChunk hc{};
-        hc.slot = u[0];
-        hc.src = u[1];
-        hc.begin = u[2] + k * unit_rows;
-        hc.end = u[2] + min(u[3], (k + 1) * unit_rows);
-        hc.part = units > 1 ? k : kNone;
-        hch[k] = hc;
-    }
-}
-
-__device__ __forceinline__ void lw_stash_units(u32 *u, FinishOp const &fo)
-{
-    u[0] = fo.small_slot;
-    u[1] = fo.src;
-    u[2] = fo.small_off;
-    u[3] = fo.small_cnt;
-}
-
-// Round start: the last round's children join the pool, then the best candidate is
-// popped (max gain, ties to the lower node id; the reference's gain_less,
-// src/grower_impl.hpp:763-770) unless the pool is empty or the leaf budget is spent,
-// its split committed (commit_split_node, :188-210) and the one partition op emitted,
-// in chunks sized to the leaf.  COUNTED (quantized): the split carries its child row
-// counts, so the children, their slots and the histogram units are set here and the
-// scatter takes each chunk's prefix from the chunk counts.  Runs as its own one-block
-// kernel for the first round and in the last workgroup of every round's split find for
-// the next; any workgroup size that is a multiple of 64.
-template <bool COUNTED>
-__device__ __forceinline__ void lw_select_round(TreeCtl *__restrict__ ctl, LwCtl *__restrict__ lw, Cand *__restrict__ cands,
-                                NodeInfo *__restrict__ kids, SplitRec const *__restrict__ kid_splits,
-                                u32 *__restrict__ free_slots, NodeInfo *__restrict__ parent_out,
-                                SplitRec *__restrict__ split_out, DevNode *__restrict__ tree, PartOp *__restrict__ ops,
-                                PartChunk *__restrict__ pch, HistChunk *__restrict__ hch,
-                                u16 const *__restrict__ n_bins, FinishOp *__restrict__ fops, GrowCfg const &cfg,
-                                double const *__restrict__ scales, u32 unit_target, u32 chunk_cap)
-{
-    __shared__ double s_wg[16];
-    __shared__ u32 s_wid[16], s_wix[16];
-    __shared__ u32 s_sel, s_go, s_n, s_units, s_urows, s_fo[4], s_ccnt, s_crow, s_nch;
-    if (ctl->done) {
-        if (threadIdx.x == 0) {
-            ctl->n_ops = 0;
-            ctl->n_part_chunks = 0;
-            ctl->n_front = 0;
-            ctl->n_finish = 0;
-            ctl->n_hist_chunks = 0;
-        }
-        return;
-    }
-    if (threadIdx.x == 0) {
-        u32 const np = lw->n_push;
-        if (np) lw_push(lw, kids, kid_splits, np, false, cands, free_slots, tree, cfg, scales);
-        lw->n_push = 0;
-        s_n = lw->n_cand;
-    }
-    __syncthreads();
-    u32 const n = s_n;
     double bg = 0.0;
     u32 bid = kNone, bix = kNone;
-    for (u32 k = threadIdx.x; k < n; k += blockDim.x) {
-        Cand const &c = cands[k];
-        double const g = c.split.gain;
-        u32 const id = c.node.id;
-        if (bix == kNone || g > bg || (g == bg && id < bid)) {
-            bg = g;
-            bid = id;
+    for (u32 k = threadIdx.x & 63u; k < n; k += 64u)
+        if (bix == kNone || val[k] > bg || (val[k] == bg && key[k] < bid)) {
+            bg = val[k];
+            bid = key[k];
             bix = k;
         }
-    }
-    // argmax (gain, then lower id: a total order, so the butterfly is exact) in each wave,
-    // then over the wave winners in wave 0
     for (int o = 32; o > 0; o >>= 1) {
         double const og = __shfl_xor(bg, o);
         u32 const oid = __shfl_xor(bid, o), oix = __shfl_xor(bix, o);
@@ -823,32 +654,383 @@ __device__ __forceinline__ void lw_select_round(TreeCtl *__restrict__ ctl, LwCtl
             bix = oix;
         }
     }
-    if ((threadIdx.x & 63u) == 0) {
-        s_wg[threadIdx.x >> 6] = bg;
-        s_wid[threadIdx.x >> 6] = bid;
-        s_wix[threadIdx.x >> 6] = bix;
+    return bix;
+}
+// One wave's LDS writes before its next reads.
+__device__ __forceinline__ void lw_wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// One expanded split of a round on its way to its children.
+struct LwSplit {
+    u32 rec;             // its record
+    u32 demoted, leaves; // one side has no rows; the children sit at max_depth
+    u32 nL, cnt, off, dst, slot, left_id, depth;
+    u32 urows, units, small_cnt, small_off, left_small;
+    u32 fresh, fin, part_first, unit_first; // from lw_place
+};
+
+__device__ __forceinline__ void lw_measure(LwSplit &x, u32 nL, GrowCfg const &cfg, u32 unit_target)
+{
+    u32 const nR = x.cnt - nL;
+    x.nL = nL;
+    x.demoted = (nL == 0) != (nR == 0) ? 1u : 0u;
+    x.leaves = static_cast<int>(x.depth) + 1 >= cfg.max_depth ? 1u : 0u;
+    x.left_small = nL <= nR ? 1u : 0u;
+    x.small_cnt = x.left_small ? nL : nR;
+    x.small_off = x.left_small ? x.off : x.off + nL;
+    x.urows = lw_unit_rows(x.small_cnt, unit_target);
+    x.units = x.demoted || x.leaves ? 0u : (x.small_cnt + x.urows - 1) / x.urows;
+}
+
+// Slots, finish ops, units and partials of the round's splits, in order (one thread);
+// fresh: the top kLwBatch free slots, top first.
+__device__ __forceinline__ void lw_place(LwSplit *x, u32 n, u32 const *fresh, u32 *free_slots, LwCtl *lw, TreeCtl *ctl)
+{
+    u32 fin = 0, units = 0, parts = 0;
+    for (u32 j = 0; j < n; ++j) {
+        if (x[j].demoted || x[j].leaves) continue;
+        x[j].fresh = fresh[fin];
+        x[j].fin = fin++;
+        x[j].unit_first = units;
+        x[j].part_first = parts;
+        units += x[j].units;
+        parts += x[j].units > 1 ? x[j].units : 0u;
     }
-    __syncthreads();
-    if (threadIdx.x < 64u) {
-        u32 const nw = blockDim.x >> 6;
-        bg = threadIdx.x < nw ? s_wg[threadIdx.x] : 0.0;
-        bid = threadIdx.x < nw ? s_wid[threadIdx.x] : kNone;
-        bix = threadIdx.x < nw ? s_wix[threadIdx.x] : kNone;
-        for (int o = 32; o > 0; o >>= 1) {
-            double const og = __shfl_xor(bg, o);
-            u32 const oid = __shfl_xor(bid, o), oix = __shfl_xor(bix, o);
-            if (oix != kNone && (bix == kNone || og > bg || (og == bg && oid < bid))) {
-                bg = og;
-                bid = oid;
-                bix = oix;
+    u32 nf = lw->n_free - fin;
+    for (u32 j = 0; j < n; ++j)
+        if (x[j].demoted || x[j].leaves) free_slots[nf++] = x[j].slot;
+    lw->n_free = nf;
+    ctl->n_front = 2u * n;
+    ctl->n_finish = fin;
+    ctl->n_hist_chunks = units;
+}
+
+// The round's children (commit_pop, src/grower_impl.hpp:370-400): the larger keeps the
+// parent's histogram slot (completed in place), the smaller gets the fresh one and the
+// histogram units.  Children at max_depth only need totals, from the split's sums, as do
+// all quantized ones (exact integers).
+template <bool Q>
+__device__ __forceinline__ void lw_children(LwSplit const *xs, u32 n, LwCtl *lw, LwRec *recs, NodeInfo *kids,
+                                            FinishOp *fops, HistChunk *hch)
+{
+    if (threadIdx.x < n) {
+        u32 const j = threadIdx.x;
+        LwSplit const x = xs[j];
+        SplitRec const s = recs[x.rec].split;
+        NodeInfo L{}, R{};
+        L.id = x.left_id;
+        R.id = x.left_id + 1u;
+        L.off = x.off;
+        L.cnt = x.nL;
+        R.off = x.off + x.nL;
+        R.cnt = x.cnt - x.nL;
+        L.src = R.src = x.dst;
+        L.depth = R.depth = x.depth + 1u;
+        if (Q || x.leaves) {
+            L.totals_ready = R.totals_ready = 1;
+            if (Q) {
+                L.itg = s.igL;
+                L.ith = s.ihL;
+                R.itg = s.igR;
+                R.ith = s.ihR;
+            } else {
+                L.tg = static_cast<float>(s.gL);
+                L.th = static_cast<float>(s.hL);
+                R.tg = static_cast<float>(s.gR);
+                R.th = static_cast<float>(s.hR);
             }
         }
+        if (x.demoted || x.leaves) {
+            L.slot = R.slot = kNone;
+        } else {
+            L.slot = x.left_small ? x.fresh : x.slot;
+            R.slot = x.left_small ? x.slot : x.fresh;
+            FinishOp fo{};
+            fo.small_slot = x.fresh;
+            fo.large_slot = x.slot;
+            fo.parent_slot = x.slot;
+            fo.part_first = x.part_first;
+            fo.part_count = x.units > 1 ? x.units : 0;
+            fo.empty = x.small_cnt == 0;
+            fops[x.fin] = fo;
+        }
+        kids[2 * j] = L;
+        kids[2 * j + 1] = R;
+        lw->batch[j] = x.rec;
+        lw->demoted[j] = x.demoted;
     }
+    for (u32 j = 0; j < n; ++j) {
+        u32 const units = xs[j].units;
+        for (u32 k = threadIdx.x; k < units; k += blockDim.x) {
+            HistChunk hc{};
+            hc.slot = xs[j].fresh;
+            hc.src = xs[j].dst;
+            hc.begin = xs[j].small_off + k * xs[j].urows;
+            hc.end = xs[j].small_off + min(xs[j].small_cnt, (k + 1) * xs[j].urows);
+            hc.part = units > 1 ? xs[j].part_first + k : kNone;
+            hch[xs[j].unit_first + k] = hc;
+        }
+    }
+}
+
+// A record's meta word: bits 0..1 the state, bit 2 a valid split, then the unit bound of
+// the child it would build.  Quantized splits whose children need no histogram are born
+// expanded (at max_depth) or demoted (one side without rows).
+constexpr u32 kLwValid = 4u;
+template <bool COUNTED> __device__ __forceinline__ u32 lw_meta(LwRec const &c, GrowCfg const &cfg, u32 unit_target)
+{
+    if (!c.split.valid) return kLwExpanded;
+    u32 const nL = c.split.n_left, nR = c.node.cnt - nL;
+    u32 state = kLwPlain;
+    if (COUNTED && (nL == 0) != (nR == 0)) state = kLwDemoted;
+    else if (COUNTED && static_cast<int>(c.node.depth) + 1 >= cfg.max_depth) state = kLwExpanded;
+    return state | kLwValid | lw_unit_bound(COUNTED ? min(nL, nR) : c.node.cnt / 2u, unit_target) << 3;
+}
+__device__ __forceinline__ bool lw_listed(u32 meta) { return (meta & 7u) == (kLwPlain | kLwValid); }
+
+// Round start: the last round's children become records, then leaves are popped while
+// the best one is expanded (max gain, ties to the lower node id; the reference's
+// gain_less, src/grower_impl.hpp:763-770), each committing its split
+// (commit_split_node, :188-210) and queueing its children (:404-428), until the pool is
+// empty, the leaf budget is spent or the best leaf has no children yet.  Then the round's
+// leaves are chosen and their partition ops emitted, in chunks sized to each leaf.
+// COUNTED (quantized): a split carries its child row counts, so the children, their slots
+// and the histogram units are set here, the scatter takes each chunk's prefix from the
+// chunk counts, and a split whose children need no histogram (at max_depth, the last one
+// of the budget, demoted) takes no round at all.  Runs as its own one-block kernel for the
+// first round and in the last workgroup of every round's split find for the next; any
+// workgroup size that is a multiple of 64.  Bound by latency, so the pops and the choice
+// run in one wave over what they need of every record in LDS, and the popped nodes, the
+// ops and the children are then written in parallel.
+template <bool COUNTED>
+__device__ __forceinline__ void lw_select_round(TreeCtl *__restrict__ ctl, LwCtl *__restrict__ lw, LwLists const &ls,
+                                                NodeInfo *__restrict__ kids, SplitRec const *__restrict__ kid_splits,
+                                                DevNode *__restrict__ tree, PartOp *__restrict__ ops,
+                                                PartChunk *__restrict__ pch, HistChunk *__restrict__ hch,
+                                                u16 const *__restrict__ n_bins, FinishOp *__restrict__ fops,
+                                                GrowCfg const &cfg, double const *__restrict__ scales)
+{
+    __shared__ double s_pg[kLwPoolCap], s_lv[kLwListCap], s_gain[kLwRecCap];
+    __shared__ u32 s_pid[kLwPoolCap], s_prec[kLwPoolCap], s_lrec[kLwListCap];
+    __shared__ u32 s_link[kLwRecCap], s_meta[kLwRecCap], s_pop_rec[kLwPoolCap], s_pop_id[kLwPoolCap];
+    __shared__ LwSplit s_x[kLwBatch];
+    __shared__ u32 s_nl, s_np, s_free, s_act, s_pops, s_n, s_sel[kLwBatch], s_fresh[kLwBatch];
+    __shared__ u32 s_chunk[kLwBatch + 1], s_crow[kLwBatch], s_deep;
+    if (ctl->done) return; // every work list is empty
+    bool const one = cfg.mono || cfg.n_groups; // final ids while expanding
+    u32 const nb = lw->n_batch, r0 = lw->n_rec, np0 = lw->n_pool, nl0 = lw->n_list;
     if (threadIdx.x == 0) {
-        bool const budget = cfg.max_leaves == 0 || ctl->live < static_cast<u32>(cfg.max_leaves);
-        s_go = (n > 0 && budget) ? 1u : 0u;
-        s_sel = bix;
-        if (!s_go) {
+        s_nl = nl0;
+        s_free = lw->n_free;
+        s_deep = ctl->max_depth_seen;
+    }
+    for (u32 k = threadIdx.x; k < np0; k += blockDim.x) {
+        s_pg[k] = ls.pool_gain[k];
+        s_pid[k] = ls.pool_id[k];
+        s_prec[k] = ls.pool_rec[k];
+    }
+    for (u32 k = threadIdx.x; k < nl0; k += blockDim.x) {
+        s_lv[k] = ls.list_prio[k];
+        s_lrec[k] = ls.list_rec[k];
+    }
+    for (u32 k = threadIdx.x; k < r0; k += blockDim.x) {
+        s_gain[k] = ls.gain[k];
+        s_link[k] = ls.link[k];
+        s_meta[k] = ls.meta[k];
+    }
+    __syncthreads();
+    // The round's children.
+    if (threadIdx.x < 2u * nb) {
+        u32 const j = threadIdx.x >> 1, e = threadIdx.x & 1u, p = lw->batch[j], r = r0 + threadIdx.x;
+        bool const gone = lw->demoted[j] != 0;
+        if (e == 0) {
+            s_link[p] = ls.link[p] = r;
+            s_meta[p] = ls.meta[p] = (s_meta[p] & ~3u) | (gone ? kLwDemoted : kLwExpanded);
+        }
+        u32 meta = 0;
+        double gain = 0.0;
+        if (!gone) {
+            LwRec &par = ls.recs[p];
+            LwRec c{};
+            c.node = kids[threadIdx.x];
+            c.split = kid_splits[threadIdx.x];
+            c.value = node_value(c.node, cfg, scales);
+            c.prio = min(par.prio, c.split.gain);
+            gain = c.split.gain;
+            meta = lw_meta<COUNTED>(c, cfg, ls.unit_target);
+            if (lw_listed(meta)) {
+                u32 const k = atomicAdd(&s_nl, 1u);
+                s_lv[k] = c.prio;
+                s_lrec[k] = r;
+            } else if (c.node.slot != kNone) {
+                ls.free_slots[atomicAdd(&s_free, 1u)] = c.node.slot;
+            }
+            ls.recs[r] = c;
+            par.kval[e] = c.value;
+            par.kcnt[e] = c.node.cnt;
+        }
+        s_gain[r] = ls.gain[r] = gain;
+        s_link[r] = ls.link[r] = kNone;
+        s_meta[r] = ls.meta[r] = meta;
+    }
+    __syncthreads();
+    // Pops, then the round's leaves: one wave, on LDS alone.
+    u32 const max_leaves = static_cast<u32>(cfg.max_leaves), limit = max_leaves + 7u; // pops of one tree
+    u32 const n_nodes = ctl->n_nodes;
+    if (threadIdx.x < 64u) {
+        u32 const lane = threadIdx.x;
+        u32 np = np0, live = ctl->live, ahead = lw->n_ahead, k = 0, act, block = 0;
+        u32 const pops = lw->pops;
+        for (;;) {
+            act = 2; // the tree is complete
+            if (np == 0 || live >= max_leaves || pops + k >= limit) break;
+            u32 const ix = lw_argmax(s_pg, s_pid, np);
+            u32 const r = s_prec[ix], id = s_pid[ix], meta = s_meta[r], link = s_link[r], lid = n_nodes + 2u * k;
+            act = 1; // waits for this leaf's children
+            block = r;
+            if ((meta & 3u) == kLwPlain && !(COUNTED && live + 1u >= max_leaves)) break;
+            np -= 1;
+            double const lg = s_pg[np];
+            u32 const li = s_pid[np], lr = s_prec[np];
+            lw_wave_sync();
+            if (lane == 0) {
+                s_pop_rec[k] = r;
+                s_pop_id[k] = id;
+                s_pg[ix] = lg;
+                s_pid[ix] = li;
+                s_prec[ix] = lr;
+            }
+            ++k;
+            if (link != kNone) ahead -= 1;
+            if ((meta & 3u) != kLwDemoted) {
+                live += 1;
+                if (link != kNone)
+                    for (u32 e = 0; e < 2; ++e)
+                        if (s_meta[link + e] & kLwValid) {
+                            if (lane == 0) {
+                                s_pg[np] = s_gain[link + e];
+                                s_pid[np] = lid + e;
+                                s_prec[np] = link + e;
+                            }
+                            np += 1;
+                        }
+            }
+            lw_wave_sync();
+        }
+        u32 n = 0, nl = s_nl;
+        if (act == 1) {
+            // The leaf the pops wait for, then the best others, while their partials fit
+            // and children are expected to be asked for.
+            u32 kmax = 1, parts = 0;
+            if (!one) {
+                u32 const left = max_leaves - live;
+                kmax = min(kLwBatch, max(1u, COUNTED ? left - 1u : left));
+                kmax = max(1u, min(kmax, kLwAhead - min(kLwAhead, ahead)));
+            }
+            while (n < kmax && nl > 0) {
+                u32 ix = kNone;
+                if (n == 0) {
+                    for (u32 q = lane; q < nl; q += 64u)
+                        if (s_lrec[q] == block) ix = q;
+                    for (int o = 32; o > 0; o >>= 1) ix = min(ix, static_cast<u32>(__shfl_xor(ix, o)));
+                } else {
+                    ix = lw_argmax(s_lv, s_lrec, nl);
+                }
+                u32 const r = s_lrec[ix], ub = s_meta[r] >> 3;
+                if (n > 0 && parts + ub > ls.max_parts) break;
+                parts += ub;
+                nl -= 1;
+                double const lv = s_lv[nl];
+                u32 const lr = s_lrec[nl];
+                lw_wave_sync();
+                if (lane == 0) {
+                    s_sel[n] = r;
+                    s_lv[ix] = lv;
+                    s_lrec[ix] = lr;
+                }
+                lw_wave_sync();
+                ++n;
+            }
+        }
+        if (lane == 0) {
+            ctl->live = live;
+            ctl->n_nodes = n_nodes + 2u * k;
+            lw->pops = pops + k;
+            lw->n_ahead = ahead + n;
+            lw->n_rec = r0 + 2u * nb;
+            lw->n_batch = n;
+            lw->n_pool = np;
+            lw->n_list = nl;
+            s_np = np;
+            s_nl = nl;
+            s_act = act;
+            s_pops = k;
+            s_n = n;
+        }
+    }
+    __syncthreads();
+    // The popped leaves' splits in the tree (commit_split_node, :188-210): children first,
+    // since a child may have been popped as well.
+    u32 const n_pops = s_pops;
+    for (u32 k = threadIdx.x; k < n_pops; k += blockDim.x) {
+        u32 const id = s_pop_id[k], lid = n_nodes + 2u * k, rid = lid + 1u, r = s_pop_rec[k];
+        LwRec const &c = ls.recs[r];
+        DevNode l{}, rr{};
+        l.feature = rr.feature = -1;
+        if ((s_meta[r] & 3u) != kLwDemoted) {
+            atomicMax(&s_deep, c.node.depth + 1u);
+            if (s_link[r] == kNone) { // never expanded: leaves from the split's sums
+                if (one) {
+                    fd_propagate_bounds(cfg, scales, id, c.split, lid, rid);
+                    fd_propagate_path(cfg, id, c.split.feature, lid, rid);
+                }
+                NodeInfo x{}, y{};
+                x.id = lid;
+                x.itg = c.split.igL;
+                x.ith = c.split.ihL;
+                y.id = rid;
+                y.itg = c.split.igR;
+                y.ith = c.split.ihR;
+                l.value = node_value(x, cfg, scales);
+                rr.value = node_value(y, cfg, scales);
+                l.cover = static_cast<float>(c.split.n_left);
+                rr.cover = static_cast<float>(c.node.cnt - c.split.n_left);
+            } else {
+                l.value = c.kval[0];
+                rr.value = c.kval[1];
+                l.cover = static_cast<float>(c.kcnt[0]);
+                rr.cover = static_cast<float>(c.kcnt[1]);
+            }
+        }
+        tree[lid] = l;
+        tree[rid] = rr;
+    }
+    __syncthreads();
+    for (u32 k = threadIdx.x; k < n_pops; k += blockDim.x) {
+        u32 const lid = n_nodes + 2u * k, r = s_pop_rec[k];
+        LwRec const &c = ls.recs[r];
+        DevNode pn{};
+        pn.cover = static_cast<float>(c.node.cnt);
+        if ((s_meta[r] & 3u) == kLwDemoted) {
+            pn.feature = -1;
+            pn.value = c.value;
+        } else {
+            pn.feature = static_cast<int32_t>(c.split.feature);
+            pn.bin = c.split.bin;
+            pn.default_left = c.split.default_left;
+            pn.left = lid;
+            pn.right = lid + 1u;
+            pn.gain = static_cast<float>(c.split.gain);
+        }
+        tree[s_pop_id[k]] = pn;
+    }
+    if (threadIdx.x == 0) ctl->max_depth_seen = s_deep;
+    u32 const n = s_n;
+    if (s_act == 2u) {
+        if (threadIdx.x == 0) {
             ctl->done = 1;
             ctl->n_ops = 0;
             ctl->n_part_chunks = 0;
@@ -856,111 +1038,107 @@ __device__ __forceinline__ void lw_select_round(TreeCtl *__restrict__ ctl, LwCtl
             ctl->n_finish = 0;
             ctl->n_hist_chunks = 0;
         }
+        return;
     }
-    __syncthreads();
-    if (!s_go) return;
-    if (threadIdx.x == 0) {
-        Cand const c = cands[s_sel];
-        u32 const crow = lw_chunk_rows(c.node.cnt, chunk_cap);
-        u32 const nch = (c.node.cnt + crow - 1) / crow;
-        s_ccnt = c.node.cnt;
-        s_crow = crow;
-        s_nch = nch;
-        // remove from the pool (order inside the pool is irrelevant)
-        cands[s_sel] = cands[n - 1];
-        lw->n_cand = n - 1;
-        u32 const lid = ctl->n_nodes, rid = lid + 1;
-        ctl->n_nodes = lid + 2;
-        DevNode pn = tree[c.node.id];
-        pn.feature = static_cast<int32_t>(c.split.feature);
-        pn.bin = c.split.bin;
-        pn.default_left = c.split.default_left;
-        pn.left = lid;
-        pn.right = rid;
-        pn.value = 0.0F;
-        pn.gain = static_cast<float>(c.split.gain);
-        tree[c.node.id] = pn;
-        DevNode leaf{};
-        leaf.feature = -1;
-        tree[lid] = leaf;
-        tree[rid] = leaf;
-        parent_out[0] = c.node;
-        split_out[0] = c.split;
-        fd_propagate_bounds(cfg, scales, c.node.id, c.split, lid, rid);
-        fd_propagate_path(cfg, c.node.id, c.split.feature, lid, rid);
-        PartOp op{};
-        op.parent = 0;
-        op.feature = c.split.feature;
-        op.bin = c.split.bin;
-        op.default_left = c.split.default_left;
-        op.last_bin = static_cast<u32>(n_bins[c.split.feature]) - 1u;
-        op.off = c.node.off;
-        op.cnt = c.node.cnt;
-        op.src = c.node.src;
-        op.dst = c.node.src == 0 ? 1u : 0u;
-        op.chunk_first = 0;
-        op.chunk_count = nch;
-        op.left_id = lid;
-        op.right_id = rid;
-        op.alive = 1;
-        lw->parent_slot = c.node.slot;
+    for (u32 k = threadIdx.x; k < s_np; k += blockDim.x) {
+        ls.pool_gain[k] = s_pg[k];
+        ls.pool_id[k] = s_pid[k];
+        ls.pool_rec[k] = s_prec[k];
+    }
+    for (u32 k = threadIdx.x; k < s_nl; k += blockDim.x) {
+        ls.list_prio[k] = s_lv[k];
+        ls.list_rec[k] = s_lrec[k];
+    }
+    if (threadIdx.x < n) {
+        u32 const j = threadIdx.x, r = s_sel[j];
+        NodeInfo const nd = ls.recs[r].node;
+        SplitRec const s = ls.recs[r].split;
+        LwSplit x{};
+        x.rec = r;
+        x.cnt = nd.cnt;
+        x.off = nd.off;
+        x.dst = nd.src == 0 ? 1u : 0u;
+        x.slot = nd.slot;
+        x.depth = nd.depth;
+        x.left_id = one ? n_nodes + 2u * n_pops : 0u;
         if (COUNTED) {
-            FinishOp fo{};
-            u32 urows = kHistChunk;
-            s_units = lw_children<true>(op, c.split.n_left, ctl, lw, c.node, c.split, free_slots, kids, tree, cfg,
-                                        scales, true, unit_target, fo, urows);
-            lw_stash_units(s_fo, fo);
-            s_urows = urows;
-            if (s_units) fops[0] = fo;
+            lw_measure(x, s.n_left, cfg, ls.unit_target);
+            s_fresh[j] = ls.free_slots[s_free - 1u - j];
         }
-        ops[0] = op;
-        ctl->n_ops = 1;
-        ctl->n_part_chunks = nch;
+        s_x[j] = x;
+        s_crow[j] = lw_chunk_rows(nd.cnt, ls.chunk_cap);
+        s_chunk[j] = (nd.cnt + s_crow[j] - 1u) / s_crow[j];
+        if (one) { // only the leaf the pops wait for: its children's ids are the next two
+            fd_propagate_bounds(cfg, scales, nd.id, s, x.left_id, x.left_id + 1u);
+            fd_propagate_path(cfg, nd.id, s.feature, x.left_id, x.left_id + 1u);
+        }
+        PartOp op{};
+        op.parent = r;
+        op.feature = s.feature;
+        op.bin = s.bin;
+        op.default_left = s.default_left;
+        op.last_bin = static_cast<u32>(n_bins[s.feature]) - 1u;
+        op.off = nd.off;
+        op.cnt = nd.cnt;
+        op.src = nd.src;
+        op.dst = x.dst;
+        op.chunk_count = s_chunk[j];
+        op.left_id = x.left_id;
+        op.n_left = COUNTED ? x.nL : 0u;
+        op.alive = 1;
+        ops[j] = op;
     }
     __syncthreads();
-    u32 const crow = s_crow, nch = s_nch, ccnt = s_ccnt;
-    for (u32 k = threadIdx.x; k < nch; k += blockDim.x) {
-        PartChunk pc;
-        pc.op = 0;
-        pc.begin = k * crow;
-        pc.end = min(ccnt, (k + 1) * crow);
-        pc.left_before = 0;
-        pch[k] = pc;
+    if (threadIdx.x == 0) {
+        u32 c = 0;
+        for (u32 j = 0; j < n; ++j) {
+            u32 const k = s_chunk[j];
+            s_chunk[j] = c;
+            c += k;
+        }
+        s_chunk[n] = c;
+        lw->n_free = s_free;
+        if (COUNTED) lw_place(s_x, n, s_fresh, ls.free_slots, lw, ctl);
+        ctl->n_ops = n;
+        ctl->n_part_chunks = c;
     }
-    if (COUNTED) lw_expand_units(s_fo, s_units, s_urows, hch);
+    __syncthreads();
+    if (threadIdx.x < n) ops[threadIdx.x].chunk_first = s_chunk[threadIdx.x];
+    for (u32 j = 0; j < n; ++j)
+        for (u32 k = threadIdx.x; k < s_chunk[j + 1] - s_chunk[j]; k += blockDim.x) {
+            PartChunk pc;
+            pc.op = j;
+            pc.begin = k * s_crow[j];
+            pc.end = min(s_x[j].cnt, (k + 1) * s_crow[j]);
+            pc.left_before = 0;
+            pch[s_chunk[j] + k] = pc;
+        }
+    if (COUNTED) lw_children<true>(s_x, n, lw, ls.recs, kids, fops, hch);
 }
 
 template <bool COUNTED>
-__global__ __launch_bounds__(256) void k_lw_select(TreeCtl *__restrict__ ctl, LwCtl *__restrict__ lw,
-                                                   Cand *__restrict__ cands, NodeInfo *__restrict__ kids,
-                                                   SplitRec const *__restrict__ kid_splits,
-                                                   u32 *__restrict__ free_slots, NodeInfo *__restrict__ parent_out,
-                                                   SplitRec *__restrict__ split_out, DevNode *__restrict__ tree,
+__global__ __launch_bounds__(256) void k_lw_select(TreeCtl *__restrict__ ctl, LwCtl *__restrict__ lw, LwLists ls,
+                                                   NodeInfo *__restrict__ kids,
+                                                   SplitRec const *__restrict__ kid_splits, DevNode *__restrict__ tree,
                                                    PartOp *__restrict__ ops, PartChunk *__restrict__ pch,
                                                    HistChunk *__restrict__ hch, u16 const *__restrict__ n_bins,
                                                    FinishOp *__restrict__ fops, GrowCfg cfg,
-                                                   double const *__restrict__ scales, u32 unit_target, u32 chunk_cap)
+                                                   double const *__restrict__ scales)
 {
-    lw_select_round<COUNTED>(ctl, lw, cands, kids, kid_splits, free_slots, parent_out, split_out, tree, ops, pch, hch,
-                             n_bins, fops, cfg, scales, unit_target, chunk_cap);
+    lw_select_round<COUNTED>(ctl, lw, ls, kids, kid_splits, tree, ops, pch, hch, n_bins, fops, cfg, scales);
 }
 
 // Split find of a round's children (k_find's body) whose last workgroup to finish -- all
-// others have stopped reading anything the select writes -- starts the next round
-// (next != 0).
+// others have stopped reading anything the select writes -- starts the next round and,
+// when the host waits for it, reports whether the tree is complete.
 struct LwNext {
-    Cand *cands;
-    u32 *free_slots;
-    NodeInfo *parent_out;
-    SplitRec *split_out;
+    LwLists ls;
     DevNode *tree;
     PartOp *ops;
     PartChunk *pch;
     HistChunk *hch;
     FinishOp *fops;
-    u32 unit_target;
-    u32 chunk_cap;
-    u32 next;
+    u32 *report; // pinned host memory, or null
 };
 
 template <bool Q, bool COUNTED, bool CON>
@@ -973,7 +1151,6 @@ __global__ __launch_bounds__(kFindThreads) void k_lw_find(NodeInfo *__restrict__
 {
     __shared__ u32 s_last_wg;
     find_node<Q, CON, kLwFindTile>(kids, ctl, hist, n_bins, F, SB, cfg, scales, splits, 0u, 0u, part, done, cnt);
-    if (!nx.next) return;
     __syncthreads();
     if (threadIdx.x == 0) {
         __threadfence();
@@ -981,29 +1158,31 @@ __global__ __launch_bounds__(kFindThreads) void k_lw_find(NodeInfo *__restrict__
     }
     __syncthreads();
     if (!s_last_wg) return;
-    if (threadIdx.x == 0) {
-        lw->grid_done = 0u;
-        __threadfence();
-    }
+    if (threadIdx.x == 0) lw->grid_done = 0u;
+    __threadfence();
     __syncthreads();
-    lw_select_round<COUNTED>(ctl, lw, nx.cands, kids, splits, nx.free_slots, nx.parent_out, nx.split_out, nx.tree,
-                             nx.ops, nx.pch, nx.hch, n_bins, nx.fops, cfg, scales, nx.unit_target, nx.chunk_cap);
+    lw_select_round<COUNTED>(ctl, lw, nx.ls, kids, splits, nx.tree, nx.ops, nx.pch, nx.hch, n_bins, nx.fops, cfg,
+                             scales);
+    if (nx.report && threadIdx.x == 0) {
+        *nx.report = ctl->done;
+        __threadfence_system();
+    }
 }
 
-// Round middle of the FP32 grower: left count from the chunk prefix, then the children
-// (lw_children) and the smaller child's histogram units.
+// Round middle of the FP32 grower: left counts from the chunk prefixes, then the
+// children and their histogram units.
 template <bool Q>
 __global__ __launch_bounds__(1024) void k_lw_scan(PartOp *__restrict__ ops, PartChunk *__restrict__ pch,
                                                   u32 const *__restrict__ chunk_left, TreeCtl *__restrict__ ctl,
-                                                  LwCtl *__restrict__ lw, NodeInfo const *__restrict__ parent_in,
-                                                  SplitRec const *__restrict__ split_in, u32 *__restrict__ free_slots,
-                                                  NodeInfo *__restrict__ kids, DevNode *__restrict__ tree,
+                                                  LwCtl *__restrict__ lw, LwLists ls, NodeInfo *__restrict__ kids,
                                                   HistChunk *__restrict__ hch, FinishOp *__restrict__ fops,
-                                                  GrowCfg cfg, double const *__restrict__ scales, u32 unit_target)
+                                                  GrowCfg cfg)
 {
     __shared__ u32 scratch[1024];
-    __shared__ u32 s_run, s_units, s_urows, s_fo[4];
-    if (ctl->n_ops == 0) return;
+    __shared__ u32 s_run, s_base[kLwBatch + 1], s_fresh[kLwBatch];
+    __shared__ LwSplit s_x[kLwBatch];
+    u32 const n = ctl->n_ops;
+    if (n == 0) return;
     u32 const n_ch = ctl->n_part_chunks;
     if (threadIdx.x == 0) s_run = 0;
     __syncthreads();
@@ -1012,54 +1191,71 @@ __global__ __launch_bounds__(1024) void k_lw_scan(PartOp *__restrict__ ops, Part
         u32 const v = c < n_ch ? chunk_left[c] : 0u;
         u32 tot;
         u32 const pre = block_exscan(v, scratch, &tot) + s_run;
-        if (c < n_ch) pch[c].left_before = pre;
+        if (c < n_ch) {
+            u32 const j = pch[c].op;
+            pch[c].left_before = pre;
+            if (c == ops[j].chunk_first) s_base[j] = pre;
+        }
         __syncthreads();
         if (threadIdx.x == 0) s_run += tot;
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        PartOp op = ops[0];
-        FinishOp fo{};
-        u32 urows = kHistChunk;
-        s_units = lw_children<Q>(op, s_run, ctl, lw, parent_in[0], split_in[0], free_slots, kids, tree, cfg, scales,
-                                 false, unit_target, fo, urows);
-        ops[0] = op;
-        lw_stash_units(s_fo, fo);
-        s_urows = urows;
-        if (s_units) fops[0] = fo;
+    if (threadIdx.x == 0) s_base[n] = s_run;
+    __syncthreads();
+    for (u32 c = threadIdx.x; c < n_ch; c += blockDim.x) pch[c].left_before -= s_base[pch[c].op];
+    if (threadIdx.x < n) {
+        PartOp op = ops[threadIdx.x];
+        LwSplit x{};
+        x.rec = op.parent;
+        x.cnt = op.cnt;
+        x.off = op.off;
+        x.dst = op.dst;
+        x.left_id = op.left_id;
+        x.slot = ls.recs[x.rec].node.slot;
+        x.depth = ls.recs[x.rec].node.depth;
+        lw_measure(x, s_base[threadIdx.x + 1] - s_base[threadIdx.x], cfg, ls.unit_target);
+        op.n_left = x.nL;
+        op.alive = x.demoted ? 0u : 1u;
+        ops[threadIdx.x] = op;
+        s_x[threadIdx.x] = x;
+        s_fresh[threadIdx.x] = ls.free_slots[lw->n_free - 1u - threadIdx.x];
     }
     __syncthreads();
-    lw_expand_units(s_fo, s_units, s_urows, hch);
+    if (threadIdx.x == 0) lw_place(s_x, n, s_fresh, ls.free_slots, lw, ctl);
+    __syncthreads();
+    lw_children<Q>(s_x, n, lw, ls.recs, kids, fops, hch);
 }
 
 // The root's split joins the pool (or the root becomes a leaf).
-__global__ void k_lw_push_root(LwCtl *__restrict__ lw, NodeInfo const *__restrict__ kids,
-                               SplitRec const *__restrict__ splits, Cand *__restrict__ cands,
-                               u32 *__restrict__ free_slots, DevNode *__restrict__ tree, GrowCfg cfg,
+template <bool COUNTED>
+__global__ void k_lw_push_root(LwCtl *__restrict__ lw, LwLists ls, NodeInfo const *__restrict__ kids,
+                               SplitRec const *__restrict__ splits, DevNode *__restrict__ tree, GrowCfg cfg,
                                double const *__restrict__ scales)
 {
     if (threadIdx.x != 0) return;
-    lw_push(lw, kids, splits, 1, true, cands, free_slots, tree, cfg, scales);
-}
-
-// Tree end: the last round's children join the pool, then what is left in the pool
-// becomes leaves (src/grower_impl.hpp:838-846).
-__global__ void k_lw_finalize(TreeCtl *__restrict__ ctl, LwCtl *__restrict__ lw, Cand *__restrict__ cands,
-                              NodeInfo const *__restrict__ kids, SplitRec const *__restrict__ kid_splits,
-                              u32 *__restrict__ free_slots, DevNode *__restrict__ tree, GrowCfg cfg,
-                              double const *__restrict__ scales)
-{
-    __shared__ u32 s_n;
-    if (threadIdx.x == 0) {
-        u32 const np = lw->n_push;
-        if (np) lw_push(lw, kids, kid_splits, np, false, cands, free_slots, tree, cfg, scales);
-        lw->n_push = 0;
-        s_n = lw->n_cand;
+    LwRec c{};
+    c.node = kids[0];
+    c.split = splits[0];
+    c.value = node_value(c.node, cfg, scales);
+    c.prio = c.split.gain;
+    if (!c.split.valid || cfg.max_depth <= 0) {
+        put_leaf(tree, c.node.id, c.value);
+        return;
     }
-    __syncthreads();
-    u32 const n = s_n;
-    for (u32 k = threadIdx.x; k < n; k += blockDim.x) put_leaf(tree, cands[k].node.id, node_value(cands[k].node, cfg, scales));
-    (void)ctl;
+    u32 const meta = lw_meta<COUNTED>(c, cfg, ls.unit_target);
+    ls.recs[0] = c;
+    ls.pool_gain[0] = ls.gain[0] = c.split.gain;
+    ls.pool_id[0] = ls.pool_rec[0] = 0;
+    ls.link[0] = kNone;
+    ls.meta[0] = meta;
+    lw->n_rec = lw->n_pool = 1;
+    if (lw_listed(meta)) {
+        ls.list_prio[0] = c.prio;
+        ls.list_rec[0] = 0;
+        lw->n_list = 1;
+    } else {
+        ls.free_slots[lw->n_free++] = c.node.slot;
+    }
 }
 
 // Leafwise tree start: root frontier (slot 0), free list 1.., pool empty.
@@ -1108,9 +1304,9 @@ __global__ __launch_bounds__(256) void k_lw_begin(TreeCtl *__restrict__ ctl, LwC
         ctl->done = 0;
         ctl->live = 1;
         ctl->max_depth_seen = 0;
-        lw->n_cand = 0;
+        lw->n_pool = lw->n_list = lw->n_rec = lw->n_batch = 0;
+        lw->pops = lw->n_ahead = 0;
         lw->n_free = n_slots - 1;
-        lw->n_push = 0;
         lw->grid_done = 0;
     }
 }
@@ -1125,18 +1321,26 @@ __global__ void k_obl_begin(TreeCtl *ctl)
 
 } // namespace
 
-hipError_t ext_alloc(ExtState &s, bh_fit_config const &f, u32 F, u32 SB, u32 max_front, u32 hist_slots)
+hipError_t ext_alloc(ExtState &s, bh_fit_config const &f, u32 F, u32 hist_slots)
 {
-    (void)SB;
-    (void)max_front;
     s.n_features = F;
     hipError_t e;
     if (f.grower == BH_LEAFWISE) {
-        s.cap = static_cast<u32>(f.max_leaves) + 8u;
-        if ((e = hipMalloc(&s.cands, sizeof(Cand) * s.cap)) != hipSuccess) return e;
-        if ((e = hipMalloc(&s.free_slots, sizeof(u32) * (hist_slots + 4))) != hipSuccess) return e;
-        if ((e = hipMalloc(&s.pending, sizeof(LwCtl))) != hipSuccess) return e;
-        if ((e = hipMalloc(&s.feat_best, sizeof(SplitRec) * 4)) != hipSuccess) return e; // parent split
+        if ((e = hipMalloc(&s.ls.recs, sizeof(LwRec) * kLwRecCap)) != hipSuccess) return e;
+        if ((e = hipMalloc(&s.ls.pool_gain, sizeof(double) * (kLwPoolCap + kLwListCap + kLwRecCap))) != hipSuccess)
+            return e;
+        if ((e = hipMalloc(&s.ls.pool_id, sizeof(u32) * (2u * kLwPoolCap + kLwListCap + 2u * kLwRecCap))) != hipSuccess)
+            return e;
+        s.ls.list_prio = s.ls.pool_gain + kLwPoolCap;
+        s.ls.gain = s.ls.list_prio + kLwListCap;
+        s.ls.pool_rec = s.ls.pool_id + kLwPoolCap;
+        s.ls.list_rec = s.ls.pool_rec + kLwPoolCap;
+        s.ls.link = s.ls.list_rec + kLwListCap;
+        s.ls.meta = s.ls.link + kLwRecCap;
+        if ((e = hipMalloc(&s.ls.free_slots, sizeof(u32) * (hist_slots + 4))) != hipSuccess) return e;
+        if ((e = hipMalloc(&s.lw, sizeof(LwCtl))) != hipSuccess) return e;
+        if ((e = hipHostMalloc(reinterpret_cast<void **>(&s.report), sizeof(u32), hipHostMallocDefault)) != hipSuccess)
+            return e;
     }
     if (f.grower == BH_LEVELWISE) {
         if ((e = hipMalloc(&s.feat_best, sizeof(SplitRec) * (F + 2))) != hipSuccess) return e;
@@ -1149,9 +1353,11 @@ hipError_t ext_alloc(ExtState &s, bh_fit_config const &f, u32 F, u32 SB, u32 max
 
 void ext_free(ExtState &s)
 {
-    void *p[] = {s.cands, s.pending, s.free_slots, s.feat_best, s.level_splits, s.level_gains};
+    void *p[] = {s.ls.recs, s.ls.pool_gain, s.ls.pool_id, s.ls.free_slots, s.lw, s.feat_best, s.level_splits,
+                 s.level_gains};
     for (void *q : p)
         if (q) (void)hipFree(q);
+    if (s.report) (void)hipHostFree(s.report);
     s = ExtState{};
 }
 
@@ -1271,78 +1477,100 @@ void launch_level_find_step(ExtState &s, hipStream_t st, bool q, GrowView const 
                            v.F, v.SB, v.splits, v.ops, v.pch, 0u, 1u, part_chunk_rows(v.Fs, v.N), 0u);
 }
 
-// LeafwiseGrower::grow as a launch sequence: the root, then max_leaves - 1 rounds
-// (plus a margin for demoted splits, which spend a round without adding a leaf); rounds
-// after the heap empties or the budget is spent are no-ops.
 template <bool Q, bool COUNTED>
-void launch_lw_find(hipStream_t st, GrowView const &v, LwCtl *lw, u32 *cnt, LwNext const &nx)
+static void launch_lw_find(hipStream_t st, GrowView const &v, LwCtl *lw, u32 *cnt, LwNext const &nx)
 {
     size_t const lds = static_cast<size_t>(kLwFindTile) * v.SB * (Q ? (cnt ? 36 : 32) : 24);
-    dim3 const grid(find_blocks_per_node(v.F, kLwFindTile), 2);
+    dim3 const grid(find_blocks_per_node(v.F, kLwFindTile), 2u * lw_batch(v));
     bool const con = v.gc.fmask || v.gc.mono || v.gc.n_groups;
     auto const fn = con ? &k_lw_find<Q, COUNTED, true> : &k_lw_find<Q, COUNTED, false>;
     hipLaunchKernelGGL(fn, grid, dim3(kFindThreads), lds, st, v.front[0], v.ctl, lw, v.hist[0], v.d_nbins, v.F, v.SB,
                        v.gc, v.scales, v.splits, v.fscr.part, v.fscr.done, cnt, nx);
 }
 
+static LwLists lw_lists(ExtState const &s, GrowView const &v)
+{
+    LwLists ls = s.ls;
+    ls.unit_target = v.lw_units;
+    ls.chunk_cap = part_chunk_rows(v.Fs, v.N);
+    ls.max_parts = v.lw_parts;
+    return ls;
+}
+
+// Leaves a round expands at most; constrained fits one (their node ids are final).
+u32 lw_batch(GrowView const &v) { return v.gc.mono || v.gc.n_groups ? 1u : kLwBatch; }
+
+u32 lw_head_rounds(GrowView const &v)
+{
+    u32 const L = static_cast<u32>(v.fc.max_leaves), K = lw_batch(v);
+    return K == 1u ? L + 7u : std::min(L + 7u, (L - 1u + K - 1u) / K + 4u);
+}
+
+// `rounds` rounds; the last one's find reports to the host whether the tree is complete.
+// A complete tree turns rounds into no-ops.
+void enqueue_leafwise_rounds(ExtState &s, hipStream_t st, bool q, GrowView const &v, u32 rounds)
+{
+    u32 const gh_bytes = q ? 4 : 8, K = lw_batch(v);
+    LwCtl *lw = s.lw;
+    NodeInfo *kids = v.front[0];
+    void *pool = v.hist[0];
+    u32 *cnt = q ? v.cnt : nullptr;
+    LwLists const ls = lw_lists(s, v);
+    u32 const pgrid = std::max(1u, std::min(v.lw_pch, tuning().part_grid));
+    u32 const hgrid = std::max(1u, std::min(v.lw_parts, 4096u));
+    for (u32 r = 0; r < rounds; ++r) {
+        launch_part_count(st, v.pch, v.ops, v.ctl, v.work[0], v.work[1], v.plane0, v.Fs, v.chunk_left, pgrid);
+        if (!q)
+            hipLaunchKernelGGL(k_lw_scan<false>, dim3(1), dim3(1024), 0, st, v.ops, v.pch, v.chunk_left, v.ctl, lw, ls,
+                               kids, v.hch, v.fops, v.gc);
+        launch_part_scatter(st, v.pch, v.ops, v.ctl, v.work[0], v.work[1], v.plane0, v.gh[0], v.gh[1], v.gh[2],
+                            v.work[0], v.work[1], const_cast<void *>(v.gh[0]), const_cast<void *>(v.gh[1]), v.Fs,
+                            gh_bytes, pgrid, q ? v.chunk_left : nullptr);
+        launch_hist(st, q, v.hch, v.ctl, v.work[0], v.work[1], v.plane0, v.gh[0], v.gh[1], v.gh[2], v.Fs, v.F, v.SB,
+                    v.fsl, v.waves, hgrid, v.partials, pool, v.fx, cnt);
+        launch_finish(st, q, v.fops, v.ctl, v.partials, pool, pool, v.F * v.SB, K, cnt, cnt, false,
+                      hist_transpose_F(q, v.Fs, v.F));
+        LwNext const nx{ls, v.tree, v.ops, v.pch, v.hch, v.fops, r + 1 == rounds ? s.report : nullptr};
+        if (q) launch_lw_find<true, true>(st, v, lw, cnt, nx);
+        else launch_lw_find<false, false>(st, v, lw, cnt, nx);
+        if (v.host_sync) (void)hipStreamSynchronize(st);
+    }
+}
+
+// LeafwiseGrower::grow as a launch sequence: the root, then lw_head_rounds rounds.  More
+// may be needed (a chain of leaves each the next best): the caller looks at *s.report
+// and adds kLwMoreRounds at a time until the tree is complete.
 void enqueue_leafwise(ExtState &s, hipStream_t st, bool q, GrowView const &v)
 {
-    u32 const gh_bytes = q ? 4 : 8;
-    LwCtl *lw = reinterpret_cast<LwCtl *>(s.pending);
+    LwCtl *lw = s.lw;
     NodeInfo *kids = v.front[0];
-    NodeInfo *parent = v.front[1];
-    SplitRec *psplit = s.feat_best;
     void *pool = v.hist[0];
     // Quantized: count cells beside the histogram pool give every split its child row
     // counts (the counted round); FP32: the chunk counts are scanned on the device.
     u32 *cnt = q ? v.cnt : nullptr;
-    u32 const pgrid = std::max(1u, std::min(v.max_pch, tuning().part_grid));
+    LwLists const ls = lw_lists(s, v);
     u32 const hgrid = std::max(1u, std::min(v.max_hch, 4096u));
-    hipLaunchKernelGGL(k_lw_begin, dim3(1), dim3(256), 0, st, v.ctl, lw, kids, v.tree, v.hch, v.fops, s.free_slots,
+    hipLaunchKernelGGL(k_lw_begin, dim3(1), dim3(256), 0, st, v.ctl, lw, kids, v.tree, v.hch, v.fops, ls.free_slots,
                        s.hist_slots, v.root, v.lw_units);
     launch_hist(st, q, v.hch, v.ctl, v.work[0], v.work[1], v.plane0, v.gh[0], v.gh[1], v.gh[2], v.Fs, v.F, v.SB,
                 v.fsl, v.waves, hgrid, v.partials, pool, v.fx, cnt);
     launch_finish(st, q, v.fops, v.ctl, v.partials, pool, pool, v.F * v.SB, 1, cnt, cnt, false,
                       hist_transpose_F(q, v.Fs, v.F));
     launch_find(st, q, kids, v.ctl, pool, v.d_nbins, v.F, v.SB, v.gc, v.scales, v.splits, 2, 0, 0, v.fscr, cnt);
-    hipLaunchKernelGGL(k_lw_push_root, dim3(1), dim3(64), 0, st, lw, kids, v.splits, s.cands, s.free_slots, v.tree,
-                       v.gc, v.scales);
     // The first round's select is a kernel of its own; every later one runs in the last
     // workgroup of the previous round's split find.
-    if (q)
-        hipLaunchKernelGGL(k_lw_select<true>, dim3(1), dim3(256), 0, st, v.ctl, lw, s.cands, kids, v.splits,
-                           s.free_slots, parent, psplit, v.tree, v.ops, v.pch, v.hch, v.d_nbins, v.fops, v.gc, v.scales,
-                           v.lw_units, part_chunk_rows(v.Fs, v.N));
-    else
-        hipLaunchKernelGGL(k_lw_select<false>, dim3(1), dim3(256), 0, st, v.ctl, lw, s.cands, kids, v.splits,
-                           s.free_slots, parent, psplit, v.tree, v.ops, v.pch, v.hch, v.d_nbins, v.fops, v.gc, v.scales,
-                           0u, part_chunk_rows(v.Fs, v.N));
-    u32 const rounds = static_cast<u32>(v.fc.max_leaves) - 1u + 8u;
-    for (u32 r = 0; r < rounds; ++r) {
-        launch_part_count(st, v.pch, v.ops, v.ctl, v.work[0], v.work[1], v.plane0, v.Fs, v.chunk_left, pgrid);
-        if (q) {
-            launch_part_scatter(st, v.pch, v.ops, v.ctl, v.work[0], v.work[1], v.plane0, v.gh[0], v.gh[1],
-                                v.gh[2], v.work[0], v.work[1], const_cast<void *>(v.gh[0]),
-                                const_cast<void *>(v.gh[1]), v.Fs, gh_bytes, pgrid, v.chunk_left);
-        } else {
-            hipLaunchKernelGGL(k_lw_scan<false>, dim3(1), dim3(1024), 0, st, v.ops, v.pch, v.chunk_left, v.ctl, lw,
-                               parent, psplit, s.free_slots, kids, v.tree, v.hch, v.fops, v.gc, v.scales, v.lw_units);
-            launch_part_scatter(st, v.pch, v.ops, v.ctl, v.work[0], v.work[1], v.plane0, v.gh[0], v.gh[1],
-                                v.gh[2], v.work[0], v.work[1], const_cast<void *>(v.gh[0]),
-                                const_cast<void *>(v.gh[1]), v.Fs, gh_bytes, pgrid);
-        }
-        launch_hist(st, q, v.hch, v.ctl, v.work[0], v.work[1], v.plane0, v.gh[0], v.gh[1], v.gh[2], v.Fs, v.F, v.SB,
-                    v.fsl, v.waves, hgrid, v.partials, pool, v.fx, cnt);
-        launch_finish(st, q, v.fops, v.ctl, v.partials, pool, pool, v.F * v.SB, 1, cnt, cnt, false,
-                      hist_transpose_F(q, v.Fs, v.F));
-        LwNext const nx{s.cands, s.free_slots, parent, psplit, v.tree, v.ops, v.pch, v.hch, v.fops, v.lw_units,
-                        part_chunk_rows(v.Fs, v.N), r + 1 < rounds ? 1u : 0u};
-        if (q) launch_lw_find<true, true>(st, v, lw, cnt, nx);
-        else launch_lw_find<false, false>(st, v, lw, cnt, nx);
-        if (v.host_sync) (void)hipStreamSynchronize(st);
+    if (q) {
+        hipLaunchKernelGGL(k_lw_push_root<true>, dim3(1), dim3(64), 0, st, lw, ls, kids, v.splits, v.tree, v.gc,
+                           v.scales);
+        hipLaunchKernelGGL(k_lw_select<true>, dim3(1), dim3(256), 0, st, v.ctl, lw, ls, kids, v.splits, v.tree, v.ops,
+                           v.pch, v.hch, v.d_nbins, v.fops, v.gc, v.scales);
+    } else {
+        hipLaunchKernelGGL(k_lw_push_root<false>, dim3(1), dim3(64), 0, st, lw, ls, kids, v.splits, v.tree, v.gc,
+                           v.scales);
+        hipLaunchKernelGGL(k_lw_select<false>, dim3(1), dim3(256), 0, st, v.ctl, lw, ls, kids, v.splits, v.tree, v.ops,
+                           v.pch, v.hch, v.d_nbins, v.fops, v.gc, v.scales);
     }
-    hipLaunchKernelGGL(k_lw_finalize, dim3(1), dim3(256), 0, st, v.ctl, lw, s.cands, kids, v.splits, s.free_slots,
-                       v.tree, v.gc, v.scales);
+    enqueue_leafwise_rounds(s, st, q, v, lw_head_rounds(v));
 }
 
 } // namespace bh

@@ -34,22 +34,49 @@ struct GrowView {
     RootSel root;  // the tree's root rows
     u32 *cnt;      // quantized leafwise: row count per (slot, feature, bin) beside the pool
     u32 lw_units;  // leafwise: histogram units per built node at most
+    u32 lw_parts, lw_pch; // leafwise: histogram units and partition chunks of a round at most
     bool host_sync;
 };
 
-// Leafwise candidate pool entry: a leaf with its best split, waiting in the gain heap
-// (grower_detail::Candidate, src/step/primitives.hpp:404-415).
-struct Cand {
+// A leaf of the tree being grown with its best split, waiting in the gain heap
+// (grower_detail::Candidate, src/step/primitives.hpp:404-415) or ahead of its parent's pop.
+struct LwRec {
     NodeInfo node;
     SplitRec split;
+    double prio;      // lowest gain on its way from the pool: when it is expected to be popped
+    float kval[2];    // its children (when expanded): value and rows
+    u32 kcnt[2];
+    float value;      // as a leaf
+    u32 pad;
+};
+
+// Device state of one leafwise tree.
+struct LwCtl {
+    u32 n_free, n_pool, n_list, n_rec;
+    u32 n_batch;      // leaves the running round expands
+    u32 pops;         // splits and demotions so far
+    u32 n_ahead;      // leaves expanded, not popped
+    u32 grid_done;    // workgroups of the running split find that have finished
+    u32 batch[kLwBatch], demoted[kLwBatch];
+};
+
+struct LwLists {
+    LwRec *recs;
+    double *gain;             // per record: its split's gain, its first child's record (kNone:
+    u32 *link, *meta;         // none) and lw_meta
+    double *pool_gain;        // leaves with final ids and a valid split
+    u32 *pool_id, *pool_rec;
+    double *list_prio;        // leaves without children yet, popped parents or not
+    u32 *list_rec;
+    u32 *free_slots;          // histogram slots
+    u32 unit_target, chunk_cap, max_parts;
 };
 
 struct ExtState {
     // leafwise
-    Cand *cands = nullptr;      // candidate pool (heap entries), capacity max_leaves + 4
-    NodeInfo *pending = nullptr;// leaves set aside (no valid split)
-    u32 *free_slots = nullptr;  // histogram slot free list
-    u32 cap = 0;
+    LwLists ls{};
+    LwCtl *lw = nullptr;
+    u32 *report = nullptr;         // pinned: 1 when the tree of the last rounds is complete
     // levelwise
     SplitRec *feat_best = nullptr; // per-feature best of the level scan
     u32 *level_splits = nullptr;   // (feature, bin, default_left) per level
@@ -58,10 +85,13 @@ struct ExtState {
     u32 hist_slots = 0;
 };
 
-hipError_t ext_alloc(ExtState &s, bh_fit_config const &f, u32 F, u32 SB, u32 max_front, u32 hist_slots);
+hipError_t ext_alloc(ExtState &s, bh_fit_config const &f, u32 F, u32 hist_slots);
 void ext_free(ExtState &s);
 hipError_t ext_set_limits();
 void enqueue_levelwise(ExtState &s, hipStream_t st, bool q, GrowView const &v);
+u32 lw_batch(GrowView const &v);
+u32 lw_head_rounds(GrowView const &v);
+void enqueue_leafwise_rounds(ExtState &s, hipStream_t st, bool q, GrowView const &v, u32 rounds);
 void enqueue_leafwise(ExtState &s, hipStream_t st, bool q, GrowView const &v);
 // The level finder as one step over a host-laid frontier (front[0 .. n), ctl->n_front =
 // n): pick[0] = the level's split, v.splits[i] = node i's child sums under it.
