@@ -101,6 +101,39 @@ __device__ __forceinline__ float fd_leaf_value(u32 id, double g, double h, GrowC
     return static_cast<float>(fd_bounded_weight(g, h, c.l1, c.l2, lo, hi));
 }
 
+// Running sums of n FP32 components in bin order, in double (v[2 b], one component of the
+// cells); each sum to out[b] when out is given.  One lane per component: the chain is
+// issue bound, so g and h run in different lanes, and the next values are read before the
+// sums of these are stored.
+__device__ __forceinline__ double fd_serial_sum(float const *v, u32 n, double *out)
+{
+    constexpr u32 W = 8;
+    double s = 0.0;
+    u32 b = 0;
+    float nx[W];
+#pragma unroll
+    for (u32 k = 0; k < W; ++k) nx[k] = k < n ? v[2u * k] : 0.0F;
+    for (; b + W <= n; b += W) {
+        float x[W];
+#pragma unroll
+        for (u32 k = 0; k < W; ++k) {
+            x[k] = nx[k];
+            u32 const q = b + W + k;
+            nx[k] = v[2u * (q < n ? q : n - 1u)];
+        }
+#pragma unroll
+        for (u32 k = 0; k < W; ++k) {
+            s += x[k];
+            if (out) out[b + k] = s;
+        }
+    }
+    for (; b < n; ++b) {
+        s += v[2u * b];
+        if (out) out[b] = s;
+    }
+    return s;
+}
+
 // CON: the feature mask and the monotone / interaction constraints are compiled in
 // (launches without any use the leaner CON = false body).
 template <bool Q, bool CON, u32 TILE = kFindTile>
@@ -120,6 +153,7 @@ __device__ void find_node(NodeInfo *__restrict__ front, TreeCtl const *__restric
     __shared__ u32 s_best_key[kFindThreads / 64];
     __shared__ double s_tot[2];
     __shared__ i64 s_itot[2];
+    __shared__ float2 s_first[Q ? 1 : 256]; // FP32: the first selected feature's cells (SB <= 256)
     __shared__ Acc s_mg[TILE], s_mh[TILE];
     __shared__ u32 s_ncut[TILE], s_dirs[TILE], s_nb[TILE], s_mc[TILE];
     __shared__ u32 s_allow[kMaxPathWords], s_cover[kMaxGroups], s_single;
@@ -163,7 +197,8 @@ __device__ void find_node(NodeInfo *__restrict__ front, TreeCtl const *__restric
     bool const had_totals = node.totals_ready != 0;
     // Quantized totals are exact integers, equal over every feature's cells: a block that
     // scans takes them from the first feature of its first tile (no extra round trip).
-    bool const tot_from_tile = Q && can && !had_totals;
+    // FP32 ones are one serial sum, run beside the first tile's prefixes.
+    bool const tot_from_tile = can && !had_totals;
     // Phase 0: node totals from the first selected feature's cells (Histogram::totals,
     // include/bonsai/histogram.hpp:76-87; SplitInput::totals skips unselected features,
     // include/bonsai/split.hpp:36-53) unless a parent split already set them.
@@ -278,8 +313,17 @@ __device__ void find_node(NodeInfo *__restrict__ front, TreeCtl const *__restric
         for (u32 k = threadIdx.x; k < nt * SB; k += blockDim.x) s_cells[k] = hcells[static_cast<size_t>(f0) * SB + k];
         if (hcnt)
             for (u32 k = threadIdx.x; k < nt * SB; k += blockDim.x) s_cn[k] = hcnt[static_cast<size_t>(f0) * SB + k];
+        u32 first = 0;
+        bool const tot_beside = !Q && tot_from_tile && f0 == bx * TILE;
+        if (tot_beside) {
+            if (CON && cfg.fmask)
+                while (first + 1u < F && !cfg.fmask[first]) ++first;
+            float2 const *cf = reinterpret_cast<float2 const *>(hcells) + static_cast<size_t>(first) * SB;
+            for (u32 k = threadIdx.x; k < SB; k += blockDim.x) s_first[k] = cf[k];
+            first = n_bins[first];
+        }
         __syncthreads();
-        if (tot_from_tile && f0 == bx * TILE) {
+        if (Q && tot_from_tile && f0 == bx * TILE) {
             if (threadIdx.x < 64) {
                 i64 g = 0, h = 0;
                 for (u32 b = threadIdx.x; b < SB; b += 64) {
@@ -299,11 +343,6 @@ __device__ void find_node(NodeInfo *__restrict__ front, TreeCtl const *__restric
                 }
             }
             __syncthreads();
-        }
-        if (f0 == bx * TILE) {
-            tg = Q ? static_cast<double>(s_itot[0]) * sg : s_tot[0];
-            th = Q ? static_cast<double>(s_itot[1]) * sh : s_tot[1];
-            node_score = fd_score_of(tg, th, cfg.l1, cfg.l2);
         }
         // Phase A: per-feature running sums in bin order (src/split.cpp:131-158).
         // Quantized: exact integers, so a wave scans a feature in parallel (the count
@@ -373,39 +412,40 @@ __device__ void find_node(NodeInfo *__restrict__ front, TreeCtl const *__restric
                 }
             }
         }
-        u32 const t = threadIdx.x;
-        if (!Q && t < TILE) {
+        if (!Q && threadIdx.x < 2u * TILE) {
+            u32 const t = threadIdx.x >> 1, e = threadIdx.x & 1u; // feature, component (g, h)
             u32 ncut = 0, dirs = 1;
             if (t < nt) {
                 u32 const nb = s_nb[t];
                 ncut = nb >= 2 ? nb - 2 : 0;
-                Acc *qg = pg + t * SB, *qh = ph + t * SB;
                 float2 const *cf = reinterpret_cast<float2 const *>(s_cells + t * SB);
                 float2 const m = nb ? cf[nb - 1] : make_float2(0.0F, 0.0F);
-                s_mg[t] = m.x;
-                s_mh[t] = m.y;
                 dirs = (m.x == 0.0F && m.y == 0.0F) ? 1 : 2;
-                double g = 0.0, h = 0.0;
-                u32 b = 0;
-                for (; b + 4 <= ncut; b += 4) {
-                    float2 const v0 = cf[b], v1 = cf[b + 1], v2 = cf[b + 2], v3 = cf[b + 3];
-                    g += v0.x; h += v0.y; qg[b] = g; qh[b] = h;
-                    g += v1.x; h += v1.y; qg[b + 1] = g; qh[b + 1] = h;
-                    g += v2.x; h += v2.y; qg[b + 2] = g; qh[b + 2] = h;
-                    g += v3.x; h += v3.y; qg[b + 3] = g; qh[b + 3] = h;
-                }
-                for (; b < ncut; ++b) {
-                    float2 const v = cf[b];
-                    g += v.x;
-                    h += v.y;
-                    qg[b] = g;
-                    qh[b] = h;
-                }
+                if (e == 0) s_mg[t] = m.x;
+                else s_mh[t] = m.y;
+                fd_serial_sum(reinterpret_cast<float const *>(cf) + e, ncut,
+                              reinterpret_cast<double *>(e == 0 ? pg : ph) + t * SB);
             }
-            s_ncut[t] = ncut;
-            s_dirs[t] = dirs;
+            if (e == 0) {
+                s_ncut[t] = ncut;
+                s_dirs[t] = dirs;
+            }
+        }
+        if (tot_beside && (threadIdx.x & ~1u) == 64u) { // Histogram::totals, stored as float
+            u32 const e = threadIdx.x & 1u;
+            s_tot[e] = static_cast<float>(fd_serial_sum(reinterpret_cast<float const *>(s_first) + e, first, nullptr));
         }
         __syncthreads();
+        if (f0 == bx * TILE) {
+            if (tot_beside) {
+                node.tg = static_cast<float>(s_tot[0]);
+                node.th = static_cast<float>(s_tot[1]);
+                node.totals_ready = 1;
+            }
+            tg = Q ? static_cast<double>(s_itot[0]) * sg : s_tot[0];
+            th = Q ? static_cast<double>(s_itot[1]) * sh : s_tot[1];
+            node_score = fd_score_of(tg, th, cfg.l1, cfg.l2);
+        }
         // Phase B: every (feature, cut bin, direction) candidate; a thread takes one
         // (feature, bin) pair and scores its directions from one prefix load.
         u32 const n_pairs = nt * SB;
