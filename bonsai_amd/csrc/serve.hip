@@ -9,6 +9,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -1275,6 +1276,9 @@ struct bh_predictor {
     SHead *d_heads = nullptr;
     float *d_w = nullptr;
     hipStream_t stream = nullptr;
+    // Buffers of small host calls (SmallCall): one call at a time.
+    std::mutex ws_busy;
+    unsigned char *ws_host = nullptr, *ws_dev = nullptr; // kWsBytes each, pinned and device
 };
 
 namespace {
@@ -1410,6 +1414,47 @@ int launch_shap(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, double *d_
         SHIP(hipGetLastError());
     }
     return 0;
+}
+
+// A host call's buffers: allocating, copying and freeing around a kernel of some 20 us took
+// about 60 us.  Calls whose rows and results fit kWsBytes take the predictor's pinned and
+// device buffers (made by the first one, freed with the predictor) unless another thread's
+// call holds them; then, and for larger batches, buffers are allocated for the call.
+constexpr size_t kWsBytes = 1u << 20;
+class SmallCall {
+public:
+    SmallCall(bh_predictor *p, size_t in, size_t out) : p_(p), out_((in + 255u) & ~static_cast<size_t>(255)), lock_(p->ws_busy, std::defer_lock)
+    {
+        if (in > kWsBytes || out > kWsBytes || out_ + out > kWsBytes || !lock_.try_lock()) return;
+        if (!p->ws_host && hipHostMalloc(reinterpret_cast<void **>(&p->ws_host), kWsBytes, hipHostMallocDefault) != hipSuccess)
+            p->ws_host = nullptr;
+        if (!p->ws_dev && hipMalloc(&p->ws_dev, kWsBytes) != hipSuccess) p->ws_dev = nullptr;
+        ready_ = p->ws_host && p->ws_dev;
+        if (!ready_) (void)hipGetLastError();
+    }
+    bool ready() const { return ready_; }
+    unsigned char *host_in() const { return p_->ws_host; }
+    unsigned char *host_out() const { return p_->ws_host + out_; }
+    unsigned char *dev_in() const { return p_->ws_dev; }
+    unsigned char *dev_out() const { return p_->ws_dev + out_; }
+
+private:
+    bh_predictor *p_;
+    size_t out_; // results' offset
+    std::unique_lock<std::mutex> lock_;
+    bool ready_ = false;
+};
+
+// Whole words (both ends lie in buffers of kWsBytes).
+__global__ void k_copy_words(u32 const *__restrict__ src, u32 *__restrict__ dst, u32 n)
+{
+    for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) dst[i] = src[i];
+}
+void launch_copy_words(hipStream_t s, void const *src, void *dst, size_t bytes)
+{
+    u32 const n = static_cast<u32>((bytes + 3u) / 4u);
+    hipLaunchKernelGGL(k_copy_words, dim3(std::min(256u, (n + 255u) / 256u)), dim3(256), 0, s,
+                       static_cast<u32 const *>(src), static_cast<u32 *>(dst), n);
 }
 
 } // namespace
@@ -1629,6 +1674,8 @@ int bh_predictor_destroy(bh_predictor *p)
                     p->d_words, p->d_tiles, p->d_ttrees, p->d_tslots, p->d_tfirst};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
+    if (p->ws_dev) (void)hipFree(p->ws_dev);
+    if (p->ws_host) (void)hipHostFree(p->ws_host);
     if (p->stream) (void)hipStreamDestroy(p->stream);
     delete p;
     return 0;
@@ -1656,6 +1703,18 @@ int bh_predict(bh_predictor *p, const uint8_t *bins, uint64_t n, uint64_t row_st
     if (row_stride < p->F) return sfail(1, "row_stride < n_features");
     if (n == 0) return 0;
     SHIP(hipSetDevice(p->device));
+    if (n < kPredTileRows) {
+        // the walk reads a row once and writes one value: both stay in host memory
+        SmallCall c(p, n * row_stride, n * sizeof(float));
+        if (c.ready()) {
+            std::memcpy(c.host_in(), bins, n * row_stride);
+            if (int rc = launch_predict(p, c.host_in(), n, row_stride, reinterpret_cast<float *>(c.host_out()), p->stream))
+                return rc;
+            SHIP(hipStreamSynchronize(p->stream));
+            std::memcpy(out, c.host_out(), n * sizeof(float));
+            return 0;
+        }
+    }
     u8 *d_bins = nullptr;
     float *d_out = nullptr;
     SHIP(hipMalloc(&d_bins, n * row_stride));
@@ -1678,6 +1737,23 @@ int bh_shap(bh_predictor *p, const uint8_t *bins, uint64_t n, uint64_t row_strid
     if (row_stride < p->F) return sfail(1, "row_stride < n_features");
     if (n == 0) return 0;
     SHIP(hipSetDevice(p->device));
+    {
+        // many workgroups read a row and add to its contributions: device buffers, with the
+        // copies in the stream
+        size_t const nb = n * row_stride, no = n * (p->F + 1) * sizeof(double);
+        SmallCall c(p, nb, no);
+        if (c.ready()) {
+            std::memcpy(c.host_in(), bins, nb);
+            launch_copy_words(p->stream, c.host_in(), c.dev_in(), nb);
+            if (int rc = launch_shap(p, c.dev_in(), n, row_stride, reinterpret_cast<double *>(c.dev_out()), p->stream))
+                return rc;
+            launch_copy_words(p->stream, c.dev_out(), c.host_out(), no);
+            SHIP(hipGetLastError());
+            SHIP(hipStreamSynchronize(p->stream));
+            std::memcpy(out, c.host_out(), no);
+            return 0;
+        }
+    }
     u8 *d_bins = nullptr;
     double *d_out = nullptr;
     SHIP(hipMalloc(&d_bins, n * row_stride));
