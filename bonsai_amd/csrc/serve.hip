@@ -499,6 +499,8 @@ struct TSlot {
 enum : u32 {
     kTEnter = 0, kTTurn = 1, kTCombine = 2, kTBlock = 3, kTSkip = 15,
     kTLeafL = 0x10000u, kTLeafR = 0x20000u, // enter / combine: that child is a leaf
+    kTOnlyL = 0x40000u, kTOnlyR = 0x80000u, // enter: the way down to a share goes there only
+    kTHeldL = 0x100000u, kTHeldR = 0x200000u, // with kTLeaf: a share's value, kept in LDS
     kTwOp = 0, kTwLv = 1, kTwSplit = 2,
     kTwZl = 3, kTwZr = 4, kTwVl = 5, kTwVr = 6,          // enter, turn, combine
     kTwZ = 9, kTwMean = 15, kTwLeaf = 19, kTwBlock = 27, // block: z of 3 nodes, means of 4, 8 leaves
@@ -523,8 +525,9 @@ struct TQuad {
     float y[kTreeShapMaxM], w[kTreeShapMaxM];
 };
 
-// U: levels above the blocks.
-template <int M, int U> struct TreeShap {
+// U: levels above the blocks.  AT: the walk may start below a tree's root (levels come
+// from the steps) and meet shares' values.
+template <int M, int U, bool AT = false> struct TreeShap {
     typedef float V[M];
     u8 const *bins;      // LDS: this lane's column of the bins
     unsigned char *phi;  // LDS: this lane's column of the sums
@@ -535,6 +538,7 @@ template <int M, int U> struct TreeShap {
     u32 at, op;          // the running step's slot in it and its first word (uniform)
     V y;                 // quadrature nodes (TQuad)
     u32 sat;             // bit l: the row satisfies the merged feature of the edge below level l
+    float *held;         // AT: LDS, this lane's column of the shares' values [share][M][64]
 
     __device__ __forceinline__ void load()
     {
@@ -749,7 +753,7 @@ template <int M, int U> struct TreeShap {
     template <int L> __device__ __forceinline__ void walk(V const &Tn, V &H)
     {
         if (L == U || (op & 3u) == kTBlock) {
-            block(Tn, H, L);
+            block(Tn, H, level_of<L>());
             advance(tree_step_slots(kTBlock));
             return;
         }
@@ -760,15 +764,21 @@ template <int M, int U> struct TreeShap {
             for (u32 side = 0; side < 2u; ++side) {
                 if (op & (kTLeafL << side)) {
                     float const v = side ? fword(kTwVr) : fword(kTwVl);
+                    if (AT && (op & (kTHeldL << side))) {
+                        float const *h = held + static_cast<u32>(v) * (M * 64u);
 #pragma unroll
-                    for (int q = 0; q < M; ++q) H[q] = v;
+                        for (int q = 0; q < M; ++q) H[q] = h[q * 64];
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < M; ++q) H[q] = v;
+                    }
                 } else {
                     V Tc;
                     V k;
                     u32 const me = side ? ~m : m;
                     consts(k, dup_of<L>());
                     descend(Tn, Tc, k, me, side ? fword(kTwZr) : fword(kTwZl));
-                    mark(me, L, dup_of<L>());
+                    mark(me, level_of<L>(), dup_of<L>());
                     advance(1);
                     fetch();
                     walk<L + 1>(Tc, H);
@@ -787,9 +797,123 @@ template <int M, int U> struct TreeShap {
     }
     template <int L> __device__ __forceinline__ Dup dup_of() const
     {
-        return Dup{L > 0 && (op & 0x100u) != 0, 1u, word(kTwLv)};
+        return Dup{(AT || L > 0) && (op & 0x100u) != 0, 1u, word(kTwLv)};
+    }
+    template <int L> __device__ __forceinline__ u32 level_of() const { return AT ? op >> 2 & 15u : L; }
+
+    // Starts reading at slot pc.
+    __device__ __forceinline__ void seek(TSlot const *slots, u32 pc)
+    {
+        ahead = slots + (pc & ~63u) + (threadIdx.x & 63u);
+        load();
+        shift();
+        at = pc & 63u;
+        sat = 0;
+    }
+    // The way from a tree's root down to the share whose steps follow.
+    __device__ __forceinline__ void go_down(V &T)
+    {
+        while ((op & 3u) == kTEnter && (op & (kTOnlyL | kTOnlyR))) {
+            bool const right = (op & kTOnlyR) != 0;
+            u32 const m = goes_left(word(kTwSplit)), me = right ? ~m : m;
+            V k, Tc;
+            consts(k, dup_of<0>());
+            descend(T, Tc, k, me, right ? fword(kTwZr) : fword(kTwZl));
+            mark(me, level_of<0>(), dup_of<0>());
+#pragma unroll
+            for (int q = 0; q < M; ++q) T[q] = Tc[q];
+            advance(1);
+            fetch();
+        }
     }
 };
+
+// Few rows or trees.  A walk is one serial chain (0.27 us a split), so a batch with fewer
+// row blocks x trees than the chip has room for waves waits for one tree's: 300 us at
+// depth 10 whatever the batch.  Here a workgroup takes one tree of a row block: its 8 waves
+// walk the tree's shares (the subtrees below a cut, each with the product T carried down to
+// it), leave their values in LDS, and the first wave walks the splits above the cut over
+// them.  Every split's arithmetic is the walk's own, so a row's bits are the same either
+// way.  One to 64 rows x 20 trees: depth 6 37 -> 29 us, depth 8 85 -> 42, depth 10
+// 297 -> 89; 65 rows x 100 depth-10 trees
+// 283 -> 72 us.
+struct SplitTree {
+    u32 share0, n_shares, top; // first share, shares, first slot of the steps above (kNone: none)
+    u32 pad;
+};
+constexpr u32 kSplitThreads = 512;   // 16 waves a workgroup spill (128 registers): a sixth slower at depth 8
+constexpr u32 kSplitLevels = 6; // cut at most this far below the root (TreePacker::cut_of)
+template <int M>
+__global__ __launch_bounds__(kSplitThreads) void k_shap_split(u8 const *__restrict__ bins, u64 n, u64 stride, u32 F,
+                                                             u16 const *__restrict__ last,
+                                                             TSlot const *__restrict__ slots,
+                                                             u32 const *__restrict__ first,
+                                                             SplitTree const *__restrict__ trees, u32 n_trees,
+                                                             TQuad quad, double *__restrict__ out)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned long long *s_phi = reinterpret_cast<unsigned long long *>(smem); // [F][64] fixed point
+    float *s_held = reinterpret_cast<float *>(s_phi + kTreeShapRows * F);      // [shares][M][64]
+    constexpr u32 nw = kSplitThreads / 64u;
+    u64 const r0 = static_cast<u64>(blockIdx.x) * kTreeShapRows;
+    u32 const nr = static_cast<u32>(min<u64>(kTreeShapRows, n - r0));
+    u32 const plane = kTreeShapRows * F;
+    u32 held = 0;
+    for (u32 t = blockIdx.y; t < n_trees; t += gridDim.y) held = max(held, trees[t].n_shares);
+    u8 *s_bins = reinterpret_cast<u8 *>(s_held + held * M * 64u); // [2][F][64]
+    for (u32 k = threadIdx.x; k < plane; k += kSplitThreads) {
+        u32 const rr = k / F, f = k - rr * F;
+        u32 const b = rr < nr ? bins[(r0 + rr) * stride + f] : 0u;
+        s_phi[k] = 0ull;
+        s_bins[f * kTreeShapRows + rr] = static_cast<u8>(b);
+        s_bins[plane + f * kTreeShapRows + rr] = static_cast<u8>(b == last[f] ? 0u : min(b + 1u, 255u));
+    }
+    __syncthreads();
+    u32 const lane = threadIdx.x & 63u;
+    u32 const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    auto begin = [&](auto &w, float(&T)[M]) {
+        w.bins = s_bins + lane;
+        w.phi = reinterpret_cast<unsigned char *>(s_phi + lane);
+        w.plane = plane;
+        w.held = s_held + lane;
+#pragma unroll
+        for (int q = 0; q < M; ++q) {
+            w.y[q] = quad.y[q];
+            T[q] = quad.w[q];
+        }
+    };
+    for (u32 t = blockIdx.y; t < n_trees; t += gridDim.y) {
+        SplitTree const tr = trees[t];
+        for (u32 j = wave; j < tr.n_shares; j += nw) {
+            TreeShap<M, 3, true> w;
+            float T[M], H[M];
+            begin(w, T);
+            w.seek(slots, __builtin_amdgcn_readfirstlane(first[tr.share0 + j]));
+            w.fetch();
+            w.go_down(T);
+            w.template walk<0>(T, H);
+#pragma unroll
+            for (int q = 0; q < M; ++q) w.held[(j * M + q) * 64u] = H[q];
+        }
+        __syncthreads();
+        if (wave == 0 && tr.top != kNone) {
+            TreeShap<M, kSplitLevels, true> w;
+            float T[M], H[M];
+            begin(w, T);
+            w.seek(slots, __builtin_amdgcn_readfirstlane(tr.top));
+            w.fetch();
+            w.template walk<0>(T, H);
+        }
+        __syncthreads();
+    }
+    // Trees of one row block meet in the zeroed output cells, as shares of k_shap_tree do.
+    unsigned long long *acc = reinterpret_cast<unsigned long long *>(out);
+    for (u32 k = threadIdx.x; k < nr * F; k += kSplitThreads) {
+        u32 const rr = k / F, f = k - rr * F;
+        unsigned long long const v = s_phi[f * kTreeShapRows + rr];
+        if (v != 0ull) atomicAdd(acc + (r0 + rr) * (F + 1) + f, v);
+    }
+}
 
 // gridDim.y workgroups share a row block; each of their waves walks a run of trees.
 template <int M, int U>
@@ -1186,6 +1310,81 @@ struct TreePacker {
         }
         step(kTCombine, level, nd, flags, vl, vr);
     }
+
+    // The split form (k_shap_split): every subtree at depth `cut`, or shallower of at most a
+    // block's levels, is a share: the steps down to it, then its own walk.
+    std::vector<u32> first;          // first slot of every share
+    std::vector<std::pair<u32, u32>> way; // (node, side) from the root
+    static u32 cut_of(u32 deepest) { return std::min(deepest - kTBlockLevels, std::max(4u, deepest / 2u)); }
+    bool is_share(u32 id, u32 level, u32 cut) const { return level == cut || levels[id] <= kTBlockLevels; }
+    void go_down(u32 id, u32 level)
+    {
+        if (level == way.size()) {
+            walk(id, level);
+            return;
+        }
+        u32 const side = way[level].second;
+        bh_node const &n = t[way[level].first];
+        Node const nd = node(way[level].first);
+        step(kTEnter, level, nd, side ? kTOnlyR : kTOnlyL, 0.0, 0.0);
+        above.push_back({static_cast<u32>(n.feature), level, nd.z * (side ? nd.zr : nd.zl)});
+        go_down(id, level + 1);
+        above.pop_back();
+    }
+    void shares(u32 id, u32 level, u32 cut)
+    {
+        if (is_share(id, level, cut)) {
+            first.push_back(static_cast<u32>(out.size()));
+            go_down(id, 0);
+            return;
+        }
+        for (u32 side = 0; side < 2; ++side) {
+            u32 const kid = side ? t[id].right : t[id].left;
+            if (t[kid].feature < 0) continue;
+            way.push_back({id, side});
+            shares(kid, level + 1, cut);
+            way.pop_back();
+        }
+    }
+    // The steps above the shares, which come in the same order.
+    void top(u32 id, u32 level, u32 cut, u32 &share)
+    {
+        bh_node const &n = t[id];
+        Node const nd = node(id);
+        u32 const kids[2] = {n.left, n.right};
+        u32 flags = 0;
+        double v[2] = {0.0, 0.0};
+        u32 next = share; // index of the side's first share
+        for (u32 side = 0; side < 2; ++side) {
+            if (t[kids[side]].feature < 0) {
+                flags |= kTLeafL << side;
+                v[side] = static_cast<double>(t[kids[side]].value) * scale;
+            } else if (is_share(kids[side], level + 1, cut)) {
+                flags |= (kTLeafL | kTHeldL) << side;
+                v[side] = next++;
+            } else if (side == 0) {
+                next += count(kids[0], level + 1, cut);
+            }
+        }
+        bool const ll = (flags & kTLeafL) != 0, rl = (flags & kTLeafR) != 0;
+        if (!ll || !rl) step(kTEnter, level, nd, flags, v[0], v[1]);
+        if (flags & kTHeldL) ++share;
+        for (u32 side = 0; side < 2; ++side) {
+            if (side ? rl : ll) continue;
+            if (side && !ll) step(kTTurn, level, nd, flags, v[0], v[1]);
+            above.push_back({static_cast<u32>(n.feature), level, nd.z * (side ? nd.zr : nd.zl)});
+            top(kids[side], level + 1, cut, share);
+            above.pop_back();
+        }
+        if (flags & kTHeldR) ++share;
+        step(kTCombine, level, nd, flags, v[0], v[1]);
+    }
+    u32 count(u32 id, u32 level, u32 cut) const
+    {
+        if (t[id].feature < 0) return 0;
+        if (is_share(id, level, cut)) return 1;
+        return count(t[id].left, level + 1, cut) + count(t[id].right, level + 1, cut);
+    }
 };
 
 // Gauss-Legendre nodes on [0, 1], ascending (Newton's method on the Legendre polynomial),
@@ -1259,11 +1458,13 @@ struct bh_predictor {
     u32 n_groups = 0;          // TreeSHAP path groups of 64
     double shap_scale = 1.0;   // fixed-point scale of the TreeSHAP accumulators
     // tree-form TreeSHAP (tree_m quadrature nodes; 0: the packed form serves the ensemble)
-    u32 tree_m = 0, tree_depth = 0, n_ttrees = 0;
+    u32 tree_m = 0, tree_depth = 0, n_ttrees = 0, max_shares = 0; // max_shares 0: no split form
     double tree_scale = 1.0;   // its fixed-point scale, times the weights' common factor
     TQuad quad{};
     TSlot *d_tslots = nullptr;
     u32 *d_tfirst = nullptr;
+    u32 *d_sfirst = nullptr;
+    SplitTree *d_split = nullptr;
     PNode *d_nodes = nullptr;
     u32 *d_roots = nullptr;
     // tile form (n_tiles 0: the ensemble does not fit it)
@@ -1334,6 +1535,13 @@ int launch_predict(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, float *
 // Workgroups that fill the chip with tree-form waves: smaller batches split their trees.
 constexpr u32 kTreeShapFill = 768;
 
+// Row blocks x trees up to which a workgroup takes one tree (k_shap_split): one round of
+// workgroups while the trees are small (depth 6, 400 walks: 42 us split, 39 whole), two from
+// depth 8 (400 walks: 70 and 87 us; 1,000: 125 and 96).
+u64 split_walks(u32 depth) { return depth >= 8 ? 512 : 256; }
+// The node count a kernel is built for (the switch of launch_shap_tree).
+u32 m_of(u32 m, u32 upper) { return upper <= 5 ? std::max(2u, std::min(m, 4u)) : std::max(4u, std::min(m, 6u)); }
+
 int launch_shap_tree(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, double *d_out, hipStream_t s)
 {
     u32 const blocks = static_cast<u32>((n + kTreeShapRows - 1) / kTreeShapRows);
@@ -1360,6 +1568,31 @@ int launch_shap_tree(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, doubl
         SHIP(hipGetLastError());
     }
     size_t const lds = tree_shap_lds(p->F);
+    size_t const split_lds = lds + static_cast<size_t>(p->max_shares) * m_of(p->tree_m, upper) * 64u * sizeof(float);
+    if (p->max_shares && static_cast<u64>(blocks) * p->n_ttrees <= split_walks(p->tree_depth) && split_lds <= 160u * 1024u) {
+        if (split <= 1) {
+            hipLaunchKernelGGL(k_shap_zero, dim3(cgrid), dim3(256), 0, s,
+                               reinterpret_cast<unsigned long long *>(d_out), cells);
+            SHIP(hipGetLastError());
+        }
+        dim3 const sgrid(blocks, p->n_ttrees);
+#define BH_SP(MV)                                                                                                  \
+    hipLaunchKernelGGL((k_shap_split<MV>), sgrid, dim3(kSplitThreads), split_lds, s, d_bins, n, stride, p->F,      \
+                       p->d_last, p->d_tslots, p->d_sfirst, p->d_split, p->n_ttrees, p->quad, d_out)
+        switch (m_of(p->tree_m, upper)) {
+        case 2: BH_SP(2); break;
+        case 3: BH_SP(3); break;
+        case 4: BH_SP(4); break;
+        case 5: BH_SP(5); break;
+        default: BH_SP(6); break;
+        }
+#undef BH_SP
+        SHIP(hipGetLastError());
+        hipLaunchKernelGGL(k_shap_to_double, dim3(cgrid), dim3(256), 0, s, d_out, n, p->F, p->lr, p->shap_bias,
+                           p->tree_scale);
+        SHIP(hipGetLastError());
+        return 0;
+    }
     dim3 const grid(blocks, split);
 #define BH_TS(MV, UV)                                                                                              \
     hipLaunchKernelGGL((k_shap_tree<MV, UV>), grid, dim3(threads), lds, s, d_bins, n, stride, p->F, p->d_last,     \
@@ -1579,6 +1812,7 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     }
     TreePacker pack{};
     std::vector<u32> tfirst;
+    std::vector<SplitTree> split;
     if (tree_form) {
         // kernels' node counts: 2, 3, 4 (up to 8 levels), 4, 5, 6 (more)
         u32 const m = std::max<u32>(deepest <= 8 ? 2u : 4u, (p->max_len + 1u) / 2u);
@@ -1606,6 +1840,7 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
         pack.F = n_features;
         pack.scale = scale;
         pack.rule = gauss_legendre(m);
+        pack.out.reserve(pn.size() * 3u + 256u); // both forms: about 1.5 slots a node each
         for (u32 t = 0; t < n_trees; ++t) {
             pack.t = nodes + tree_offsets[t];
             pack.levels = levels[t].data();
@@ -1614,6 +1849,24 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
             pack.walk(0, 0);
         }
         tfirst.push_back(static_cast<u32>(pack.out.size()));
+        if (deepest > kTBlockLevels + 1u) {
+            u32 const cut = TreePacker::cut_of(deepest);
+            for (u32 t = 0; t < n_trees; ++t) {
+                pack.t = nodes + tree_offsets[t];
+                pack.levels = levels[t].data();
+                if (pack.t[0].feature < 0) continue;
+                SplitTree st{static_cast<u32>(pack.first.size()), 0u, kNone, 0u};
+                pack.shares(0, 0, cut);
+                st.n_shares = static_cast<u32>(pack.first.size()) - st.share0;
+                if (!pack.is_share(0, 0, cut)) {
+                    u32 share = 0;
+                    st.top = static_cast<u32>(pack.out.size());
+                    pack.top(0, 0, cut, share);
+                }
+                p->max_shares = std::max(p->max_shares, st.n_shares);
+                split.push_back(st);
+            }
+        }
         pack.out.resize((pack.out.size() / 64u + 3u) * 64u); // the kernel reads whole groups, two ahead
         double g = 1.0;
         p->quad = tree_quad(pack.rule, g);
@@ -1655,6 +1908,12 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
         al(reinterpret_cast<void **>(&p->d_tslots), pack.out.size() * sizeof(TSlot));
         al(reinterpret_cast<void **>(&p->d_tfirst), tfirst.size() * sizeof(u32));
         if (e == hipSuccess) e = hipMemcpy(p->d_tslots, pack.out.data(), pack.out.size() * sizeof(TSlot), hipMemcpyHostToDevice);
+        if (!split.empty()) {
+            al(reinterpret_cast<void **>(&p->d_sfirst), pack.first.size() * sizeof(u32));
+            al(reinterpret_cast<void **>(&p->d_split), split.size() * sizeof(SplitTree));
+            if (e == hipSuccess) e = hipMemcpy(p->d_sfirst, pack.first.data(), pack.first.size() * sizeof(u32), hipMemcpyHostToDevice);
+            if (e == hipSuccess) e = hipMemcpy(p->d_split, split.data(), split.size() * sizeof(SplitTree), hipMemcpyHostToDevice);
+        }
         if (e == hipSuccess && !tfirst.empty()) e = hipMemcpy(p->d_tfirst, tfirst.data(), tfirst.size() * sizeof(u32), hipMemcpyHostToDevice);
     }
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking);
@@ -1671,7 +1930,7 @@ int bh_predictor_destroy(bh_predictor *p)
     if (!p) return 0;
     (void)hipSetDevice(p->device);
     void *ptrs[] = {p->d_nodes, p->d_roots, p->d_last,   p->d_elems, p->d_heads, p->d_w,
-                    p->d_words, p->d_tiles, p->d_ttrees, p->d_tslots, p->d_tfirst};
+                    p->d_words, p->d_tiles, p->d_ttrees, p->d_tslots, p->d_tfirst, p->d_sfirst, p->d_split};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     if (p->ws_dev) (void)hipFree(p->ws_dev);

@@ -224,6 +224,22 @@ def test_shap_tree_form_matches_packed_form(hip, orc, depth, n_features, used, n
             assert np.max(np.abs(got - ref) / mass) <= 1e-5
 
 
+@pytest.mark.parametrize("depth,used,p_leaf", [
+    (4, 28, 0.0), (5, 28, 0.0), (6, 3, 0.3), (7, 28, 0.2), (8, 28, 0.0), (9, 6, 0.3), (10, 10, 0.1), (11, 28, 0.4),
+    (12, 12, 0.35), (12, 3, 0.25)])
+def test_shap_split_trees_equal_whole_walks(hip, depth, used, p_leaf):
+    """Few row blocks x trees give each tree a workgroup whose waves walk its subtrees (from
+    5 levels up); 1,300 rows x 60 trees walk whole trees.  The same bits for every row."""
+    rng = np.random.default_rng([7, depth, used])
+    nb = rng.integers(2, 257, 28).astype(np.uint16)
+    trees = random_trees(rng, 57, depth, used, nb, p_leaf, True) + random_trees(rng, 3, 2, used, nb, 0.2)
+    rows = (rng.random((1300, 28)) * nb).astype(np.uint8)
+    p = hip.Predictor(trees, nb, 0.3, 0.25)
+    whole = p.shap(rows)
+    for a, b in ((0, 1), (3, 68), (1200, 1300)):
+        assert np.array_equal(p.shap(rows[a:b]).view(np.uint64), whole[a:b].view(np.uint64)), (a, b)
+
+
 @pytest.mark.parametrize("depth,n_features,n_trees,p_leaf", [
     (1, 1, 3, 0.0), (4, 28, 1, 0.0), (8, 28, 37, 0.0), (9, 28, 130, 0.3), (6, 256, 70, 0.1), (12, 60, 9, 0.2),
     (3, 257, 5, 0.0), (13, 5, 2, 0.0)])
