@@ -1468,7 +1468,7 @@ int bh_set_bernoulli(bh_context *c, float subsample, uint64_t seed)
     c->samp_kind = c->samp_n = 0;
     drop_graphs(c);
     if (subsample >= 1.0F) return 0; // the reference keeps every row for p >= 1
-    if (!c->samp_cnt) HIP_TRY(dalloc(&c->samp_cnt, c->N / kPartChunk + 2));
+    if (!c->samp_cnt) HIP_TRY(dalloc(&c->samp_cnt, c->N / part_chunk_rows(4u, c->N) + 2));
     double const t = std::floor(static_cast<double>(subsample) * 4294967296.0);
     c->samp_thr = static_cast<u32>(std::min(t, 4294967295.0));
     c->samp_seed = seed;

@@ -2889,15 +2889,16 @@ __device__ __forceinline__ bool bern_keep(u64 seed, u32 iter, u32 row, u32 thr)
     return static_cast<u32>(splitmix64(key) >> 32) < thr;
 }
 
-// Kept rows per kPartChunk-row chunk.
+// Kept rows per chunk (of part_chunk_rows(4, n) rows: a chunk is one workgroup's serial
+// chain; 1M rows in 4,096-row chunks: k_bern_gather 34.2 us, in 1,024-row ones BERNUS).
 __global__ __launch_bounds__(256) void k_bern_count(TreeCtl const *__restrict__ ctl, u32 n, u64 seed, u32 thr,
-                                                    u32 *__restrict__ chunk_cnt)
+                                                    u32 *__restrict__ chunk_cnt, u32 chunk)
 {
     __shared__ u32 red[4];
     u32 const iter = ctl->iter;
-    u32 const n_ch = (n + kPartChunk - 1) / kPartChunk;
+    u32 const n_ch = (n + chunk - 1) / chunk;
     for (u32 c = blockIdx.x; c < n_ch; c += gridDim.x) {
-        u32 const r0 = c * kPartChunk, r1 = min(n, r0 + kPartChunk);
+        u32 const r0 = c * chunk, r1 = min(n, r0 + chunk);
         u32 k = 0;
         for (u32 r = r0 + threadIdx.x; r < r1; r += blockDim.x) k += bern_keep(seed, iter, r, thr) ? 1u : 0u;
         for (int o = 32; o > 0; o >>= 1) k += __shfl_xor(k, o);
@@ -2932,15 +2933,15 @@ __global__ __launch_bounds__(1024) void k_bern_scan(u32 *__restrict__ chunk_cnt,
 __global__ __launch_bounds__(256) void k_bern_gather(TreeCtl const *__restrict__ ctl, u32 n, u64 seed, u32 thr,
                                                      u32 const *__restrict__ chunk_off, u8 const *__restrict__ plane,
                                                      u32 Fs, void const *__restrict__ gh, u32 gh_bytes,
-                                                     u8 *__restrict__ out_plane, void *__restrict__ out_gh)
+                                                     u8 *__restrict__ out_plane, void *__restrict__ out_gh, u32 chunk)
 {
     __shared__ u32 s_w[4];
     u32 const iter = ctl->iter;
     u32 const lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     u32 const D = Fs / 4u;
-    u32 const n_ch = (n + kPartChunk - 1) / kPartChunk;
+    u32 const n_ch = (n + chunk - 1) / chunk;
     for (u32 c = blockIdx.x; c < n_ch; c += gridDim.x) {
-        u32 const r0 = c * kPartChunk, r1 = min(n, r0 + kPartChunk);
+        u32 const r0 = c * chunk, r1 = min(n, r0 + chunk);
         u32 run = chunk_off[c];
         for (u32 p0 = r0; p0 < r1; p0 += blockDim.x) {
             u32 const r = p0 + threadIdx.x;
@@ -2972,12 +2973,13 @@ __global__ __launch_bounds__(256) void k_bern_gather(TreeCtl const *__restrict__
 void launch_bernoulli(hipStream_t s, TreeCtl *ctl, u32 n, u64 seed, u32 thr, u32 *chunk_cnt, u8 const *plane,
                       u32 Fs, void const *gh, u32 gh_bytes, u8 *out_plane, void *out_gh)
 {
-    u32 const n_ch = (n + kPartChunk - 1) / kPartChunk;
+    u32 const chunk = part_chunk_rows(4u, n);
+    u32 const n_ch = (n + chunk - 1) / chunk;
     u32 const grid = std::max(1u, std::min(n_ch, 2048u));
-    hipLaunchKernelGGL(k_bern_count, dim3(grid), dim3(256), 0, s, ctl, n, seed, thr, chunk_cnt);
+    hipLaunchKernelGGL(k_bern_count, dim3(grid), dim3(256), 0, s, ctl, n, seed, thr, chunk_cnt, chunk);
     hipLaunchKernelGGL(k_bern_scan, dim3(1), dim3(1024), 0, s, chunk_cnt, n_ch, ctl);
     hipLaunchKernelGGL(k_bern_gather, dim3(grid), dim3(256), 0, s, ctl, n, seed, thr, chunk_cnt, plane, Fs, gh,
-                       gh_bytes, out_plane, out_gh);
+                       gh_bytes, out_plane, out_gh, chunk);
 }
 
 // ---------------------------------------------------------------------------------

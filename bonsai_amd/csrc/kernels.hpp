@@ -86,7 +86,8 @@ void launch_tree_begin(hipStream_t s, TreeCtl *ctl, NodeInfo *front, DevNode *tr
                        FinishOp *fops, RootSel const &root, u32 unit_rows = kHistChunk);
 // Device Bernoulli row sampler: the rows of [0, n) kept in this iteration (threshold
 // thr on 32 random bits), ascending, with their gradient words, into out_plane/out_gh;
-// their count into ctl->root_n.  chunk_cnt: n / kPartChunk + 1 words of scratch.
+// their count into ctl->root_n.  chunk_cnt: n / part_chunk_rows(4, n) + 1 words of
+// scratch.
 void launch_bernoulli(hipStream_t s, TreeCtl *ctl, u32 n, u64 seed, u32 thr, u32 *chunk_cnt, u8 const *plane,
                       u32 Fs, void const *gh, u32 gh_bytes, u8 *out_plane, void *out_gh);
 // Per-tree feature selection for iteration ctl->iter: mask[f] = 1 for the k smallest
