@@ -1,9 +1,12 @@
 // Predict / TreeSHAP plans and the continuous-batching serving loop (H15, H16, cfg4).
 //
-// A bh_predictor holds one ensemble resident in HBM in two packed forms:
-//   walk nodes (8 B each) for the bin-space predict walk, and
-//   leaf paths (8 B elements, 12 B heads) for TreeSHAP's closed form,
-// and is immutable after creation, so serving streams share it.
+// A bh_predictor holds one ensemble resident in HBM, packed for each kernel:
+//   walk nodes (8 B each) for the bin-space walk of few rows, and LDS tiles of 4-byte nodes
+//   for the walk of many,
+//   step streams (32 B slots) of whole trees and of their subtrees for TreeSHAP, or leaf
+//   paths (8 B elements, 12 B heads) where the ensemble does not fit the tree form.
+// Its device data is immutable after creation, so serving streams share it; the buffers of
+// small host calls are taken by one call at a time.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <chrono>
