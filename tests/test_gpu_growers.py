@@ -229,6 +229,46 @@ def test_train_graph_equals_eager(hip, orc, tall, grower):
 
 
 @pytest.mark.parametrize("quantized", [True, False])
+@pytest.mark.parametrize("leaves", [2, 9, 10, 13])
+def test_grow_leafwise_chain(hip, orc, leaves, quantized):
+    """Labels that triple from group to group: every split peels one group off, so each pop
+    waits for the last one's children and 13 leaves need more rounds than a tree is first
+    given (6); leaf counts around one round's eight.  The tree, then a fit by graph and
+    eagerly, bit-exact."""
+    n, f = 6500, 3
+    rng = np.random.default_rng(5)
+    group = rng.integers(0, 13, n)
+    bins = np.stack([group, rng.integers(0, 13, n), rng.integers(0, 13, n)], axis=1).astype(np.uint8)
+    nb = np.full(f, 14, np.uint16)
+    y = (3.0 ** group).astype(np.float32)
+    g, h = orc.mse_grad(np.zeros(n, np.float32), y)
+    kw = dict(grower="hip_leafwise", quantized=quantized, max_depth=12, max_leaves=leaves, min_data_in_leaf=1)
+    c = orc_cfg(max_depth=12, max_leaves=leaves, min_data=1)
+    ctx = ctx_for(hip, bins, nb, **kw)
+    if quantized:
+        gq, hq, sc = ctx.set_gradients(g, h)
+        ref, rlor = orc.grow_leafwise(bins, nb, gq=gq, hq=hq, scales=sc, c=c, mode=HIST_INT)
+    else:
+        ctx.set_gradients(g, h)
+        ref, rlor = orc.grow_leafwise(bins, nb, g=g, h=h, c=c, mode=HIST_F32_FIXED, chunk=LW_F32_CHUNK)
+    nodes, lor = ctx.grow_tree()
+    ctx.close()
+    assert_same_tree(nodes, ref)
+    assert np.array_equal(lor, rlor)
+    fits = []
+    for use_graph in (True, False):
+        ctx = ctx_for(hip, bins, nb, use_graph=use_graph, learning_rate=0.5, **kw)
+        ctx.upload_labels(y)
+        ctx.set_scores(np.zeros(n, np.float32))
+        ctx.train(3)
+        fits.append((ctx.trees(), ctx.get_scores()))
+        ctx.close()
+    for a, b in zip(fits[0][0], fits[1][0]):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+    assert np.array_equal(fits[0][1].view(np.uint32), fits[1][1].view(np.uint32))
+
+
+@pytest.mark.parametrize("quantized", [True, False])
 def test_grow_leafwise_wide_rows(hip, orc, quantized):
     """1,500-byte rows: partition chunks are capped at 128 rows by bytes, below the
     leaf-sized rule's 256-row minimum."""
