@@ -230,6 +230,7 @@ struct bh_context {
     // leafwise: the iteration past its growth, and the extra rounds of an unfinished tree
     hipGraph_t graph_tail = nullptr, graph_more = nullptr;
     hipGraphExec_t tail_exec = nullptr, more_exec = nullptr;
+    hipError_t build_err = hipSuccess; // a histogram launch refused while enqueueing (enqueued)
     // histogram profiling (per-launch hipEvents, non-graph iterations only)
     bool prof = false;
     double prof_ms = 0.0, prof_bytes = 0.0, prof_scanned_bytes = 0.0;
@@ -278,12 +279,13 @@ struct bh_context {
     size_t part_bytes() const { return quant ? 12 : 8; }
     // Rows per histogram work unit of the counted (quantized depthwise) path on levels
     // that scan every live row (the root and routed levels): groups of hist_group
-    // sub-units, unless the feature-in-lane layout (single sub-units) is set.  Levels that
-    // build the small children only keep single sub-units: their fewer units would leave
-    // workgroup slots idle.
+    // sub-units, unless the feature-in-lane layout or the wide-row kernel (single sub-units
+    // both) serves them.  Levels that build the small children only keep single sub-units:
+    // their fewer units would leave workgroup slots idle.
     u32 unit_rows() const
     {
-        return quant && tune.hist_layout != 1u && tune.hist_group > 1u ? kHistChunk * tune.hist_group : small_unit();
+        bool const group = quant && Fs <= 64u && tune.hist_layout != 1u && tune.hist_group > 1u;
+        return group ? kHistChunk * tune.hist_group : small_unit();
     }
     // Rows per unit of its other levels: kHistChunk, halved down to kHistUnitMin until
     // the rows make kHistUnitFill units (exact integer sums: the unit size does not show;
@@ -569,9 +571,10 @@ hipError_t host_sync_point(bh_context *c)
 float profiled_hist(bh_context *c, void *hist_next, u32 grid_units, u32 *cnt_next, PartOp const *routes, bool group)
 {
     (void)hipEventRecord(c->ev0, c->stream);
-    launch_hist(c->stream, c->quant, c->hch, c->ctl, c->work[0], c->work[1], c->plane0, gh_src(c, 0),
+    hipError_t const e = launch_hist(c->stream, c->quant, c->hch, c->ctl, c->work[0], c->work[1], c->plane0, gh_src(c, 0),
                 gh_src(c, 1), gh_src(c, 2), c->Fs, c->F, c->SB, c->hist_fsl(), c->hist_waves(), grid_units,
                 c->partials, hist_next, c->fx, cnt_next, routes, group);
+    if (e != hipSuccess) c->build_err = e;
     (void)hipEventRecord(c->ev1, c->stream);
     (void)hipEventSynchronize(c->ev1);
     float ms = 0.0F;
@@ -626,15 +629,28 @@ void enqueue_build(bh_context *c, void *hist_cur, void *hist_next, u32 max_ops, 
                    PartOp const *routes = nullptr, bool group = false)
 {
     float ms = 0.0F;
-    if (c->prof)
+    if (c->prof) {
         ms = profiled_hist(c, hist_next, grid_units, cnt_next, routes, group);
-    else
-        launch_hist(c->stream, c->quant, c->hch, c->ctl, c->work[0], c->work[1], c->plane0, gh_src(c, 0),
-                    gh_src(c, 1), gh_src(c, 2), c->Fs, c->F, c->SB, c->hist_fsl(), c->hist_waves(), grid_units,
-                    c->partials, hist_next, c->fx, cnt_next, routes, group);
+    } else {
+        hipError_t const e = launch_hist(c->stream, c->quant, c->hch, c->ctl, c->work[0], c->work[1], c->plane0,
+                                         gh_src(c, 0), gh_src(c, 1), gh_src(c, 2), c->Fs, c->F, c->SB, c->hist_fsl(),
+                                         c->hist_waves(), grid_units, c->partials, hist_next, c->fx, cnt_next, routes,
+                                         group);
+        if (e != hipSuccess) c->build_err = e;
+    }
     launch_finish(c->stream, c->quant, c->fops, c->ctl, c->partials, hist_cur, hist_next, c->node_cells(), max_ops,
                   cnt_cur, cnt_next, advance, hist_transpose_F(c->quant, c->Fs, c->F, group));
     if (c->prof) profiled_count(c, ms, cnt_next);
+}
+
+// The error of the launches enqueued so far, refused histogram launches included.
+int enqueued(bh_context *c)
+{
+    hipError_t const e = c->build_err;
+    c->build_err = hipSuccess;
+    HIP_TRY(e);
+    HIP_TRY(hipGetLastError());
+    return 0;
 }
 
 u32 hist_grid(bh_context *c) { return std::max(1u, std::min(c->max_hch, 4096u)); }
@@ -684,6 +700,7 @@ void enqueue_depthwise_counted(bh_context *c)
     bool const group = unit_rows > kHistChunk;
     launch_tree_begin(s, c->ctl, c->front[0], c->tree, c->hch, c->fops, root_sel(c), unit_rows);
     enqueue_build(c, c->hist[1], c->hist[0], 1, hist_grid(c), c->cnt[1], c->cnt[0], false, nullptr, group);
+    if (c->build_err != hipSuccess) return; // no histogram: nothing below may plan from it
     for (u32 d = 0; d < D; ++d) {
         NodeInfo *cur = c->front[d & 1u], *nxt = c->front[(d + 1) & 1u];
         void *hcur = c->hist[d & 1u], *hnext = c->hist[(d + 1) & 1u];
@@ -858,6 +875,7 @@ int capture(bh_context *c, hipGraph_t &g, hipGraphExec_t &ge, void (*enqueue)(bh
     enqueue(c);
     hipError_t const e = hipStreamEndCapture(c->stream, &g);
     if (e != hipSuccess) return fail(-1, std::string("hip: capture: ") + hipGetErrorString(e));
+    if (int r = enqueued(c)) return r;
     HIP_TRY(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
     return 0;
 }
@@ -1632,7 +1650,7 @@ int bh_train(bh_context *c, uint32_t n_iters)
         }
         c->trees_done += k;
     }
-    HIP_TRY(hipGetLastError());
+    if (int r = enqueued(c)) return r;
     HIP_TRY(hipStreamSynchronize(c->stream));
     if (int r = check_partition(c)) return r;
     return 0;
@@ -1738,6 +1756,7 @@ int bh_autotune(bh_context *c, uint32_t iters, bh_tuning *chosen, float *ms_per_
                                  {&Tuning::hist_layout, hl_c, 6},  {&Tuning::pair_levels, pl_c, 2},
                                  {&Tuning::hist_group, hg_c, 3}};
     for (Knob const &kn : knobs) {
+        if (kn.field == &Tuning::hist_group && c->Fs > 64) continue; // unit_rows
         for (int k = 0; rc == 0 && k < kn.n; ++k) {
             Tuning t = best;
             u32 &slot = t.*kn.field;
@@ -1875,7 +1894,7 @@ int bh_grow_tree(bh_context *c, bh_node *nodes, uint32_t cap, uint32_t *n_nodes,
     if (int r = finish_growth(c)) return r;
     launch_score_update(c->stream, c->plane0, c->Fs, c->N, c->tree, c->ctl, c->d_nbins, c->F, 0.0F, nullptr,
                         c->leaf_rows, c->max_nodes);
-    HIP_TRY(hipGetLastError());
+    if (int r = enqueued(c)) return r;
     HIP_TRY(hipStreamSynchronize(c->stream));
     if (int r = check_partition(c)) return r;
     TreeCtl ctl;
@@ -1921,7 +1940,7 @@ int bh_histogram(bh_context *c, const uint32_t *rows, uint64_t n, float *out_f32
     HIP_TRY(hipMemcpy(c->fops, &fo, sizeof(fo), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->ctl, &ctl, sizeof(ctl), hipMemcpyHostToDevice));
     enqueue_build(c, c->hist[0], c->hist[0], 1, std::max(1u, std::min(units, 4096u)));
-    HIP_TRY(hipGetLastError());
+    if (int r = enqueued(c)) return r;
     HIP_TRY(hipStreamSynchronize(c->stream));
     hipFree(d_rows);
     size_t const nc = c->node_cells();
@@ -2085,7 +2104,7 @@ int bh_profile_hist(bh_context *c, uint32_t n_iters, double *ms_total, double *b
     for (u32 it = 0; it < n_iters; ++it)
         if (int r = enqueue_iteration(c)) return r;
     c->prof = false;
-    HIP_TRY(hipGetLastError());
+    if (int r = enqueued(c)) return r;
     HIP_TRY(hipStreamSynchronize(c->stream));
     if (int r = check_partition(c)) return r;
     c->trees_done += n_iters;

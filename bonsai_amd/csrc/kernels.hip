@@ -3339,7 +3339,8 @@ hipError_t launch_hist(hipStream_t s, bool q, HistChunk const *chunks, TreeCtl c
                        u32 *cnt_next, PartOp const *routes, bool group, void const *hist_cur)
 {
     if (Fs > 64u) {
-        if (!q && !fx) return hipErrorInvalidValue;
+        // k_hist_wide adds a whole unit into packed cells, which hold one sub-unit's rows.
+        if (group || routes || (!q && !fx)) return hipErrorInvalidValue;
         size_t const wlds = static_cast<size_t>((fsl + 3u) / 4u * 4u) * hist_wide_stride(SB) * (q ? 8u : 16u);
         dim3 const wgrid((F + fsl - 1) / fsl, grid_x);
         u32 const magic = static_cast<u32>(((1ull << 32) + SB - 1u) / SB); // exact quotients below 2^16 cells

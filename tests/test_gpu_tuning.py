@@ -3,7 +3,8 @@ found it (scores, trees, iteration counter)."""
 import numpy as np
 import pytest
 
-from test_gpu_depthwise import ctx_for, tall_data
+from oracle_lib import HIST_INT, cfg as orc_cfg
+from test_gpu_depthwise import assert_same_tree, ctx_for, tall_data
 
 pytestmark = pytest.mark.gpu
 
@@ -78,6 +79,51 @@ def test_launch_shapes_do_not_change_results(hip, orc, tall, quantized):
         for a, b in zip(trees, ref_trees):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
         assert np.array_equal(scores.view(np.uint32), ref_scores.view(np.uint32))
+
+
+@pytest.fixture(scope="module")
+def wide():
+    """70 features (rows of more than 64 bytes), several 32,768-row histogram units."""
+    n, f = 70_001, 70
+    rng = np.random.default_rng(11)
+    nb = np.full(f, 256, np.uint16)
+    nb[::7] = 18
+    bins = (rng.random((n, f)) * nb).astype(np.uint8)
+    y = (bins[:, 1] + 0.5 * bins[:, 2] + rng.normal(0, 40, n) > 190).astype(np.float32)
+    return bins, nb, y
+
+
+@pytest.mark.parametrize("quantized", [True, False])
+def test_launch_shapes_do_not_change_wide_row_results(hip, orc, wide, quantized):
+    """Rows of more than 64 bytes take single sub-units whatever hist_group says; a
+    grouped tree is the oracle's."""
+    bins, nb, y = wide
+    ref_trees, ref_scores = fit(hip, orc, bins, nb, y, quantized, iters=2)
+    if quantized:
+        ctx = ctx_for(hip, bins, nb, quantized=True, max_depth=6)
+        g, h = orc.logloss_grad(np.full(y.size, orc.init_score(1, y), np.float32), y)
+        gq, hq, sc = ctx.set_gradients(g, h)
+        want, rows = orc.grow_depthwise(bins, nb, gq=gq, hq=hq, scales=sc, c=orc_cfg(max_depth=6), mode=HIST_INT)
+        ctx.set_tuning(hist_group=4)
+        got, got_rows = ctx.grow_tree()
+        ctx.close()
+        assert_same_tree(got, want)
+        assert np.array_equal(got_rows, rows)
+    for shape in SHAPES:
+        trees, scores = fit(hip, orc, bins, nb, y, quantized, tuning=shape, iters=2)
+        assert len(trees) == len(ref_trees)
+        for a, b in zip(trees, ref_trees):
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+        assert np.array_equal(scores.view(np.uint32), ref_scores.view(np.uint32))
+
+
+def test_autotune_wide_rows(hip, orc, wide):
+    bins, nb, y = wide
+    ref_trees, ref_scores = fit(hip, orc, bins, nb, y, True)
+    trees, scores = fit(hip, orc, bins, nb, y, True, autotune=True)
+    for a, b in zip(trees, ref_trees):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+    assert np.array_equal(scores.view(np.uint32), ref_scores.view(np.uint32))
 
 
 def test_autotune_keeps_model_state(hip, orc, tall):
