@@ -1719,6 +1719,10 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     std::vector<std::vector<u32>> levels(n_trees);
     std::vector<u32> feats;
     u32 deepest = 0;
+    // Leaf magnitudes: the largest of every tree, and whether all are finite (with one that
+    // is not, every contribution is NaN).
+    std::vector<double> leaf_top(n_trees, 0.0);
+    bool leaves_finite = true;
     for (u32 t = 0; t < n_trees; ++t) {
         bh_node const *tn = nodes + tree_offsets[t];
         u32 const end = t + 1 < n_trees ? tree_offsets[t + 1] : 0;
@@ -1729,7 +1733,10 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
             u32 const i = stack.back();
             stack.pop_back();
             count = std::max(count, i + 1);
-            if (tn[i].feature >= 0) {
+            if (tn[i].feature < 0) {
+                leaves_finite = leaves_finite && std::isfinite(tn[i].value);
+                leaf_top[t] = std::max(leaf_top[t], std::fabs(static_cast<double>(tn[i].value)));
+            } else {
                 if (static_cast<u32>(tn[i].feature) >= n_features || tn[i].bin > 255) {
                     delete p;
                     return sfail(1, "tree node out of range (feature id or bin)");
@@ -1821,19 +1828,12 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
         u32 const m = std::max<u32>(deepest <= 8 ? 2u : 4u, (p->max_len + 1u) / 2u);
         // A contribution is at most 4 max|leaf| of its tree, and one level's together too.
         double top = 0.0, sum = 0.0;
-        for (u32 t = 0; t < n_trees; ++t) {
-            u32 const count = (t + 1 < n_trees ? roots[t + 1] : static_cast<u32>(pn.size())) - roots[t];
-            double v = 0.0;
-            for (u32 i = 0; i < count; ++i)
-                if (nodes[tree_offsets[t] + i].feature < 0) {
-                    double const a = std::fabs(static_cast<double>(nodes[tree_offsets[t] + i].value));
-                    v = a <= v ? v : a; // keeps a NaN
-                }
-            top = v <= top ? top : v;
+        for (double v : leaf_top) {
+            top = std::max(top, v);
             sum += v;
         }
         double scale = 1.0;
-        if (std::isfinite(sum) && sum > 0.0) {
+        if (leaves_finite && sum > 0.0) {
             int e1 = 0, e2 = 0;
             (void)std::frexp(top, &e1);
             (void)std::frexp(sum * std::max(1u, deepest), &e2);
@@ -1876,7 +1876,7 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
         p->tree_m = m;
         p->tree_depth = deepest;
         p->n_ttrees = static_cast<u32>(tfirst.size() - 1);
-        p->tree_scale = std::isfinite(sum) ? scale * g : std::nan("");
+        p->tree_scale = leaves_finite ? scale * g : std::nan("");
     }
     std::vector<u32> words;
     std::vector<Tile> tiles;

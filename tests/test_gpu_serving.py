@@ -263,3 +263,19 @@ def test_predict_tiles_match_the_walk(hip, orc, depth, n_features, n_trees, p_le
         ref = orc.predict(trees, rows, nb, 0.1, -0.5)
         assert np.array_equal(dev.view(np.uint32), ref.view(np.uint32)), n
     p.close()
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("at", [0, 1, -1])
+@pytest.mark.parametrize("depth,n_rows", [(3, 5), (6, 70), (6, 20_000)])
+def test_shap_nonfinite_leaf(hip, depth, n_rows, at, value):
+    """A leaf that is not finite, wherever it stands, makes every contribution NaN."""
+    rng = np.random.default_rng([depth, n_rows])
+    nb = np.full(9, 60, np.uint16)
+    trees = random_trees(rng, 4, depth, 9, nb, 0.2)
+    leaves = np.flatnonzero(trees[2]["feature"] < 0)
+    trees[2]["value"][leaves[at]] = value
+    rows = (rng.random((n_rows, 9)) * nb).astype(np.uint8)
+    p = hip.Predictor(trees, nb, 0.3, 0.25)
+    assert np.isnan(p.shap(rows)[:, :-1]).all()
+    p.close()
