@@ -739,7 +739,7 @@ __global__ __launch_bounds__(1024) void k_hist_wide(
         }
         __syncthreads();
         for (u32 i = threadIdx.x; i < cells; i += blockDim.x) {
-            u32 const fl = __umulhi(i, sb_magic), b = i - fl * SB; // i / SB
+            u32 const fl = sb_magic ? __umulhi(i, sb_magic) : i, b = i - fl * SB; // i / SB
             unsigned long long const *p = lh + ((fl & 3u) * Dw + (fl >> 2)) * SL + b;
             if (ch.part != kNone) {
                 size_t const o = static_cast<size_t>(ch.part) * node_cells + cell0 + i;
@@ -3343,7 +3343,8 @@ hipError_t launch_hist(hipStream_t s, bool q, HistChunk const *chunks, TreeCtl c
         if (group || routes || (!q && !fx)) return hipErrorInvalidValue;
         size_t const wlds = static_cast<size_t>((fsl + 3u) / 4u * 4u) * hist_wide_stride(SB) * (q ? 8u : 16u);
         dim3 const wgrid((F + fsl - 1) / fsl, grid_x);
-        u32 const magic = static_cast<u32>(((1ull << 32) + SB - 1u) / SB); // exact quotients below 2^16 cells
+        // exact quotients below 2^16 cells; SB 1 has no 32-bit magic (0: the cell is the feature's)
+        u32 const magic = SB == 1u ? 0u : static_cast<u32>(((1ull << 32) + SB - 1u) / SB);
         hipLaunchKernelGGL(q ? k_hist_wide<true> : k_hist_wide<false>, wgrid, dim3(t_tune.hist_threads), wlds, s, chunks,
                            ctl, pl0, pl1, plp, g0, g1, gp, Fs, F, SB, magic, fsl, partials, hist_cur, hist_next,
                            cnt_next, fx);

@@ -6,7 +6,7 @@ against the oracle restating the device's fixed summation order.
 import numpy as np
 import pytest
 
-from oracle_lib import CHUNK_ADAPTIVE, HIST_F32_FIXED, HIST_INT, cfg as orc_cfg
+from oracle_lib import CHUNK_ADAPTIVE, DEVICE_CHUNK, HIST_F32_FIXED, HIST_INT, cfg as orc_cfg
 from test_gpu_depthwise import assert_same_tree, ctx_for, grad_of, tall_data
 
 pytestmark = pytest.mark.gpu
@@ -206,6 +206,38 @@ def test_wide_row_edges(hip, orc, f, n, depth, quantized):
         ctx.close()
         assert_same_tree(nodes, ref)
         assert np.array_equal(lor[rows], rlor)
+
+
+@pytest.mark.parametrize("quantized", [True, False])
+@pytest.mark.parametrize("f,n", [(65, 100), (70, 8192), (131, 20_001)])
+def test_wide_single_bin_histogram(hip, orc, f, n, quantized):
+    """Planes of more than 64 features with one bin each: every feature's only cell holds
+    the rows' sums, which a finder that skips the first features takes its totals from."""
+    rng = np.random.default_rng(f)
+    bins, nb = np.zeros((n, f), np.uint8), np.ones(f, np.uint16)
+    g, h = orc.mse_grad(np.zeros(n, np.float32), rng.normal(0, 1, n).astype(np.float32))
+    ctx = ctx_for(hip, bins, nb, quantized=quantized, max_depth=2)
+    gq, hq, sc = ctx.set_gradients(g, h)
+    rows = np.arange(n, dtype=np.uint32)
+    got = ctx.histogram(rows)
+    mask = np.zeros(f, np.uint8)
+    mask[f - 1] = 1
+    ctx.set_feature_mask(mask)
+    nodes, _ = ctx.grow_tree()
+    ctx.close()
+    orc.set_feature_mask(mask)
+    try:
+        if quantized:
+            want = orc.hist_int(bins, rows, gq, hq, 1)
+            ref, _ = orc.grow_depthwise(bins, nb, gq=gq, hq=hq, scales=sc, c=orc_cfg(max_depth=2), mode=HIST_INT)
+        else:
+            want = orc.hist_f32(bins, rows, g, h, 1, HIST_F32_FIXED, DEVICE_CHUNK)
+            ref, _ = orc.grow_depthwise(bins, nb, g=g, h=h, c=orc_cfg(max_depth=2), mode=HIST_F32_FIXED,
+                                        scales=(orc.fx_shift(g), orc.fx_shift(h)))
+    finally:
+        orc.set_feature_mask(None)
+    assert np.array_equal(got.reshape(f, 2), np.reshape(want, (f, 2)))
+    assert_same_tree(nodes, ref)
 
 
 @pytest.mark.parametrize("grower", ["hip_leafwise", "hip_levelwise"])
