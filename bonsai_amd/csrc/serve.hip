@@ -477,9 +477,12 @@ __global__ __launch_bounds__(256) void k_shap(u8 const *__restrict__ bins, u64 n
 // issue: 14,900 wave instructions per 255-node tree and 64 rows (about 58 a node, against
 // some 265 a path of the packed form) at 4 clocks each are 6.2 of the 7.6 ms that 16,384
 // rows of 1,000 such trees take (packed form 28.4 ms).  Contributions go through float to
-// 64-bit fixed point (one FP64 add against 1.5 * 2^52)
-// and into LDS with conflict-free integer atomics: exact in any order, so a row's result
-// depends neither on the batch nor on how trees are dealt to waves and workgroups.
+// 64-bit fixed point and into LDS with conflict-free integer atomics: exact in any order, so
+// a row's result depends neither on the batch nor on how trees are dealt to waves and
+// workgroups.  The grid is never coarser than the packed form's (tree_grid): where the
+// largest leaf stands among many (Sum |leaf| of some 2^11 of it) one FP64 add against
+// 1.5 * 2^52 rounds to it, otherwise (WIDE: few trees, or one leaf far above the rest) a
+// conversion of the whole 64 bits does, which takes the batch above 5% longer (8.0 ms).
 // ---------------------------------------------------------------------------------
 // A tree is stored as the steps of its depth-first walk, read as one sequential stream:
 //   block    a subtree of at most three levels, as seven nodes in one straight run of
@@ -528,9 +531,9 @@ struct TQuad {
     float y[kTreeShapMaxM], w[kTreeShapMaxM];
 };
 
-// U: levels above the blocks.  AT: the walk may start below a tree's root (levels come
-// from the steps) and meet shares' values.
-template <int M, int U, bool AT = false> struct TreeShap {
+// U: levels above the blocks.  WIDE: contributions of up to 63 bits (tree_grid).  AT: the
+// walk may start below a tree's root (levels come from the steps) and meet shares' values.
+template <int M, int U, bool WIDE, bool AT = false> struct TreeShap {
     typedef float V[M];
     u8 const *bins;      // LDS: this lane's column of the bins
     unsigned char *phi;  // LDS: this lane's column of the sums
@@ -594,10 +597,16 @@ template <int M, int U, bool AT = false> struct TreeShap {
     __device__ __forceinline__ void add(u32 split, float c)
     {
         u32 const col = split & 0xFFFFu;
-        // |c| < 2^51: the sum's low 52 bits hold round(c) beside 1.5 * 2^52's own
-        double const v = static_cast<double>(c) + 6755399441055744.0;
-        atomicAdd(reinterpret_cast<unsigned long long *>(phi + min(col, col - plane) * 8u),
-                  static_cast<unsigned long long>(__double_as_longlong(v)) - 0x4338000000000000ull);
+        unsigned long long q;
+        if (WIDE) { // round(c) as hi * 2^32 + lo, exactly
+            double const v = __builtin_rintf(c), hi = __builtin_floor(v * 0x1p-32);
+            u32 const lo = static_cast<u32>(__builtin_fma(hi, -0x1p32, v));
+            q = static_cast<unsigned long long>(static_cast<u32>(static_cast<int>(hi))) << 32 | lo;
+        } else { // |c| < 2^51: the sum's low 52 bits hold round(c) beside 1.5 * 2^52's own
+            double const v = static_cast<double>(c) + 6755399441055744.0;
+            q = static_cast<unsigned long long>(__double_as_longlong(v)) - 0x4338000000000000ull;
+        }
+        atomicAdd(reinterpret_cast<unsigned long long *>(phi + min(col, col - plane) * 8u), q);
     }
 
     static constexpr bool past_half(int q) { return 2 * q >= M + (M & 1); }
@@ -846,7 +855,7 @@ struct SplitTree {
 };
 constexpr u32 kSplitThreads = 512;   // 16 waves a workgroup spill (128 registers): a sixth slower at depth 8
 constexpr u32 kSplitLevels = 6; // cut at most this far below the root (TreePacker::cut_of)
-template <int M>
+template <int M, bool WIDE>
 __global__ __launch_bounds__(kSplitThreads) void k_shap_split(u8 const *__restrict__ bins, u64 n, u64 stride, u32 F,
                                                              u16 const *__restrict__ last,
                                                              TSlot const *__restrict__ slots,
@@ -888,7 +897,7 @@ __global__ __launch_bounds__(kSplitThreads) void k_shap_split(u8 const *__restri
     for (u32 t = blockIdx.y; t < n_trees; t += gridDim.y) {
         SplitTree const tr = trees[t];
         for (u32 j = wave; j < tr.n_shares; j += nw) {
-            TreeShap<M, 3, true> w;
+            TreeShap<M, 3, WIDE, true> w;
             float T[M], H[M];
             begin(w, T);
             w.seek(slots, __builtin_amdgcn_readfirstlane(first[tr.share0 + j]));
@@ -900,7 +909,7 @@ __global__ __launch_bounds__(kSplitThreads) void k_shap_split(u8 const *__restri
         }
         __syncthreads();
         if (wave == 0 && tr.top != kNone) {
-            TreeShap<M, kSplitLevels, true> w;
+            TreeShap<M, kSplitLevels, WIDE, true> w;
             float T[M], H[M];
             begin(w, T);
             w.seek(slots, __builtin_amdgcn_readfirstlane(tr.top));
@@ -919,7 +928,7 @@ __global__ __launch_bounds__(kSplitThreads) void k_shap_split(u8 const *__restri
 }
 
 // gridDim.y workgroups share a row block; each of their waves walks a run of trees.
-template <int M, int U>
+template <int M, int U, bool WIDE>
 __global__ __launch_bounds__(kTreeShapThreads, tree_shap_waves(U)) void k_shap_tree(
     u8 const *__restrict__ bins, u64 n, u64 stride, u32 F, u16 const *__restrict__ last,
     TSlot const *__restrict__ slots, u32 const *__restrict__ first, u32 n_trees, TQuad quad, float lr, double bias,
@@ -942,7 +951,7 @@ __global__ __launch_bounds__(kTreeShapThreads, tree_shap_waves(U)) void k_shap_t
     __syncthreads();
     u32 const lane = threadIdx.x & 63u;
     u32 const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    TreeShap<M, U> w;
+    TreeShap<M, U, WIDE> w;
     w.bins = s_bins + lane;
     w.phi = reinterpret_cast<unsigned char *>(s_phi + lane);
     w.plane = plane;
@@ -1438,6 +1447,36 @@ TQuad tree_quad(GaussRule const &r, double &g)
     return q;
 }
 
+// Leaf magnitudes of an ensemble.
+struct LeafStats {
+    std::vector<double> top; // the largest of every tree
+    double sum = 0.0;        // of all
+    bool finite = true;      // with one leaf that is not, every contribution is NaN
+    bool covers = true;      // every node's children hold fractions of it that sum to 1 at most
+};
+
+// log2 of the tree form's fixed-point scale.  The packed form's grid is 2^61 / (4 Sum |leaf|),
+// the next power of two at least what 63-bit contributions take (wide).  The 52-bit add takes
+// contributions below 2^51: each is at most 4 max |leaf| of its tree, and one level's of a
+// tree together too, if the covers are proper; it serves where its grid is as fine.
+int tree_grid(LeafStats const &s, u32 deepest, bool &wide)
+{
+    double top = 0.0, tops = 0.0;
+    for (double v : s.top) {
+        top = std::max(top, v);
+        tops += v;
+    }
+    wide = false;
+    if (!s.finite || s.sum <= 0.0) return 0;
+    int e_all = 0, e_top = 0, e_tops = 0;
+    (void)std::frexp(s.sum, &e_all);
+    (void)std::frexp(top, &e_top);
+    (void)std::frexp(tops * std::max(1u, deepest), &e_tops);
+    int const narrow = std::min(48 - e_top, 60 - e_tops);
+    wide = !s.covers || narrow < 60 - e_all;
+    return wide ? 60 - e_all : narrow;
+}
+
 // tree_expected_value (src/shap.cpp:246-292): cover-weighted mean of the leaves.
 double expected_value(bh_node const *t, u32 id)
 {
@@ -1463,6 +1502,7 @@ struct bh_predictor {
     // tree-form TreeSHAP (tree_m quadrature nodes; 0: the packed form serves the ensemble)
     u32 tree_m = 0, tree_depth = 0, n_ttrees = 0, max_shares = 0; // max_shares 0: no split form
     double tree_scale = 1.0;   // its fixed-point scale, times the weights' common factor
+    bool tree_wide = false;    // TreeShap's WIDE
     TQuad quad{};
     TSlot *d_tslots = nullptr;
     u32 *d_tfirst = nullptr;
@@ -1580,8 +1620,9 @@ int launch_shap_tree(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, doubl
         }
         dim3 const sgrid(blocks, p->n_ttrees);
 #define BH_SP(MV)                                                                                                  \
-    hipLaunchKernelGGL((k_shap_split<MV>), sgrid, dim3(kSplitThreads), split_lds, s, d_bins, n, stride, p->F,      \
-                       p->d_last, p->d_tslots, p->d_sfirst, p->d_split, p->n_ttrees, p->quad, d_out)
+    hipLaunchKernelGGL((p->tree_wide ? k_shap_split<MV, true> : k_shap_split<MV, false>), sgrid,                   \
+                       dim3(kSplitThreads), split_lds, s, d_bins, n, stride, p->F, p->d_last,                      \
+                       p->d_tslots, p->d_sfirst, p->d_split, p->n_ttrees, p->quad, d_out)
         switch (m_of(p->tree_m, upper)) {
         case 2: BH_SP(2); break;
         case 3: BH_SP(3); break;
@@ -1598,8 +1639,9 @@ int launch_shap_tree(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, doubl
     }
     dim3 const grid(blocks, split);
 #define BH_TS(MV, UV)                                                                                              \
-    hipLaunchKernelGGL((k_shap_tree<MV, UV>), grid, dim3(threads), lds, s, d_bins, n, stride, p->F, p->d_last,     \
-                       p->d_tslots, p->d_tfirst, p->n_ttrees, p->quad, p->lr, p->shap_bias, p->tree_scale, d_out)
+    hipLaunchKernelGGL((p->tree_wide ? k_shap_tree<MV, UV, true> : k_shap_tree<MV, UV, false>), grid,              \
+                       dim3(threads), lds, s, d_bins, n, stride, p->F, p->d_last, p->d_tslots, p->d_tfirst,        \
+                       p->n_ttrees, p->quad, p->lr, p->shap_bias, p->tree_scale, d_out)
     if (upper <= 5) {
         if (p->tree_m <= 2) BH_TS(2, 5);
         else if (p->tree_m == 3) BH_TS(3, 5);
@@ -1719,10 +1761,8 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     std::vector<std::vector<u32>> levels(n_trees);
     std::vector<u32> feats;
     u32 deepest = 0;
-    // Leaf magnitudes: the largest of every tree, and whether all are finite (with one that
-    // is not, every contribution is NaN).
-    std::vector<double> leaf_top(n_trees, 0.0);
-    bool leaves_finite = true;
+    LeafStats leaves;
+    leaves.top.assign(n_trees, 0.0);
     for (u32 t = 0; t < n_trees; ++t) {
         bh_node const *tn = nodes + tree_offsets[t];
         u32 const end = t + 1 < n_trees ? tree_offsets[t + 1] : 0;
@@ -1734,13 +1774,17 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
             stack.pop_back();
             count = std::max(count, i + 1);
             if (tn[i].feature < 0) {
-                leaves_finite = leaves_finite && std::isfinite(tn[i].value);
-                leaf_top[t] = std::max(leaf_top[t], std::fabs(static_cast<double>(tn[i].value)));
+                double const a = std::fabs(static_cast<double>(tn[i].value));
+                leaves.finite = leaves.finite && std::isfinite(a);
+                leaves.top[t] = std::max(leaves.top[t], a);
+                leaves.sum += a;
             } else {
                 if (static_cast<u32>(tn[i].feature) >= n_features || tn[i].bin > 255) {
                     delete p;
                     return sfail(1, "tree node out of range (feature id or bin)");
                 }
+                double const c = tn[i].cover, l = tn[tn[i].left].cover, r = tn[tn[i].right].cover;
+                leaves.covers = leaves.covers && (c <= 0.0 || (l >= 0.0 && r >= 0.0 && l + r <= c * 1.0001));
                 stack.push_back(tn[i].left);
                 stack.push_back(tn[i].right);
             }
@@ -1826,19 +1870,8 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     if (tree_form) {
         // kernels' node counts: 2, 3, 4 (up to 8 levels), 4, 5, 6 (more)
         u32 const m = std::max<u32>(deepest <= 8 ? 2u : 4u, (p->max_len + 1u) / 2u);
-        // A contribution is at most 4 max|leaf| of its tree, and one level's together too.
-        double top = 0.0, sum = 0.0;
-        for (double v : leaf_top) {
-            top = std::max(top, v);
-            sum += v;
-        }
-        double scale = 1.0;
-        if (leaves_finite && sum > 0.0) {
-            int e1 = 0, e2 = 0;
-            (void)std::frexp(top, &e1);
-            (void)std::frexp(sum * std::max(1u, deepest), &e2);
-            scale = std::ldexp(1.0, std::min(48 - e1, 60 - e2));
-        }
+        int const bits = tree_grid(leaves, deepest, p->tree_wide);
+        double const scale = std::ldexp(1.0, bits);
         pack.last = last_bin;
         pack.F = n_features;
         pack.scale = scale;
@@ -1876,7 +1909,7 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
         p->tree_m = m;
         p->tree_depth = deepest;
         p->n_ttrees = static_cast<u32>(tfirst.size() - 1);
-        p->tree_scale = leaves_finite ? scale * g : std::nan("");
+        p->tree_scale = leaves.finite ? scale * g : std::nan("");
     }
     std::vector<u32> words;
     std::vector<Tile> tiles;

@@ -279,3 +279,33 @@ def test_shap_nonfinite_leaf(hip, depth, n_rows, at, value):
     p = hip.Predictor(trees, nb, 0.3, 0.25)
     assert np.isnan(p.shap(rows)[:, :-1]).all()
     p.close()
+
+
+@pytest.mark.parametrize("depth,n_rows", [(4, 3), (4, 20_000), (7, 5), (7, 20_000), (10, 70)])
+def test_shap_small_leaves_beside_a_large_one(hip, orc, depth, n_rows):
+    """One leaf of 1e6 and a subtree of leaves around 1e-6 on the root's other side: the
+    grid is Sum |leaf| / 2^59 or finer, so the subtree's features (each on at most 2^(depth
+    - 1) nodes, half a grid step apiece) keep their digits: that and 64 float roundings
+    of terms that sum to at most twice the subtree's largest leaf."""
+    rng = np.random.default_rng([depth, n_rows])
+    nb = np.full(9, 60, np.uint16)
+    sub = random_trees(rng, 1, depth - 1, 8, nb[1:], 0.1)[0]
+    small = sub["value"] * 1e-5
+    sub["value"] = small
+    inner = sub["feature"] >= 0
+    sub["feature"][inner] += 1
+    sub["left"][inner] += 2
+    sub["right"][inner] += 2
+    root = np.array([(0, 30, 1, 1, 2, 0.0, 3e6, 1.0), (-1, 0, 0, 0, 0, 1e6, 2e6, 0.0)], NODE_DTYPE)
+    trees = [np.concatenate([root, sub])]
+    rows = (rng.random((n_rows, 9)) * nb).astype(np.uint8)
+    rows[:, 0] = np.where(np.arange(n_rows) % 2 == 0, 40, 3)  # into the subtree, or beside it
+    p = hip.Predictor(trees, nb, 1.0, 0.0)
+    got = p.shap(rows)
+    m = min(n_rows, 300)
+    ref = orc.pred_contribs(trees, rows[:m], nb, 1.0, 0.0, depth)
+    leaf_sum = float(np.abs(trees[0]["value"][trees[0]["feature"] < 0]).sum())
+    tol = 2 ** (depth - 1) * 0.5 * leaf_sum / 2 ** 59 + 64 * 2 ** -24 * 2 * float(np.abs(small).max())
+    assert np.max(np.abs(got[:m, 1:9] - ref[:, 1:9])) <= tol
+    assert np.array_equal(p.shap(rows[:2]), got[:2])
+    p.close()
