@@ -309,3 +309,22 @@ def test_shap_small_leaves_beside_a_large_one(hip, orc, depth, n_rows):
     assert np.max(np.abs(got[:m, 1:9] - ref[:, 1:9])) <= tol
     assert np.array_equal(p.shap(rows[:2]), got[:2])
     p.close()
+
+
+@pytest.mark.parametrize("used,longest", [(8, 8), (9, 9), (16, 12)])
+@pytest.mark.parametrize("n_rows", [1, 33, 3_000])
+def test_shap_packed_path_lengths(hip, orc, used, longest, n_rows):
+    """The packed form's kernels for paths of up to 8 and up to 16 features, on either side
+    of the line (257 features keep the tree form off), within 1e-5 of the row's mass."""
+    rng = np.random.default_rng([used, n_rows])
+    nb = rng.integers(3, 257, 257).astype(np.uint16)
+    trees = random_trees(rng, 6, longest, used, nb, 0.3)
+    rows = (rng.random((n_rows, 257)) * nb).astype(np.uint8)
+    p = hip.Predictor(trees, nb, 0.3, 0.25)
+    got = p.shap(rows)
+    m = min(n_rows, 200)
+    ref = orc.pred_contribs(trees, rows[:m], nb, 0.3, 0.25, longest)
+    mass = np.abs(ref).sum(axis=1, keepdims=True)
+    assert np.max(np.abs(got[:m] - ref) / mass) <= 1e-5
+    assert np.array_equal(p.shap(rows[-1:])[0], got[-1])
+    p.close()
