@@ -82,20 +82,18 @@ constexpr int kMaxPath = 16;
 // tree) pairs of one tree tile from global memory into LDS, then one thread per row adds
 // the tile in tree order.  Latency bound: the walk's dependent node loads and the ordered
 // float sum (about 3 us per 1,000 trees); one row per workgroup while the rows alone do
-// not fill the chip.
+// not fill the chip (walk_shape).
 // ---------------------------------------------------------------------------------
-constexpr u32 kPredTile = 1024;    // trees whose values wait in LDS
-constexpr u32 kPredMaxRows = 8;    // rows of a workgroup
 
 __global__ __launch_bounds__(1024) void k_predict_direct(u8 const *__restrict__ bins, u64 n, u64 stride, u32 F,
-                                                         u32 rows, PNode const *__restrict__ nodes,
+                                                         u32 rows, u32 tile, PNode const *__restrict__ nodes,
                                                          u32 const *__restrict__ roots, u32 n_trees,
                                                          u16 const *__restrict__ last, float lr, float init,
                                                          float *__restrict__ out)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    float *s_val = reinterpret_cast<float *>(smem);                          // [rows][kPredTile]
-    u16 *s_last = reinterpret_cast<u16 *>(s_val + rows * kPredTile);         // [F]
+    float *s_val = reinterpret_cast<float *>(smem);                  // [rows][tile]
+    u16 *s_last = reinterpret_cast<u16 *>(s_val + rows * tile);      // [F]
     u8 *s_rows = reinterpret_cast<u8 *>(s_last + F);                         // [rows][F]
     u64 const r0 = static_cast<u64>(blockIdx.x) * rows;
     u32 const nr = static_cast<u32>(min<u64>(rows, n - r0));
@@ -106,8 +104,8 @@ __global__ __launch_bounds__(1024) void k_predict_direct(u8 const *__restrict__ 
     for (u32 f = threadIdx.x; f < F; f += blockDim.x) s_last[f] = last[f];
     __syncthreads();
     float acc = 0.0F;
-    for (u32 t0 = 0; t0 < n_trees; t0 += kPredTile) {
-        u32 const tt = min(kPredTile, n_trees - t0);
+    for (u32 t0 = 0; t0 < n_trees; t0 += tile) {
+        u32 const tt = min(tile, n_trees - t0);
         for (u32 k = threadIdx.x; k < nr * tt; k += blockDim.x) {
             u32 const rr = k / tt, t = k - rr * tt;
             PNode const *tn = nodes + roots[t0 + t];
@@ -118,11 +116,11 @@ __global__ __launch_bounds__(1024) void k_predict_direct(u8 const *__restrict__ 
                 bool const left = b == s_last[nd.feature] ? (nd.dl != 0) : (b <= nd.bin);
                 nd = tn[left ? nd.u.c.left : nd.u.c.right];
             }
-            s_val[rr * kPredTile + t] = nd.u.value;
+            s_val[rr * tile + t] = nd.u.value;
         }
         __syncthreads();
         if (threadIdx.x < nr) {
-            float const *v = s_val + threadIdx.x * kPredTile;
+            float const *v = s_val + threadIdx.x * tile;
             u32 t = 0;
             for (; t + 16 <= tt; t += 16) {
                 float4 q[4];
@@ -1513,6 +1511,7 @@ struct bh_predictor {
     u32 *d_roots = nullptr;
     // tile form (n_tiles 0: the ensemble does not fit it)
     u32 n_tiles = 0;
+    double mean_levels = 0.0;  // splits above a leaf if the mean tree were full
     u32 *d_words = nullptr;
     Tile *d_tiles = nullptr;
     TileTree *d_ttrees = nullptr;
@@ -1528,50 +1527,96 @@ struct bh_predictor {
 
 namespace {
 
-// Rows from which a batch is served from tiles: below, walking from global memory with a
-// few rows per workgroup answers sooner (2,000 rows x 1,000 depth-8 trees: 153 us against
-// 145 from tiles, whose time is flat up to 16,384 rows; 1,000 rows: 82 us).
-constexpr u64 kPredTileRows = 2048;
+constexpr size_t kPredLdsMax = 160u * 1024u;
+
+// Microseconds of a batch served from tiles, and the rows a workgroup takes: one workgroup
+// per CU (LDS), so rounds of 256 of them; a round costs a tile's barriers and loads and its
+// trees' walks (1,000 depth-8 trees, 63 tiles: 145, 235 and 595 us with 64, 256 and 1,024
+// rows; 20 of depth 12, a tile each: 39, 45 and 50).
+struct TileShape {
+    double us;
+    u32 rows;
+};
+size_t tile_lds(bh_predictor const *p, u32 rows)
+{
+    u32 const split = kTileThreads / rows;
+    return static_cast<size_t>(2u * kTileNodes * 4u) + (split > 1 ? 2u * split * 4u * rows * 4u : 0u) +
+           rows * tile_row_stride(p->F);
+}
+TileShape tile_shape(bh_predictor const *p, u64 n)
+{
+    static const struct {
+        u32 rows;
+        double tile, tree;
+    } shapes[] = {{64, 1.9, 0.045}, {256, 2.2, 0.1}, {1024, 2.4, 0.44}};
+    TileShape best{1e300, 0u};
+    for (auto const &q : shapes) {
+        u64 const rounds = ((n + q.rows - 1) / q.rows + 255) / 256;
+        double const us = static_cast<double>(rounds) * (p->n_tiles * q.tile + p->n_trees * q.tree);
+        if (us < best.us && tile_lds(p, q.rows) <= kPredLdsMax) best = TileShape{us, q.rows};
+    }
+    return best;
+}
+
+// Walking from memory costs about 6 ps a level, tree and row (2 to 7 over 1 to 100 trees of
+// 3 to 13 levels, 2,048 to 65,536 rows), 9 with kManyTrees (a row's ordered sum is long), so
+// tiles serve from where their rounds cost less: 1,000 depth-8 trees from 2,300 rows (146 us),
+// 20 of depth 12 (39 us from tiles, 20 walked at 16,384 rows) from 32,000; and never an
+// ensemble they do not hold.
+constexpr u32 kManyTrees = 500;
+bool served_from_tiles(bh_predictor const *p, u64 n)
+{
+    double const per = p->n_trees >= kManyTrees ? 9e-6 : 6e-6;
+    return p->n_tiles && static_cast<double>(n) * p->n_trees * p->mean_levels * per > tile_shape(p, n).us;
+}
+
+// Rows of a workgroup, trees whose values wait in its LDS and its threads at most.  Of many
+// trees, rows a lane each (64) share a tree's nodes, and few values a row keep workgroups on
+// a CU while one thread a row adds: 1,000 depth-8 trees, 300 features: 65,536 rows 4,483 ->
+// 2,202 us against 8 rows and 1,024 trees, 4,096 rows (16 and 256) 299 -> 232; fewer rows
+// have the chip to fill first, and of 100 trees 8 rows take as long or less.  A tile of the
+// trees there are: 262,144 rows of 4 depth-13 trees 470 -> 104 us.
+struct WalkShape {
+    u32 rows, tile, threads;
+};
+WalkShape walk_shape(u64 n, u32 n_trees, u32 F)
+{
+    u32 const lanes = 64u / std::min(64u, std::max(1u, n_trees)); // rows that fill a wave
+    WalkShape w{static_cast<u32>(std::min<u64>(8u, std::max<u64>(lanes, n / 1024))), 1024u, 1024u};
+    if (n >= 16384 && n_trees >= kManyTrees) w = WalkShape{64u, 64u, 256u};
+    else if (n >= 2560 && n_trees >= kManyTrees) w = WalkShape{16u, 256u, 256u};
+    w.tile = std::min(w.tile, (std::max(1u, n_trees) + 15u) / 16u * 16u); // float4 reads of a row's values
+    while (w.rows > 1 && static_cast<size_t>(w.rows) * (w.tile * sizeof(float) + F) > kPredLdsMax / 4) w.rows /= 2;
+    // A thread a walk; with few trees 256 to load the rows while the chip has room for them
+    // (4 depth-13 trees, 300 features: 16,384 rows 12.7 -> 10.2 us, but 200,000 80.7 -> 118.6).
+    u32 const walks = w.rows * std::min(w.tile, std::max(1u, n_trees));
+    u32 const load = n / w.rows <= 4096u ? std::min(256u, w.rows * F) : 64u;
+    w.threads = std::min(w.threads, (std::max(walks, load) + 63u) / 64u * 64u);
+    return w;
+}
 
 int launch_predict(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, float *d_out, hipStream_t s)
 {
     if (n == 0) return 0;
-    constexpr size_t kLdsMax = 160u * 1024u;
-    if (p->n_tiles && n >= kPredTileRows) {
-        auto const lds = [&](u32 rows) {
-            u32 const split = kTileThreads / rows;
-            return static_cast<size_t>(2u * kTileNodes * 4u) + (split > 1 ? 2u * split * 4u * rows * 4u : 0u) +
-                   rows * tile_row_stride(p->F);
-        };
+    if (served_from_tiles(p, n)) {
+        u32 const rows = tile_shape(p, n).rows;
 #define BH_PT(R)                                                                                                    \
-    hipLaunchKernelGGL(k_predict_tile<R>, dim3(static_cast<u32>((n + R - 1) / R)), dim3(kTileThreads), lds(R), s,   \
-                       d_bins, n, stride, p->F, p->d_words, p->d_tiles, p->n_tiles, p->d_ttrees, p->d_last, p->lr,  \
-                       p->init, d_out)
-        // One workgroup per CU (LDS): a round of 256 workgroups over 1,000 depth-8 trees
-        // takes 145 us with 64 rows each, 235 with 256 and 595 with 1,024.  The cheapest
-        // rounds win.
-        auto const cost = [&](u32 rows, u64 round) { return ((n + rows - 1) / rows + 255) / 256 * round; };
-        u64 const c64 = cost(64, 145), c256 = lds(256) <= kLdsMax ? cost(256, 235) : ~0ull,
-                  c1024 = lds(1024) <= kLdsMax ? cost(1024, 595) : ~0ull;
-        if (c64 <= c256 && c64 <= c1024) BH_PT(64);
-        else if (c256 <= c1024) BH_PT(256);
+    hipLaunchKernelGGL(k_predict_tile<R>, dim3(static_cast<u32>((n + R - 1) / R)), dim3(kTileThreads),              \
+                       tile_lds(p, R), s, d_bins, n, stride, p->F, p->d_words, p->d_tiles, p->n_tiles,              \
+                       p->d_ttrees, p->d_last, p->lr, p->init, d_out)
+        if (rows == 64) BH_PT(64);
+        else if (rows == 256) BH_PT(256);
         else BH_PT(1024);
 #undef BH_PT
         SHIP(hipGetLastError());
         return 0;
     }
-    u32 rows = static_cast<u32>(std::min<u64>(kPredMaxRows, std::max<u64>(1, n / 1024)));
-    auto const lds_of = [&](u32 r) {
-        return static_cast<size_t>(r) * (kPredTile * sizeof(float) + p->F) + p->F * sizeof(u16);
-    };
-    while (rows > 1 && lds_of(rows) > kLdsMax / 4) rows /= 2;
-    size_t const lds = lds_of(rows);
-    if (lds > kLdsMax) return sfail(1, "predict: too many features for one row in LDS");
-    u32 const blocks = static_cast<u32>((n + rows - 1) / rows);
-    u32 const walks = rows * std::min(kPredTile, std::max(1u, p->n_trees));
-    u32 const threads = std::min(1024u, (walks + 63u) / 64u * 64u);
-    hipLaunchKernelGGL(k_predict_direct, dim3(blocks), dim3(threads), lds, s, d_bins, n, stride, p->F, rows, p->d_nodes,
-                       p->d_roots, p->n_trees, p->d_last, p->lr, p->init, d_out);
+    WalkShape const w = walk_shape(n, p->n_trees, p->F);
+    size_t const lds = static_cast<size_t>(w.rows) * (w.tile * sizeof(float) + p->F) + p->F * sizeof(u16);
+    if (lds > kPredLdsMax) return sfail(1, "predict: too many features for one row in LDS");
+    hipLaunchKernelGGL(k_predict_direct, dim3(static_cast<u32>((n + w.rows - 1) / w.rows)), dim3(w.threads), lds, s,
+                       d_bins, n, stride, p->F, w.rows, w.tile, p->d_nodes, p->d_roots, p->n_trees, p->d_last, p->lr,
+                       p->init, d_out);
     SHIP(hipGetLastError());
     return 0;
 }
@@ -1868,6 +1913,7 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
                 w[rr * nn / 2 + i] = static_cast<float>(1.0 / (static_cast<double>(nn) * binom[i]));
         }
     }
+    if (n_trees) p->mean_levels = std::log2((static_cast<double>(pn.size()) / n_trees + 1.0) / 2.0);
     TreePacker pack{};
     std::vector<u32> tfirst;
     std::vector<SplitTree> split;
@@ -2002,7 +2048,7 @@ int bh_predict(bh_predictor *p, const uint8_t *bins, uint64_t n, uint64_t row_st
     if (row_stride < p->F) return sfail(1, "row_stride < n_features");
     if (n == 0) return 0;
     SHIP(hipSetDevice(p->device));
-    if (n < kPredTileRows) {
+    if (!served_from_tiles(p, n)) {
         // the walk reads a row once and writes one value: both stay in host memory
         SmallCall c(p, n * row_stride, n * sizeof(float));
         if (c.ready()) {

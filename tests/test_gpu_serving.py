@@ -244,9 +244,9 @@ def test_shap_split_trees_equal_whole_walks(hip, depth, used, p_leaf):
     (1, 1, 3, 0.0), (4, 28, 1, 0.0), (8, 28, 37, 0.0), (9, 28, 130, 0.3), (6, 256, 70, 0.1), (12, 60, 9, 0.2),
     (3, 257, 5, 0.0), (13, 5, 2, 0.0)])
 def test_predict_tiles_match_the_walk(hip, orc, depth, n_features, n_trees, p_leaf):
-    """Batches from 2,048 rows walk trees from LDS tiles (64, 256 or 1,024 rows per
-    workgroup); smaller ones, more than 256 features and trees past a tile walk from
-    memory.  Every row is bit-equal to the oracle's walk in each."""
+    """Large batches walk trees from LDS tiles (256 or 1,024 rows per workgroup here);
+    smaller ones, more than 256 features and trees past a tile walk from memory.  Every
+    row is bit-equal to the oracle's walk in each."""
     rng = np.random.default_rng([depth, n_features, n_trees])
     nb = rng.integers(2, 257, n_features).astype(np.uint16)
     trees = random_trees(rng, n_trees, depth, n_features, nb, p_leaf)
@@ -327,4 +327,24 @@ def test_shap_packed_path_lengths(hip, orc, used, longest, n_rows):
     mass = np.abs(ref).sum(axis=1, keepdims=True)
     assert np.max(np.abs(got[:m] - ref) / mass) <= 1e-5
     assert np.array_equal(p.shap(rows[-1:])[0], got[-1])
+    p.close()
+
+
+@pytest.mark.parametrize("depth,n_features,n_trees,sizes", [
+    (8, 28, 37, (2_500, 5_003, 17_000, 300_000)),   # walked, then tiles of 64, 256 and 1,024 rows
+    (12, 28, 5, (5_003, 16_385, 90_000)),           # a tile a tree: walked until the rows pay for it
+    (13, 28, 4, (1_000, 16_383, 70_000)),           # trees past a tile
+    (3, 100, 1, (33, 8_192, 100_001)),              # fewer values a row than a tile of trees
+    (4, 257, 70, (2_049, 16_383, 16_384)),          # 8 rows a workgroup at most
+    (3, 257, 500, (2_559, 2_560, 16_383, 16_385)),  # 16 rows and 256 trees, then a row per lane
+    (3, 9_000, 3, (1, 9, 16_385))])                 # rows that leave LDS for few of them
+def test_predict_shapes_match_the_walk(hip, orc, depth, n_features, n_trees, sizes):
+    """Both sides of every line between the launch shapes, bit-equal to the oracle."""
+    rng = np.random.default_rng([depth, n_features, n_trees])
+    nb = rng.integers(2, 257, n_features).astype(np.uint16)
+    trees = random_trees(rng, n_trees, depth, n_features, nb, 0.05)
+    p = hip.Predictor(trees, nb, 0.1, -0.5)
+    for n in sizes:
+        rows = (rng.random((n, n_features), np.float32) * nb).astype(np.uint8)
+        assert np.array_equal(p.predict(rows).view(np.uint32), orc.predict(trees, rows, nb, 0.1, -0.5).view(np.uint32)), n
     p.close()
