@@ -1139,21 +1139,21 @@ void pack_paths(bh_node const *t, u16 const *last, u32 id, std::vector<ActiveEle
     else act[idx] = saved;
 }
 
-// Levels of splits below every node of a tree, and the most distinct features on a path.
-u32 tree_levels(bh_node const *t, u32 id, std::vector<u32> &levels, std::vector<u32> &feats, size_t &max_len)
+// Levels of splits below every node of a tree, and the most distinct features on a path
+// (seen: per feature, its splits on the way; distinct: the features among them).
+u32 tree_levels(bh_node const *t, u32 id, std::vector<u32> &levels, std::vector<u32> &seen, size_t distinct,
+                size_t &max_len)
 {
-    if (levels.size() <= id) levels.resize(id + 1, 0u);
     bh_node const &nd = t[id];
     if (nd.feature < 0) {
-        max_len = std::max(max_len, feats.size());
+        max_len = std::max(max_len, distinct);
         return 0;
     }
-    u32 const f = static_cast<u32>(nd.feature);
-    bool const fresh = std::find(feats.begin(), feats.end(), f) == feats.end();
-    if (fresh) feats.push_back(f);
-    u32 const l = tree_levels(t, nd.left, levels, feats, max_len);
-    u32 const r = tree_levels(t, nd.right, levels, feats, max_len);
-    if (fresh) feats.pop_back();
+    u32 &on_path = seen[static_cast<u32>(nd.feature)];
+    distinct += on_path++ == 0 ? 1u : 0u;
+    u32 const l = tree_levels(t, nd.left, levels, seen, distinct, max_len);
+    u32 const r = tree_levels(t, nd.right, levels, seen, distinct, max_len);
+    --on_path;
     return levels[id] = 1u + std::max(l, r);
 }
 
@@ -1172,6 +1172,7 @@ struct TreePacker {
     double scale;
     GaussRule rule;
     std::vector<TSlot> out;
+    std::vector<std::pair<u32, u32>> spans; // of every node walked: its subtree's slots in out
     struct Edge { // on the way down: feature, level and merged cover fraction of its latest edge
         u32 feature, level;
         double z;
@@ -1183,6 +1184,7 @@ struct TreePacker {
         u32 split = 0, level = 0; // level: of the same-feature edge above
         bool dup = false, leaf = false;
         double z = 1.0;           // and its merged fraction
+        float k[kTreeShapMaxM], l[kTreeShapMaxM]; // then its k_q (1 - k_q past the half) and l_q
         double zl = 0.5, zr = 0.5, value = 0.0;
     };
     Node node(u32 id) const
@@ -1208,6 +1210,11 @@ struct TreePacker {
                 r.dup = true;
                 r.level = above[k].level;
                 r.z = above[k].z;
+                for (u32 q = 0; q < rule.m; ++q) {
+                    double const x = rule.x[q], a = r.z + x * (1.0 - r.z);
+                    r.k[q] = static_cast<float>(past_half(q, rule.m) ? r.z * (1.0 - x) / a : x / a);
+                    r.l[q] = static_cast<float>(r.z / (a * a));
+                }
                 break;
             }
         return r;
@@ -1215,12 +1222,9 @@ struct TreePacker {
     static void put(TSlot *s, u32 word, float v) { std::memcpy(&s[word / 8u].w[word % 8u], &v, sizeof(v)); }
     static void put(TSlot *s, u32 word, double v) { put(s, word, static_cast<float>(v)); }
 
-    // Room for a step and the constants of its n nodes; returns its first slot.
-    size_t open(u32 kind, Node const *nodes, u32 n)
+    // Room for a step of `need` slots inside a group; returns its first slot.
+    size_t room(u32 need)
     {
-        u32 const ds = tree_dup_slots(rule.m);
-        u32 need = tree_step_slots(kind);
-        for (u32 i = 0; i < n; ++i) need += nodes[i].dup ? ds : 0u;
         while ((out.size() & 63u) + need > 64u) {
             TSlot skip{};
             skip.w[kTwOp] = kTSkip << 2;
@@ -1228,15 +1232,22 @@ struct TreePacker {
         }
         size_t const at = out.size();
         out.resize(at + need);
+        return at;
+    }
+
+    // Room for a step and the constants of its n nodes; returns its first slot.
+    size_t open(u32 kind, Node const *nodes, u32 n)
+    {
+        u32 const ds = tree_dup_slots(rule.m);
+        u32 need = tree_step_slots(kind);
+        for (u32 i = 0; i < n; ++i) need += nodes[i].dup ? ds : 0u;
+        size_t const at = room(need);
         size_t o = at + tree_step_slots(kind);
         for (u32 i = 0; i < n; ++i) {
             if (!nodes[i].dup) continue;
-            double const z = nodes[i].z;
-            for (u32 q = 0; q < rule.m; ++q) {
-                double const x = rule.x[q], a = z + x * (1.0 - z);
-                put(&out[o], q, past_half(q, rule.m) ? z * (1.0 - x) / a : x / a);
-                put(&out[o], rule.m + q, z / (a * a));
-            }
+            auto *const to = reinterpret_cast<unsigned char *>(out.data() + o);
+            std::memcpy(to, nodes[i].k, rule.m * sizeof(float));
+            std::memcpy(to + rule.m * sizeof(float), nodes[i].l, rule.m * sizeof(float));
             o += ds;
         }
         return at;
@@ -1301,6 +1312,12 @@ struct TreePacker {
 
     void walk(u32 id, u32 level)
     {
+        u32 const begin = static_cast<u32>(out.size());
+        walk_steps(id, level);
+        spans[id] = {begin, static_cast<u32>(out.size())};
+    }
+    void walk_steps(u32 id, u32 level)
+    {
         if (levels[id] <= kTBlockLevels) {
             block(id, level);
             return;
@@ -1322,8 +1339,24 @@ struct TreePacker {
         step(kTCombine, level, nd, flags, vl, vr);
     }
 
+    // Appends a walked subtree's steps again, in a third of the time packing them takes.
+    void copy_steps(u32 id)
+    {
+        for (u32 at = spans[id].first; at < spans[id].second;) {
+            u32 const op = out[at].w[kTwOp];
+            if ((op >> 2 & 15u) == kTSkip) {
+                ++at;
+                continue;
+            }
+            u32 const need = tree_step_slots(op & 3u) + static_cast<u32>(__builtin_popcount(op >> 8 & 0x7Fu)) * tree_dup_slots(rule.m);
+            size_t const to = room(need);
+            std::copy_n(out.begin() + at, need, out.begin() + static_cast<std::ptrdiff_t>(to));
+            at += need;
+        }
+    }
+
     // The split form (k_shap_split): every subtree at depth `cut`, or shallower of at most a
-    // block's levels, is a share: the steps down to it, then its own walk.
+    // block's levels, is a share: the steps down to it, then its own walk's.
     std::vector<u32> first;          // first slot of every share
     std::vector<std::pair<u32, u32>> way; // (node, side) from the root
     static u32 cut_of(u32 deepest) { return std::min(deepest - kTBlockLevels, std::max(4u, deepest / 2u)); }
@@ -1331,7 +1364,7 @@ struct TreePacker {
     void go_down(u32 id, u32 level)
     {
         if (level == way.size()) {
-            walk(id, level);
+            copy_steps(id);
             return;
         }
         u32 const side = way[level].second;
@@ -1519,6 +1552,7 @@ struct bh_predictor {
     SElem *d_elems = nullptr;
     SHead *d_heads = nullptr;
     float *d_w = nullptr;
+    unsigned char *d_all = nullptr; // the allocation all of them lie in (Upload)
     hipStream_t stream = nullptr;
     // Buffers of small host calls (SmallCall): one call at a time.
     std::mutex ws_busy;
@@ -1630,6 +1664,11 @@ constexpr u32 kTreeShapFill = 768;
 u64 split_walks(u32 depth) { return depth >= 8 ? 512 : 256; }
 // The node count a kernel is built for (the switch of launch_shap_tree).
 u32 m_of(u32 m, u32 upper) { return upper <= 5 ? std::max(2u, std::min(m, 4u)) : std::max(4u, std::min(m, 6u)); }
+// LDS of a k_shap_split workgroup whose trees have up to `shares` shares.
+size_t split_lds(u32 F, u32 shares, u32 m, u32 upper)
+{
+    return tree_shap_lds(F) + static_cast<size_t>(shares) * m_of(m, upper) * 64u * sizeof(float);
+}
 
 int launch_shap_tree(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, double *d_out, hipStream_t s)
 {
@@ -1657,8 +1696,7 @@ int launch_shap_tree(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, doubl
         SHIP(hipGetLastError());
     }
     size_t const lds = tree_shap_lds(p->F);
-    size_t const split_lds = lds + static_cast<size_t>(p->max_shares) * m_of(p->tree_m, upper) * 64u * sizeof(float);
-    if (p->max_shares && static_cast<u64>(blocks) * p->n_ttrees <= split_walks(p->tree_depth) && split_lds <= 160u * 1024u) {
+    if (p->max_shares && static_cast<u64>(blocks) * p->n_ttrees <= split_walks(p->tree_depth)) {
         if (split <= 1) {
             hipLaunchKernelGGL(k_shap_zero, dim3(cgrid), dim3(256), 0, s,
                                reinterpret_cast<unsigned long long *>(d_out), cells);
@@ -1667,7 +1705,7 @@ int launch_shap_tree(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, doubl
         dim3 const sgrid(blocks, p->n_ttrees);
 #define BH_SP(MV)                                                                                                  \
     hipLaunchKernelGGL((p->tree_wide ? k_shap_split<MV, true> : k_shap_split<MV, false>), sgrid,                   \
-                       dim3(kSplitThreads), split_lds, s, d_bins, n, stride, p->F, p->d_last,                      \
+                       dim3(kSplitThreads), split_lds(p->F, p->max_shares, p->tree_m, upper), s, d_bins, n, stride, p->F, p->d_last,                      \
                        p->d_tslots, p->d_sfirst, p->d_split, p->n_ttrees, p->quad, d_out)
         switch (m_of(p->tree_m, upper)) {
         case 2: BH_SP(2); break;
@@ -1772,6 +1810,40 @@ private:
     bool ready_ = false;
 };
 
+// A predictor's device data: one allocation, and one copy while it is small (13 of each took
+// 60 us of the 200 a small predictor takes to create).
+class Upload {
+public:
+    template <typename T> void add(T *&dev, T const *src, size_t count)
+    {
+        parts_.push_back({reinterpret_cast<void **>(&dev), src, count * sizeof(T), bytes_});
+        bytes_ += (std::max<size_t>(count * sizeof(T), 16) + 255u) & ~static_cast<size_t>(255);
+    }
+    hipError_t run(unsigned char *&base)
+    {
+        hipError_t e = hipMalloc(&base, bytes_);
+        bool const small = bytes_ <= (1u << 20);
+        std::vector<unsigned char> host(small ? bytes_ : 0u);
+        for (Part const &q : parts_) {
+            if (e != hipSuccess) return e;
+            *q.dev = base + q.at;
+            if (q.bytes == 0) continue;
+            if (small) std::memcpy(host.data() + q.at, q.src, q.bytes);
+            else e = hipMemcpy(base + q.at, q.src, q.bytes, hipMemcpyHostToDevice);
+        }
+        return e == hipSuccess && small ? hipMemcpy(base, host.data(), bytes_, hipMemcpyHostToDevice) : e;
+    }
+
+private:
+    struct Part {
+        void **dev;
+        void const *src;
+        size_t bytes, at;
+    };
+    std::vector<Part> parts_;
+    size_t bytes_ = 0;
+};
+
 // Whole words (both ends lie in buffers of kWsBytes).
 __global__ void k_copy_words(u32 const *__restrict__ src, u32 *__restrict__ dst, u32 n)
 {
@@ -1808,7 +1880,7 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     size_t max_len = 0;
     double ev_sum = 0.0;
     std::vector<std::vector<u32>> levels(n_trees);
-    std::vector<u32> feats;
+    std::vector<u32> seen(n_features, 0u);
     u32 deepest = 0;
     LeafStats leaves;
     leaves.top.assign(n_trees, 0.0);
@@ -1859,7 +1931,7 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
             pn.push_back(q);
         }
         levels[t].assign(count, 0u);
-        deepest = std::max(deepest, tree_levels(tn, 0, levels[t], feats, max_len));
+        deepest = std::max(deepest, tree_levels(tn, 0, levels[t], seen, 0, max_len));
         ev_sum += expected_value(tn, 0);
     }
     if (max_len > static_cast<size_t>(kMaxPath)) {
@@ -1917,6 +1989,7 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     TreePacker pack{};
     std::vector<u32> tfirst;
     std::vector<SplitTree> split;
+    std::vector<std::vector<std::pair<u32, u32>>> spans;
     if (tree_form) {
         // kernels' node counts: 2, 3, 4 (up to 8 levels), 4, 5, 6 (more)
         u32 const m = std::max<u32>(deepest <= 8 ? 2u : 4u, (p->max_len + 1u) / 2u);
@@ -1926,32 +1999,43 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
         pack.F = n_features;
         pack.scale = scale;
         pack.rule = gauss_legendre(m);
-        pack.out.reserve(pn.size() * 3u + 256u); // both forms: about 1.5 slots a node each
+        u32 const cut = deepest > kTBlockLevels + 1u ? TreePacker::cut_of(deepest) : 0u;
+        u32 walked = 0, most = 0; // trees with splits; shares of one
         for (u32 t = 0; t < n_trees; ++t) {
             pack.t = nodes + tree_offsets[t];
             pack.levels = levels[t].data();
             if (pack.t[0].feature < 0) continue; // a single leaf has no contributions
+            ++walked;
+            if (cut) most = std::max(most, pack.count(0, 0, cut));
+        }
+        // The split form serves up to split_walks trees whose shares' values fit LDS.
+        u32 const upper = deepest > kTBlockLevels ? deepest - kTBlockLevels : 0u;
+        if (walked <= split_walks(deepest) && split_lds(n_features, most, m, upper) <= 160u * 1024u) p->max_shares = most;
+        pack.out.reserve(pn.size() * (p->max_shares ? 3u : 2u) + 256u); // about 1.5 slots a node each
+        for (u32 t = 0; t < n_trees; ++t) {
+            pack.t = nodes + tree_offsets[t];
+            pack.levels = levels[t].data();
+            if (pack.t[0].feature < 0) continue;
+            pack.spans.assign(levels[t].size(), {0u, 0u});
             tfirst.push_back(static_cast<u32>(pack.out.size()));
             pack.walk(0, 0);
+            if (p->max_shares) spans.push_back(std::move(pack.spans));
         }
         tfirst.push_back(static_cast<u32>(pack.out.size()));
-        if (deepest > kTBlockLevels + 1u) {
-            u32 const cut = TreePacker::cut_of(deepest);
-            for (u32 t = 0; t < n_trees; ++t) {
-                pack.t = nodes + tree_offsets[t];
-                pack.levels = levels[t].data();
-                if (pack.t[0].feature < 0) continue;
-                SplitTree st{static_cast<u32>(pack.first.size()), 0u, kNone, 0u};
-                pack.shares(0, 0, cut);
-                st.n_shares = static_cast<u32>(pack.first.size()) - st.share0;
-                if (!pack.is_share(0, 0, cut)) {
-                    u32 share = 0;
-                    st.top = static_cast<u32>(pack.out.size());
-                    pack.top(0, 0, cut, share);
-                }
-                p->max_shares = std::max(p->max_shares, st.n_shares);
-                split.push_back(st);
+        for (u32 t = 0, k = 0; p->max_shares && t < n_trees; ++t) {
+            pack.t = nodes + tree_offsets[t];
+            pack.levels = levels[t].data();
+            if (pack.t[0].feature < 0) continue;
+            pack.spans = std::move(spans[k++]);
+            SplitTree st{static_cast<u32>(pack.first.size()), 0u, kNone, 0u};
+            pack.shares(0, 0, cut);
+            st.n_shares = static_cast<u32>(pack.first.size()) - st.share0;
+            if (!pack.is_share(0, 0, cut)) {
+                u32 share = 0;
+                st.top = static_cast<u32>(pack.out.size());
+                pack.top(0, 0, cut, share);
             }
+            split.push_back(st);
         }
         pack.out.resize((pack.out.size() / 64u + 3u) * 64u); // the kernel reads whole groups, two ahead
         double g = 1.0;
@@ -1966,42 +2050,21 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     std::vector<TileTree> ttrees;
     if (pack_tiles(nodes, tree_offsets, n_trees, n_features, words, tiles, ttrees))
         p->n_tiles = static_cast<u32>(tiles.size());
-    hipError_t e = hipSuccess;
-    auto al = [&](void **ptr, size_t bytes) {
-        if (e == hipSuccess) e = hipMalloc(ptr, std::max<size_t>(bytes, 16));
-    };
-    al(reinterpret_cast<void **>(&p->d_nodes), pn.size() * sizeof(PNode));
-    al(reinterpret_cast<void **>(&p->d_roots), roots.size() * sizeof(u32));
-    al(reinterpret_cast<void **>(&p->d_last), n_features * sizeof(u16));
-    al(reinterpret_cast<void **>(&p->d_elems), el.size() * sizeof(SElem));
-    al(reinterpret_cast<void **>(&p->d_heads), hd.size() * sizeof(SHead));
-    al(reinterpret_cast<void **>(&p->d_w), w.size() * sizeof(float));
-    if (e == hipSuccess && !pn.empty()) e = hipMemcpy(p->d_nodes, pn.data(), pn.size() * sizeof(PNode), hipMemcpyHostToDevice);
-    if (e == hipSuccess && n_trees) e = hipMemcpy(p->d_roots, roots.data(), roots.size() * sizeof(u32), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(p->d_last, last_bin, n_features * sizeof(u16), hipMemcpyHostToDevice);
-    if (e == hipSuccess && !el.empty()) e = hipMemcpy(p->d_elems, el.data(), el.size() * sizeof(SElem), hipMemcpyHostToDevice);
-    if (e == hipSuccess && !hd.empty()) e = hipMemcpy(p->d_heads, hd.data(), hd.size() * sizeof(SHead), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(p->d_w, w.data(), w.size() * sizeof(float), hipMemcpyHostToDevice);
-    if (p->n_tiles) {
-        al(reinterpret_cast<void **>(&p->d_words), words.size() * sizeof(u32));
-        al(reinterpret_cast<void **>(&p->d_tiles), tiles.size() * sizeof(Tile));
-        al(reinterpret_cast<void **>(&p->d_ttrees), ttrees.size() * sizeof(TileTree));
-        if (e == hipSuccess) e = hipMemcpy(p->d_words, words.data(), words.size() * sizeof(u32), hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(p->d_tiles, tiles.data(), tiles.size() * sizeof(Tile), hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(p->d_ttrees, ttrees.data(), ttrees.size() * sizeof(TileTree), hipMemcpyHostToDevice);
-    }
-    if (p->tree_m) {
-        al(reinterpret_cast<void **>(&p->d_tslots), pack.out.size() * sizeof(TSlot));
-        al(reinterpret_cast<void **>(&p->d_tfirst), tfirst.size() * sizeof(u32));
-        if (e == hipSuccess) e = hipMemcpy(p->d_tslots, pack.out.data(), pack.out.size() * sizeof(TSlot), hipMemcpyHostToDevice);
-        if (!split.empty()) {
-            al(reinterpret_cast<void **>(&p->d_sfirst), pack.first.size() * sizeof(u32));
-            al(reinterpret_cast<void **>(&p->d_split), split.size() * sizeof(SplitTree));
-            if (e == hipSuccess) e = hipMemcpy(p->d_sfirst, pack.first.data(), pack.first.size() * sizeof(u32), hipMemcpyHostToDevice);
-            if (e == hipSuccess) e = hipMemcpy(p->d_split, split.data(), split.size() * sizeof(SplitTree), hipMemcpyHostToDevice);
-        }
-        if (e == hipSuccess && !tfirst.empty()) e = hipMemcpy(p->d_tfirst, tfirst.data(), tfirst.size() * sizeof(u32), hipMemcpyHostToDevice);
-    }
+    Upload up;
+    up.add(p->d_nodes, pn.data(), pn.size());
+    up.add(p->d_roots, roots.data(), roots.size());
+    up.add(p->d_last, last_bin, n_features);
+    up.add(p->d_elems, el.data(), el.size());
+    up.add(p->d_heads, hd.data(), hd.size());
+    up.add(p->d_w, w.data(), w.size());
+    up.add(p->d_words, words.data(), words.size());
+    up.add(p->d_tiles, tiles.data(), tiles.size());
+    up.add(p->d_ttrees, ttrees.data(), ttrees.size());
+    up.add(p->d_tslots, pack.out.data(), pack.out.size());
+    up.add(p->d_tfirst, tfirst.data(), tfirst.size());
+    up.add(p->d_sfirst, pack.first.data(), pack.first.size());
+    up.add(p->d_split, split.data(), split.size());
+    hipError_t e = up.run(p->d_all);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
         bh_predictor_destroy(p);
@@ -2015,10 +2078,7 @@ int bh_predictor_destroy(bh_predictor *p)
 {
     if (!p) return 0;
     (void)hipSetDevice(p->device);
-    void *ptrs[] = {p->d_nodes, p->d_roots, p->d_last,   p->d_elems, p->d_heads, p->d_w,
-                    p->d_words, p->d_tiles, p->d_ttrees, p->d_tslots, p->d_tfirst, p->d_sfirst, p->d_split};
-    for (void *q : ptrs)
-        if (q) (void)hipFree(q);
+    if (p->d_all) (void)hipFree(p->d_all);
     if (p->ws_dev) (void)hipFree(p->ws_dev);
     if (p->ws_host) (void)hipHostFree(p->ws_host);
     if (p->stream) (void)hipStreamDestroy(p->stream);
