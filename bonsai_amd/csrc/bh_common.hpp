@@ -67,7 +67,8 @@ constexpr u32 kLwAhead = 32;      // leaves expanded before their pop at most (e
 constexpr u32 kLwMoreRounds = 4;  // rounds added at a time to a tree the first ones left unfinished
 constexpr u32 kLwPoolCap = 1024 + 8;                       // max_leaves and its last round's children
 constexpr u32 kLwListCap = kLwPoolCap + kLwAhead + 2 * kLwBatch;
-constexpr u32 kLwRecCap = 1 + 2 * (kLwPoolCap + kLwAhead + kLwBatch); // two a leaf expanded
+constexpr u32 lw_records(u32 max_leaves) { return 1 + 2 * (max_leaves + 8 + kLwAhead + kLwBatch); } // two a leaf expanded
+constexpr u32 kLwRecCap = lw_records(1024);
 // Tail padding of planes (bytes) and gradient buffers (elements): kernels that read
 // aligned 16-byte words around a row range may touch up to 15 bytes past its end.
 constexpr size_t kTailPadBytes = 64;
@@ -256,7 +257,8 @@ struct GrowCfg {
     u8 const *fmask;
     // Monotone constraints (tree.monotone_constraints, include/bonsai/config/tree_config.hpp:
     // 20-22): per-feature direction (+1, -1, 0), nullptr for none; then bounds holds the
-    // [lo, hi] leaf-weight box of every tree node id (2 doubles per node).
+    // [lo, hi] leaf-weight box of every tree node id (2 doubles per node; leafwise rounds:
+    // of every record, NodeInfo::id there).
     int8_t const *mono;
     double *bounds;
     // Interaction constraints (tree.interaction_constraints, tree_config.hpp:23-26):

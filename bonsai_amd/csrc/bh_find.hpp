@@ -45,12 +45,12 @@ __device__ __forceinline__ double fd_bounded_weight(double g, double h, double l
 // parent's box; a split on a monotone feature fences them at the midpoint of the two
 // child weights, each bounded by the parent's box.  The child sums are the ones the
 // finder scored (exact integers times the scales when quantized).
-__device__ __forceinline__ void fd_propagate_bounds(GrowCfg const &c, double const *__restrict__ scales, u32 pid,
-                                                    SplitRec const &s, u32 lid, u32 rid)
+__device__ __forceinline__ void fd_child_bounds(GrowCfg const &c, double const *__restrict__ scales, u32 pid,
+                                                SplitRec const &s, double &llo, double &lhi, double &rlo, double &rhi)
 {
-    if (!c.mono) return;
     double const plo = c.bounds[2 * pid], phi = c.bounds[2 * pid + 1];
-    double llo = plo, lhi = phi, rlo = plo, rhi = phi;
+    llo = rlo = plo;
+    lhi = rhi = phi;
     int const mc = c.mono[s.feature];
     if (mc != 0) {
         double gL = s.gL, hL = s.hL, gR = s.gR, hR = s.hR;
@@ -71,6 +71,13 @@ __device__ __forceinline__ void fd_propagate_bounds(GrowCfg const &c, double con
             rhi = mid < rhi ? mid : rhi;
         }
     }
+}
+__device__ __forceinline__ void fd_propagate_bounds(GrowCfg const &c, double const *__restrict__ scales, u32 pid,
+                                                    SplitRec const &s, u32 lid, u32 rid)
+{
+    if (!c.mono) return;
+    double llo, lhi, rlo, rhi;
+    fd_child_bounds(c, scales, pid, s, llo, lhi, rlo, rhi);
     c.bounds[2 * lid] = llo;
     c.bounds[2 * lid + 1] = lhi;
     c.bounds[2 * rid] = rlo;

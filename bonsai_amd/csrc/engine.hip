@@ -214,11 +214,11 @@ struct bh_context {
     // monotone constraints (bh_set_monotone): directions by sign, per-node boxes
     std::vector<int8_t> mono_host;
     int8_t *mono_dev = nullptr;  // [F]
-    double *bounds = nullptr;    // [max_nodes][2]
+    double *bounds = nullptr;    // [constraint_slots][2]
     // interaction constraints (bh_set_interaction): groups as feature bitmasks, node paths
     std::vector<std::vector<u32>> groups_host;
     u32 *groups_dev = nullptr;   // [n_groups][path_words]
-    u32 *paths = nullptr;        // [max_nodes][path_words]
+    u32 *paths = nullptr;        // [constraint_slots][path_words]
     // configuration
     bh_fit_config fc{};
     GrowCfg gc{};
@@ -370,6 +370,13 @@ u32 tree_capacity(bh_fit_config const &f)
     return std::min<u32>(kMaxTreeNodes, (2u << static_cast<u32>(f.max_depth)) + 2u);
 }
 
+// Ids that own a box or a path: tree nodes, and the records of leafwise rounds.
+u32 constraint_slots(bh_context const *c)
+{
+    u32 const records = c->fc.grower == BH_LEAFWISE ? lw_records(static_cast<u32>(c->fc.max_leaves)) : 0u;
+    return std::max(c->max_nodes, records);
+}
+
 // Device copies of the monotone directions and the per-node boxes for the configured
 // fit; none when every direction is 0.  The levelwise grower refuses constraints
 // (src/grower_impl.hpp:583-588).
@@ -388,7 +395,7 @@ int arm_monotone(bh_context *c)
     std::vector<int8_t> d(c->F, 0);
     for (size_t f = 0; f < c->mono_host.size() && f < c->F; ++f) d[f] = c->mono_host[f];
     HIP_TRY(dalloc(&c->mono_dev, c->F));
-    HIP_TRY(dalloc(&c->bounds, 2 * static_cast<size_t>(c->max_nodes)));
+    HIP_TRY(dalloc(&c->bounds, 2 * static_cast<size_t>(constraint_slots(c))));
     HIP_TRY(hipMemcpy(c->mono_dev, d.data(), c->F, hipMemcpyHostToDevice));
     c->gc.mono = c->mono_dev;
     c->gc.bounds = c->bounds;
@@ -417,7 +424,7 @@ int arm_interaction(bh_context *c)
             bits[g * W + f / 32u] |= 1u << (f % 32u);
         }
     HIP_TRY(dalloc(&c->groups_dev, bits.size()));
-    HIP_TRY(dalloc(&c->paths, static_cast<size_t>(c->max_nodes) * W));
+    HIP_TRY(dalloc(&c->paths, static_cast<size_t>(constraint_slots(c)) * W));
     HIP_TRY(hipMemcpy(c->groups_dev, bits.data(), bits.size() * sizeof(u32), hipMemcpyHostToDevice));
     c->gc.groups = c->groups_dev;
     c->gc.paths = c->paths;

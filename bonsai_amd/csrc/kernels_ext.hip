@@ -602,8 +602,9 @@ __global__ __launch_bounds__(1024) void k_oblivious_tree(NodeInfo const *__restr
 // the logistic table (of 32 possible), 31 take 7; 16M x 28, 255
 // leaves, 3 trees: 44.5 -> 22.2 ms; 1M x 28 FP32, 31 leaves, 10 trees: 23.9 -> 13.1 ms.
 //
-// Constrained fits (monotone or interaction) keep one leaf a round: their split finder
-// reads per-node bounds and paths, which exist under the final node ids only.
+// NodeInfo::id is the leaf's record here: a child may be searched before its node id is
+// known, and monotone boxes and interaction paths are kept by it (1M x 28, 255 leaves,
+// monotone: 10.4 ms a quantized tree by one leaf a round, 12.4 by one of these a round).
 // ---------------------------------------------------------------------------------
 // Rows per partition chunk of a leaf of `rows` rows: about kLwChunkTarget chunks,
 // multiples of 256 rows, kLwMinChunk..kPartChunk, and at most cap (the chunk of wide
@@ -821,7 +822,6 @@ __device__ __forceinline__ void lw_select_round(TreeCtl *__restrict__ ctl, LwCtl
     __shared__ u32 s_nl, s_np, s_free, s_act, s_pops, s_n, s_sel[kLwBatch], s_fresh[kLwBatch];
     __shared__ u32 s_chunk[kLwBatch + 1], s_crow[kLwBatch], s_deep;
     if (ctl->done) return; // every work list is empty
-    bool const one = cfg.mono || cfg.n_groups; // final ids while expanding
     u32 const nb = lw->n_batch, r0 = lw->n_rec, np0 = lw->n_pool, nl0 = lw->n_list;
     if (threadIdx.x == 0) {
         s_nl = nl0;
@@ -925,12 +925,9 @@ __device__ __forceinline__ void lw_select_round(TreeCtl *__restrict__ ctl, LwCtl
         if (act == 1) {
             // The leaf the pops wait for, then the best others, while their partials fit
             // and children are expected to be asked for.
-            u32 kmax = 1, parts = 0;
-            if (!one) {
-                u32 const left = max_leaves - live;
-                kmax = min(kLwBatch, max(1u, COUNTED ? left - 1u : left));
-                kmax = max(1u, min(kmax, kLwAhead - min(kLwAhead, ahead)));
-            }
+            u32 const left = max_leaves - live;
+            u32 kmax = min(kLwBatch, max(1u, COUNTED ? left - 1u : left)), parts = 0;
+            kmax = max(1u, min(kmax, kLwAhead - min(kLwAhead, ahead)));
             while (n < kmax && nl > 0) {
                 u32 ix = kNone;
                 if (n == 0) {
@@ -977,26 +974,26 @@ __device__ __forceinline__ void lw_select_round(TreeCtl *__restrict__ ctl, LwCtl
     // since a child may have been popped as well.
     u32 const n_pops = s_pops;
     for (u32 k = threadIdx.x; k < n_pops; k += blockDim.x) {
-        u32 const id = s_pop_id[k], lid = n_nodes + 2u * k, rid = lid + 1u, r = s_pop_rec[k];
+        u32 const lid = n_nodes + 2u * k, rid = lid + 1u, r = s_pop_rec[k];
         LwRec const &c = ls.recs[r];
         DevNode l{}, rr{};
         l.feature = rr.feature = -1;
         if ((s_meta[r] & 3u) != kLwDemoted) {
             atomicMax(&s_deep, c.node.depth + 1u);
-            if (s_link[r] == kNone) { // never expanded: leaves from the split's sums
-                if (one) {
-                    fd_propagate_bounds(cfg, scales, id, c.split, lid, rid);
-                    fd_propagate_path(cfg, id, c.split.feature, lid, rid);
+            if (COUNTED && s_link[r] == kNone) { // never expanded: leaves from the split's sums
+                double const gl = static_cast<double>(c.split.igL) * scales[0],
+                             hl = static_cast<double>(c.split.ihL) * scales[1],
+                             gr = static_cast<double>(c.split.igR) * scales[0],
+                             hr = static_cast<double>(c.split.ihR) * scales[1];
+                if (cfg.mono) {
+                    double llo, lhi, rlo, rhi;
+                    fd_child_bounds(cfg, scales, r, c.split, llo, lhi, rlo, rhi);
+                    l.value = static_cast<float>(fd_bounded_weight(gl, hl, cfg.l1, cfg.l2, llo, lhi));
+                    rr.value = static_cast<float>(fd_bounded_weight(gr, hr, cfg.l1, cfg.l2, rlo, rhi));
+                } else {
+                    l.value = leaf_weight(gl, hl, cfg.l1, cfg.l2);
+                    rr.value = leaf_weight(gr, hr, cfg.l1, cfg.l2);
                 }
-                NodeInfo x{}, y{};
-                x.id = lid;
-                x.itg = c.split.igL;
-                x.ith = c.split.ihL;
-                y.id = rid;
-                y.itg = c.split.igR;
-                y.ith = c.split.ihR;
-                l.value = node_value(x, cfg, scales);
-                rr.value = node_value(y, cfg, scales);
                 l.cover = static_cast<float>(c.split.n_left);
                 rr.cover = static_cast<float>(c.node.cnt - c.split.n_left);
             } else {
@@ -1061,7 +1058,7 @@ __device__ __forceinline__ void lw_select_round(TreeCtl *__restrict__ ctl, LwCtl
         x.dst = nd.src == 0 ? 1u : 0u;
         x.slot = nd.slot;
         x.depth = nd.depth;
-        x.left_id = one ? n_nodes + 2u * n_pops : 0u;
+        x.left_id = r0 + 2u * nb + 2u * j; // its children's records (NodeInfo::id here)
         if (COUNTED) {
             lw_measure(x, s.n_left, cfg, ls.unit_target);
             s_fresh[j] = ls.free_slots[s_free - 1u - j];
@@ -1069,10 +1066,8 @@ __device__ __forceinline__ void lw_select_round(TreeCtl *__restrict__ ctl, LwCtl
         s_x[j] = x;
         s_crow[j] = lw_chunk_rows(nd.cnt, ls.chunk_cap);
         s_chunk[j] = (nd.cnt + s_crow[j] - 1u) / s_crow[j];
-        if (one) { // only the leaf the pops wait for: its children's ids are the next two
-            fd_propagate_bounds(cfg, scales, nd.id, s, x.left_id, x.left_id + 1u);
-            fd_propagate_path(cfg, nd.id, s.feature, x.left_id, x.left_id + 1u);
-        }
+        fd_propagate_bounds(cfg, scales, r, s, x.left_id, x.left_id + 1u);
+        fd_propagate_path(cfg, r, s.feature, x.left_id, x.left_id + 1u);
         PartOp op{};
         op.parent = r;
         op.feature = s.feature;
@@ -1482,7 +1477,7 @@ template <bool Q, bool COUNTED>
 static void launch_lw_find(hipStream_t st, GrowView const &v, LwCtl *lw, u32 *cnt, LwNext const &nx)
 {
     size_t const lds = static_cast<size_t>(kLwFindTile) * v.SB * (Q ? (cnt ? 36 : 32) : 24);
-    dim3 const grid(find_blocks_per_node(v.F, kLwFindTile), 2u * lw_batch(v));
+    dim3 const grid(find_blocks_per_node(v.F, kLwFindTile), 2u * kLwBatch);
     bool const con = v.gc.fmask || v.gc.mono || v.gc.n_groups;
     auto const fn = con ? &k_lw_find<Q, COUNTED, true> : &k_lw_find<Q, COUNTED, false>;
     hipLaunchKernelGGL(fn, grid, dim3(kFindThreads), lds, st, v.front[0], v.ctl, lw, v.hist[0], v.d_nbins, v.F, v.SB,
@@ -1498,20 +1493,17 @@ static LwLists lw_lists(ExtState const &s, GrowView const &v)
     return ls;
 }
 
-// Leaves a round expands at most; constrained fits one (their node ids are final).
-u32 lw_batch(GrowView const &v) { return v.gc.mono || v.gc.n_groups ? 1u : kLwBatch; }
-
 u32 lw_head_rounds(GrowView const &v)
 {
-    u32 const L = static_cast<u32>(v.fc.max_leaves), K = lw_batch(v);
-    return K == 1u ? L + 7u : std::min(L + 7u, (L - 1u + K - 1u) / K + 4u);
+    u32 const L = static_cast<u32>(v.fc.max_leaves);
+    return std::min(L + 7u, (L - 1u + kLwBatch - 1u) / kLwBatch + 4u);
 }
 
 // `rounds` rounds; the last one's find reports to the host whether the tree is complete.
 // A complete tree turns rounds into no-ops.
 void enqueue_leafwise_rounds(ExtState &s, hipStream_t st, bool q, GrowView const &v, u32 rounds)
 {
-    u32 const gh_bytes = q ? 4 : 8, K = lw_batch(v);
+    u32 const gh_bytes = q ? 4 : 8;
     LwCtl *lw = s.lw;
     NodeInfo *kids = v.front[0];
     void *pool = v.hist[0];
@@ -1529,7 +1521,7 @@ void enqueue_leafwise_rounds(ExtState &s, hipStream_t st, bool q, GrowView const
                             gh_bytes, pgrid, q ? v.chunk_left : nullptr);
         launch_hist(st, q, v.hch, v.ctl, v.work[0], v.work[1], v.plane0, v.gh[0], v.gh[1], v.gh[2], v.Fs, v.F, v.SB,
                     v.fsl, v.waves, hgrid, v.partials, pool, v.fx, cnt);
-        launch_finish(st, q, v.fops, v.ctl, v.partials, pool, pool, v.F * v.SB, K, cnt, cnt, false,
+        launch_finish(st, q, v.fops, v.ctl, v.partials, pool, pool, v.F * v.SB, kLwBatch, cnt, cnt, false,
                       hist_transpose_F(q, v.Fs, v.F));
         LwNext const nx{ls, v.tree, v.ops, v.pch, v.hch, v.fops, r + 1 == rounds ? s.report : nullptr};
         if (q) launch_lw_find<true, true>(st, v, lw, cnt, nx);

@@ -89,7 +89,6 @@ hipError_t ext_alloc(ExtState &s, bh_fit_config const &f, u32 F, u32 hist_slots)
 void ext_free(ExtState &s);
 hipError_t ext_set_limits();
 void enqueue_levelwise(ExtState &s, hipStream_t st, bool q, GrowView const &v);
-u32 lw_batch(GrowView const &v);
 u32 lw_head_rounds(GrowView const &v);
 void enqueue_leafwise_rounds(ExtState &s, hipStream_t st, bool q, GrowView const &v, u32 rounds);
 void enqueue_leafwise(ExtState &s, hipStream_t st, bool q, GrowView const &v);

@@ -119,3 +119,33 @@ def test_fit_config_fields_equal_the_setters(hip, orc, tall):
     assert a.tobytes() == b.tobytes()
     with pytest.raises(hip.ConfigError):
         ctx_for(hip, bins, nb, grower="hip_levelwise", quantized=True, max_depth=4, monotone_constraints=(1,))
+
+
+@pytest.mark.parametrize("quantized", [True, False])
+@pytest.mark.parametrize("leaves,depth", [(2, 12), (3, 2), (9, 12), (10, 4), (40, 6), (255, 12)])
+def test_leafwise_constraints_by_round(hip, orc, tall, leaves, depth, quantized):
+    """Boxes and paths of leaves expanded before their pop, of children that are never
+    expanded (the budget's last and those at max_depth) and of more leaves than one round
+    takes, both kinds of constraint at once, bit-exact."""
+    bins, nb, X, y = tall
+    g, h = grad_of(orc, y, seed=37)
+    dirs = np.zeros(28, np.int8)
+    dirs[[0, 2, 5, 24]] = [1, -1, 1, -1]
+    kw = dict(max_depth=depth, max_leaves=leaves)
+    ctx = ctx_for(hip, bins, nb, grower="hip_leafwise", quantized=quantized, **kw)
+    gq = hq = sc = None
+    if quantized:
+        gq, hq, sc = ctx.set_gradients(g, h)
+    else:
+        ctx.set_gradients(g, h)
+    ctx.set_interaction_constraints(GROUPS)
+    ctx.set_monotone(dirs)
+    nodes, lor = ctx.grow_tree()
+    ctx.close()
+    orc.set_monotone(dirs)
+    try:
+        ref, rlor = oracle_tree(orc, "hip_leafwise", bins, nb, g, h, gq, hq, sc, quantized, orc_cfg(**kw))
+    finally:
+        orc.set_monotone(None)
+    assert_same_tree(nodes, ref)
+    assert np.array_equal(lor, rlor)
