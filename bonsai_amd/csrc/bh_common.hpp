@@ -35,6 +35,7 @@ constexpr u32 kHistChunk  = 8192;
 // (cells x 8 bytes each) cost about as much as 1,000 rows.  100,000 rows x 28
 // features x 256 bins: full-scan levels 22.9 -> 9.3 us, routed ones 22.5 -> 11.4.
 constexpr u32 kHistUnitMin = 1024, kHistUnitFill = 128;
+constexpr u32 kFxWideUnits = 128; // 8,192-row units from which FP32 histograms of rows over 40 bytes take wider slices
 constexpr u32 kPackCntShift = 28;
 constexpr u32 kPackGShift = 42;
 constexpr u64 kPackHMask = (1ull << 28) - 1ull;

@@ -265,6 +265,14 @@ struct bh_context {
         }
         u32 f = round_up4(F);
         while (f > 4 && static_cast<size_t>(f) * SB * cell > (128u << 10)) f -= 4;
+        // FP32: 8 features, whose 32 KiB of cells let four workgroups share a CU where whole
+        // rows of 28 (114 KiB) left it one, and few units still fill the chip: 500,009 rows x
+        // 28 49 -> 17.9 us (4 features: no faster, slower on full levels), 10 rounds of
+        // 4,000,003 rows 16.75 -> 16.13 ms.  Rows over 40 bytes are read by many slices, so
+        // with units enough they take 16: 8M x 64, depth 7, 5.20 (8), 4.29 (16) and 4.49 ms
+        // (32) a round, x 52 4.15, 3.80 and 3.92, x 40 2.95 and 2.90; 300,000 x 64 0.66 (8)
+        // and 0.72.
+        if (!quant) f = std::min(f, Fs > 40 && N / kHistChunk >= kFxWideUnits ? 16u : 8u);
         return f;
     }
     u32 hist_waves() const

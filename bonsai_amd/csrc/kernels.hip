@@ -3331,8 +3331,6 @@ u32 hist_transpose_F(bool q, u32 Fs, u32 F, bool group)
     return q && !group && Fs <= 64u && (t_tune.hist_layout == 3u || t_tune.hist_layout == 5u) ? F : 0u;
 }
 
-constexpr u32 kFxSlice = 8; // features of a k_hist_fx workgroup at most
-
 hipError_t launch_hist(hipStream_t s, bool q, HistChunk const *chunks, TreeCtl const *ctl, u8 const *pl0,
                        u8 const *pl1, u8 const *plp, void const *g0, void const *g1, void const *gp, u32 Fs, u32 F,
                        u32 SB, u32 fsl, u32 n_waves, u32 grid_x, void *partials, void *hist_next, u32 const *fx,
@@ -3410,12 +3408,7 @@ hipError_t launch_hist(hipStream_t s, bool q, HistChunk const *chunks, TreeCtl c
                            Fs, F, SB, fsl, partials, hist_next, cnt_next, routes);
     } else {
         if (!fx) return hipErrorInvalidValue;
-        // Slices of 8 features: 32 KiB of cells let four workgroups share a CU where whole
-        // rows of 28 features (114 KiB) left it one, and few units still fill the chip.  The
-        // slices of a unit are adjacent workgroups, so its rows come from memory once.
-        // 500,009 rows x 28: 49 -> 17.9 us (4 features a slice: no faster, and slower on
-        // full levels); 10 rounds of 4,000,003 rows 16.75 -> 16.13 ms.
-        fsl = std::min(fsl, kFxSlice);
+        // The slices of a unit are adjacent workgroups, so its rows come from memory once.
         dim3 const fgrid((F + fsl - 1) / fsl, std::min(grid_x, 65535u));
         hipLaunchKernelGGL(k_hist_fx, fgrid, dim3(t_tune.hist_threads), static_cast<size_t>(fsl) * SB * 16u, s, chunks, ctl, pl0, pl1, plp, g0,
                            g1, gp, Fs, F, SB, fsl, partials, hist_next, fx);
