@@ -209,6 +209,30 @@ def test_wide_row_edges(hip, orc, f, n, depth, quantized):
 
 
 @pytest.mark.parametrize("quantized", [True, False])
+@pytest.mark.parametrize("f,top", [(65, 256), (66, 17), (100, 255), (257, 64), (513, 3)])
+def test_wide_histogram_of_row_lists(hip, orc, f, top, quantized):
+    """Row lists of one to several histogram units over more than 64 features: slices are
+    narrowed by the units there are, cells bit for bit."""
+    rng = np.random.default_rng(f)
+    n = 40_000
+    nb = rng.integers(1, top + 1, f).astype(np.uint16)
+    nb[f // 2] = top
+    bins = (rng.random((n, f)) * nb).astype(np.uint8)
+    g, h = orc.mse_grad(np.zeros(n, np.float32), rng.normal(0, 1, n).astype(np.float32))
+    ctx = ctx_for(hip, bins, nb, quantized=quantized, max_depth=3)
+    gq, hq, _ = ctx.set_gradients(g, h)
+    for m in (1, 100, 8_193, 40_000):
+        rows = np.sort(rng.permutation(n)[:m]).astype(np.uint32)
+        got = ctx.histogram(rows)
+        if quantized:
+            assert np.array_equal(got.ravel(), np.asarray(orc.hist_int(bins, rows, gq, hq, top)).ravel())
+        else:
+            want = orc.hist_f32(bins, rows, g, h, top, HIST_F32_FIXED, DEVICE_CHUNK)
+            assert np.array_equal(got.view(np.uint32).ravel(), want.view(np.uint32).ravel())
+    ctx.close()
+
+
+@pytest.mark.parametrize("quantized", [True, False])
 @pytest.mark.parametrize("f,n", [(65, 100), (70, 8192), (131, 20_001)])
 def test_wide_single_bin_histogram(hip, orc, f, n, quantized):
     """Planes of more than 64 features with one bin each: every feature's only cell holds
