@@ -1552,7 +1552,7 @@ struct bh_predictor {
     SElem *d_elems = nullptr;
     SHead *d_heads = nullptr;
     float *d_w = nullptr;
-    unsigned char *d_all = nullptr; // the allocation all of them lie in (Upload)
+    std::vector<void *> owned; // the allocations they lie in (Upload)
     hipStream_t stream = nullptr;
     // Buffers of small host calls (SmallCall): one call at a time.
     std::mutex ws_busy;
@@ -1810,38 +1810,49 @@ private:
     bool ready_ = false;
 };
 
-// A predictor's device data: one allocation, and one copy while it is small (13 of each took
-// 60 us of the 200 a small predictor takes to create).
+// A predictor's device data: the small arrays share one allocation and one copy (13 of each
+// took 60 us of the 200 a small predictor takes to create), large ones have their own (in
+// one allocation of 20 MB the first TreeSHAP pass took 12.0 ms where it takes 10.1 so).
 class Upload {
 public:
     template <typename T> void add(T *&dev, T const *src, size_t count)
     {
-        parts_.push_back({reinterpret_cast<void **>(&dev), src, count * sizeof(T), bytes_});
-        bytes_ += (std::max<size_t>(count * sizeof(T), 16) + 255u) & ~static_cast<size_t>(255);
+        parts_.push_back({reinterpret_cast<void **>(&dev), src, count * sizeof(T)});
     }
-    hipError_t run(unsigned char *&base)
+    // The allocations, also after an error, go to `owned`.
+    hipError_t run(std::vector<void *> &owned)
     {
-        hipError_t e = hipMalloc(&base, bytes_);
-        bool const small = bytes_ <= (1u << 20);
-        std::vector<unsigned char> host(small ? bytes_ : 0u);
-        for (Part const &q : parts_) {
-            if (e != hipSuccess) return e;
-            *q.dev = base + q.at;
-            if (q.bytes == 0) continue;
-            if (small) std::memcpy(host.data() + q.at, q.src, q.bytes);
-            else e = hipMemcpy(base + q.at, q.src, q.bytes, hipMemcpyHostToDevice);
+        std::vector<unsigned char> host;
+        auto const get = [&](void **ptr, size_t bytes) {
+            hipError_t const e = hipMalloc(ptr, bytes);
+            if (e == hipSuccess) owned.push_back(*ptr);
+            return e;
+        };
+        for (Part &q : parts_) {
+            if (q.bytes > kLarge) {
+                if (hipError_t const e = get(q.dev, q.bytes); e != hipSuccess) return e;
+                if (hipError_t const e = hipMemcpy(*q.dev, q.src, q.bytes, hipMemcpyHostToDevice); e != hipSuccess) return e;
+                continue;
+            }
+            q.at = host.size();
+            host.resize(host.size() + ((std::max<size_t>(q.bytes, 16) + 255u) & ~static_cast<size_t>(255)));
+            if (q.bytes) std::memcpy(host.data() + q.at, q.src, q.bytes);
         }
-        return e == hipSuccess && small ? hipMemcpy(base, host.data(), bytes_, hipMemcpyHostToDevice) : e;
+        void *base = nullptr;
+        if (hipError_t const e = get(&base, std::max<size_t>(host.size(), 16)); e != hipSuccess) return e;
+        for (Part const &q : parts_)
+            if (q.bytes <= kLarge) *q.dev = static_cast<unsigned char *>(base) + q.at;
+        return hipMemcpy(base, host.data(), host.size(), hipMemcpyHostToDevice);
     }
 
 private:
+    static constexpr size_t kLarge = 256u << 10;
     struct Part {
         void **dev;
         void const *src;
-        size_t bytes, at;
+        size_t bytes, at = 0;
     };
     std::vector<Part> parts_;
-    size_t bytes_ = 0;
 };
 
 // Whole words (both ends lie in buffers of kWsBytes).
@@ -2064,7 +2075,7 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     up.add(p->d_tfirst, tfirst.data(), tfirst.size());
     up.add(p->d_sfirst, pack.first.data(), pack.first.size());
     up.add(p->d_split, split.data(), split.size());
-    hipError_t e = up.run(p->d_all);
+    hipError_t e = up.run(p->owned);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
         bh_predictor_destroy(p);
@@ -2078,7 +2089,7 @@ int bh_predictor_destroy(bh_predictor *p)
 {
     if (!p) return 0;
     (void)hipSetDevice(p->device);
-    if (p->d_all) (void)hipFree(p->d_all);
+    for (void *q : p->owned) (void)hipFree(q);
     if (p->ws_dev) (void)hipFree(p->ws_dev);
     if (p->ws_host) (void)hipHostFree(p->ws_host);
     if (p->stream) (void)hipStreamDestroy(p->stream);
