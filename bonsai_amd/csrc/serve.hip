@@ -530,72 +530,30 @@ struct TQuad {
     float y[kTreeShapMaxM], w[kTreeShapMaxM];
 };
 
-// U: levels above the blocks.  WIDE: contributions of up to 63 bits (tree_grid).  AT: the
-// walk may start below a tree's root (levels come from the steps) and meet shares' values.
-template <int M, int U, bool WIDE, bool AT = false> struct TreeShap {
+// A row's arithmetic at a split, and at the seven of a block; D reads the running step's
+// words (word, dup_word), the row's bin and its sum of the column a split names (bin_at,
+// phi_at).  WIDE: contributions of up to 63 bits (tree_grid).
+template <class D, int M, bool WIDE> struct ShapRow {
     typedef float V[M];
-    u8 const *bins;      // LDS: this lane's column of the bins
-    unsigned char *phi;  // LDS: this lane's column of the sums
-    u32 plane;           // bytes of one plane of bins
-    TSlot const *ahead;  // this lane's slot of the group after the next
-    uint4 nx0, nx1;      // its slot of the next group, in flight
-    u32 cur[8];          // its slot of the current group
-    u32 at, op;          // the running step's slot in it and its first word (uniform)
+    u32 op;              // the running step's first word
     V y;                 // quadrature nodes (TQuad)
     u32 sat;             // bit l: the row satisfies the merged feature of the edge below level l
-    float *held;         // AT: LDS, this lane's column of the shares' values [share][M][64]
 
-    __device__ __forceinline__ void load()
-    {
-        uint4 const *p = reinterpret_cast<uint4 const *>(ahead);
-        nx0 = p[0];
-        nx1 = p[1];
-        ahead += 64;
-    }
-    __device__ __forceinline__ void shift()
-    {
-        cur[0] = nx0.x;
-        cur[1] = nx0.y;
-        cur[2] = nx0.z;
-        cur[3] = nx0.w;
-        cur[4] = nx1.x;
-        cur[5] = nx1.y;
-        cur[6] = nx1.z;
-        cur[7] = nx1.w;
-        load(); // whole groups of 64 slots are allocated, and two past the last
-    }
-    // The step at `at`: a skip or the group's end moves on to the next group.
-    __device__ __forceinline__ void fetch()
-    {
-        op = at < 64u ? __builtin_amdgcn_readlane(cur[kTwOp], at & 63u) : kTSkip << 2;
-        if ((op >> 2 & 15u) == kTSkip) {
-            shift();
-            at = 0;
-            op = __builtin_amdgcn_readlane(cur[kTwOp], 0);
-        }
-    }
-    __device__ __forceinline__ void advance(u32 slots)
-    {
-        at += slots + __popc(op >> 8 & 0x7Fu) * tree_dup_slots(M);
-    }
-
-    // word j (a constant) of the slots from `slot` after the step's first
-    __device__ __forceinline__ u32 word(u32 j, u32 slot = 0) const
-    {
-        return __builtin_amdgcn_readlane(cur[j & 7u], at + slot + (j >> 3));
-    }
-    __device__ __forceinline__ float fword(u32 j, u32 slot = 0) const { return __uint_as_float(word(j, slot)); }
+    __device__ __forceinline__ D const &d() const { return static_cast<D const &>(*this); }
+    __device__ __forceinline__ float fword(u32 j) const { return __uint_as_float(d().word(j)); }
     static __device__ __forceinline__ float keep(float v, u32 m) { return __uint_as_float(__float_as_uint(v) & m); }
     static __device__ __forceinline__ float pick(u32 m, float a, float b)
     {
         return __uint_as_float((__float_as_uint(a) & m) | (__float_as_uint(b) & ~m));
     }
 
-    __device__ __forceinline__ u32 goes_left(u32 split) const { return bins[split & 0xFFFFu] < split >> 16 ? ~0u : 0u; }
+    __device__ __forceinline__ u32 goes_left(u32 split) const
+    {
+        return d().bin_at(split & 0xFFFFu) < split >> 16 ? ~0u : 0u;
+    }
 
     __device__ __forceinline__ void add(u32 split, float c)
     {
-        u32 const col = split & 0xFFFFu;
         unsigned long long q;
         if (WIDE) { // round(c) as hi * 2^32 + lo, exactly
             double const v = __builtin_rintf(c), hi = __builtin_floor(v * 0x1p-32);
@@ -605,7 +563,7 @@ template <int M, int U, bool WIDE, bool AT = false> struct TreeShap {
             double const v = static_cast<double>(c) + 6755399441055744.0;
             q = static_cast<unsigned long long>(__double_as_longlong(v)) - 0x4338000000000000ull;
         }
-        atomicAdd(reinterpret_cast<unsigned long long *>(phi + min(col, col - plane) * 8u), q);
+        atomicAdd(d().phi_at(split & 0xFFFFu), q);
     }
 
     static constexpr bool past_half(int q) { return 2 * q >= M + (M & 1); }
@@ -629,10 +587,10 @@ template <int M, int U, bool WIDE, bool AT = false> struct TreeShap {
     // its k_q (or 1 - k_q) there, else k_q = 0
     __device__ __forceinline__ float dup_k(Dup const &u, int q, u32 o) const
     {
-        u32 const k = word(q, u.slot);
+        u32 const k = d().dup_word(q, u.slot);
         return __uint_as_float(past_half(q) ? (k & o) | (0x3F800000u & ~o) : k & o);
     }
-    __device__ __forceinline__ float dup_l(Dup const &u, int q) const { return fword(M + q, u.slot); }
+    __device__ __forceinline__ float dup_l(Dup const &u, int q) const { return __uint_as_float(d().dup_word(M + q, u.slot)); }
 
     // A node's k_q (1 - k_q past the half) for every row.
     __device__ __forceinline__ void consts(V &k, Dup const &u) const
@@ -719,13 +677,13 @@ template <int M, int U, bool WIDE, bool AT = false> struct TreeShap {
     // Seven nodes in preorder (r; a, a0, a1; b, b0, b1) below the product Tr.
     __device__ __forceinline__ void block(V const &Tr, V &H, u32 level)
     {
-        u32 const lv = word(kTwLv);
+        u32 const lv = d().word(kTwLv);
         u32 split[7], m[7];
         Dup u[7];
         u32 slot = tree_step_slots(kTBlock);
 #pragma unroll
         for (int i = 0; i < 7; ++i) {
-            split[i] = word(kTwSplit + i);
+            split[i] = d().word(kTwSplit + i);
             m[i] = goes_left(split[i]);
             u[i] = Dup{(op >> (8 + i) & 1u) != 0, slot, lv >> (4 * i) & 15u};
             slot += u[i].is ? tree_dup_slots(M) : 0u;
@@ -758,18 +716,83 @@ template <int M, int U, bool WIDE, bool AT = false> struct TreeShap {
         }
         join(Tr, kr, Ha, H, H, m[0], z[0], z[1], split[0], u[0]);
     }
+};
+
+// A wave's walk.  U: levels above the blocks.  AT: the walk may start below a tree's root
+// (levels come from the steps) and meet shares' values.
+template <int M, int U, bool WIDE, bool AT = false>
+struct TreeShap : ShapRow<TreeShap<M, U, WIDE, AT>, M, WIDE> {
+    using Row = ShapRow<TreeShap<M, U, WIDE, AT>, M, WIDE>;
+    using typename Row::Dup;
+    using typename Row::V;
+    using Row::fword;
+    using Row::op; // uniform
+    u8 const *bins;      // LDS: this lane's column of the bins
+    unsigned char *phi;  // LDS: this lane's column of the sums
+    u32 plane;           // bytes of one plane of bins
+    TSlot const *ahead;  // this lane's slot of the group after the next
+    uint4 nx0, nx1;      // its slot of the next group, in flight
+    u32 cur[8];          // its slot of the current group
+    u32 at;              // the running step's slot in it (uniform)
+    float *held;         // AT: LDS, this lane's column of the shares' values [share][M][64]
+
+    __device__ __forceinline__ u32 bin_at(u32 col) const { return bins[col]; }
+    __device__ __forceinline__ unsigned long long *phi_at(u32 col) const
+    {
+        return reinterpret_cast<unsigned long long *>(phi + min(col, col - plane) * 8u);
+    }
+    __device__ __forceinline__ void load()
+    {
+        uint4 const *p = reinterpret_cast<uint4 const *>(ahead);
+        nx0 = p[0];
+        nx1 = p[1];
+        ahead += 64;
+    }
+    __device__ __forceinline__ void shift()
+    {
+        cur[0] = nx0.x;
+        cur[1] = nx0.y;
+        cur[2] = nx0.z;
+        cur[3] = nx0.w;
+        cur[4] = nx1.x;
+        cur[5] = nx1.y;
+        cur[6] = nx1.z;
+        cur[7] = nx1.w;
+        load(); // whole groups of 64 slots are allocated, and two past the last
+    }
+    // The step at `at`: a skip or the group's end moves on to the next group.
+    __device__ __forceinline__ void fetch()
+    {
+        op = at < 64u ? __builtin_amdgcn_readlane(cur[kTwOp], at & 63u) : kTSkip << 2;
+        if ((op >> 2 & 15u) == kTSkip) {
+            shift();
+            at = 0;
+            op = __builtin_amdgcn_readlane(cur[kTwOp], 0);
+        }
+    }
+    __device__ __forceinline__ void advance(u32 slots)
+    {
+        at += slots + __popc(op >> 8 & 0x7Fu) * tree_dup_slots(M);
+    }
+
+    // word j (a constant) of the slots from `slot` after the step's first
+    __device__ __forceinline__ u32 word(u32 j, u32 slot = 0) const
+    {
+        return __builtin_amdgcn_readlane(cur[j & 7u], at + slot + (j >> 3));
+    }
+    __device__ __forceinline__ u32 dup_word(u32 j, u32 slot) const { return word(j, slot); }
 
     // The subtree whose first step is fetched, at level L below the product Tn.  Each
     // level is one copy of this code: its two children are two trips of a loop.
     template <int L> __device__ __forceinline__ void walk(V const &Tn, V &H)
     {
         if (L == U || (op & 3u) == kTBlock) {
-            block(Tn, H, level_of<L>());
+            this->block(Tn, H, level_of<L>());
             advance(tree_step_slots(kTBlock));
             return;
         }
         if constexpr (L < U) {
-            u32 const m = goes_left(word(kTwSplit));
+            u32 const m = this->goes_left(word(kTwSplit));
             V HL;
 #pragma clang loop unroll(disable)
             for (u32 side = 0; side < 2u; ++side) {
@@ -787,9 +810,9 @@ template <int M, int U, bool WIDE, bool AT = false> struct TreeShap {
                     V Tc;
                     V k;
                     u32 const me = side ? ~m : m;
-                    consts(k, dup_of<L>());
-                    descend(Tn, Tc, k, me, side ? fword(kTwZr) : fword(kTwZl));
-                    mark(me, level_of<L>(), dup_of<L>());
+                    this->consts(k, dup_of<L>());
+                    Row::descend(Tn, Tc, k, me, side ? fword(kTwZr) : fword(kTwZl));
+                    this->mark(me, level_of<L>(), dup_of<L>());
                     advance(1);
                     fetch();
                     walk<L + 1>(Tc, H);
@@ -801,8 +824,8 @@ template <int M, int U, bool WIDE, bool AT = false> struct TreeShap {
                 }
             }
             V k;
-            consts(k, dup_of<L>());
-            join(Tn, k, HL, H, H, m, fword(kTwZl), fword(kTwZr), word(kTwSplit), dup_of<L>());
+            this->consts(k, dup_of<L>());
+            this->join(Tn, k, HL, H, H, m, fword(kTwZl), fword(kTwZr), word(kTwSplit), dup_of<L>());
             advance(1);
         }
     }
@@ -819,18 +842,18 @@ template <int M, int U, bool WIDE, bool AT = false> struct TreeShap {
         load();
         shift();
         at = pc & 63u;
-        sat = 0;
+        this->sat = 0;
     }
     // The way from a tree's root down to the share whose steps follow.
     __device__ __forceinline__ void go_down(V &T)
     {
         while ((op & 3u) == kTEnter && (op & (kTOnlyL | kTOnlyR))) {
             bool const right = (op & kTOnlyR) != 0;
-            u32 const m = goes_left(word(kTwSplit)), me = right ? ~m : m;
+            u32 const m = this->goes_left(word(kTwSplit)), me = right ? ~m : m;
             V k, Tc;
-            consts(k, dup_of<0>());
-            descend(T, Tc, k, me, right ? fword(kTwZr) : fword(kTwZl));
-            mark(me, level_of<0>(), dup_of<0>());
+            this->consts(k, dup_of<0>());
+            Row::descend(T, Tc, k, me, right ? fword(kTwZr) : fword(kTwZl));
+            this->mark(me, level_of<0>(), dup_of<0>());
 #pragma unroll
             for (int q = 0; q < M; ++q) T[q] = Tc[q];
             advance(1);
@@ -839,15 +862,16 @@ template <int M, int U, bool WIDE, bool AT = false> struct TreeShap {
     }
 };
 
-// Few rows or trees.  A walk is one serial chain (0.27 us a split), so a batch with fewer
-// row blocks x trees than the chip has room for waves waits for one tree's: 300 us at
-// depth 10 whatever the batch.  Here a workgroup takes one tree of a row block: its 8 waves
-// walk the tree's shares (the subtrees below a cut, each with the product T carried down to
-// it), leave their values in LDS, and the first wave walks the splits above the cut over
-// them.  Every split's arithmetic is the walk's own, so a row's bits are the same either
-// way.  One to 64 rows x 20 trees: depth 6 37 -> 29 us, depth 8 85 -> 42, depth 10
-// 297 -> 89; 65 rows x 100 depth-10 trees
-// 283 -> 72 us.
+// Deep trees (past kSplitAbove levels), few row blocks x trees.  A walk is one serial chain
+// (0.27 us a split), so a batch with fewer of them than the chip has room for waves waits
+// for one tree's: 280 us at depth 10 whatever the batch.  Here a workgroup takes one tree of
+// a row block: its 8 waves walk the tree's shares (the subtrees below a cut, each with the
+// product T carried down to it), leave their values in LDS, and the first wave walks the
+// splits above the cut over them.  Every split's arithmetic is the walk's own, so a row's
+// bits are the same either way.  128 rows x 100 depth-10 trees 283 -> 76 us, 64 rows x 100
+// of depth 12 1,170 -> 250.  Shallower trees' few rows take k_shap_lanes at less (depth 8,
+// 256 rows x 100 trees: 33 us, 54 so).
+constexpr u32 kSplitAbove = 8;
 struct SplitTree {
     u32 share0, n_shares, top; // first share, shares, first slot of the steps above (kNone: none)
     u32 pad;
@@ -923,6 +947,193 @@ __global__ __launch_bounds__(kSplitThreads) void k_shap_split(u8 const *__restri
         u32 const rr = k / F, f = k - rr * F;
         unsigned long long const v = s_phi[f * kTreeShapRows + rr];
         if (v != 0ull) atomicAdd(acc + (r0 + rr) * (F + 1) + f, v);
+    }
+}
+
+// A handful of rows.  In a walk a row has one lane of 64, and its splits are one chain.  Here
+// a lane takes one block of a tree for one row: it forms the products T down its own way
+// from the root, runs the block, and the blocks' values are joined level by level through
+// LDS, every split by the lane of the first block below it.  A split's arithmetic is the
+// walk's own (ShapRow), so a row's bits are the same either way.  A workgroup's lanes are the
+// rows of `per` trees' blocks at a time.  Bound by latency (records from L2, a barrier a
+// level) with few lanes, by its instructions with many: the way down is taken again for
+// every block.  One row x 20 trees: depth 8 28 (k_shap_split) -> 14 us, depth 10 74 -> 20,
+// 5 of depth 12 245 -> 21; 16 rows x 1,000 depth-8 trees 78 (k_shap_tree) -> 35.
+constexpr u32 lane_threads(u32 m) { return m <= 5u ? 1024u : 512u; } // of a workgroup at most
+// Four waves a SIMD (a few spills with 5 nodes): 64 rows x 100 depth-10 trees 82 -> 73 us,
+// one row 17.4 -> 19.4; with 6 nodes they would cost more than they give.
+constexpr u32 lane_waves(u32 m) { return m <= 5u ? 4u : 3u; }
+constexpr u32 kLaneLevels = kTreeShapMaxDepth - kTBlockLevels; // splits above a block at most
+struct alignas(16) LaneUnit {
+    u32 block, info;            // the block's slot; splits above | right turns << 4 | own splits << 13
+    u32 node[kLaneLevels];      // by level: the split's step (kTEnter)
+    u32 other[kLaneLevels];     // own splits: the unit that owns the other child, kNone: a leaf
+};
+
+template <int M, bool WIDE> struct LaneShap : ShapRow<LaneShap<M, WIDE>, M, WIDE> {
+    u8 const *bins;      // LDS: [2][F][rows], this lane's row
+    unsigned char *phi;  // LDS: [F][rows], this lane's row
+    u32 plane, rs;       // bytes of a plane of bins in the steps' columns; log2 of the rows
+    TSlot const *step, *next;
+    uint4 nx0, nx1;
+    u32 cur[8 * tree_step_slots(kTBlock)]; // its words (of a split: the first slot's)
+
+    __device__ __forceinline__ u32 word(u32 j) const { return cur[j]; }
+    __device__ __forceinline__ u32 dup_word(u32 j, u32 slot) const { return step[slot + (j >> 3)].w[j & 7u]; }
+    __device__ __forceinline__ u32 bin_at(u32 col) const { return bins[col / kTreeShapRows << rs]; }
+    __device__ __forceinline__ unsigned long long *phi_at(u32 col) const
+    {
+        return reinterpret_cast<unsigned long long *>(phi) + (min(col, col - plane) / kTreeShapRows << rs);
+    }
+    // A step's first slot into flight (fetch), then it is the running step (take); rest():
+    // a block's other slots.
+    __device__ __forceinline__ void fetch(TSlot const *s)
+    {
+        next = s;
+        nx0 = reinterpret_cast<uint4 const *>(s)[0];
+        nx1 = reinterpret_cast<uint4 const *>(s)[1];
+    }
+    __device__ __forceinline__ void put(u32 k, uint4 const &v)
+    {
+        cur[4 * k] = v.x;
+        cur[4 * k + 1] = v.y;
+        cur[4 * k + 2] = v.z;
+        cur[4 * k + 3] = v.w;
+    }
+    __device__ __forceinline__ void take()
+    {
+        step = next;
+        put(0, nx0);
+        put(1, nx1);
+        this->op = cur[kTwOp];
+    }
+    __device__ __forceinline__ void rest()
+    {
+#pragma unroll
+        for (u32 k = 2; k < 2u * tree_step_slots(kTBlock); ++k) put(k, reinterpret_cast<uint4 const *>(step)[k]);
+    }
+};
+
+template <int M, int U, bool WIDE>
+__global__ __launch_bounds__(lane_threads(M), lane_waves(M)) void k_shap_lanes(
+    u8 const *__restrict__ bins, u64 n, u64 stride, u32 F, u16 const *__restrict__ last,
+    TSlot const *__restrict__ slots, LaneUnit const *__restrict__ units, u32 const *__restrict__ first, u32 n_trees,
+    u32 per, u32 rs, u32 upper, TQuad quad, float lr, double bias, double scale, double *__restrict__ out)
+{
+    typedef float V[M];
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned long long *s_phi = reinterpret_cast<unsigned long long *>(smem); // [F][rows] fixed point
+    float *s_held = reinterpret_cast<float *>(s_phi + (F << rs));              // [2][M][threads] values
+    u32 const threads = blockDim.x, rows = 1u << rs;
+    u8 *s_bins = reinterpret_cast<u8 *>(s_held + 2u * M * threads);            // [2][F][rows]
+    u64 const r0 = static_cast<u64>(blockIdx.x) << rs;
+    u32 const nr = static_cast<u32>(min<u64>(rows, n - r0));
+    for (u32 k = threadIdx.x; k < F << rs; k += threads) {
+        u32 const rr = k / F, f = k - rr * F;
+        u32 const b = rr < nr ? bins[(r0 + rr) * stride + f] : 0u;
+        s_phi[k] = 0ull;
+        s_bins[(f << rs) + rr] = static_cast<u8>(b);
+        s_bins[((F + f) << rs) + rr] = static_cast<u8>(b == last[f] ? 0u : min(b + 1u, 255u));
+    }
+    __syncthreads();
+    u32 const rr = threadIdx.x & (rows - 1u), unit = threadIdx.x >> rs;
+    LaneShap<M, WIDE> w;
+    w.bins = s_bins + rr;
+    w.phi = reinterpret_cast<unsigned char *>(s_phi + rr);
+    w.plane = kTreeShapRows * F;
+    w.rs = rs;
+#pragma unroll
+    for (int q = 0; q < M; ++q) w.y[q] = quad.y[q];
+    u32 const chunks = (n_trees + per - 1u) / per;
+    u32 buf = 0;
+    for (u32 c = blockIdx.y; c < chunks; c += gridDim.y) {
+        u32 const u0 = first[c * per], u1 = first[min(n_trees, (c + 1u) * per)];
+        bool const live = rr < nr && unit < u1 - u0;
+        V Ts[U], H; // products at the splits above; the value of the child last joined
+        u32 info = 0u, len = 0u, node[U]; // the steps down to the block
+        if (live) {
+            LaneUnit const *un = units + u0 + unit;
+            info = un->info;
+            len = info & 15u;
+#pragma unroll
+            for (int L = 0; L < U; ++L) node[L] = un->node[L];
+            u32 const block = un->block;
+            w.fetch(slots + (len ? node[0] : block));
+            V T;
+            w.sat = 0;
+#pragma unroll
+            for (int q = 0; q < M; ++q) T[q] = quad.w[q];
+#pragma unroll
+            for (int L = 0; L < U; ++L)
+                if (L < static_cast<int>(len)) {
+                    w.take();
+                    w.fetch(slots + (L + 1 < U && L + 1 < static_cast<int>(len) ? node[L + 1] : block));
+                    typename LaneShap<M, WIDE>::Dup const u{L > 0 && (w.op & 0x100u) != 0, 1u, w.word(kTwLv)};
+                    bool const right = (info >> (4 + L) & 1u) != 0;
+                    u32 const m = w.goes_left(w.word(kTwSplit)), me = right ? ~m : m;
+                    V k, Tc;
+                    w.consts(k, u);
+                    w.descend(T, Tc, k, me, right ? w.fword(kTwZr) : w.fword(kTwZl));
+                    w.mark(me, L, u);
+#pragma unroll
+                    for (int q = 0; q < M; ++q) {
+                        Ts[L][q] = T[q];
+                        T[q] = Tc[q];
+                    }
+                }
+            w.take();
+            w.rest();
+            w.block(T, H, len);
+        }
+#pragma unroll
+        for (int L = U - 1; L >= 0; --L) {
+            if (L >= static_cast<int>(upper)) continue;
+            bool const own = (info >> (13 + L) & 1u) != 0;
+            u32 other = kNone;
+            if (own) {
+                w.fetch(slots + node[L]);
+                other = units[u0 + unit].other[L];
+            }
+            float *held = s_held + buf * M * threads;
+            buf ^= 1u; // the next level writes beside what this one still reads
+            if (live) {
+#pragma unroll
+                for (int q = 0; q < M; ++q) held[q * threads + threadIdx.x] = H[q];
+            }
+            __syncthreads();
+            if (own) {
+                w.take();
+                typename LaneShap<M, WIDE>::Dup const u{L > 0 && (w.op & 0x100u) != 0, 1u, w.word(kTwLv)};
+                bool const right = (info >> (4 + L) & 1u) != 0;
+                u32 const at = ((other - u0) << rs) + rr;
+                float const leaf = right ? w.fword(kTwVl) : w.fword(kTwVr);
+                V k, HL, HR;
+#pragma unroll
+                for (int q = 0; q < M; ++q) {
+                    float const x = other == kNone ? leaf : held[q * threads + at];
+                    HL[q] = right ? x : H[q];
+                    HR[q] = right ? H[q] : x;
+                }
+                w.consts(k, u);
+                w.join(Ts[L], k, HL, HR, H, w.goes_left(w.word(kTwSplit)), w.fword(kTwZl), w.fword(kTwZr),
+                       w.word(kTwSplit), u);
+            }
+        }
+    }
+    __syncthreads();
+    if (gridDim.y > 1) {
+        // Trees of one row block meet in the zeroed output cells, as k_shap_tree's do.
+        unsigned long long *acc = reinterpret_cast<unsigned long long *>(out);
+        for (u32 k = threadIdx.x; k < nr * F; k += threads) {
+            u32 const r = k / F, f = k - r * F;
+            unsigned long long const v = s_phi[(f << rs) + r];
+            if (v != 0ull) atomicAdd(acc + (r0 + r) * (F + 1) + f, v);
+        }
+        return;
+    }
+    for (u32 k = threadIdx.x; k < nr * (F + 1); k += threads) {
+        u32 const r = k / (F + 1), f = k - r * (F + 1);
+        out[(r0 + r) * (F + 1) + f] = f == F ? bias : shap_from_fixed(s_phi[(f << rs) + r], scale, lr);
     }
 }
 
@@ -1173,6 +1384,8 @@ struct TreePacker {
     GaussRule rule;
     std::vector<TSlot> out;
     std::vector<std::pair<u32, u32>> spans; // of every node walked: its subtree's slots in out
+    std::vector<LaneUnit> units;     // k_shap_lanes: the blocks, in the walk's order
+    std::vector<std::pair<u32, u32>> down; // (step, side) of the splits above the walk
     struct Edge { // on the way down: feature, level and merged cover fraction of its latest edge
         u32 feature, level;
         double z;
@@ -1211,9 +1424,9 @@ struct TreePacker {
                 r.level = above[k].level;
                 r.z = above[k].z;
                 for (u32 q = 0; q < rule.m; ++q) {
-                    double const x = rule.x[q], a = r.z + x * (1.0 - r.z);
-                    r.k[q] = static_cast<float>(past_half(q, rule.m) ? r.z * (1.0 - x) / a : x / a);
-                    r.l[q] = static_cast<float>(r.z / (a * a));
+                    double const x = rule.x[q], inv = 1.0 / (r.z + x * (1.0 - r.z)), zi = r.z * inv;
+                    r.k[q] = static_cast<float>(past_half(q, rule.m) ? zi * (1.0 - x) : x * inv);
+                    r.l[q] = static_cast<float>(zi * inv);
                 }
                 break;
             }
@@ -1253,7 +1466,7 @@ struct TreePacker {
         return at;
     }
 
-    void step(u32 kind, u32 level, Node const &nd, u32 flags, double vl, double vr)
+    size_t step(u32 kind, u32 level, Node const &nd, u32 flags, double vl, double vr)
     {
         size_t const at = open(kind, &nd, 1);
         TSlot *s = &out[at];
@@ -1264,6 +1477,7 @@ struct TreePacker {
         put(s, kTwZr, nd.zr);
         put(s, kTwVl, vl);
         put(s, kTwVr, vr);
+        return at;
     }
 
     // Nodes of a block in preorder: `depth` more levels below id.
@@ -1283,7 +1497,7 @@ struct TreePacker {
         }
     }
 
-    void block(u32 id, u32 level)
+    size_t block(u32 id, u32 level)
     {
         Node nd[7], *np = nd;
         double leaf[8], *lp = leaf;
@@ -1308,35 +1522,53 @@ struct TreePacker {
             put(s, kTwLeaf + 2 * i, leaf[2 * i]);
             put(s, kTwLeaf + 2 * i + 1, leaf[2 * i + 1]);
         }
+        return at;
     }
 
-    void walk(u32 id, u32 level)
+    // Returns the first unit below id, which owns it.
+    u32 walk(u32 id, u32 level)
     {
         u32 const begin = static_cast<u32>(out.size());
-        walk_steps(id, level);
+        u32 const own = levels[id] <= kTBlockLevels ? leaf_block(id, level) : inner(id, level);
         spans[id] = {begin, static_cast<u32>(out.size())};
+        return own;
     }
-    void walk_steps(u32 id, u32 level)
+    u32 leaf_block(u32 id, u32 level)
     {
-        if (levels[id] <= kTBlockLevels) {
-            block(id, level);
-            return;
+        LaneUnit u{};
+        u.block = static_cast<u32>(block(id, level));
+        u.info = level;
+        for (u32 l = 0; l < level; ++l) {
+            u.node[l] = down[l].first;
+            u.info |= down[l].second << (4 + l);
         }
+        units.push_back(u);
+        return static_cast<u32>(units.size() - 1);
+    }
+    u32 inner(u32 id, u32 level)
+    {
         bh_node const &n = t[id];
         Node const nd = node(id);
         bool const ll = t[n.left].feature < 0, rl = t[n.right].feature < 0;
         double const vl = ll ? static_cast<double>(t[n.left].value) * scale : 0.0;
         double const vr = rl ? static_cast<double>(t[n.right].value) * scale : 0.0;
         u32 const flags = (ll ? kTLeafL : 0u) | (rl ? kTLeafR : 0u);
-        step(kTEnter, level, nd, flags, vl, vr);
+        u32 const at = static_cast<u32>(step(kTEnter, level, nd, flags, vl, vr));
+        u32 kid[2] = {kNone, kNone};
         for (u32 side = 0; side < 2; ++side) {
             if (side ? rl : ll) continue;
             if (side && !ll) step(kTTurn, level, nd, flags, vl, vr);
             above.push_back({static_cast<u32>(n.feature), level, nd.z * (side ? nd.zr : nd.zl)});
-            walk(side ? n.right : n.left, level + 1);
+            down.push_back({at, side});
+            kid[side] = walk(side ? n.right : n.left, level + 1);
+            down.pop_back();
             above.pop_back();
         }
         step(kTCombine, level, nd, flags, vl, vr);
+        u32 const own = ll ? kid[1] : kid[0];
+        units[own].info |= 1u << (13 + level);
+        units[own].other[level] = ll ? kNone : kid[1];
+        return own;
     }
 
     // Appends a walked subtree's steps again, in a third of the time packing them takes.
@@ -1533,6 +1765,7 @@ struct bh_predictor {
     double shap_scale = 1.0;   // fixed-point scale of the TreeSHAP accumulators
     // tree-form TreeSHAP (tree_m quadrature nodes; 0: the packed form serves the ensemble)
     u32 tree_m = 0, tree_depth = 0, n_ttrees = 0, max_shares = 0; // max_shares 0: no split form
+    u32 max_units = 1;         // blocks of a tree at most
     double tree_scale = 1.0;   // its fixed-point scale, times the weights' common factor
     bool tree_wide = false;    // TreeShap's WIDE
     TQuad quad{};
@@ -1540,6 +1773,8 @@ struct bh_predictor {
     u32 *d_tfirst = nullptr;
     u32 *d_sfirst = nullptr;
     SplitTree *d_split = nullptr;
+    LaneUnit *d_units = nullptr;
+    u32 *d_ufirst = nullptr;
     PNode *d_nodes = nullptr;
     u32 *d_roots = nullptr;
     // tile form (n_tiles 0: the ensemble does not fit it)
@@ -1658,88 +1893,160 @@ int launch_predict(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, float *
 // Workgroups that fill the chip with tree-form waves: smaller batches split their trees.
 constexpr u32 kTreeShapFill = 768;
 
-// Row blocks x trees up to which a workgroup takes one tree (k_shap_split): one round of
-// workgroups while the trees are small (depth 6, 400 walks: 42 us split, 39 whole), two from
-// depth 8 (400 walks: 70 and 87 us; 1,000: 125 and 96).
-u64 split_walks(u32 depth) { return depth >= 8 ? 512 : 256; }
-// The node count a kernel is built for (the switch of launch_shap_tree).
-u32 m_of(u32 m, u32 upper) { return upper <= 5 ? std::max(2u, std::min(m, 4u)) : std::max(4u, std::min(m, 6u)); }
+// Row blocks x trees up to which a workgroup takes one tree (k_shap_split): two rounds of
+// workgroups (depth 10, 400 walks: 148 us split, 287 whole; 1,600: 574 whole).
+constexpr u64 kSplitWalks = 512;
 // LDS of a k_shap_split workgroup whose trees have up to `shares` shares.
-size_t split_lds(u32 F, u32 shares, u32 m, u32 upper)
+size_t split_lds(u32 F, u32 shares, u32 m) { return tree_shap_lds(F) + static_cast<size_t>(shares) * m * 64u * sizeof(float); }
+
+// Launch of k_shap_lanes: rows and trees of a workgroup's lanes, and the workgroups that
+// share the trees.  256 lanes where a tree's blocks allow it: more workgroups, and more of
+// them on a CU (64 rows x 20 depth-10 trees 28 -> 20 us against 512); up to 1,024 where one
+// workgroup then takes the batch and writes its output itself.
+constexpr u32 kLaneFill = 1024;
+struct LaneShape {
+    u32 rs, per, threads, split;
+    u64 blocks;
+    size_t lds;
+};
+LaneShape lane_shape(bh_predictor const *p, u64 n)
 {
-    return tree_shap_lds(F) + static_cast<size_t>(shares) * m_of(m, upper) * 64u * sizeof(float);
+    LaneShape s{};
+    u32 most = (p->max_units <= 256u ? 256u : 512u) / p->max_units; // rows x trees of full lanes
+    if (n * p->n_ttrees * p->max_units <= lane_threads(p->tree_m)) most = lane_threads(p->tree_m) / p->max_units;
+    auto const lds = [&](u32 rs, u32 threads) {
+        return (static_cast<size_t>(p->F) * 10u << rs) + 2u * p->tree_m * threads * sizeof(float);
+    };
+    while ((2u << s.rs) <= most && (1u << s.rs) < n && lds(s.rs + 1, 512u) <= 64u * 1024u) ++s.rs;
+    s.per = std::max(1u, std::min(p->n_ttrees, most >> s.rs));
+    u32 const lanes = (s.per * p->max_units) << s.rs;
+    s.threads = (std::max(lanes, std::min(256u, p->F << s.rs)) + 63u) / 64u * 64u; // some to load the rows with
+    s.lds = lds(s.rs, s.threads);
+    s.blocks = (n + (1u << s.rs) - 1u) >> s.rs;
+    s.split = static_cast<u32>(std::min<u64>((p->n_ttrees + s.per - 1u) / s.per, std::max<u64>(1, kLaneFill / s.blocks)));
+    return s;
 }
+
+// Microseconds of a batch, measured over 1 to 1,000 trees of 4 to 12 levels x 1 to 1,024 rows
+// of 28 and 200 features.  Several workgroups a row block (shares) zero the output, add to
+// it and convert it.
+double shares_us(bh_predictor const *p, u64 n, u32 shares)
+{
+    return shares > 1 ? 6.0 + static_cast<double>(n) * (p->F + 1) * 8.0 * (2.0 + shares) / 3e6 : 0.0;
+}
+// Whole walks: a wave's trees one after the other, 2.1 us a block of seven splits.
+double whole_us(bh_predictor const *p, u64 n, u32 split)
+{
+    u64 const wgs = (n + kTreeShapRows - 1) / kTreeShapRows * split;
+    u32 const cu = std::max<u32>(1u, std::min<size_t>(kTreeShapFill / 256u, 160u * 1024u / tree_shap_lds(p->F)));
+    u32 const trees = (p->n_ttrees + split * (kTreeShapThreads / 64u) - 1u) / (split * (kTreeShapThreads / 64u));
+    return static_cast<double>((wgs + 256u * cu - 1) / (256u * cu)) * (2.1 * p->max_units * trees + 0.08 * p->F) +
+           shares_us(p, n, split);
+}
+// A tree a workgroup: 256 at a time.
+double split_us(bh_predictor const *p, u64 n)
+{
+    u64 const walks = (n + kTreeShapRows - 1) / kTreeShapRows * p->n_ttrees;
+    if (!p->max_shares || walks > kSplitWalks) return 1e300;
+    return static_cast<double>((walks + 255) / 256) * (7.0 + 0.47 * p->max_units + 0.04 * p->F) + shares_us(p, n, 2);
+}
+// A lane a block and row: 8 ps and more by the levels of the way down; its rows' loads.
+double lanes_us(bh_predictor const *p, u64 n, u32 upper, LaneShape const &s)
+{
+    double const lanes = static_cast<double>(n) * p->n_ttrees * p->max_units;
+    double const per = std::max(20.0, 7.0 + 1.2 * upper * upper) * (p->tree_m <= 5 ? 1.0 : 1.3);
+    double const load = 0.1 * (p->F << s.rs) / s.threads * ((s.blocks * s.split + 1023) / 1024);
+    return 7.0 + 0.6 * upper + load + lanes * 1e-6 * per + shares_us(p, n, s.split);
+}
+
+// The node counts and levels the tree form's kernels are built for.
+#define BH_FORMS(LAUNCH)                       \
+    if (upper <= 5) {                          \
+        if (p->tree_m <= 2) LAUNCH(2, 5);      \
+        else if (p->tree_m == 3) LAUNCH(3, 5); \
+        else LAUNCH(4, 5);                     \
+    } else if (p->tree_m <= 4) {               \
+        LAUNCH(4, 9);                          \
+    } else if (p->tree_m == 5) {               \
+        LAUNCH(5, 9);                          \
+    } else {                                   \
+        LAUNCH(6, 9);                          \
+    }
 
 int launch_shap_tree(bh_predictor *p, u8 const *d_bins, u64 n, u64 stride, double *d_out, hipStream_t s)
 {
     u32 const blocks = static_cast<u32>((n + kTreeShapRows - 1) / kTreeShapRows);
     u32 const upper = p->tree_depth > kTBlockLevels ? p->tree_depth - kTBlockLevels : 0u;
-    u32 const threads = kTreeShapThreads, waves = threads / 64u;
-    // Trees of a row block over `split` workgroups: the fewest rounds of kTreeShapFill
-    // workgroups per share of the trees, then the fewest shares.
+    // Every launch gives a row the same bits: the cheapest one.
+    // Whole walks: the trees of a row block over `shares` workgroups, the fewest rounds of
+    // kTreeShapFill workgroups per share of the trees, then the fewest shares; or one, where
+    // adding to the output costs more than that saves.
+    u32 const waves = kTreeShapThreads / 64u;
     u32 const most = std::min(std::max(1u, kTreeShapFill / std::min(blocks, kTreeShapFill)) + 7u,
                               std::max(1u, (p->n_ttrees + waves - 1) / waves));
-    u32 split = 1;
+    u32 shares = 1;
     u64 rounds = (static_cast<u64>(blocks) + kTreeShapFill - 1) / kTreeShapFill;
     for (u32 k = 2; k <= most && blocks < 16u * kTreeShapFill; ++k) {
         u64 const r = (static_cast<u64>(blocks) * k + kTreeShapFill - 1) / kTreeShapFill;
-        if (r * split < rounds * k) {
+        if (r * shares < rounds * k) {
             rounds = r;
-            split = k;
+            shares = k;
         }
+    }
+    double us = whole_us(p, n, shares);
+    if (double const one = whole_us(p, n, 1); one < us) {
+        us = one;
+        shares = 1;
+    }
+    LaneShape const ls = lane_shape(p, n);
+    enum { kWhole, kSplit, kLanes } form = kWhole;
+    if (split_us(p, n) < us) {
+        us = split_us(p, n);
+        form = kSplit;
+        shares = 2; // at least: the output is added to
+    }
+    if (p->n_ttrees && lanes_us(p, n, upper, ls) < 0.9 * us && ls.blocks <= 0x7FFFFFFFu) {
+        form = kLanes;
+        shares = ls.split;
     }
     u64 const cells = n * (p->F + 1);
     u32 const cgrid = static_cast<u32>(std::min<u64>((cells + 255) / 256, 4096));
-    if (split > 1) {
+    if (shares > 1) {
         hipLaunchKernelGGL(k_shap_zero, dim3(cgrid), dim3(256), 0, s, reinterpret_cast<unsigned long long *>(d_out),
                            cells);
         SHIP(hipGetLastError());
     }
     size_t const lds = tree_shap_lds(p->F);
-    if (p->max_shares && static_cast<u64>(blocks) * p->n_ttrees <= split_walks(p->tree_depth)) {
-        if (split <= 1) {
-            hipLaunchKernelGGL(k_shap_zero, dim3(cgrid), dim3(256), 0, s,
-                               reinterpret_cast<unsigned long long *>(d_out), cells);
-            SHIP(hipGetLastError());
-        }
-        dim3 const sgrid(blocks, p->n_ttrees);
+    if (form == kLanes) {
+        dim3 const grid(static_cast<u32>(ls.blocks), ls.split);
+#define BH_SL(MV, UV)                                                                                              \
+    hipLaunchKernelGGL((p->tree_wide ? k_shap_lanes<MV, UV, true> : k_shap_lanes<MV, UV, false>), grid,            \
+                       dim3(ls.threads), ls.lds, s, d_bins, n, stride, p->F, p->d_last, p->d_tslots, p->d_units,   \
+                       p->d_ufirst, p->n_ttrees, ls.per, ls.rs, upper, p->quad, p->lr, p->shap_bias,               \
+                       p->tree_scale, d_out)
+        BH_FORMS(BH_SL)
+#undef BH_SL
+    } else if (form == kSplit) {
+        dim3 const grid(blocks, p->n_ttrees);
 #define BH_SP(MV)                                                                                                  \
-    hipLaunchKernelGGL((p->tree_wide ? k_shap_split<MV, true> : k_shap_split<MV, false>), sgrid,                   \
-                       dim3(kSplitThreads), split_lds(p->F, p->max_shares, p->tree_m, upper), s, d_bins, n, stride, p->F, p->d_last,                      \
-                       p->d_tslots, p->d_sfirst, p->d_split, p->n_ttrees, p->quad, d_out)
-        switch (m_of(p->tree_m, upper)) {
-        case 2: BH_SP(2); break;
-        case 3: BH_SP(3); break;
-        case 4: BH_SP(4); break;
-        case 5: BH_SP(5); break;
-        default: BH_SP(6); break;
-        }
+    hipLaunchKernelGGL((p->tree_wide ? k_shap_split<MV, true> : k_shap_split<MV, false>), grid,                    \
+                       dim3(kSplitThreads), split_lds(p->F, p->max_shares, p->tree_m), s, d_bins, n, stride, p->F, \
+                       p->d_last, p->d_tslots, p->d_sfirst, p->d_split, p->n_ttrees, p->quad, d_out)
+        if (p->tree_m <= 4) BH_SP(4); // deep trees have 4 nodes at least
+        else if (p->tree_m == 5) BH_SP(5);
+        else BH_SP(6);
 #undef BH_SP
-        SHIP(hipGetLastError());
-        hipLaunchKernelGGL(k_shap_to_double, dim3(cgrid), dim3(256), 0, s, d_out, n, p->F, p->lr, p->shap_bias,
-                           p->tree_scale);
-        SHIP(hipGetLastError());
-        return 0;
-    }
-    dim3 const grid(blocks, split);
+    } else {
+        dim3 const grid(blocks, shares);
 #define BH_TS(MV, UV)                                                                                              \
     hipLaunchKernelGGL((p->tree_wide ? k_shap_tree<MV, UV, true> : k_shap_tree<MV, UV, false>), grid,              \
-                       dim3(threads), lds, s, d_bins, n, stride, p->F, p->d_last, p->d_tslots, p->d_tfirst,        \
-                       p->n_ttrees, p->quad, p->lr, p->shap_bias, p->tree_scale, d_out)
-    if (upper <= 5) {
-        if (p->tree_m <= 2) BH_TS(2, 5);
-        else if (p->tree_m == 3) BH_TS(3, 5);
-        else BH_TS(4, 5);
-    } else if (p->tree_m <= 4) {
-        BH_TS(4, 9);
-    } else if (p->tree_m == 5) {
-        BH_TS(5, 9);
-    } else {
-        BH_TS(6, 9);
-    }
+                       dim3(kTreeShapThreads), lds, s, d_bins, n, stride, p->F, p->d_last, p->d_tslots,            \
+                       p->d_tfirst, p->n_ttrees, p->quad, p->lr, p->shap_bias, p->tree_scale, d_out)
+        BH_FORMS(BH_TS)
 #undef BH_TS
+    }
     SHIP(hipGetLastError());
-    if (split > 1) {
+    if (shares > 1) {
         hipLaunchKernelGGL(k_shap_to_double, dim3(cgrid), dim3(256), 0, s, d_out, n, p->F, p->lr, p->shap_bias,
                            p->tree_scale);
         SHIP(hipGetLastError());
@@ -1954,9 +2261,11 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     p->shap_bias = ev_sum * static_cast<double>(learning_rate) + static_cast<double>(init_score);
     p->max_len = static_cast<u32>(std::max<size_t>(max_len, 1));
     // The tree form serves every ensemble whose trees, paths and feature count fit its
-    // kernels; the packed form the rest.
+    // kernels; the packed form the rest, and deep trees on few features: past 8 levels the
+    // walk runs one wave a SIMD, and paths of at most 8 features take the short body (4
+    // features, 5 depth-12 trees: 16,384 rows 2,437 -> 1,645 us, 64 rows 255 -> 41).
     bool const tree_form = deepest <= kTreeShapMaxDepth && max_len <= 2 * kTreeShapMaxM &&
-                           tree_shap_lds(n_features) <= 160u * 1024u;
+                           tree_shap_lds(n_features) <= 160u * 1024u && (deepest <= 8u || max_len > 8u);
     if (!tree_form) {
         std::vector<ActiveElem> act;
         size_t longest = 0;
@@ -2000,6 +2309,7 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     TreePacker pack{};
     std::vector<u32> tfirst;
     std::vector<SplitTree> split;
+    std::vector<u32> ufirst; // of every tree: its first unit
     std::vector<std::vector<std::pair<u32, u32>>> spans;
     if (tree_form) {
         // kernels' node counts: 2, 3, 4 (up to 8 levels), 4, 5, 6 (more)
@@ -2010,7 +2320,7 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
         pack.F = n_features;
         pack.scale = scale;
         pack.rule = gauss_legendre(m);
-        u32 const cut = deepest > kTBlockLevels + 1u ? TreePacker::cut_of(deepest) : 0u;
+        u32 const cut = deepest > kSplitAbove ? TreePacker::cut_of(deepest) : 0u;
         u32 walked = 0, most = 0; // trees with splits; shares of one
         for (u32 t = 0; t < n_trees; ++t) {
             pack.t = nodes + tree_offsets[t];
@@ -2019,9 +2329,8 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
             ++walked;
             if (cut) most = std::max(most, pack.count(0, 0, cut));
         }
-        // The split form serves up to split_walks trees whose shares' values fit LDS.
-        u32 const upper = deepest > kTBlockLevels ? deepest - kTBlockLevels : 0u;
-        if (walked <= split_walks(deepest) && split_lds(n_features, most, m, upper) <= 160u * 1024u) p->max_shares = most;
+        // The split form serves up to kSplitWalks trees whose shares' values fit LDS.
+        if (walked <= kSplitWalks && split_lds(n_features, most, m) <= 160u * 1024u) p->max_shares = most;
         pack.out.reserve(pn.size() * (p->max_shares ? 3u : 2u) + 256u); // about 1.5 slots a node each
         for (u32 t = 0; t < n_trees; ++t) {
             pack.t = nodes + tree_offsets[t];
@@ -2029,10 +2338,13 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
             if (pack.t[0].feature < 0) continue;
             pack.spans.assign(levels[t].size(), {0u, 0u});
             tfirst.push_back(static_cast<u32>(pack.out.size()));
+            ufirst.push_back(static_cast<u32>(pack.units.size()));
             pack.walk(0, 0);
+            p->max_units = std::max(p->max_units, static_cast<u32>(pack.units.size()) - ufirst.back());
             if (p->max_shares) spans.push_back(std::move(pack.spans));
         }
         tfirst.push_back(static_cast<u32>(pack.out.size()));
+        ufirst.push_back(static_cast<u32>(pack.units.size()));
         for (u32 t = 0, k = 0; p->max_shares && t < n_trees; ++t) {
             pack.t = nodes + tree_offsets[t];
             pack.levels = levels[t].data();
@@ -2075,6 +2387,8 @@ int bh_predictor_create(int device, const bh_node *nodes, const uint32_t *tree_o
     up.add(p->d_tfirst, tfirst.data(), tfirst.size());
     up.add(p->d_sfirst, pack.first.data(), pack.first.size());
     up.add(p->d_split, split.data(), split.size());
+    up.add(p->d_units, pack.units.data(), pack.units.size());
+    up.add(p->d_ufirst, ufirst.data(), ufirst.size());
     hipError_t e = up.run(p->owned);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {

@@ -228,8 +228,9 @@ def test_shap_tree_form_matches_packed_form(hip, orc, depth, n_features, used, n
     (4, 28, 0.0), (5, 28, 0.0), (6, 3, 0.3), (7, 28, 0.2), (8, 28, 0.0), (9, 6, 0.3), (10, 10, 0.1), (11, 28, 0.4),
     (12, 12, 0.35), (12, 3, 0.25)])
 def test_shap_split_trees_equal_whole_walks(hip, depth, used, p_leaf):
-    """Few row blocks x trees give each tree a workgroup whose waves walk its subtrees (from
-    5 levels up); 1,300 rows x 60 trees walk whole trees.  The same bits for every row."""
+    """A handful of rows take a lane a block, few row blocks x trees may give each tree a
+    workgroup whose waves walk its subtrees; 1,300 rows x 60 trees walk whole trees.  The
+    same bits for every row."""
     rng = np.random.default_rng([7, depth, used])
     nb = rng.integers(2, 257, 28).astype(np.uint16)
     trees = random_trees(rng, 57, depth, used, nb, p_leaf, True) + random_trees(rng, 3, 2, used, nb, 0.2)
@@ -348,3 +349,26 @@ def test_predict_shapes_match_the_walk(hip, orc, depth, n_features, n_trees, siz
         rows = (rng.random((n, n_features), np.float32) * nb).astype(np.uint8)
         assert np.array_equal(p.predict(rows).view(np.uint32), orc.predict(trees, rows, nb, 0.1, -0.5).view(np.uint32)), n
     p.close()
+
+
+@pytest.mark.parametrize("depth,used,n_features,n_trees,p_leaf", [
+    (1, 1, 1, 3, 0.0), (3, 5, 5, 70, 0.2), (4, 28, 28, 300, 0.0), (5, 9, 9, 40, 0.5), (6, 28, 28, 130, 0.0),
+    (7, 3, 28, 33, 0.2), (8, 28, 28, 60, 0.0), (8, 200, 200, 20, 0.1), (9, 12, 12, 30, 0.3), (10, 28, 28, 40, 0.0),
+    (10, 40, 256, 9, 0.1), (11, 10, 28, 7, 0.3), (12, 28, 28, 12, 0.2), (12, 28, 28, 1, 0.0)])
+def test_shap_bits_do_not_depend_on_the_batch(hip, depth, used, n_features, n_trees, p_leaf):
+    """Batches of 1 to 700 rows go to lanes, subtrees or whole walks by what they cost, and
+    share their trees over one or several workgroups: every row has the bits it has among
+    1,500 rows, with leaves of one size and with one far above the others (either grid)."""
+    rng = np.random.default_rng([11, depth, used, n_trees])
+    nb = rng.integers(2, 257, n_features).astype(np.uint16)
+    rows = (rng.random((1500, n_features)) * nb).astype(np.uint8)
+    for large in (False, True):
+        trees = random_trees(rng, n_trees, depth, used, nb, p_leaf, True)
+        trees.insert(1, np.array([(-1, 0, 0, 0, 0, 0.5, 10.0, 0.0)], NODE_DTYPE))  # a single leaf
+        if large:
+            trees[0]["value"][np.flatnonzero(trees[0]["feature"] < 0)[0]] = 1e5
+        p = hip.Predictor(trees, nb, 0.3, 0.25)
+        whole = p.shap(rows).view(np.uint64)
+        for a, b in ((0, 1), (5, 7), (9, 16), (0, 33), (64, 128), (100, 165), (0, 130), (200, 450), (0, 700)):
+            assert np.array_equal(p.shap(rows[a:b]).view(np.uint64), whole[a:b]), (a, b)
+        p.close()
