@@ -43,13 +43,13 @@ u32 find_blocks_per_node(u32 F, u32 tile); // workgroups per node for tile-featu
 void launch_plan_level(hipStream_t s, NodeInfo const *front, SplitRec const *splits, TreeCtl *ctl, DevNode *tree,
                        PartOp *ops, PartChunk *pch, u16 const *n_bins, GrowCfg const &cfg, double const *scales,
                        u32 dst, u32 chunk_rows);
-// fuse (wide rows): single-unit nodes name their sibling and parent for the histogram
-// kernel, which then completes both children (launch_hist's hist_cur).
 // Rows per partition chunk for n rows of Fs bytes: kPartChunk, halved down to
 // kPartChunkMin until there are kPartChunkFill chunks; kWideChunk for wide rows.
 u32 part_chunk_rows(u32 Fs, u64 n);
 void launch_part_count(hipStream_t s, PartChunk const *pch, PartOp const *ops, TreeCtl const *ctl, u8 const *pl0,
                        u8 const *pl1, u8 const *plp, u32 Fs, u32 *chunk_left, u32 grid);
+// fuse (wide rows): single-unit nodes name their sibling and parent for the histogram
+// kernel, which then completes both children (launch_hist's hist_cur).
 void launch_part_scan(hipStream_t s, bool q, PartOp *ops, PartChunk *pch, u32 const *chunk_left, TreeCtl *ctl,
                       NodeInfo const *front, NodeInfo *next, SplitRec const *splits, DevNode *tree, HistChunk *hch,
                       FinishOp *fops, GrowCfg const &cfg, double const *scales, u32 is_last, u32 oblivious,

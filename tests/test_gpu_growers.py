@@ -325,9 +325,33 @@ def test_grow_leafwise_chain(hip, orc, leaves, quantized):
 
 
 @pytest.mark.parametrize("quantized", [True, False])
+def test_grow_leafwise_wide_row_chunks(hip, orc, quantized):
+    """Leaves on both sides of the wide rows' cap of 1,024 rows a chunk: the leaf-sized rule
+    reaches it past 262,144 rows."""
+    n, f = 300_000, 66
+    rng = np.random.default_rng(66)
+    bins = rng.integers(0, 32, (n, f), dtype=np.uint8)
+    nb = np.full(f, 33, np.uint16)
+    y = ((bins[:, 3] > 4) * 2.0 + bins[:, 7] / 16.0 + rng.normal(0, 0.3, n)).astype(np.float32)
+    g, h = orc.mse_grad(np.zeros(n, np.float32), y)
+    ctx = ctx_for(hip, bins, nb, grower="hip_leafwise", quantized=quantized, max_depth=6, max_leaves=12)
+    c = orc_cfg(max_depth=6, max_leaves=12)
+    if quantized:
+        gq, hq, sc = ctx.set_gradients(g, h)
+        ref, rlor = orc.grow_leafwise(bins, nb, gq=gq, hq=hq, scales=sc, c=c, mode=HIST_INT)
+    else:
+        ctx.set_gradients(g, h)
+        ref, rlor = orc.grow_leafwise(bins, nb, g=g, h=h, c=c, mode=HIST_F32_FIXED, chunk=LW_F32_CHUNK)
+    nodes, lor = ctx.grow_tree()
+    ctx.close()
+    assert_same_tree(nodes, ref)
+    assert np.array_equal(lor, rlor)
+
+
+@pytest.mark.parametrize("quantized", [True, False])
 def test_grow_leafwise_wide_rows(hip, orc, quantized):
-    """1,500-byte rows: partition chunks are capped at 128 rows by bytes, below the
-    leaf-sized rule's 256-row minimum."""
+    """1,500-byte rows: partitions order row ids, in chunks of the leaf-sized rule's 256-row
+    minimum at this many rows."""
     bins, nb, X, y = wide_data(n=4000, f=1500)
     rng = np.random.default_rng(6)
     g, h = orc.mse_grad(rng.normal(0, 1, y.size).astype(np.float32), y)

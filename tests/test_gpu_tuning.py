@@ -84,7 +84,7 @@ def test_launch_shapes_do_not_change_results(hip, orc, tall, quantized):
 @pytest.fixture(scope="module")
 def wide():
     """70 features (rows of more than 64 bytes), several 32,768-row histogram units."""
-    n, f = 70_001, 70
+    n, f = 40_001, 70
     rng = np.random.default_rng(11)
     nb = np.full(f, 256, np.uint16)
     nb[::7] = 18
